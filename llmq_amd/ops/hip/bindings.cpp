@@ -217,6 +217,47 @@ void rope_and_cache(at::Tensor q, at::Tensor k, at::Tensor value,
 
 // ------------------------------------------------------------ attention --
 
+// The matrix-core kernel of paged_decode.hip. Waves: as many as are resident at
+// the variant's register use, so that every range is in work at once.
+template <int D, typename TC, int NK, int OCC>
+void launch_paged_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor& kc,
+                         const at::Tensor& vc, const at::Tensor& bt,
+                         const at::Tensor& cl, double scale, double softcap,
+                         long window) {
+  using Shape = PdShape<D, TC, NK>;
+  constexpr double kLog2e = 1.4426950408889634;
+  const int B = q.size(0), KVH = kc.size(1), G = q.size(1) / KVH;
+  const int bs_shift = kc.size(2) == 32 ? 5 : 4;
+  int cus = 0;
+  TORCH_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
+                                    q.get_device()) == hipSuccess);
+  const long most = (long)B * KVH * ((bt.size(1) << bs_shift) / Shape::kKeys + 1);
+  const int wgs = (int)std::min<long>((long)cus * OCC, (most + 3) / 4);
+  const int waves = wgs * 4;
+  auto opts = q.options().dtype(at::kFloat);
+  at::Tensor part_o = at::empty({2L * waves, G, D}, opts);
+  at::Tensor part_ml = at::empty({2L * waves, G, 2}, opts);
+  auto go = [&]<bool CAP>() {
+    hipLaunchKernelGGL((paged_decode_kernel<D, TC, NK, OCC, CAP>), dim3(wgs), dim3(256),
+                       Shape::kLds, stream(),
+                       reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), out.stride(0),
+                       reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()), q.stride(0),
+                       reinterpret_cast<const TC*>(kc.data_ptr()),
+                       reinterpret_cast<const TC*>(vc.data_ptr()), bt.data_ptr<int>(),
+                       (int)bt.stride(0), cl.data_ptr<int>(), B, KVH, G, bs_shift, (int)window,
+                       (float)(scale * kLog2e), (float)(softcap * kLog2e),
+                       softcap > 0 ? (float)(2 * scale / softcap * kLog2e) : 0.f,
+                       part_o.data_ptr<float>(), part_ml.data_ptr<float>());
+  };
+  if (softcap > 0) go.template operator()<true>();
+  else go.template operator()<false>();
+  hipLaunchKernelGGL((paged_decode_merge_kernel<D, Shape::kTileShift>), dim3(B, q.size(1)),
+                     dim3(256), 0, stream(),
+                     reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), out.stride(0),
+                     part_o.data_ptr<float>(), part_ml.data_ptr<float>(), cl.data_ptr<int>(), B,
+                     KVH, G, (int)window, waves);
+}
+
 template <typename T>
 void launch_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor& kc,
                    const at::Tensor& vc, const at::Tensor& bt,
@@ -225,160 +266,41 @@ void launch_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor& kc,
   const int B = q.size(0), H = q.size(1), D = q.size(2);
   const int KVH = kc.size(1);
   const int bs = kc.size(2);
-  const int max_blocks = bt.size(1);
   const int G = H / KVH;
   TORCH_CHECK(H % KVH == 0, "num_heads must divide num_kv_heads");
   TORCH_CHECK(bs == 16 || bs == 32, "block_size must be 16 or 32");
-  dim3 grid(B, KVH);
-  // bf16 + MFMA-supported head dims → matrix-core kernel (G padded to 16).
-  // NW = waves per workgroup (keys-per-chunk = 16·NW); 8 halves the
-  // barriers per token vs 4 at the same waves/SIMD (A/B-able via
-  // LLMQ_DECODE_NW).
-  if constexpr (std::is_same_v<T, __hip_bfloat16>) {
-    if ((D == 128 || D == 256) && G <= 16) {
-      static const int nw_env = [] {
-        const char* e = getenv("LLMQ_DECODE_NW");
-        return e ? atoi(e) : 8;
-      }();
-      // Split-KV: when B×KVH under-fills the chip (TP ranks hold few kv
-      // heads; small batches), split the context across z-workgroups and
-      // merge fp32 partials. Target ≥512 workgroups (2 resident per CU).
-      int nsplit = 1;
-      while (B * KVH * nsplit < 512 && nsplit < 16) nsplit *= 2;
-      at::Tensor scratch;
-      float* scratch_ptr = nullptr;
-      if (nsplit > 1) {
-        scratch = at::empty({(long)B, KVH, nsplit, G, D + 2},
-                            q.options().dtype(at::kFloat));
-        scratch_ptr = scratch.data_ptr<float>();
-      }
-      dim3 sgrid(B, KVH, nsplit);
-      const bool fp8_cache = kc.scalar_type() == at::kFloat8_e4m3fn;
-      // Software-pipelined glds kernel (default): LLMQ_DECODE_PIPE selects
-      // the chunk size (64 | 128 keys) or 0 = the plain-staged kernel.
-      // Read per call so microbenches can A/B in-process. Preconditions:
-      // bf16 cache (glds cannot convert fp8 during the LDS write) and the
-      // whole block table staged in LDS (no per-granule LDS-vs-global
-      // select — guide §5 trap 4c).
-      const char* pe = getenv("LLMQ_DECODE_PIPE");
-      const int pipe_kt = pe ? atoi(pe) : 64;
-      if (fp8_cache && pipe_kt > 0 && max_blocks <= PD_MAX_BT) {
-        // fp8 glds pipeline: raw-fp8 staging + native packed cvt VOPs
-        auto lf8 = [&]<int HD>() {
-          hipLaunchKernelGGL((paged_decode_pipe_fp8_kernel<HD, 8>), sgrid,
-                             dim3(8 * 64), 0, stream(),
-                             reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-                             reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
-                             reinterpret_cast<const __hip_fp8_e4m3*>(kc.data_ptr()),
-                             reinterpret_cast<const __hip_fp8_e4m3*>(vc.data_ptr()),
-                             bt.data_ptr<int>(), cl.data_ptr<int>(), scratch_ptr,
-                             H, KVH, bs, max_blocks, (float)scale,
-                             (float)softcap, (int)window, q.stride(0),
-                             out.stride(0));
-          if (nsplit > 1) {
-            hipLaunchKernelGGL((decode_splitkv_merge_kernel<HD>),
-                               dim3(B, KVH, G), dim3(64), 0, stream(),
-                               reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-                               scratch_ptr, KVH, G, nsplit, out.stride(0));
-          }
-        };
-        if (D == 128) lf8.template operator()<128>();
-        else lf8.template operator()<256>();
-        return;
-      }
-      if (!fp8_cache && pipe_kt > 0 && max_blocks <= PD_MAX_BT) {
-        auto lp = [&]<int HD, int KT>() {
-          hipLaunchKernelGGL((paged_decode_pipe_kernel<HD, 8, KT>), sgrid,
-                             dim3(8 * 64), 0, stream(),
-                             reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-                             reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
-                             reinterpret_cast<const __hip_bfloat16*>(kc.data_ptr()),
-                             reinterpret_cast<const __hip_bfloat16*>(vc.data_ptr()),
-                             bt.data_ptr<int>(), cl.data_ptr<int>(), scratch_ptr,
-                             H, KVH, bs, max_blocks, (float)scale,
-                             (float)softcap, (int)window, q.stride(0),
-                             out.stride(0));
-          if (nsplit > 1) {
-            hipLaunchKernelGGL((decode_splitkv_merge_kernel<HD>),
-                               dim3(B, KVH, G), dim3(64), 0, stream(),
-                               reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-                               scratch_ptr, KVH, G, nsplit, out.stride(0));
-          }
-        };
-        if (pipe_kt == 32) {  // ring variant: separate K/V slots, 32-key
-          auto lr = [&]<int HD>() {
-            hipLaunchKernelGGL((paged_decode_ring_kernel<HD, 8>), sgrid,
-                               dim3(8 * 64), 0, stream(),
-                               reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-                               reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
-                               reinterpret_cast<const __hip_bfloat16*>(kc.data_ptr()),
-                               reinterpret_cast<const __hip_bfloat16*>(vc.data_ptr()),
-                               bt.data_ptr<int>(), cl.data_ptr<int>(), scratch_ptr,
-                               H, KVH, bs, max_blocks, (float)scale,
-                               (float)softcap, (int)window, q.stride(0),
-                               out.stride(0));
-            if (nsplit > 1) {
-              hipLaunchKernelGGL((decode_splitkv_merge_kernel<HD>),
-                                 dim3(B, KVH, G), dim3(64), 0, stream(),
-                                 reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-                                 scratch_ptr, KVH, G, nsplit, out.stride(0));
-            }
-          };
-          if (D == 128) lr.template operator()<128>();
-          else lr.template operator()<256>();
-          return;
-        }
-        if (D == 128) {
-          if (pipe_kt >= 128) lp.template operator()<128, 128>();
-          else lp.template operator()<128, 64>();
-        } else {
-          if (pipe_kt >= 128) lp.template operator()<256, 128>();
-          else lp.template operator()<256, 64>();
-        }
-        return;
-      }
-      auto lm = [&]<int HD, int NW, typename TC>() {
-        hipLaunchKernelGGL((paged_decode_mfma_kernel<HD, NW, TC>), sgrid,
-                           dim3(NW * 64), 0, stream(),
-                           reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-                           reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
-                           reinterpret_cast<const TC*>(kc.data_ptr()),
-                           reinterpret_cast<const TC*>(vc.data_ptr()),
-                           bt.data_ptr<int>(), cl.data_ptr<int>(), scratch_ptr,
-                           H, KVH, bs, max_blocks, (float)scale,
-                           (float)softcap, (int)window, q.stride(0),
-                           out.stride(0));
-        if (nsplit > 1) {
-          hipLaunchKernelGGL((decode_splitkv_merge_kernel<HD>),
-                             dim3(B, KVH, G), dim3(64), 0, stream(),
-                             reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-                             scratch_ptr, KVH, G, nsplit, out.stride(0));
-        }
-      };
-      using BF = __hip_bfloat16;
-      using F8 = __hip_fp8_e4m3;
-      if (fp8_cache) {  // fp8 KV rides the default NW=8 configuration
-        if (D == 128) lm.template operator()<128, 8, F8>();
-        else lm.template operator()<256, 8, F8>();
-      } else if (D == 128) {
-        // NW=16 needs D/NW >= 16 (a full MFMA dim tile per wave)
-        if (nw_env == 2) lm.template operator()<128, 2, BF>();
-        else if (nw_env == 4) lm.template operator()<128, 4, BF>();
-        else lm.template operator()<128, 8, BF>();
-      } else {
-        if (nw_env == 2) lm.template operator()<256, 2, BF>();
-        else if (nw_env == 4) lm.template operator()<256, 4, BF>();
-        else if (nw_env == 16) lm.template operator()<256, 16, BF>();
-        else lm.template operator()<256, 8, BF>();
-      }
-      return;
-    }
-  }
-  // The VALU fallback reads the cache as T; an fp8 cache reaching it would
-  // be silently reinterpreted as bf16 (garbage, no error).
-  TORCH_CHECK(kc.scalar_type() != at::kFloat8_e4m3fn,
+  if (B == 0) return;
+  const bool fp8 = kc.scalar_type() == at::kFloat8_e4m3fn;
+  TORCH_CHECK(!fp8 || (std::is_same_v<T, __hip_bfloat16> && (D == 128 || D == 256) && G <= 16),
               "fp8 KV cache requires the MFMA decode path (bf16 q, head_dim "
               "128/256, GQA group <= 16); got head_dim=", D, " group=", G);
+  TORCH_CHECK(D == 64 || D == 128 || D == 256, "unsupported head_dim ", D);
+  if constexpr (std::is_same_v<T, __hip_bfloat16>) {
+    TORCH_CHECK(G <= (D == 64 ? 8 : 16), "GQA group must be <= 8 at head_dim 64, else <= 16");
+    // 16-byte query loads and 8-byte stores: rows that start elsewhere go
+    // through a copy
+    auto aligned = [](const at::Tensor& t, long bytes) {
+      return reinterpret_cast<uintptr_t>(t.data_ptr()) % bytes == 0 &&
+             t.stride(0) * (long)t.element_size() % bytes == 0;
+    };
+    const at::Tensor qa = aligned(q, 16) ? q : q.clone(at::MemoryFormat::Contiguous);
+    const at::Tensor bta = bt.stride(1) == 1 ? bt : bt.contiguous();
+    at::Tensor oa = aligned(out, 8) ? out : out.clone(at::MemoryFormat::Contiguous);
+    auto go = [&]<int HD, typename TC, int NK, int OCC>() {
+      launch_paged_decode<HD, TC, NK, OCC>(oa, qa, kc, vc, bta, cl, scale, softcap, window);
+    };
+    using BF = __hip_bfloat16;
+    using F8 = __hip_fp8_e4m3;
+    if (D == 64) go.template operator()<64, BF, 4, 3>();
+    else if (D == 128 && !fp8) go.template operator()<128, BF, 2, 2>();
+    else if (D == 256 && !fp8) go.template operator()<256, BF, 1, 1>();
+    else if (D == 128) go.template operator()<128, F8, 2, 3>();
+    else go.template operator()<256, F8, 1, 2>();
+    if (!oa.is_same(out)) out.copy_(oa);
+    return;
+  } else {
+  const int max_blocks = bt.size(1);
+  dim3 grid(B, KVH);
   TORCH_CHECK(G <= 8, "GQA group must be <= 8 for the VALU decode kernel");
   const int subs = 256 / (32 * G);
   const int lds = (G * D + DECODE_CHUNK * G + subs * G * (D + 2)) * sizeof(float) +
@@ -397,7 +319,7 @@ void launch_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor& kc,
     case 64: l.template operator()<64>(); break;
     case 128: l.template operator()<128>(); break;
     case 256: l.template operator()<256>(); break;
-    default: TORCH_CHECK(false, "unsupported head_dim ", D);
+  }
   }
 }
 

@@ -3,6 +3,7 @@
 #include "elementwise.hip"
 #include "kvcache.hip"
 #include "attention.hip"
+#include "paged_decode.hip"
 #include "skinny_gemm.hip"
 #include "sampling.hip"
 #include "bindings.cpp"

@@ -211,6 +211,40 @@ class TestDecodeAttention:
         assert_close_to_f32_ref(out.cpu(), ref, 2e-2, 1e-1)
 
 
+class TestDecodeRanges:
+    """The matrix-core decode kernel deals the batch's key tiles to waves in
+    equal ranges: ranges that open, close and cross (sequence, kv head) pairs,
+    empty rows, batches over one wave's scan, block tables of any width."""
+
+    @pytest.mark.parametrize("D,G,KVH,fp8", [
+        (64, 4, 3, False), (64, 8, 1, False), (128, 1, 2, False), (128, 16, 1, False),
+        (256, 2, 2, False), (128, 6, 2, True), (256, 16, 1, True),
+    ])
+    @pytest.mark.parametrize("BS,window,softcap", [(16, 0, 0.0), (32, 50, 0.0), (16, 70, 30.0)])
+    @pytest.mark.parametrize("lens", [
+        [1], [16, 17, 0, 33], [4000, 1, 63, 64, 65, 129], [(i * 37) % 150 for i in range(131)],
+    ])
+    def test_vs_ref(self, D, G, KVH, fp8, BS, window, softcap, lens):
+        B, H = len(lens), G * KVH
+        kc, vc, bt = _build_cache(B, KVH, D, BS, max(lens), torch.bfloat16)
+        bt = torch.nn.functional.pad(bt, (0, 1200))
+        if fp8:
+            kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+        ctx = torch.tensor(lens, dtype=torch.int32, device=DEV)
+        # a query view inside a wider row, as the packed projection gives it
+        q = torch.randn(B, H * D + 64, device=DEV, dtype=torch.bfloat16)[:, :H * D].view(B, H, D)
+        scale = D ** -0.5
+        out = ops.paged_decode_attention(q, kc, vc, bt, ctx, scale, softcap, window)
+        live = torch.tensor([n > 0 for n in lens])
+        ref = torch_ref.paged_decode_attention(
+            q.float().cpu()[live], kc.float().cpu(), vc.float().cpu(), bt.cpu()[live],
+            ctx.cpu()[live], scale, softcap, window,
+        )
+        # the output's bf16 rounding (2^-9 of the value, twice that allowed) and
+        # fp32 sums over up to 4000 keys of unit values
+        assert_close_to_f32_ref(out.cpu()[live], ref, 2e-4, 2 ** -8)
+
+
 class TestPrefillAttention:
     @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
     @pytest.mark.parametrize("H,KVH,D", [(8, 2, 128), (16, 8, 256), (4, 4, 64)])
