@@ -337,6 +337,28 @@ void paged_decode_attention(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   });
 }
 
+template <int D, int HP, int WR, int KT, int MINW>
+void launch_flash_prefill(at::Tensor& out, const at::Tensor& q, const at::Tensor& k,
+                          const at::Tensor& v, const at::Tensor& cu, const at::Tensor& cu_k,
+                          int B, double scale, double softcap, long window, long max_seqlen) {
+  constexpr double kLog2e = 1.4426950408889634;
+  const int H = q.size(1), KVH = k.size(1);
+  const int n_qt = (int)((std::max<long>(max_seqlen, 1) + 32 * WR - 1) / (32 * WR));
+  auto go = [&]<bool CAP>() {
+    hipLaunchKernelGGL((flash_prefill_kernel<D, HP, WR, KT, MINW, CAP>),
+                       dim3((unsigned)(n_qt * (H / HP) * B)), dim3(64 * HP * WR), 0, stream(),
+                       reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), out.stride(0),
+                       reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()), q.stride(0),
+                       reinterpret_cast<const __hip_bfloat16*>(k.data_ptr()), k.stride(0),
+                       reinterpret_cast<const __hip_bfloat16*>(v.data_ptr()), v.stride(0),
+                       cu.data_ptr<int>(), cu_k.data_ptr<int>(), B, H, KVH, (int)window,
+                       (float)(scale * kLog2e), (float)(softcap * kLog2e),
+                       softcap > 0 ? (float)(2 * scale / softcap * kLog2e) : 0.f, n_qt);
+  };
+  if (softcap > 0) go.template operator()<true>();
+  else go.template operator()<false>();
+}
+
 template <typename T>
 void launch_prefill(at::Tensor& out, const at::Tensor& q, const at::Tensor& k,
                     const at::Tensor& v, const at::Tensor& cu,
@@ -344,44 +366,36 @@ void launch_prefill(at::Tensor& out, const at::Tensor& q, const at::Tensor& k,
                     double scale, double softcap, long window, long max_seqlen) {
   const int H = q.size(1), D = q.size(2);
   const int KVH = k.size(1);
+  if (B == 0) return;
+  TORCH_CHECK(D == 64 || D == 128 || D == 256, "unsupported head_dim ", D);
   if constexpr (std::is_same_v<T, __hip_bfloat16>) {
-    // MFMA flash path (bf16): grid (seq, head, q-tile). Default: the glds
-    // software-pipelined kernel; LLMQ_PREFILL_PIPE=0 selects the plain-
-    // staged one (A/B). Read per call for in-process microbenches.
-    const int qtiles = (int)((max_seqlen + 63) / 64);
-    dim3 fgrid(B, H, std::max(qtiles, 1));
-    const char* ppe = getenv("LLMQ_PREFILL_PIPE");
-    const bool use_pipe = !ppe || atoi(ppe) != 0;
-    auto lf = [&]<int HD>() {
-      if (use_pipe) {
-        hipLaunchKernelGGL((flash_prefill_pipe_kernel<HD>), fgrid, dim3(256), 0,
-                           stream(),
-                           reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-                           reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
-                           reinterpret_cast<const __hip_bfloat16*>(k.data_ptr()),
-                           reinterpret_cast<const __hip_bfloat16*>(v.data_ptr()),
-                           cu.data_ptr<int>(), cu_k.data_ptr<int>(), H, KVH,
-                           (float)scale, (float)softcap, (int)window,
-                           q.stride(0), k.stride(0), v.stride(0), out.stride(0));
-        return;
-      }
-      hipLaunchKernelGGL((flash_prefill_bf16_kernel<HD>), fgrid, dim3(256), 0,
-                         stream(),
-                         reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-                         reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
-                         reinterpret_cast<const __hip_bfloat16*>(k.data_ptr()),
-                         reinterpret_cast<const __hip_bfloat16*>(v.data_ptr()),
-                         cu.data_ptr<int>(), cu_k.data_ptr<int>(), H, KVH,
-                         (float)scale, (float)softcap, (int)window,
-                         q.stride(0), k.stride(0), v.stride(0), out.stride(0));
+    // 16-byte loads and 8-byte stores: rows that start elsewhere go through a copy
+    auto aligned = [](const at::Tensor& t, long bytes) {
+      return reinterpret_cast<uintptr_t>(t.data_ptr()) % bytes == 0 &&
+             t.stride(0) * (long)t.element_size() % bytes == 0;
     };
-    switch (D) {
-      case 64: lf.template operator()<64>(); return;
-      case 128: lf.template operator()<128>(); return;
-      case 256: lf.template operator()<256>(); return;
-      default: TORCH_CHECK(false, "unsupported head_dim ", D);
-    }
-  }
+    auto rows16 = [&](const at::Tensor& t) {
+      return aligned(t, 16) ? t : t.clone(at::MemoryFormat::Contiguous);
+    };
+    const at::Tensor qa = rows16(q), ka = rows16(k), va = rows16(v);
+    at::Tensor oa = aligned(out, 8) ? out : out.clone(at::MemoryFormat::Contiguous);
+    auto go = [&]<int HD, int HP, int WR, int KT, int MINW>() {
+      launch_flash_prefill<HD, HP, WR, KT, MINW>(oa, qa, ka, va, cu, cu_k, B, scale, softcap,
+                                                 window, max_seqlen);
+    };
+    // Two heads of a kv head on one stream of tiles where the group is even
+    // (2 x 64 rows at head size 64, 2 x 128 at 256: 138 against 147 us for
+    // 8 x 1024 tokens). Tiles of 32 keys where that buys a third wave per SIMD
+    // (head size 128: 160 against 187 us for 16 x 1024) or the registers (256).
+    const bool even = (H / KVH) % 2 == 0;
+    if (D == 64 && even) go.template operator()<64, 2, 2, 64, 3>();
+    else if (D == 64) go.template operator()<64, 1, 4, 64, 3>();
+    else if (D == 128) go.template operator()<128, 1, 4, 32, 3>();
+    else if (even) go.template operator()<256, 2, 4, 32, 1>();
+    else go.template operator()<256, 1, 8, 32, 1>();
+    if (!oa.is_same(out)) out.copy_(oa);
+    return;
+  } else {
   dim3 grid(B, H);
   auto l = [&]<int HD>() {
     hipLaunchKernelGGL((varlen_prefill_attention_kernel<T, HD>), grid,
@@ -398,7 +412,7 @@ void launch_prefill(at::Tensor& out, const at::Tensor& q, const at::Tensor& k,
     case 64: l.template operator()<64>(); break;
     case 128: l.template operator()<128>(); break;
     case 256: l.template operator()<256>(); break;
-    default: TORCH_CHECK(false, "unsupported head_dim ", D);
+  }
   }
 }
 

@@ -1,0 +1,296 @@
+// Causal attention of packed bf16 prompt portions on the matrix cores (gfx950),
+// head size 64, 128 or 256, grouped query heads, optional score cap and sliding
+// window; a portion may continue cached context (more keys than queries).
+//
+// Bound by the matrix cores and by the softmax beside them: at head size 128 the
+// products take 40% of the SIMD cycles and the vector work 50%, at the 1.9 GHz that
+// the clock falls to. Measured (us; before = 64-row workgroups whose softmax went
+// through lane exchanges and whose weights went through LDS): 8192 tokens, 24 heads
+// of 128: 1717 -> 510 (807 TFLOP/s); 16 x 1024, 32 heads of 64: 322 -> 123;
+// 8 x 1024, 16 heads of 256, capped: 273 -> 131; 7000, the same: 1483 -> 546;
+// 40 ragged up to 170, 12 heads of 128: 34 -> 18.
+//
+//
+//   - Both products run TRANSPOSED on v_mfma_f32_32x32x16_bf16, S^T = K Q^T and
+//     O^T = V^T P^T (A: row = lane%32, k = 8*(lane/32)..+7; B: column = lane%32;
+//     C: column = lane%32, rows 8*(r/4) + 4*(lane/32) + r%4): a lane owns one
+//     query, its softmax state never leaves it, and its weights are already the
+//     second product's operand (slot 8h+4b+i of 16 keys = key 8b+4h+i).
+//   - K and V tiles go from memory to LDS without passing registers
+//     (global_load_lds), row-major in 16-byte granules whose order within a row
+//     depends on the key: K operands are 16-byte reads, V operands transposing
+//     reads (ds_read_b64_tr_b16), both without bank conflicts. Two buffers, one
+//     barrier per tile: the next tile travels during the current one's products.
+//   - A workgroup takes HP query heads of one kv head times WR blocks of 32 rows,
+//     a wave each, on one stream of K/V tiles.
+//   - Workgroups that share keys land on the same XCD (the dispatcher deals
+//     consecutive ids out in turn), latest = longest query tiles first.
+
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(4))) short fp_s16x4;
+typedef __attribute__((ext_vector_type(8))) short fp_s16x8;
+typedef __attribute__((ext_vector_type(2))) unsigned fp_u32x2;
+typedef __attribute__((ext_vector_type(4))) unsigned fp_u32x4;
+typedef __attribute__((ext_vector_type(16))) float fp_f32x16;
+typedef __attribute__((ext_vector_type(2))) float fp_f32x2;
+typedef __attribute__((ext_vector_type(2))) __bf16 fp_bf16x2;
+typedef __attribute__((ext_vector_type(4))) __bf16 fp_bf16x4;
+typedef __attribute__((address_space(3))) fp_bf16x4 fp_lds_bf16x4;
+
+// 16 bytes per lane from memory to LDS (lane-linear from a uniform LDS address, in
+// M0), in inline asm: with the builtin the compiler waits for all of them before
+// the first LDS read that may alias, which would drain the next tile's loads.
+// pipe_barrier_vm is the only wait for them.
+DEVINL void glds16(const void* src, void* lds_dst_uniform) {
+  unsigned lds_off = (unsigned)(unsigned long)(
+      (__attribute__((address_space(3))) char*)lds_dst_uniform);
+  lds_off = __builtin_amdgcn_readfirstlane(lds_off);
+  unsigned keep;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(keep)
+      : "v"(src), "s"(lds_off)
+      : "memory");
+}
+
+// The wave's loads have landed but the last N, everyone's LDS reads are done.
+template <int N>
+DEVINL void pipe_barrier_vm() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "i"(N) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// glds16 with a uniform base and a 32-bit byte offset per lane.
+DEVINL void glds16_at(const void* base, unsigned off, void* lds_dst_uniform) {
+  unsigned lds_off = (unsigned)(unsigned long)(
+      (__attribute__((address_space(3))) char*)lds_dst_uniform);
+  lds_off = __builtin_amdgcn_readfirstlane(lds_off);
+  unsigned keep;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %3\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(keep)
+      : "v"(off), "s"(base), "s"(lds_off)
+      : "memory");
+}
+
+// Place of granule g of key row `key`: 16 consecutive keys' equal granules in 16
+// different 16-byte bank groups (K) ...
+template <int D>
+DEVINL int fp_kswz(int key) { return D >= 128 ? key & 15 : (key >> 1) & 7; }
+// ... and 8 consecutive keys' 32-byte groups in 8 different ones (V).
+template <int D>
+DEVINL int fp_vswz(int key) { return D >= 128 ? (key & 7) << 1 : ((key >> 1) & 3) << 1; }
+
+template <int D, int HP, int WR, int KT, int MINW, bool CAP>
+__global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
+    __hip_bfloat16* __restrict__ out, long o_stride,
+    const __hip_bfloat16* __restrict__ q, long q_stride,
+    const __hip_bfloat16* __restrict__ k, long k_stride,
+    const __hip_bfloat16* __restrict__ v, long v_stride,
+    const int* __restrict__ cu_q, const int* __restrict__ cu_k, int B, int H, int KVH,
+    int window, float scale_log2, float cap_log2, float cap_in, int n_qt) {
+  constexpr int NW = HP * WR, QT = 32 * WR, NT = KT / 32;
+  constexpr int KS = D / 16, DT = D / 32, GPR = D / 8;
+  constexpr int NI = KT * GPR / 64;                    // 1 KiB loads of a tile's K (and V)
+  __shared__ __align__(16) short lds[4 * KT * D];      // [buffer][K | V][KT][D]
+
+  const int hg = H / HP;                               // head groups
+  const int nb = hg * B;
+  const int id = blockIdx.x % nb;
+  const int pair = nb % 8 == 0 ? (id % 8) * (nb / 8) + id / 8 : id;
+  const int b = pair / hg, h0 = (pair % hg) * HP;
+  const int r0 = (n_qt - 1 - (int)(blockIdx.x / nb)) * QT;
+  const int row0 = cu_q[b];
+  const int nq = cu_q[b + 1] - row0;
+  if (r0 >= nq) return;
+  const int k0 = cu_k[b];
+  const int nk = cu_k[b + 1] - k0;
+  const int rows = min(QT, nq - r0);
+  const int pos0 = nk - nq + r0;                       // position of the tile's first row
+  const int pos_last = pos0 + rows - 1;
+  const int kvh = h0 / (H / KVH);
+
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = h0 + w % HP, wr = w / HP;
+  const int col = lane & 31, half = lane >> 5;
+
+  const int qrow = wr * 32 + col;
+  const int ipos = qrow < rows ? pos0 + qrow : -1;     // -1: sees nothing
+  const int lpos = window > 0 ? max(0, ipos - window + 1) : 0;
+  fp_s16x8 qf[KS];
+  {
+    const __hip_bfloat16* qr =
+        q + (long)(row0 + r0 + min(qrow, rows - 1)) * q_stride + (long)h * D + half * 8;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      qf[ks] = *reinterpret_cast<const fp_s16x8*>(qr + ks * 16);
+      asm volatile("" : "+v"(qf[ks]));                 // landed before the first tile's loads
+    }
+  }
+  const int wave_first = pos0 + wr * 32;
+  const int wave_last = min(pos_last, wave_first + 31);
+  const int wave_lo = window > 0 ? max(0, wave_first - window + 1) : 0;  // first key any row sees
+  const int wave_all = window > 0 ? max(0, wave_last - window + 1) : 0;  // first key all rows see
+  const bool idle = wr * 32 >= rows;
+
+  // Staging: load i = w + j NW of a tile (K rows, then V rows) is 1 KiB = KPL key
+  // rows. A wave's loads lie a multiple of 16 keys apart, so its lanes' place in a
+  // row and their offset from the load's first row are the same for all of them.
+  constexpr int KPL = 64 / GPR, STEP = NW * KPL;
+  static_assert(NI % NW == 0 && STEP % 16 == 0, "a wave's loads share their swizzle");
+  const int skey = w * KPL + lane / GPR;
+  const int kgran = ((lane % GPR) ^ fp_kswz<D>(skey)) << 3;
+  const int vgran = ((lane % GPR) ^ fp_vswz<D>(skey)) << 3;
+  const unsigned koff = ((unsigned)skey * (unsigned)k_stride + kgran) * 2;
+  const unsigned voff = ((unsigned)skey * (unsigned)v_stride + vgran) * 2;
+  const __hip_bfloat16* kb = k + (long)k0 * k_stride + (long)kvh * D;
+  const __hip_bfloat16* vb = v + (long)k0 * v_stride + (long)kvh * D;
+  auto fetch = [&](int kt, bool is_v, short* dst) {
+    const bool whole = kt + KT <= nk;
+    const long stride = is_v ? v_stride : k_stride;
+#pragma unroll
+    for (int j = 0; j < NI / NW; ++j) {
+      const int first = kt + j * STEP;                 // row of this wave's key 0
+      const __hip_bfloat16* base = (is_v ? vb : kb) + (long)first * stride;
+      short* const to = dst + (w + j * NW) * 512;
+      if (whole) {
+        glds16_at(base, is_v ? voff : koff, to);
+      } else {                                         // rows past the end: masked below
+        const int row = min(first + skey, nk - 1) - first;
+        glds16(base + (long)row * stride + (is_v ? vgran : kgran), to);
+      }
+    }
+  };
+
+  // this lane's part of the operand reads
+  const int kbase = col * D, ksw = fp_kswz<D>(col);
+  const int vkey = half * 4 + ((lane & 15) >> 2);
+  const int vbase = vkey * D + (lane & 1) * 4;
+  const int vg = ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1);
+
+  float m = -INFINITY, l = 0.f;                        // log2 domain
+  fp_f32x16 o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
+
+  const int kt0 = window > 0 ? max(0, pos0 - window + 1) / KT * KT : 0;
+  if (kt0 <= pos_last) {
+    fetch(kt0, false, lds);
+    fetch(kt0, true, lds + KT * D);
+  }
+  int cur = 0;
+  for (int kt = kt0; kt <= pos_last; kt += KT, cur ^= 1) {
+    short* const Kt = lds + cur * (2 * KT * D);
+    short* const Vt = Kt + KT * D;
+    pipe_barrier_vm<0>();                              // tile landed, the other buffer is read
+    if (kt + KT <= pos_last) {
+      short* const next = lds + (cur ^ 1) * (2 * KT * D);
+      fetch(kt + KT, false, next);
+      fetch(kt + KT, true, next + KT * D);
+    }
+    if (idle || kt > wave_last || kt + KT - 1 < wave_lo) continue;
+
+    // the products first: at head size 256 the other wave's softmax would hold
+    // them up (547 against 580 us for 7000 tokens, 16 heads)
+    __builtin_amdgcn_s_setprio(1);
+    fp_f32x16 s[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[t][r] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const fp_s16x8 kf = *reinterpret_cast<const fp_s16x8*>(
+            Kt + t * 32 * D + kbase + (((ks * 2 + half) ^ ksw) << 3));
+        s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], s[t], 0, 0, 0);
+      }
+    __builtin_amdgcn_s_setprio(0);
+    if constexpr (CAP) {   // cap tanh(x / cap) = cap - 2 cap / (e^(2 x / cap) + 1), log2 domain
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          s[t][r] = fmaf(-2.f * cap_log2, __builtin_amdgcn_rcpf(
+              __builtin_amdgcn_exp2f(s[t][r] * cap_in) + 1.f), cap_log2);
+    }
+    if (kt + KT - 1 > wave_first || kt < wave_all) {
+      asm volatile("");                                // a branch, not selects on every tile
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int key = kt + t * 32 + (r >> 2) * 8 + half * 4 + (r & 3);
+          s[t][r] = key <= ipos && key >= lpos ? s[t][r] : -INFINITY;
+        }
+    }
+    float tmax = s[0][0];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[t][r]);
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
+    const float sc = CAP ? 1.f : scale_log2;           // > 0
+    const float m_new = fmaxf(m, tmax * sc);
+    const float mb = m_new > -INFINITY ? m_new : 0.f;
+    if (__any(m_new > m)) {
+      const float alpha = __builtin_amdgcn_exp2f(m - mb);    // m = -inf -> 0
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
+      m = m_new;
+    }
+#pragma unroll
+    for (int j = 0; j < KT / 16; ++j) {                // 16 keys per step
+      const int t = j >> 1, u = (j & 1) * 8;
+      fp_u32x4 pw;
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(s[t][u + e], sc, -mb));
+        const float p1 = __builtin_amdgcn_exp2f(fmaf(s[t][u + e + 1], sc, -mb));
+        l += p0 + p1;
+        pw[e / 2] = __builtin_bit_cast(
+            unsigned, __builtin_convertvector((fp_f32x2{p0, p1}), fp_bf16x2));
+      }
+      const fp_s16x8 pf = __builtin_bit_cast(fp_s16x8, pw);
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const short* at = Vt + j * 16 * D + vbase + (((dt * 4 + vg) ^ fp_vswz<D>(vkey)) << 3);
+        const fp_s16x4 v0 = __builtin_bit_cast(fp_s16x4,
+            __builtin_amdgcn_ds_read_tr16_b64_v4bf16((fp_lds_bf16x4*)at));
+        const fp_s16x4 v1 = __builtin_bit_cast(fp_s16x4,
+            __builtin_amdgcn_ds_read_tr16_b64_v4bf16((fp_lds_bf16x4*)(at + 8 * D)));
+        const fp_s16x8 vf = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf, o[dt], 0, 0, 0);
+      }
+    }
+  }
+  l += __shfl_xor(l, 32, WAVE);
+  if (qrow >= rows) return;
+  const float f = l > 0.f ? 1.0f / l : 0.f;
+  __hip_bfloat16* orow = out + (long)(row0 + r0 + qrow) * o_stride + (long)h * D + half * 4;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; r += 4) {
+      Vec4<__hip_bfloat16> y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y.data[e] = __float2bfloat16(o[dt][r + e] * f);
+      *reinterpret_cast<int2*>(orow + dt * 32 + (r >> 2) * 8) =
+          *reinterpret_cast<const int2*>(y.data);
+    }
+}

@@ -4,6 +4,7 @@
 #include "kvcache.hip"
 #include "attention.hip"
 #include "paged_decode.hip"
+#include "flash_prefill.hip"
 #include "skinny_gemm.hip"
 #include "sampling.hip"
 #include "bindings.cpp"

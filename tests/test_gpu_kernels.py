@@ -306,6 +306,37 @@ class TestPrefillAttention:
         assert_close_to_f32_ref(out.cpu(), ref, 2e-2, 1e-1)
 
 
+class TestPrefillRanges:
+    """The matrix-core prompt kernel at the edges of its row blocks (32, 64, 128,
+    256) and key tiles (32, 64), on continued contexts, odd and even head groups,
+    windows that open inside a tile, and rows inside a wider projection."""
+
+    @pytest.mark.parametrize("D,H,KVH", [(64, 6, 3), (64, 3, 1), (128, 3, 1), (128, 4, 2),
+                                         (256, 4, 2), (256, 3, 3)])
+    @pytest.mark.parametrize("window,softcap", [(0, 0.0), (40, 0.0), (130, 30.0)])
+    @pytest.mark.parametrize("past", [0, 1, 100])
+    def test_vs_ref(self, D, H, KVH, window, softcap, past):
+        lens = [1, 31, 32, 33, 64, 127, 129, 257]
+        cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32, device=DEV)
+        lens_k = [n + past * (i % 3 != 1) for i, n in enumerate(lens)]
+        cu_k = torch.tensor([0] + list(torch.tensor(lens_k).cumsum(0)), dtype=torch.int32,
+                            device=DEV)
+        T, Tk = sum(lens), sum(lens_k)
+        q = torch.randn(T, (H + 1) * D, device=DEV, dtype=torch.bfloat16)[:, D:].view(T, H, D)
+        kv = torch.randn(Tk, 2 * KVH * D, device=DEV, dtype=torch.bfloat16)
+        k, v = (kv[:, i * KVH * D:(i + 1) * KVH * D].view(Tk, KVH, D) for i in (0, 1))
+        scale = D ** -0.5
+        out = ops.varlen_prefill_attention(q, k, v, cu, max(lens), scale, softcap, window,
+                                           cu_seqlens_k=cu_k)
+        ref = torch_ref.varlen_prefill_attention(
+            q.float().cpu(), k.float().cpu(), v.float().cpu(), cu.cpu(), scale, softcap, window,
+            cu_seqlens_k=cu_k.cpu(),
+        )
+        # weights rounded to bf16: at most 2^-9 of the largest value (under 5 among
+        # unit normals); the output's own rounding 2^-9 of it, twice that allowed
+        assert_close_to_f32_ref(out.cpu(), ref, 5 * 2 ** -9, 2 ** -8)
+
+
 class TestEngineGPU:
     def test_engine_generates_and_graphs_match_eager(self):
         from llmq_amd.engine.config import EngineConfig
