@@ -228,6 +228,70 @@ class CausalLM:
             s.attn_softcap, window, cu_seqlens_k=g.cu_seqlens_k,
         )
 
+    def _attention(self, i: int, qkv, positions, kv_cache, meta) -> torch.Tensor:
+        """Layer i between its projections: RoPE, cache write, attention of each
+        segment. qkv [T, q+2kv] -> [T, q]."""
+        s = self.spec
+        T = qkv.shape[0]
+        q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
+        q = q.view(T, self.heads, s.head_dim)
+        k = k.view(T, self.kv_heads, s.head_dim)
+        v = v.view(T, self.kv_heads, s.head_dim)
+        ops.rope_and_cache(
+            q, k, v, kv_cache.k[i], kv_cache.v[i], positions,
+            self.rope_cache, meta.slot_mapping,
+        )
+        window = s.sliding_window if s.layer_uses_sliding_window(i) else 0
+        if meta.is_prefill:
+            attn = self._prefill_attn(q, k, v, meta, kv_cache, i, window)
+        elif meta.is_mixed:
+            # per-segment attention; GEMMs/norms already ran packed
+            nd = meta.n_decode
+            attn_d = ops.paged_decode_attention(
+                q[:nd], kv_cache.k[i], kv_cache.v[i],
+                meta.decode.block_tables, meta.decode.context_lens,
+                s.scale, s.attn_softcap, window,
+            )
+            attn_p = self._prefill_attn(
+                q[nd:], k[nd:], v[nd:], meta.prefill, kv_cache, i, window
+            )
+            attn = torch.cat([attn_d, attn_p], dim=0)
+        else:
+            attn = ops.paged_decode_attention(
+                q, kv_cache.k[i], kv_cache.v[i], meta.block_tables,
+                meta.context_lens, s.scale, s.attn_softcap, window,
+            )
+        return attn.reshape(T, self.q_size)
+
+    def _forward_few_rows(self, residual, positions, kv_cache, meta) -> torch.Tensor:
+        """The layers for up to ops.FEW_ROWS rows (a decode step of few
+        sequences): norms, activation and residual addition ride on the
+        projections, which stream the weights once."""
+        s = self.spec
+        act = "gelu_tanh" if s.gelu else "silu"
+        n_layers = len(self.layers)
+        h = self._norm(residual, self.layers[0].input_norm) if s.post_norms else None
+        for i, lw in enumerate(self.layers):
+            if s.post_norms:
+                qkv = ops.few_rows_linear(h, lw.qkv, lw.qkv_bias)
+                y = ops.few_rows_linear(
+                    self._attention(i, qkv, positions, kv_cache, meta), lw.o)
+                h, residual = ops.norm_add_norm(
+                    y, residual, lw.post_attn_norm, lw.pre_mlp_norm, s.rms_eps, self.norm_offset)
+                y = ops.few_rows_linear(ops.few_rows_linear(h, lw.gate_up, act=act), lw.down)
+                w_next = self.layers[i + 1].input_norm if i + 1 < n_layers else self.final_norm
+                h, residual = ops.norm_add_norm(
+                    y, residual, lw.post_mlp_norm, w_next, s.rms_eps, self.norm_offset)
+                continue
+            qkv = ops.few_rows_linear(residual, lw.qkv, lw.qkv_bias, lw.input_norm,
+                                      s.rms_eps, self.norm_offset)
+            ops.few_rows_linear(self._attention(i, qkv, positions, kv_cache, meta), lw.o,
+                                residual=residual)
+            a = ops.few_rows_linear(residual, lw.gate_up, None, lw.pre_mlp_norm,
+                                    s.rms_eps, self.norm_offset, act=act)
+            ops.few_rows_linear(a, lw.down, residual=residual)
+        return h if s.post_norms else self._norm(residual, self.final_norm)
+
     @torch.no_grad()
     def forward(
         self,
@@ -242,6 +306,9 @@ class CausalLM:
         if s.embedding_scale:
             x = x * math.sqrt(s.hidden_size)
             x = x.to(self.dtype)
+        l0 = self.layers[0]
+        if tp is None and ops.few_rows_ok(x, (l0.qkv, l0.o, l0.gate_up, l0.down)):
+            return self._forward_few_rows(x, positions, kv_cache, meta)
         residual = x
         h = self._norm(x, self.layers[0].input_norm)
         n_layers = len(self.layers)
@@ -249,36 +316,7 @@ class CausalLM:
             # ---- attention block (h = normed input, set by the previous
             # block's fused norm — launch count is the decode-step bound)
             qkv = _proj(h, lw.qkv, lw.qkv_bias)
-            q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
-            T = q.shape[0]
-            q = q.view(T, self.heads, s.head_dim)
-            k = k.view(T, self.kv_heads, s.head_dim)
-            v = v.view(T, self.kv_heads, s.head_dim)
-            ops.rope_and_cache(
-                q, k, v, kv_cache.k[i], kv_cache.v[i], positions,
-                self.rope_cache, meta.slot_mapping,
-            )
-            window = s.sliding_window if s.layer_uses_sliding_window(i) else 0
-            if meta.is_prefill:
-                attn = self._prefill_attn(q, k, v, meta, kv_cache, i, window)
-            elif meta.is_mixed:
-                # per-segment attention; GEMMs/norms already ran packed
-                nd = meta.n_decode
-                attn_d = ops.paged_decode_attention(
-                    q[:nd], kv_cache.k[i], kv_cache.v[i],
-                    meta.decode.block_tables, meta.decode.context_lens,
-                    s.scale, s.attn_softcap, window,
-                )
-                attn_p = self._prefill_attn(
-                    q[nd:], k[nd:], v[nd:], meta.prefill, kv_cache, i, window
-                )
-                attn = torch.cat([attn_d, attn_p], dim=0)
-            else:
-                attn = ops.paged_decode_attention(
-                    q, kv_cache.k[i], kv_cache.v[i], meta.block_tables,
-                    meta.context_lens, s.scale, s.attn_softcap, window,
-                )
-            attn_out = _proj(attn.reshape(T, self.q_size), lw.o)
+            attn_out = _proj(self._attention(i, qkv, positions, kv_cache, meta), lw.o)
             if tp is not None:
                 attn_out = tp.all_reduce(attn_out)
             if s.post_norms:

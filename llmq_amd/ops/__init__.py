@@ -259,6 +259,48 @@ def skinny_gemm(
     return out
 
 
+# ------------------------------------------------- projections of few rows --
+
+FEW_ROWS = 16
+_FEW_ACTS = {"silu": 2, "gelu_tanh": 3}
+
+
+def few_rows_ok(x: torch.Tensor, weights) -> bool:
+    """Whether few_rows_linear's kernel takes these rows and weights [N, K]."""
+    return (
+        x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= FEW_ROWS
+        and x.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0
+        and all(w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] % 128 == 0
+                and w.shape[0] % 32 == 0 and w.data_ptr() % 16 == 0 for w in weights)
+    )
+
+
+def few_rows_linear(
+    x: torch.Tensor,                        # [M, K], M <= FEW_ROWS
+    w: torch.Tensor,                        # [N, K]
+    bias: Optional[torch.Tensor] = None,    # [N]
+    norm: Optional[torch.Tensor] = None,    # [K]: x is RMS-normalised first
+    eps: float = 0.0,
+    offset: float = 0.0,                    # added to the norm's weights
+    act: str = "",                          # "silu" / "gelu_tanh": act(x gate^T) * (x up^T)
+    residual: Optional[torch.Tensor] = None,  # [M, N]: added to in place and returned
+) -> torch.Tensor:
+    """out = rmsnorm(x) @ w.T (+ bias), activated or added to the residual, in
+    one launch that streams the weights once (w = [gate | up] rows with act)."""
+    if _use_hip(x):
+        cols = w.shape[0] // 2 if act else w.shape[0]
+        out = residual if residual is not None else torch.empty(
+            x.shape[0], cols, dtype=x.dtype, device=x.device)
+        epi = 1 if residual is not None else _FEW_ACTS[act] if act else 0
+        _EXT.stream_gemm(out, x, w, bias, norm, eps, offset, epi)
+        return out
+    h = x if norm is None else torch_ref.rmsnorm(x, norm, eps, offset)
+    y = torch.nn.functional.linear(h, w, bias)
+    if act:
+        return torch_ref.silu_and_mul(y) if act == "silu" else torch_ref.gelu_tanh_and_mul(y)
+    return y if residual is None else residual.add_(y)
+
+
 # ------------------------------------------------------------- sampling --
 
 

@@ -492,6 +492,79 @@ void skinny_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
                      slabs.data_ptr<float>(), bias_ptr, z, MN, N);
 }
 
+// --------------------------------------------------- projections, few rows --
+
+// out = f(x) W^T for up to 16 rows: see stream_gemm.hip. norm_w: x is RMS-normalised
+// first; epi: 0 plain, 1 added to out in place, 2 / 3 SiLU / tanh-GELU of the first
+// half of W's rows times the second half.
+void stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
+                 c10::optional<at::Tensor> bias, c10::optional<at::Tensor> norm_w,
+                 double eps, double offset, long epi) {
+  CHECK_GPU(x);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2, "x, w and out must be matrices");
+  const int M = x.size(0), K = x.size(1), N = w.size(0);
+  const bool pair = epi >= kSgSilu;
+  const int cols = pair ? N / 2 : N;
+  auto bf16 = [](const at::Tensor& t) { return t.scalar_type() == at::kBFloat16; };
+  auto start16 = [](const at::Tensor& t) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  TORCH_CHECK(epi >= kSgPlain && epi <= kSgGelu, "unknown epilogue");
+  TORCH_CHECK(bf16(x) && bf16(w) && bf16(out), "x, w and out must be bfloat16");
+  TORCH_CHECK(M >= 1 && M <= 16, "1 to 16 rows");
+  TORCH_CHECK(w.size(1) == K && out.size(0) == M && out.size(1) == cols, "shapes differ");
+  TORCH_CHECK(K > 0 && K % 128 == 0 && N % 32 == 0, "K must be a multiple of 128, N of 32");
+  TORCH_CHECK(w.is_contiguous() && x.stride(1) == 1 && x.stride(0) % 8 == 0 &&
+                  out.stride(1) == 1 && start16(x) && start16(w),
+              "w must be contiguous, x's rows start on 16 bytes, rows packed");
+  const __hip_bfloat16 *bp = nullptr, *np = nullptr;
+  if (bias.has_value() && bias->defined()) {
+    TORCH_CHECK(bf16(*bias) && bias->is_contiguous() && bias->numel() == N && !pair,
+                "bias must be bfloat16 [N], without an activation");
+    bp = reinterpret_cast<const __hip_bfloat16*>(bias->data_ptr());
+  }
+  if (norm_w.has_value() && norm_w->defined()) {
+    TORCH_CHECK(bf16(*norm_w) && norm_w->is_contiguous() && norm_w->numel() == K &&
+                    start16(*norm_w), "norm weights must be bfloat16 [K]");
+    np = reinterpret_cast<const __hip_bfloat16*>(norm_w->data_ptr());
+  }
+  auto go = [&]<int KH, int NW, int KU, bool NORM, int EPI>() {
+    constexpr int RO = EPI >= kSgSilu ? 8 / KH : 16 / KH;
+    hipLaunchKernelGGL((stream_gemm_kernel<KH, NW, KU, NORM, EPI>), dim3(cols / RO),
+                       dim3(64 * NW), 0, stream(),
+                       reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), out.stride(0),
+                       reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()), x.stride(0),
+                       reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()), bp, np,
+                       (float)eps, (float)offset, M, N, K);
+  };
+  // Slices: as many as the tokens leave room for, up to four (2048 x 8192, one
+  // token: 13.0 us with one slice, 8.9 with four; eight gain nothing), because a
+  // small matrix then has more workgroups; a large one has enough of them anyway
+  // and saves the second reading of x (16384 x 3072, three tokens: 22.2 us with
+  // one slice and 16 waves, 23.3 with two, 23.8 with four).
+  const bool large = (long)N * K >= (48L << 20);
+  auto chunk = [&]<int KH, int NW, bool NORM, int EPI>() {
+    const int ks = K / KH;
+    if (ks % 128 == 0) go.template operator()<KH, NW, 4, NORM, EPI>();
+    else if (ks % 64 == 0) go.template operator()<KH, NW, 2, NORM, EPI>();
+    else go.template operator()<KH, NW, 1, NORM, EPI>();
+  };
+  auto slices = [&]<bool NORM, int EPI>() {
+    if (large) chunk.template operator()<1, 16, NORM, EPI>();
+    else if (M <= 4) chunk.template operator()<4, 8, NORM, EPI>();
+    else if (M <= 8) chunk.template operator()<2, 8, NORM, EPI>();
+    else chunk.template operator()<1, 8, NORM, EPI>();
+  };
+  auto epilogue = [&]<bool NORM>() {
+    if (epi == kSgPlain) slices.template operator()<NORM, kSgPlain>();
+    else if (epi == kSgResidual) slices.template operator()<NORM, kSgResidual>();
+    else if (epi == kSgSilu) slices.template operator()<NORM, kSgSilu>();
+    else slices.template operator()<NORM, kSgGelu>();
+  };
+  if (np) epilogue.template operator()<true>();
+  else epilogue.template operator()<false>();
+}
+
 // ------------------------------------------------------------- sampling --
 
 void topk_topp_bound(at::Tensor out_bound, at::Tensor logits, at::Tensor temps,
@@ -554,6 +627,7 @@ TORCH_LIBRARY(llmq_amd, m) {
   m.def("sample_gumbel_argmax(Tensor(a!) out, Tensor(b!) keys, Tensor logits, Tensor temps, Tensor req_seeds, Tensor req_pos, int seed, int step, Tensor? bounds=None) -> ()");
   m.def("topk_topp_bound(Tensor(a!) out_bound, Tensor logits, Tensor temps, Tensor top_ps, Tensor top_ks) -> ()");
   m.def("skinny_gemm(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int splitk) -> ()");
+  m.def("stream_gemm(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, Tensor? norm_w, float eps, float offset, int epi) -> ()");
   m.def("norm_add_norm(Tensor(a!) x, Tensor(b!) residual, Tensor w_post, Tensor w_pre, float eps, float offset) -> ()");
   m.def("rope_and_cache(Tensor(a!) q, Tensor(b!) k, Tensor value, Tensor(c!) k_cache, Tensor(d!) v_cache, Tensor positions, Tensor cos_sin, Tensor slot_mapping) -> ()");
 }
@@ -570,6 +644,7 @@ TORCH_LIBRARY_IMPL(llmq_amd, CUDA, m) {
   m.impl("sample_gumbel_argmax", &sample_gumbel_argmax);
   m.impl("topk_topp_bound", &topk_topp_bound);
   m.impl("skinny_gemm", &skinny_gemm);
+  m.impl("stream_gemm", &stream_gemm);
   m.impl("norm_add_norm", &norm_add_norm);
   m.impl("rope_and_cache", &rope_and_cache);
 }

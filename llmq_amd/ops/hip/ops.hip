@@ -6,5 +6,6 @@
 #include "paged_decode.hip"
 #include "flash_prefill.hip"
 #include "skinny_gemm.hip"
+#include "stream_gemm.hip"
 #include "sampling.hip"
 #include "bindings.cpp"

@@ -1,0 +1,150 @@
+// Projections of up to 16 rows, out[M, N] = f(x[M, K]) W[N, K]^T in bf16 with fp32
+// sums: the products of a decode step of few sequences (gfx950).
+//
+// Bound by the weights' bytes, each needed once, and below about 30 MB by the fixed
+// costs of a launch; so one launch does what surrounds the product too, and even a
+// matrix of a few MB is in flight on the whole chip at once.
+//
+//   - Operands go straight from memory into the layout of
+//     v_mfma_f32_16x16x32_bf16 (A = weights: row = lane%16, k = 8*(lane/16)..+7;
+//     B = tokens: column = lane%16; C: column = lane%16, rows 4*(lane/16)+r).
+//   - With M tokens only 16/KH >= M of the 16 columns are needed, so K is cut in KH
+//     slices that take the rest: A's rows are 16/KH weight rows times KH slices, B's
+//     columns 16/KH tokens times KH slices, and the result is the sum of the
+//     blocks on C's diagonal. That sets a workgroup's share to 16, 8, 4, 2 or 1
+//     weight rows without a masked lane.
+//   - The workgroup's waves share out the slices in chunks and add up through LDS.
+//   - NORM: the tokens are RMS-normalised on the way in: x is multiplied by the
+//     norm's weights (and rounded, as a normalised row is), its squares are summed
+//     beside, and the row's factor meets the fp32 sums at the end.
+//   - RES: the sums are added to the residual in place. ACT: half of the weight
+//     rows are gates, half the values that they act on (x = [gate | up]).
+
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(8))) short sg_s16x8;
+typedef __attribute__((ext_vector_type(4))) unsigned sg_u32x4;
+typedef __attribute__((ext_vector_type(4))) float sg_f32x4;
+typedef __attribute__((ext_vector_type(2))) float sg_f32x2;
+typedef __attribute__((ext_vector_type(2))) __bf16 sg_bf16x2;
+
+enum : int { kSgPlain = 0, kSgResidual = 1, kSgSilu = 2, kSgGelu = 3 };
+
+// KH: slices of K (16 / KH >= M); NW: waves; KU: 32-wide K steps of a chunk.
+template <int KH, int NW, int KU, bool NORM, int EPI>
+__global__ __launch_bounds__(64 * NW) void stream_gemm_kernel(
+    __hip_bfloat16* __restrict__ out, long out_stride,
+    const __hip_bfloat16* __restrict__ x, long x_stride,
+    const __hip_bfloat16* __restrict__ wt, const __hip_bfloat16* __restrict__ bias,
+    const __hip_bfloat16* __restrict__ norm_w, float eps, float offset,
+    int M, int N, int K) {
+  constexpr int R = 16 / KH, MP = 16 / KH, KC = 32 * KU;   // weight rows, token places
+  constexpr bool PAIR = EPI == kSgSilu || EPI == kSgGelu;
+  constexpr int RO = PAIR ? R / 2 : R;                     // output columns
+  constexpr int RP = 17;
+  __shared__ float red[NW][16 * RP];
+  __shared__ float sums[NW][16];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  const int ks = K / KH;
+  const int n0 = blockIdx.x * RO;
+  const int i = col % R;
+  const int wrow = PAIR ? (i < RO ? n0 + i : N / 2 + n0 + i - RO) : n0 + i;
+  const long kslice = (long)(col / R) * ks + grp * 8;
+  const __hip_bfloat16* wp = wt + (long)wrow * K + kslice;
+  const __hip_bfloat16* xp = x + (long)min(col % MP, M - 1) * x_stride + kslice;
+  const __hip_bfloat16* np = NORM ? norm_w + kslice : nullptr;
+  sg_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  float ss = 0.f;
+
+  sg_s16x8 wf[KU], wn[KU];
+  auto fetch = [&](sg_s16x8 (&f)[KU], int k0) {
+#pragma unroll
+    for (int u = 0; u < KU; ++u)
+      f[u] = __builtin_nontemporal_load(reinterpret_cast<const sg_s16x8*>(wp + k0 + u * 32));
+  };
+  int k0 = w * KC;
+  if (k0 < ks) fetch(wf, k0);
+  for (; k0 < ks; k0 += NW * KC) {
+    sg_s16x8 xf[KU];
+#pragma unroll
+    for (int u = 0; u < KU; ++u)
+      xf[u] = *reinterpret_cast<const sg_s16x8*>(xp + k0 + u * 32);
+    const int next = k0 + NW * KC;
+    if (next < ks) fetch(wn, next);
+    if constexpr (NORM) {
+#pragma unroll
+      for (int u = 0; u < KU; ++u) {
+        const Vec8<__hip_bfloat16> nv = load16(np + k0 + u * 32);
+        sg_u32x4 y;
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+          const float a = __uint_as_float((unsigned)(unsigned short)xf[u][e] << 16);
+          const float b = __uint_as_float((unsigned)(unsigned short)xf[u][e + 1] << 16);
+          ss += a * a + b * b;
+          y[e / 2] = __builtin_bit_cast(unsigned, __builtin_convertvector(
+              (sg_f32x2{a * (to_f32(nv.data[e]) + offset), b * (to_f32(nv.data[e + 1]) + offset)}),
+              sg_bf16x2));
+        }
+        xf[u] = __builtin_bit_cast(sg_s16x8, y);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < KU; ++u)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], xf[u], acc, 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < KU; ++u) wf[u] = wn[u];
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) red[w][(grp * 4 + r) * RP + col] = acc[r];
+  if constexpr (NORM) {
+    ss += __shfl_xor(ss, 16, WAVE);
+    ss += __shfl_xor(ss, 32, WAVE);
+    if (grp == 0) sums[w][col] = ss;
+  }
+  __syncthreads();
+  // four threads per sum: each takes every fourth wave
+  auto total = [&](int m, int row, int part) {
+    float s = 0.f;
+#pragma unroll
+    for (int v = 0; v < NW / 4; ++v)
+#pragma unroll
+      for (int h = 0; h < KH; ++h)
+        s += red[part + v * 4][(h * R + row) * RP + h * MP + m];
+    s += __shfl_xor(s, 1, WAVE);
+    s += __shfl_xor(s, 2, WAVE);
+    return s;
+  };
+  for (int t = threadIdx.x; t < 4 * RO * MP; t += 64 * NW) {
+    const int part = t & 3, row = (t >> 2) % RO, m = (t >> 2) / RO;
+    float y = total(m, row, part);
+    float up = 0.f, inv = 1.f;
+    if constexpr (PAIR) up = total(m, row + RO, part);
+    if constexpr (NORM) {
+      float q = 0.f;
+#pragma unroll
+      for (int v = 0; v < NW / 4; ++v)
+#pragma unroll
+        for (int h = 0; h < KH; ++h) q += sums[part + v * 4][h * MP + m];
+      q += __shfl_xor(q, 1, WAVE);
+      q += __shfl_xor(q, 2, WAVE);
+      inv = rsqrtf(q / K + eps);
+    }
+    if (part != 0 || m >= M) continue;
+    const int n = n0 + row;
+    y *= inv;
+    if (bias) y += to_f32(bias[n]);
+    if constexpr (PAIR) {
+      up *= inv;
+      if constexpr (EPI == kSgSilu) {
+        y = y / (1.0f + __expf(-y)) * up;
+      } else {               // tanh form of GELU
+        y = 0.5f * y * (1.0f + tanhf(0.7978845608028654f * (y + 0.044715f * y * y * y))) * up;
+      }
+    }
+    __hip_bfloat16* o = out + (long)m * out_stride + n;
+    if constexpr (EPI == kSgResidual) y += to_f32(*o);
+    *o = __float2bfloat16(y);
+  }
+}

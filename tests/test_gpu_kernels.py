@@ -337,6 +337,44 @@ class TestPrefillRanges:
         assert_close_to_f32_ref(out.cpu(), ref, 5 * 2 ** -9, 2 ** -8)
 
 
+class TestFewRowsLinear:
+    """Streaming projections of up to 16 rows: each split of K (rows <= 4, 8, 16;
+    large matrices), chunk remainders, norm, bias, activation and residual."""
+
+    @pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
+    @pytest.mark.parametrize("N,K", [(32, 128), (96, 384), (1536, 640), (16384, 3072)])
+    @pytest.mark.parametrize("norm", [False, True])
+    @pytest.mark.parametrize("what", ["plain", "bias", "residual", "silu", "gelu_tanh"])
+    def test_vs_64_bits(self, M, N, K, norm, what):
+        x = torch.randn(M, K + 8, device=DEV, dtype=torch.bfloat16)[:, :K] * 2
+        w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) * K ** -0.5
+        nw = torch.randn(K, device=DEV, dtype=torch.bfloat16) if norm else None
+        bias = torch.randn(N, device=DEV, dtype=torch.bfloat16) if what == "bias" else None
+        res = torch.randn(M, N, device=DEV, dtype=torch.bfloat16)
+        h = x.double()
+        if norm:   # the kernel's operands: weighted in fp32, rounded, scaled after the sum
+            inv = torch.rsqrt(h.square().mean(-1, keepdim=True) + 1e-5)
+            h = (x.float() * (nw.float() + 1.0)).bfloat16().double() * inv
+        ref = h @ w.double().t()
+        mag = h.norm(dim=-1, keepdim=True) * K ** -0.5       # of one sum
+        act = what if what in ("silu", "gelu_tanh") else ""
+        if bias is not None:
+            ref = ref + bias.double()
+        if what == "residual":
+            ref = ref + res.double()
+        if act:
+            g, u = ref.chunk(2, -1)
+            ref = (torch.nn.functional.silu(g) if act == "silu"
+                   else torch.nn.functional.gelu(g, approximate="tanh")) * u
+            mag = mag * (u.abs() + 1.2 * g.abs())            # |act'| < 1.2, |act(g)| <= |g|
+        got = ops.few_rows_linear(x, w, bias, nw, 1e-5, 1.0, act=act,
+                                  residual=res if what == "residual" else None)
+        # the output's rounding (half a step of bf16 is up to 2^-8 of the value) and
+        # fp32 sums
+        tol = 2 ** -8 * ref.abs() + 1e-5 * mag + 1e-6
+        assert ((got.double() - ref).abs() <= tol).all()
+
+
 class TestEngineGPU:
     def test_engine_generates_and_graphs_match_eager(self):
         from llmq_amd.engine.config import EngineConfig
