@@ -355,8 +355,4 @@ class CausalLM:
     @torch.no_grad()
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
         """hidden [N, hidden] → logits [N, vocab] (fp32)."""
-        logits = _proj(hidden, self.lm_head).float()
-        cap = self.spec.final_softcap
-        if cap and cap > 0:
-            logits = torch.tanh(logits / cap) * cap
-        return logits
+        return ops.softcap_logits(_proj(hidden, self.lm_head), self.spec.final_softcap)

@@ -304,6 +304,17 @@ def few_rows_linear(
 # ------------------------------------------------------------- sampling --
 
 
+def softcap_logits(x: torch.Tensor, cap: float) -> torch.Tensor:
+    """fp32 logits: cap * tanh(x / cap), or x as it is with cap 0."""
+    if not cap or cap <= 0:
+        return x.float()
+    if x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and _use_hip(x):
+        out = torch.empty(x.shape, dtype=torch.float32, device=x.device)
+        _EXT.softcap_logits(out, x, float(cap))
+        return out
+    return torch.tanh(x.float() / cap) * cap
+
+
 def sample_gumbel_argmax(
     out: torch.Tensor,        # [B] int64
     keys: torch.Tensor,       # [B] int64 scratch (packed value|~index)

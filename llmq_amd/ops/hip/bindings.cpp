@@ -567,6 +567,32 @@ void stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
 
 // ------------------------------------------------------------- sampling --
 
+// Chunks of a logits row: enough workgroups to fill the chip at few rows, whole
+// 16-byte loads where every row allows them (the return value).
+bool row_chunks(const at::Tensor& logits, int B, int V, int& chunk, int& splits) {
+  int n = 1;
+  while (B * n < 2048 && n < 64 && (V / n) > 4096) n *= 2;
+  chunk = ((V + n - 1) / n + 3) / 4 * 4;
+  splits = (V + chunk - 1) / chunk;
+  return V % 4 == 0 && logits.stride(0) % 4 == 0 &&
+         reinterpret_cast<uintptr_t>(logits.data_ptr()) % 16 == 0;
+}
+
+// out = cap * tanh(in / cap) in fp32 of bf16 logits
+void softcap_logits(at::Tensor out, at::Tensor in, double cap) {
+  CHECK_GPU(in);
+  TORCH_CHECK(in.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kFloat);
+  TORCH_CHECK(in.is_contiguous() && out.is_contiguous() && in.numel() == out.numel());
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(in.data_ptr()) % 16 == 0 &&
+              reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0);
+  const long n = in.numel();
+  if (n == 0) return;
+  const int grid = (int)std::min<long>((n + 2047) / 2048, 8192);
+  hipLaunchKernelGGL(softcap_logits_kernel, dim3(grid), dim3(256), 0, stream(),
+                     out.data_ptr<float>(),
+                     reinterpret_cast<const __hip_bfloat16*>(in.data_ptr()), n, (float)cap);
+}
+
 void topk_topp_bound(at::Tensor out_bound, at::Tensor logits, at::Tensor temps,
                      at::Tensor top_ps, at::Tensor top_ks) {
   CHECK_GPU(logits);
@@ -575,10 +601,28 @@ void topk_topp_bound(at::Tensor out_bound, at::Tensor logits, at::Tensor temps,
   TORCH_CHECK(top_ps.scalar_type() == at::kFloat);
   TORCH_CHECK(top_ks.scalar_type() == at::kLong);
   const int B = logits.size(0), V = logits.size(1);
-  hipLaunchKernelGGL(topk_topp_bound_kernel, dim3(B), dim3(256), 0, stream(),
-                     out_bound.data_ptr<float>(), logits.data_ptr<float>(),
-                     temps.data_ptr<float>(), top_ps.data_ptr<float>(),
-                     top_ks.data_ptr<long>(), V, logits.stride(0));
+  if (B == 0) return;
+  TORCH_CHECK(logits.stride(1) == 1, "logits rows must be packed");
+  int chunk, splits;
+  const bool vec = row_chunks(logits, B, V, chunk, splits);
+  at::Tensor ws = at::zeros({(long)B * (long)sizeof(ThRow) / 4}, logits.options().dtype(at::kInt));
+  ThRow* rows = reinterpret_cast<ThRow*>(ws.data_ptr());
+  float* bound = out_bound.data_ptr<float>();
+  const float *lp = logits.data_ptr<float>(), *tp = temps.data_ptr<float>(),
+              *pp = top_ps.data_ptr<float>();
+  const long* kp = top_ks.data_ptr<long>();
+  const long stride = logits.stride(0);
+  const dim3 grid(B, splits), wg(256);
+  hipLaunchKernelGGL(topk_topp_max_kernel, grid, wg, 0, stream(), bound, rows, lp, tp, pp, kp, V,
+                     stride, chunk, vec);
+  hipLaunchKernelGGL((topk_topp_hist_kernel<0>), grid, wg, 0, stream(), rows, lp, tp, pp, kp, V,
+                     stride, chunk, vec);
+  hipLaunchKernelGGL((topk_topp_scan_kernel<0>), dim3(B), wg, 0, stream(), bound, rows, tp, pp, kp,
+                     V);
+  hipLaunchKernelGGL((topk_topp_hist_kernel<1>), grid, wg, 0, stream(), rows, lp, tp, pp, kp, V,
+                     stride, chunk, vec);
+  hipLaunchKernelGGL((topk_topp_scan_kernel<1>), dim3(B), wg, 0, stream(), bound, rows, tp, pp, kp,
+                     V);
 }
 
 void sample_gumbel_argmax(at::Tensor out, at::Tensor keys, at::Tensor logits,
@@ -597,16 +641,17 @@ void sample_gumbel_argmax(at::Tensor out, at::Tensor keys, at::Tensor logits,
     TORCH_CHECK(bounds->scalar_type() == at::kFloat && bounds->numel() == B);
     bounds_ptr = bounds->data_ptr<float>();
   }
-  // enough splits to fill the chip at small B
-  int nsplit = 1;
-  while (B * nsplit < 2048 && nsplit < 64 && (V / nsplit) > 4096) nsplit *= 2;
-  hipLaunchKernelGGL(sample_argmax_kernel, dim3(B, nsplit), dim3(256), 0,
+  if (B == 0) return;
+  TORCH_CHECK(logits.is_contiguous(), "logits must be contiguous");
+  int chunk, splits;
+  const bool vec = row_chunks(logits, B, V, chunk, splits);
+  hipLaunchKernelGGL(sample_argmax_kernel, dim3(B, splits), dim3(256), 0,
                      stream(),
                      reinterpret_cast<unsigned long long*>(keys.data_ptr()),
                      logits.data_ptr<float>(), temps.data_ptr<float>(),
                      reinterpret_cast<const unsigned int*>(req_seeds.data_ptr()),
                      reinterpret_cast<const unsigned int*>(req_pos.data_ptr()),
-                     bounds_ptr, V, (unsigned int)seed, (unsigned int)step);
+                     bounds_ptr, V, (unsigned int)seed, (unsigned int)step, chunk, vec);
   hipLaunchKernelGGL(unpack_keys_kernel, dim3((B + 255) / 256), dim3(256), 0,
                      stream(), out.data_ptr<long>(),
                      reinterpret_cast<const unsigned long long*>(keys.data_ptr()),
@@ -626,6 +671,7 @@ TORCH_LIBRARY(llmq_amd, m) {
   m.def("varlen_prefill_attention(Tensor(a!) out, Tensor q, Tensor k, Tensor v, Tensor cu_seqlens, Tensor cu_seqlens_k, int max_seqlen, float scale, float softcap, int window) -> ()");
   m.def("sample_gumbel_argmax(Tensor(a!) out, Tensor(b!) keys, Tensor logits, Tensor temps, Tensor req_seeds, Tensor req_pos, int seed, int step, Tensor? bounds=None) -> ()");
   m.def("topk_topp_bound(Tensor(a!) out_bound, Tensor logits, Tensor temps, Tensor top_ps, Tensor top_ks) -> ()");
+  m.def("softcap_logits(Tensor(a!) out, Tensor input, float cap) -> ()");
   m.def("skinny_gemm(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int splitk) -> ()");
   m.def("stream_gemm(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, Tensor? norm_w, float eps, float offset, int epi) -> ()");
   m.def("norm_add_norm(Tensor(a!) x, Tensor(b!) residual, Tensor w_post, Tensor w_pre, float eps, float offset) -> ()");
@@ -643,6 +689,7 @@ TORCH_LIBRARY_IMPL(llmq_amd, CUDA, m) {
   m.impl("varlen_prefill_attention", &varlen_prefill_attention);
   m.impl("sample_gumbel_argmax", &sample_gumbel_argmax);
   m.impl("topk_topp_bound", &topk_topp_bound);
+  m.impl("softcap_logits", &softcap_logits);
   m.impl("skinny_gemm", &skinny_gemm);
   m.impl("stream_gemm", &stream_gemm);
   m.impl("norm_add_norm", &norm_add_norm);

@@ -572,6 +572,52 @@ class TestFusedSampler:
             counts, expected)
 
 
+class TestTruncationRanges:
+    """topk_topp_bound and the sampler over chunked rows: odd row lengths (4-byte
+    loads), few rows (many chunks), each way a top-k narrows the histogram (up to
+    64, up to 64 per chunk, beyond), peaked and flat rows."""
+
+    @pytest.mark.parametrize("B,V", [(1, 50000), (3, 1003), (2, 16384), (300, 257)])
+    @pytest.mark.parametrize("k,p", [(1, 1.0), (50, 0.9), (64, 1.0), (65, 1.0), (600, 0.97),
+                                     (0, 0.5), (0, 0.9), (5000, 1.0)])
+    @pytest.mark.parametrize("spread", [0.01, 1.5, 12.0])
+    def test_bound_and_argmax(self, B, V, k, p, spread):
+        logits = torch.randn(B, V, device=DEV) * spread
+        temps = torch.rand(B, device=DEV) + 0.3
+        temps[-1] = 0.0                                       # greedy: keeps all
+        tps = torch.full((B,), p, device=DEV)
+        tks = torch.full((B,), k, dtype=torch.int64, device=DEV)
+        bound = ops.topk_topp_bound(logits, temps, tps, tks).double()
+        live = temps > 0
+        T = temps.double().where(live, torch.ones((), dtype=torch.double, device=DEV))
+        x = (logits.double() / T[:, None]).sort(1, descending=True)[0]
+        mass = x.softmax(1).cumsum(1)
+        n_k = torch.full((B,), k if 0 < k < V else V, device=DEV)
+        n_p = ((mass < p).sum(1) + 1).clamp(max=V) if p < 1.0 else torch.full((B,), V, device=DEV)
+        want = torch.minimum(n_k, n_p)
+        edge = x.gather(1, want[:, None] - 1)[:, 0] * T       # the last logit to keep
+        none = (~live) | (want == V)
+        # not above the last one to keep and at most a sub-bin, 32 / 512^2, below it,
+        # where that is told from its neighbours by more than 1e-5 of the mass (fp32
+        # sums of fp32 exponentials); rounding of x = (l - max) / T
+        def reached(share):
+            n = (mass < p * share).sum(1) if p < 1.0 else n_k - 1
+            return x.gather(1, torch.minimum(n, n_k - 1).clamp(max=V - 1)[:, None])[:, 0] * T
+        near, far = reached(1 - 1e-5), reached(1 + 1e-5)
+        # beyond 32 below the maximum nothing is told apart
+        deep = (x[:, 0] - edge / T) > 31.9
+        ok = none | deep | ((bound <= near + 1e-5 * spread) &
+                            (bound >= far - T * 32 / 512 ** 2 * 1.01 - 1e-5 * spread))
+        assert ok.all()
+        assert (bound[~live] < -1e38).all()
+        out = torch.empty(B, dtype=torch.int64, device=DEV)
+        keys = torch.empty(B, dtype=torch.int64, device=DEV)
+        zeros = torch.zeros(B, dtype=torch.int32, device=DEV)
+        ops.sample_gumbel_argmax(out, keys, logits, torch.zeros(B, device=DEV), zeros, zeros, 1, 1,
+                                 bound.float())
+        assert torch.equal(out, logits.argmax(1))
+
+
 class TestFusedNormSandwich:
     @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
     def test_norm_add_norm(self, dtype):
