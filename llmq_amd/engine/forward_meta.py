@@ -41,6 +41,9 @@ class PrefillMeta:
     gather: "ChunkGather | None" = None  # set when any entry is a chunk
     # models whose prefill attention reads the paged cache directly:
     block_tables: "torch.Tensor | None" = None  # [B, max_blocks] int32
+    # with block_tables and no gather: portions that continue cached contexts,
+    # attention reads the cache in place
+    cu_seqlens_k: "torch.Tensor | None" = None  # [B+1] int32 context offsets
     q_start: "torch.Tensor | None" = None       # [B] int32 first query position
     recurrent: "RecurrentMeta | None" = None
 

@@ -71,6 +71,11 @@ class ModelRunner:
         # the block table (no gathered K/V copy), and models with recurrent
         # layers (per-sequence state slots), get the extra step metadata.
         self.paged_prefill = bool(getattr(model, "paged_prefill", False))
+        # Portions on cached context, other models: attention reads a bf16 cache
+        # in place; a cache of another type is gathered into packed rows.
+        self.paged_portions = not self.paged_prefill and device.type == "cuda" and all(
+            t is not None and t.dtype == torch.bfloat16 and model.dtype == torch.bfloat16
+            for t in kv_cache.k + kv_cache.v)
         self.recurrent = kv_cache.recurrent if (
             kv_cache.recurrent is not None and kv_cache.recurrent.active) else None
         if self.use_graphs:
@@ -180,7 +185,8 @@ class ModelRunner:
         cu = [0]
         cu_k = [0]
         rel_last: List[int] = []
-        any_chunk = (not self.paged_prefill) and any(start > 0 for (start, _e) in chunks)
+        continued = (not self.paged_prefill) and any(start > 0 for (start, _e) in chunks)
+        any_chunk = continued and not self.paged_portions
         g_blocks: List[int] = []
         g_offs: List[int] = []
         past_dst: List[int] = []
@@ -222,6 +228,9 @@ class ModelRunner:
             slot_mapping=slot_mapping,
             gather=gather,
         )
+        if continued and self.paged_portions:
+            meta.block_tables = self._block_table_tensor(pseqs, dev)
+            meta.cu_seqlens_k = torch.tensor(cu_k, dtype=torch.int32, device=dev)
         if self.paged_prefill:
             meta.block_tables = self._block_table_tensor(pseqs, dev)
             meta.q_start = torch.tensor([st for (st, _e) in chunks], dtype=torch.int32, device=dev)

@@ -205,9 +205,15 @@ class CausalLM:
         return ops.rmsnorm(x, w, self.spec.rms_eps, self.norm_offset)
 
     def _prefill_attn(self, q, k, v, pmeta, kv_cache, layer: int, window: int):
-        """Packed varlen attention; chunk continuations assemble their full
-        context (gathered past from the paged cache + fresh rows)."""
+        """Packed varlen attention; chunk continuations read their full context
+        from the paged cache, or assemble it (gathered past + fresh rows)."""
         s = self.spec
+        if pmeta.cu_seqlens_k is not None:
+            return ops.paged_prefill_attention(
+                q, kv_cache.k[layer], kv_cache.v[layer], pmeta.block_tables,
+                pmeta.cu_seqlens, pmeta.cu_seqlens_k, pmeta.max_seqlen, s.scale,
+                s.attn_softcap, window,
+            )
         g = pmeta.gather
         if g is None:
             return ops.varlen_prefill_attention(

@@ -231,6 +231,27 @@ def varlen_prefill_attention(
     )
 
 
+def paged_prefill_attention(
+    q: torch.Tensor,             # [Tq, H, D]
+    k_cache: torch.Tensor,       # [blocks, KVH, block, D], the portions' rows included
+    v_cache: torch.Tensor,
+    block_tables: torch.Tensor,  # [B, max_blocks] int32
+    cu_seqlens: torch.Tensor,    # [B+1] int32 query offsets
+    cu_seqlens_k: torch.Tensor,  # [B+1] int32 context offsets
+    max_seqlen: int,
+    scale: float,
+    softcap: float = 0.0,
+    window: int = 0,
+) -> torch.Tensor:
+    """varlen_prefill_attention with keys and values read from the paged cache:
+    portions that continue a cached context. GPU, bf16 cache."""
+    assert _use_hip(q)
+    out = torch.empty_like(q)
+    _EXT.paged_prefill_attention(out, q, k_cache, v_cache, block_tables, cu_seqlens,
+                                 cu_seqlens_k, int(max_seqlen), scale, softcap, window)
+    return out
+
+
 # ---------------------------------------------------------- skinny GEMM --
 
 

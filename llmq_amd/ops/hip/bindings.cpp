@@ -217,6 +217,15 @@ void rope_and_cache(at::Tensor q, at::Tensor k, at::Tensor value,
 
 // ------------------------------------------------------------ attention --
 
+// 16-byte loads and 8-byte stores: rows that start elsewhere go through a copy.
+bool rows_start_on(const at::Tensor& t, long bytes) {
+  return reinterpret_cast<uintptr_t>(t.data_ptr()) % bytes == 0 &&
+         t.stride(0) * (long)t.element_size() % bytes == 0;
+}
+at::Tensor rows_on_16(const at::Tensor& t) {
+  return rows_start_on(t, 16) ? t : t.clone(at::MemoryFormat::Contiguous);
+}
+
 // The matrix-core kernel of paged_decode.hip. Waves: as many as are resident at
 // the variant's register use, so that every range is in work at once.
 template <int D, typename TC, int NK, int OCC>
@@ -277,15 +286,9 @@ void launch_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor& kc,
   TORCH_CHECK(D == 64 || D == 128 || D == 256, "unsupported head_dim ", D);
   if constexpr (std::is_same_v<T, __hip_bfloat16>) {
     TORCH_CHECK(G <= (D == 64 ? 8 : 16), "GQA group must be <= 8 at head_dim 64, else <= 16");
-    // 16-byte query loads and 8-byte stores: rows that start elsewhere go
-    // through a copy
-    auto aligned = [](const at::Tensor& t, long bytes) {
-      return reinterpret_cast<uintptr_t>(t.data_ptr()) % bytes == 0 &&
-             t.stride(0) * (long)t.element_size() % bytes == 0;
-    };
-    const at::Tensor qa = aligned(q, 16) ? q : q.clone(at::MemoryFormat::Contiguous);
+    const at::Tensor qa = rows_on_16(q);
     const at::Tensor bta = bt.stride(1) == 1 ? bt : bt.contiguous();
-    at::Tensor oa = aligned(out, 8) ? out : out.clone(at::MemoryFormat::Contiguous);
+    at::Tensor oa = rows_start_on(out, 8) ? out : out.clone(at::MemoryFormat::Contiguous);
     auto go = [&]<int HD, typename TC, int NK, int OCC>() {
       launch_paged_decode<HD, TC, NK, OCC>(oa, qa, kc, vc, bta, cl, scale, softcap, window);
     };
@@ -337,26 +340,61 @@ void paged_decode_attention(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   });
 }
 
+// The matrix-core kernel of flash_prefill.hip on packed rows, or with a block table
+// on cache blocks [blocks, kv heads, block, D].
+struct PrefillArgs {
+  const at::Tensor &q, &k, &v, &cu, &cu_k;
+  const at::Tensor* block_tables;            // null: packed rows
+  int B, KVH;
+  double scale, softcap;
+  long window, max_seqlen;
+};
+
 template <int D, int HP, int WR, int KT, int MINW>
-void launch_flash_prefill(at::Tensor& out, const at::Tensor& q, const at::Tensor& k,
-                          const at::Tensor& v, const at::Tensor& cu, const at::Tensor& cu_k,
-                          int B, double scale, double softcap, long window, long max_seqlen) {
+void launch_flash_prefill(at::Tensor& out, const PrefillArgs& a) {
   constexpr double kLog2e = 1.4426950408889634;
-  const int H = q.size(1), KVH = k.size(1);
-  const int n_qt = (int)((std::max<long>(max_seqlen, 1) + 32 * WR - 1) / (32 * WR));
-  auto go = [&]<bool CAP>() {
-    hipLaunchKernelGGL((flash_prefill_kernel<D, HP, WR, KT, MINW, CAP>),
-                       dim3((unsigned)(n_qt * (H / HP) * B)), dim3(64 * HP * WR), 0, stream(),
+  const int H = a.q.size(1);
+  const int n_qt = (int)((std::max<long>(a.max_seqlen, 1) + 32 * WR - 1) / (32 * WR));
+  auto go = [&]<bool CAP, bool PAGED>() {
+    hipLaunchKernelGGL((flash_prefill_kernel<D, HP, WR, KT, MINW, CAP, PAGED>),
+                       dim3((unsigned)(n_qt * (H / HP) * a.B)), dim3(64 * HP * WR), 0, stream(),
                        reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), out.stride(0),
-                       reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()), q.stride(0),
-                       reinterpret_cast<const __hip_bfloat16*>(k.data_ptr()), k.stride(0),
-                       reinterpret_cast<const __hip_bfloat16*>(v.data_ptr()), v.stride(0),
-                       cu.data_ptr<int>(), cu_k.data_ptr<int>(), B, H, KVH, (int)window,
-                       (float)(scale * kLog2e), (float)(softcap * kLog2e),
-                       softcap > 0 ? (float)(2 * scale / softcap * kLog2e) : 0.f, n_qt);
+                       reinterpret_cast<const __hip_bfloat16*>(a.q.data_ptr()), a.q.stride(0),
+                       reinterpret_cast<const __hip_bfloat16*>(a.k.data_ptr()), a.k.stride(0),
+                       reinterpret_cast<const __hip_bfloat16*>(a.v.data_ptr()), a.v.stride(0),
+                       a.cu.data_ptr<int>(), a.cu_k.data_ptr<int>(),
+                       PAGED ? a.block_tables->data_ptr<int>() : nullptr,
+                       PAGED ? (int)a.block_tables->stride(0) : 0,
+                       PAGED && a.k.size(2) == 32 ? 5 : 4, a.B, H, a.KVH, (int)a.window,
+                       (float)(a.scale * kLog2e), (float)(a.softcap * kLog2e),
+                       a.softcap > 0 ? (float)(2 * a.scale / a.softcap * kLog2e) : 0.f, n_qt);
   };
-  if (softcap > 0) go.template operator()<true>();
-  else go.template operator()<false>();
+  if (a.block_tables) {
+    if (a.softcap > 0) go.template operator()<true, true>();
+    else go.template operator()<false, true>();
+  } else {
+    if (a.softcap > 0) go.template operator()<true, false>();
+    else go.template operator()<false, false>();
+  }
+}
+
+void launch_flash_prefill_any(at::Tensor& out, const PrefillArgs& args) {
+  const int H = args.q.size(1), D = args.q.size(2);
+  const at::Tensor qa = rows_on_16(args.q), ka = rows_on_16(args.k), va = rows_on_16(args.v);
+  at::Tensor oa = rows_start_on(out, 8) ? out : out.clone(at::MemoryFormat::Contiguous);
+  const PrefillArgs a{qa, ka, va, args.cu, args.cu_k, args.block_tables, args.B, args.KVH,
+                      args.scale, args.softcap, args.window, args.max_seqlen};
+  // Two heads of a kv head on one stream of tiles where the group is even
+  // (2 x 64 rows at head size 64, 2 x 128 at 256: 138 against 147 us for
+  // 8 x 1024 tokens). Tiles of 32 keys where that buys a third wave per SIMD
+  // (head size 128: 160 against 187 us for 16 x 1024) or the registers (256).
+  const bool even = (H / args.KVH) % 2 == 0;
+  if (D == 64 && even) launch_flash_prefill<64, 2, 2, 64, 3>(oa, a);
+  else if (D == 64) launch_flash_prefill<64, 1, 4, 64, 3>(oa, a);
+  else if (D == 128) launch_flash_prefill<128, 1, 4, 32, 3>(oa, a);
+  else if (even) launch_flash_prefill<256, 2, 4, 32, 1>(oa, a);
+  else launch_flash_prefill<256, 1, 8, 32, 1>(oa, a);
+  if (!oa.is_same(out)) out.copy_(oa);
 }
 
 template <typename T>
@@ -369,31 +407,8 @@ void launch_prefill(at::Tensor& out, const at::Tensor& q, const at::Tensor& k,
   if (B == 0) return;
   TORCH_CHECK(D == 64 || D == 128 || D == 256, "unsupported head_dim ", D);
   if constexpr (std::is_same_v<T, __hip_bfloat16>) {
-    // 16-byte loads and 8-byte stores: rows that start elsewhere go through a copy
-    auto aligned = [](const at::Tensor& t, long bytes) {
-      return reinterpret_cast<uintptr_t>(t.data_ptr()) % bytes == 0 &&
-             t.stride(0) * (long)t.element_size() % bytes == 0;
-    };
-    auto rows16 = [&](const at::Tensor& t) {
-      return aligned(t, 16) ? t : t.clone(at::MemoryFormat::Contiguous);
-    };
-    const at::Tensor qa = rows16(q), ka = rows16(k), va = rows16(v);
-    at::Tensor oa = aligned(out, 8) ? out : out.clone(at::MemoryFormat::Contiguous);
-    auto go = [&]<int HD, int HP, int WR, int KT, int MINW>() {
-      launch_flash_prefill<HD, HP, WR, KT, MINW>(oa, qa, ka, va, cu, cu_k, B, scale, softcap,
-                                                 window, max_seqlen);
-    };
-    // Two heads of a kv head on one stream of tiles where the group is even
-    // (2 x 64 rows at head size 64, 2 x 128 at 256: 138 against 147 us for
-    // 8 x 1024 tokens). Tiles of 32 keys where that buys a third wave per SIMD
-    // (head size 128: 160 against 187 us for 16 x 1024) or the registers (256).
-    const bool even = (H / KVH) % 2 == 0;
-    if (D == 64 && even) go.template operator()<64, 2, 2, 64, 3>();
-    else if (D == 64) go.template operator()<64, 1, 4, 64, 3>();
-    else if (D == 128) go.template operator()<128, 1, 4, 32, 3>();
-    else if (even) go.template operator()<256, 2, 4, 32, 1>();
-    else go.template operator()<256, 1, 8, 32, 1>();
-    if (!oa.is_same(out)) out.copy_(oa);
+    launch_flash_prefill_any(out, PrefillArgs{q, k, v, cu, cu_k, nullptr, B, KVH, scale, softcap,
+                                              window, max_seqlen});
     return;
   } else {
   dim3 grid(B, H);
@@ -430,6 +445,31 @@ void varlen_prefill_attention(at::Tensor out, at::Tensor q, at::Tensor k,
     launch_prefill<T>(out, q, k, v, cu_seqlens, cu_seqlens_k, B, scale,
                       softcap, window, max_seqlen);
   });
+}
+
+// Prompt portions over the paged bf16 cache: the last rows of contexts of
+// cu_k[b+1] - cu_k[b] keys.
+void paged_prefill_attention(at::Tensor out, at::Tensor q, at::Tensor k_cache,
+                             at::Tensor v_cache, at::Tensor block_tables, at::Tensor cu_seqlens,
+                             at::Tensor cu_seqlens_k, long max_seqlen, double scale,
+                             double softcap, long window) {
+  CHECK_GPU(q);
+  CHECK_LASTDIM(q);
+  TORCH_CHECK(cu_seqlens.scalar_type() == at::kInt && cu_seqlens_k.scalar_type() == at::kInt &&
+              block_tables.scalar_type() == at::kInt);
+  TORCH_CHECK(q.scalar_type() == at::kBFloat16 && k_cache.scalar_type() == at::kBFloat16 &&
+                  v_cache.scalar_type() == at::kBFloat16, "bfloat16 queries and cache");
+  const int D = q.size(2), B = cu_seqlens.size(0) - 1, KVH = k_cache.size(1);
+  const long bs = k_cache.size(2);
+  TORCH_CHECK(D == 64 || D == 128 || D == 256, "unsupported head_dim ", D);
+  TORCH_CHECK(bs == 16 || bs == 32, "block_size must be 16 or 32");
+  TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous() && block_tables.stride(1) == 1);
+  TORCH_CHECK(q.size(1) % KVH == 0 && block_tables.size(0) == B &&
+              cu_seqlens_k.size(0) == B + 1);
+  if (B == 0 || q.size(0) == 0) return;
+  launch_flash_prefill_any(out, PrefillArgs{q, k_cache, v_cache, cu_seqlens, cu_seqlens_k,
+                                            &block_tables, B, KVH, scale, softcap, window,
+                                            max_seqlen});
 }
 
 // ---------------------------------------------------------- skinny GEMM --
@@ -669,6 +709,7 @@ TORCH_LIBRARY(llmq_amd, m) {
   m.def("reshape_and_cache(Tensor key, Tensor value, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor slot_mapping) -> ()");
   m.def("paged_decode_attention(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor context_lens, float scale, float softcap, int window) -> ()");
   m.def("varlen_prefill_attention(Tensor(a!) out, Tensor q, Tensor k, Tensor v, Tensor cu_seqlens, Tensor cu_seqlens_k, int max_seqlen, float scale, float softcap, int window) -> ()");
+  m.def("paged_prefill_attention(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor cu_seqlens, Tensor cu_seqlens_k, int max_seqlen, float scale, float softcap, int window) -> ()");
   m.def("sample_gumbel_argmax(Tensor(a!) out, Tensor(b!) keys, Tensor logits, Tensor temps, Tensor req_seeds, Tensor req_pos, int seed, int step, Tensor? bounds=None) -> ()");
   m.def("topk_topp_bound(Tensor(a!) out_bound, Tensor logits, Tensor temps, Tensor top_ps, Tensor top_ks) -> ()");
   m.def("softcap_logits(Tensor(a!) out, Tensor input, float cap) -> ()");
@@ -687,6 +728,7 @@ TORCH_LIBRARY_IMPL(llmq_amd, CUDA, m) {
   m.impl("reshape_and_cache", &reshape_and_cache);
   m.impl("paged_decode_attention", &paged_decode_attention);
   m.impl("varlen_prefill_attention", &varlen_prefill_attention);
+  m.impl("paged_prefill_attention", &paged_prefill_attention);
   m.impl("sample_gumbel_argmax", &sample_gumbel_argmax);
   m.impl("topk_topp_bound", &topk_topp_bound);
   m.impl("softcap_logits", &softcap_logits);

@@ -23,6 +23,9 @@
 //     barrier per tile: the next tile travels during the current one's products.
 //   - A workgroup takes HP query heads of one kv head times WR blocks of 32 rows,
 //     a wave each, on one stream of K/V tiles.
+//   - K and V are rows of the packed projection, or cache blocks (a portion that
+//     continues a cached context reads it in place: gathering and interleaving it
+//     took 3.7 ms of an 11000-token prompt's second portion).
 //   - Workgroups that share keys land on the same XCD (the dispatcher deals
 //     consecutive ids out in turn), latest = longest query tiles first.
 
@@ -91,13 +94,14 @@ DEVINL int fp_kswz(int key) { return D >= 128 ? key & 15 : (key >> 1) & 7; }
 template <int D>
 DEVINL int fp_vswz(int key) { return D >= 128 ? (key & 7) << 1 : ((key >> 1) & 3) << 1; }
 
-template <int D, int HP, int WR, int KT, int MINW, bool CAP>
+template <int D, int HP, int WR, int KT, int MINW, bool CAP, bool PAGED>
 __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
     __hip_bfloat16* __restrict__ out, long o_stride,
     const __hip_bfloat16* __restrict__ q, long q_stride,
     const __hip_bfloat16* __restrict__ k, long k_stride,
     const __hip_bfloat16* __restrict__ v, long v_stride,
-    const int* __restrict__ cu_q, const int* __restrict__ cu_k, int B, int H, int KVH,
+    const int* __restrict__ cu_q, const int* __restrict__ cu_k,
+    const int* __restrict__ block_tables, int bt_stride, int bs_shift, int B, int H, int KVH,
     int window, float scale_log2, float cap_log2, float cap_in, int n_qt) {
   constexpr int NW = HP * WR, QT = 32 * WR, NT = KT / 32;
   constexpr int KS = D / 16, DT = D / 32, GPR = D / 8;
@@ -152,23 +156,47 @@ __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
   const int skey = w * KPL + lane / GPR;
   const int kgran = ((lane % GPR) ^ fp_kswz<D>(skey)) << 3;
   const int vgran = ((lane % GPR) ^ fp_vswz<D>(skey)) << 3;
-  const unsigned koff = ((unsigned)skey * (unsigned)k_stride + kgran) * 2;
-  const unsigned voff = ((unsigned)skey * (unsigned)v_stride + vgran) * 2;
-  const __hip_bfloat16* kb = k + (long)k0 * k_stride + (long)kvh * D;
-  const __hip_bfloat16* vb = v + (long)k0 * v_stride + (long)kvh * D;
+  constexpr int NJ = NI / NW;                          // a wave's K loads per tile
+  const int lrow = PAGED ? lane / GPR : skey;          // row that the lane's offset counts
+  const unsigned krow = PAGED ? D : (unsigned)k_stride, vrow = PAGED ? D : (unsigned)v_stride;
+  const unsigned koff = ((unsigned)lrow * krow + kgran) * 2;
+  const unsigned voff = ((unsigned)lrow * vrow + vgran) * 2;
+  const __hip_bfloat16* kb = PAGED ? k : k + (long)k0 * k_stride + (long)kvh * D;
+  const __hip_bfloat16* vb = PAGED ? v : v + (long)k0 * v_stride + (long)kvh * D;
+  // Paged: a load's rows lie in one cache block (blocks hold 16 or 32 keys); its id
+  // is read a tile ahead. Rows past the end repeat the last one, masked below.
+  const int* bt = PAGED ? block_tables + (long)b * bt_stride : nullptr;
+  const int bs_mask = (1 << bs_shift) - 1;
+  int bid[NJ];
+  auto blocks = [&](int kt) {
+    if constexpr (PAGED)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        bid[j] = bt[__builtin_amdgcn_readfirstlane(
+            min(kt + j * STEP + w * KPL, nk - 1) >> bs_shift)];
+  };
   auto fetch = [&](int kt, bool is_v, short* dst) {
     const bool whole = kt + KT <= nk;
-    const long stride = is_v ? v_stride : k_stride;
 #pragma unroll
-    for (int j = 0; j < NI / NW; ++j) {
-      const int first = kt + j * STEP;                 // row of this wave's key 0
-      const __hip_bfloat16* base = (is_v ? vb : kb) + (long)first * stride;
+    for (int j = 0; j < NJ; ++j) {
       short* const to = dst + (w + j * NW) * 512;
-      if (whole) {
-        glds16_at(base, is_v ? voff : koff, to);
-      } else {                                         // rows past the end: masked below
-        const int row = min(first + skey, nk - 1) - first;
-        glds16(base + (long)row * stride + (is_v ? vgran : kgran), to);
+      const int gran = is_v ? vgran : kgran;
+      if constexpr (PAGED) {
+        const int first = kt + j * STEP + w * KPL;
+        const __hip_bfloat16* base =
+            (is_v ? vb : kb) + (((long)bid[j] * KVH + kvh) << bs_shift) * D;
+        if (whole)
+          glds16_at(base + (first & bs_mask) * D, is_v ? voff : koff, to);
+        else
+          glds16(base + (min(first + lrow, nk - 1) & bs_mask) * D + gran, to);
+      } else {
+        const int first = kt + j * STEP;               // row of the workgroup's key 0
+        const long stride = is_v ? v_stride : k_stride;
+        const __hip_bfloat16* base = (is_v ? vb : kb) + (long)first * stride;
+        if (whole)
+          glds16_at(base, is_v ? voff : koff, to);
+        else
+          glds16(base + (long)(min(first + skey, nk - 1) - first) * stride + gran, to);
       }
     }
   };
@@ -188,8 +216,10 @@ __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
 
   const int kt0 = window > 0 ? max(0, pos0 - window + 1) / KT * KT : 0;
   if (kt0 <= pos_last) {
+    blocks(kt0);
     fetch(kt0, false, lds);
     fetch(kt0, true, lds + KT * D);
+    blocks(kt0 + KT);
   }
   int cur = 0;
   for (int kt = kt0; kt <= pos_last; kt += KT, cur ^= 1) {
@@ -200,6 +230,7 @@ __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
       short* const next = lds + (cur ^ 1) * (2 * KT * D);
       fetch(kt + KT, false, next);
       fetch(kt + KT, true, next + KT * D);
+      blocks(kt + 2 * KT);
     }
     if (idle || kt > wave_last || kt + KT - 1 < wave_lo) continue;
 

@@ -337,6 +337,43 @@ class TestPrefillRanges:
         assert_close_to_f32_ref(out.cpu(), ref, 5 * 2 ** -9, 2 ** -8)
 
 
+class TestPagedPrefill:
+    """The prompt kernel on cache blocks gives what it gives on packed rows, bit for
+    bit: the same tiles, whatever the blocks' order and the rows past the end hold."""
+
+    @pytest.mark.parametrize("D,H,KVH,BS", [(64, 4, 2, 16), (64, 3, 3, 32), (128, 6, 2, 16),
+                                            (128, 2, 2, 32), (256, 4, 2, 16), (256, 3, 1, 32)])
+    @pytest.mark.parametrize("window,softcap", [(0, 0.0), (70, 30.0)])
+    def test_equals_packed(self, D, H, KVH, BS, window, softcap):
+        lens = [1, 33, 128, 200, 16]
+        lens_k = [1, 70, 128, 431, 516]
+        cu, cu_k = (torch.tensor([0] + list(torch.tensor(x).cumsum(0)), dtype=torch.int32,
+                                 device=DEV) for x in (lens, lens_k))
+        nb = sum(-(-n // BS) for n in lens_k)
+        kc, vc = (torch.randn(nb + 2, KVH, BS, D, device=DEV, dtype=torch.bfloat16)
+                  for _ in range(2))
+        kc[-1] = vc[-1] = float("nan")                        # never to be read
+        ids = torch.randperm(nb) + 1
+        kc[0] = vc[0] = float("nan")
+        bt = torch.full((len(lens), 40), nb + 1, dtype=torch.int32)
+        rows, at = [], 0
+        for b, n in enumerate(lens_k):
+            m = -(-n // BS)
+            bt[b, :m] = ids[at:at + m].int()
+            rows += [(int(ids[at + j // BS]), j % BS) for j in range(n)]
+            if n % BS:                                        # unwritten rows of the last block
+                kc[ids[at + m - 1], :, n % BS:] = float("nan")
+                vc[ids[at + m - 1], :, n % BS:] = float("nan")
+            at += m
+        blk, off = (torch.tensor(x, device=DEV) for x in zip(*rows))
+        q = torch.randn(sum(lens), H, D, device=DEV, dtype=torch.bfloat16)
+        args = (max(lens), D ** -0.5, softcap, window)
+        want = ops.varlen_prefill_attention(q, kc[blk, :, off], vc[blk, :, off], cu, *args,
+                                            cu_seqlens_k=cu_k)
+        got = ops.paged_prefill_attention(q, kc, vc, bt.to(DEV), cu, cu_k, *args)
+        assert torch.isfinite(got).all() and torch.equal(got, want)
+
+
 class TestFewRowsLinear:
     """Streaming projections of up to 16 rows: each split of K (rows <= 4, 8, 16;
     large matrices), chunk remainders, norm, bias, activation and residual."""
