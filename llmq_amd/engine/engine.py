@@ -416,8 +416,10 @@ class LLMEngine:
                 offs[s.request_id] = (at, at + len(wants[s.request_id]))
                 at += len(wants[s.request_id])
             order = [i for ent in entries for i in range(*offs[ent["id"]])]
-            out = logits[torch.tensor(order, dtype=torch.long, device=logits.device)] \
-                if order else logits[:0]
+            out = logits
+            if order != list(range(logits.shape[0])):
+                out = logits[torch.tensor(order, dtype=torch.long, device=logits.device)] \
+                    if order else logits[:0]
         for rid in end or []:
             seq = self._seqs.pop(rid, None)
             if seq is not None:

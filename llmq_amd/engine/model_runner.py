@@ -173,82 +173,115 @@ class ModelRunner:
 
     # -- prefill / mixed (chunk-aware, eager) ----------------------------
 
-    def _build_prefill_meta(self, pseqs, chunks, dev) -> tuple:
+    def _stage(self, arrays: List[np.ndarray]) -> List[torch.Tensor]:
+        """Small int arrays to the device in ONE copy that does not wait for the
+        stream (a copy out of pageable memory would, once per array)."""
+        at, spans = 0, []
+        for a in arrays:
+            words = (a.size * a.itemsize + 7) // 8
+            spans.append((at, words))
+            at += words
+        on_gpu = self.device.type == "cuda"
+        host = torch.empty(at, dtype=torch.long, pin_memory=on_gpu)
+        flat = host.numpy()
+        for a, (first, words) in zip(arrays, spans):
+            flat[first:first + words].view(a.dtype)[:a.size] = a.reshape(-1)
+        # the pinned block returns to torch's pool once the copy's stream has passed it
+        device = host.to(self.device, non_blocking=True) if on_gpu else host
+        kinds = {np.dtype(np.int64): torch.long, np.dtype(np.int32): torch.int32}
+        return [device[first:first + words].view(kinds[a.dtype])[:a.size].view(a.shape)
+                for a, (first, words) in zip(arrays, spans)]
+
+    def _build_prefill_meta(self, pseqs, chunks, extra=()) -> tuple:
         """Packed ids/pos/slots for the prefill segment + optional gather
-        plan for chunk continuations. Returns (ids, pos, slots, meta,
-        rel_last_idx) where rel_last_idx are within-segment row indices of
-        FINAL chunks (the rows that sample)."""
+        plan for chunk continuations. Returns (ids, pos, slots, meta, extra)
+        on the device; ``extra`` (int arrays of the caller) travels with them."""
         bs = self.block_size
-        ids: List[int] = []
-        pos: List[int] = []
-        slots: List[int] = []
-        cu = [0]
-        cu_k = [0]
-        rel_last: List[int] = []
+        lens = np.array([e - st for st, e in chunks], dtype=np.int64)
+        cu = np.zeros(len(chunks) + 1, dtype=np.int32)
+        cu[1:] = np.cumsum(lens)
+        ids = np.empty(int(cu[-1]), dtype=np.int64)
+        pos = np.empty_like(ids)
+        slots = np.empty_like(ids)
         continued = (not self.paged_prefill) and any(start > 0 for (start, _e) in chunks)
         any_chunk = continued and not self.paged_portions
-        g_blocks: List[int] = []
-        g_offs: List[int] = []
-        past_dst: List[int] = []
-        fresh_dst: List[int] = []
+        past_blocks, past_offs, past_dst, fresh_dst = [], [], [], []
         krow = 0
-        for seq, (start, end) in zip(pseqs, chunks):
-            n = end - start
-            ids.extend(seq.token_ids[start:end])
-            pos.extend(range(start, end))
-            bt = seq.block_table
-            slots.extend(bt[p // bs] * bs + (p % bs) for p in range(start, end))
-            if end == seq.num_tokens:
-                rel_last.append(cu[-1] + n - 1)
-            cu.append(cu[-1] + n)
-            if any_chunk:
-                for p in range(start):  # past rows gathered from the cache
-                    g_blocks.append(bt[p // bs])
-                    g_offs.append(p % bs)
-                    past_dst.append(krow)
-                    krow += 1
-                for i in range(cu[-2], cu[-1]):
-                    fresh_dst.append(krow)
-                    krow += 1
-            cu_k.append(cu_k[-1] + end)  # keys = full context so far
-        slot_mapping = torch.tensor(slots, dtype=torch.long, device=dev)
+        for i, (seq, (start, end)) in enumerate(zip(pseqs, chunks)):
+            rows = slice(int(cu[i]), int(cu[i + 1]))
+            bt = np.asarray(seq.block_table, dtype=np.int64)
+            p = np.arange(start, end, dtype=np.int64)
+            ids[rows] = seq.token_ids[start:end]
+            pos[rows] = p
+            slots[rows] = bt[p // bs] * bs + p % bs
+            if any_chunk:  # past rows gathered from the cache
+                past = np.arange(start, dtype=np.int64)
+                past_blocks.append(bt[past // bs])
+                past_offs.append(past % bs)
+                past_dst.append(krow + past)
+                fresh_dst.append(krow + p)
+                krow += end  # keys = full context so far
+        cu_k = np.zeros_like(cu)
+        cu_k[1:] = np.cumsum([e for _st, e in chunks])
+        arrays = [ids, pos, slots, cu]
+        names = ["ids", "pos", "slots", "cu"]
+
+        def add(name, a):
+            names.append(name)
+            arrays.append(a)
+
+        if any_chunk:
+            add("blocks", np.concatenate(past_blocks))
+            add("offs", np.concatenate(past_offs))
+            add("past_dst", np.concatenate(past_dst))
+            add("fresh_dst", np.concatenate(fresh_dst))
+        if continued:
+            add("cu_k", cu_k)
+        if self.paged_prefill or (continued and self.paged_portions):
+            add("tables", self._block_tables(pseqs))
+        if self.paged_prefill:
+            add("q_start", np.array([st for (st, _e) in chunks], dtype=np.int32))
+        if self.recurrent is not None:
+            add("state_slots", np.array([s.state_slot for s in pseqs], dtype=np.int32))
+            add("fresh", np.array([int(st == 0) for (st, _e) in chunks], dtype=np.int32))
+        staged = self._stage(arrays + list(extra))
+        t = dict(zip(names, staged))
         gather = None
         if any_chunk:
             gather = ChunkGather(
-                cu_seqlens_k=torch.tensor(cu_k, dtype=torch.int32, device=dev),
-                blocks=torch.tensor(g_blocks, dtype=torch.long, device=dev),
-                offs=torch.tensor(g_offs, dtype=torch.long, device=dev),
-                past_dst=torch.tensor(past_dst, dtype=torch.long, device=dev),
-                fresh_dst=torch.tensor(fresh_dst, dtype=torch.long, device=dev),
-                total_k=krow,
+                cu_seqlens_k=t["cu_k"], blocks=t["blocks"], offs=t["offs"],
+                past_dst=t["past_dst"], fresh_dst=t["fresh_dst"], total_k=krow,
             )
         meta = PrefillMeta(
-            cu_seqlens=torch.tensor(cu, dtype=torch.int32, device=dev),
-            max_seqlen=max(e - st for (st, e) in chunks),
-            slot_mapping=slot_mapping,
+            cu_seqlens=t["cu"],
+            max_seqlen=int(lens.max()),
+            slot_mapping=t["slots"],
             gather=gather,
+            block_tables=t.get("tables"),
+            cu_seqlens_k=None if any_chunk else t.get("cu_k"),
+            q_start=t.get("q_start"),
         )
-        if continued and self.paged_portions:
-            meta.block_tables = self._block_table_tensor(pseqs, dev)
-            meta.cu_seqlens_k = torch.tensor(cu_k, dtype=torch.int32, device=dev)
-        if self.paged_prefill:
-            meta.block_tables = self._block_table_tensor(pseqs, dev)
-            meta.q_start = torch.tensor([st for (st, _e) in chunks], dtype=torch.int32, device=dev)
         if self.recurrent is not None:
-            meta.recurrent = RecurrentMeta(
-                cu=meta.cu_seqlens,
-                slots=torch.tensor([s.state_slot for s in pseqs], dtype=torch.int32, device=dev),
-                fresh=torch.tensor([int(st == 0) for (st, _e) in chunks], dtype=torch.int32,
-                                   device=dev),
-            )
-        return ids, pos, slot_mapping, meta, rel_last
+            meta.recurrent = RecurrentMeta(cu=t["cu"], slots=t["state_slots"], fresh=t["fresh"])
+        return t["ids"], t["pos"], t["slots"], meta, staged[len(names):]
 
-    def _block_table_tensor(self, seqs, dev) -> torch.Tensor:
+    @staticmethod
+    def _final_rows(chunks, pseqs) -> List[int]:
+        """Within-segment last rows of FINAL chunks (the rows that sample)."""
+        rows, at = [], 0
+        for seq, (start, end) in zip(pseqs, chunks):
+            at += end - start
+            if end == seq.num_tokens:
+                rows.append(at - 1)
+        return rows
+
+    @staticmethod
+    def _block_tables(seqs) -> np.ndarray:
         width = max(1, max(len(s.block_table) for s in seqs))
-        bt_np = np.zeros((len(seqs), width), dtype=np.int32)
+        out = np.zeros((len(seqs), width), dtype=np.int32)
         for i, s in enumerate(seqs):
-            bt_np[i, : len(s.block_table)] = s.block_table
-        return torch.from_numpy(bt_np).to(dev)
+            out[i, : len(s.block_table)] = s.block_table
+        return out
 
     def _decode_recurrent_meta(self, seqs, dev):
         if self.recurrent is None:
@@ -260,14 +293,18 @@ class ModelRunner:
             fresh=torch.zeros(n, dtype=torch.int32, device=dev),
         )
 
-    def _logits_at(self, hidden: torch.Tensor, rows: List[int]) -> torch.Tensor:
+    def _logits_at(self, hidden: torch.Tensor, rows: List[int],
+                   idx: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Logits of the given rows of a step (teacher-forced replay: the
-        caller asks for positions instead of sampling)."""
+        caller asks for positions instead of sampling). idx: rows, staged
+        with the step's other indices."""
         if not rows:
             return torch.empty(0, self.model.spec.vocab_size, dtype=torch.float32,
                                device=hidden.device)
-        idx = torch.tensor(rows, dtype=torch.long, device=hidden.device)
-        return self.model.compute_logits(hidden[idx]).float()
+        if rows != list(range(hidden.shape[0])):
+            hidden = hidden[self._stage([np.array(rows, dtype=np.int64)])[0]
+                            if idx is None else idx]
+        return self.model.compute_logits(hidden).float()
 
     @torch.no_grad()
     def execute_prefill(self, seqs: List[Sequence], chunks=None, buf_name: str = "main",
@@ -278,22 +315,22 @@ class ModelRunner:
         sampled: the logits of those rows are returned, in that order."""
         if chunks is None:
             chunks = [(0, s.num_tokens) for s in seqs]
-        dev = self.device
-        ids, pos, slot_mapping, meta, rel_last = self._build_prefill_meta(
-            seqs, chunks, dev
+        if want is None:
+            rows = self._final_rows(chunks, seqs)
+        else:
+            rows, at = [], 0
+            for (st, e), ws in zip(chunks, want):
+                rows += [at + w for w in ws]
+                at += e - st
+        input_ids, positions, _slots, meta, (idx,) = self._build_prefill_meta(
+            seqs, chunks, extra=[np.array(rows, dtype=np.int64)]
         )
-        input_ids = torch.tensor(ids, dtype=torch.long, device=dev)
-        positions = torch.tensor(pos, dtype=torch.long, device=dev)
         hidden = self.model.forward(input_ids, positions, self.kv_cache, meta)
         if want is not None:
-            cu = [0]
-            for st, e in chunks:
-                cu.append(cu[-1] + e - st)
-            return self._logits_at(hidden, [cu[b] + w for b, ws in enumerate(want) for w in ws])
-        if not rel_last:
-            return torch.empty(0, dtype=torch.long, device=dev)
-        last_hidden = hidden[torch.tensor(rel_last, dtype=torch.long, device=dev)]
-        logits = self.model.compute_logits(last_hidden)
+            return self._logits_at(hidden, rows, idx)
+        if not rows:
+            return torch.empty(0, dtype=torch.long, device=self.device)
+        logits = self.model.compute_logits(hidden[idx])
         sample_seqs = [s for s, (st, e) in zip(seqs, chunks) if e == s.num_tokens]
         return self._sample(logits, sample_seqs, buf_name)
 
@@ -312,30 +349,21 @@ class ModelRunner:
         bs = self.block_size
         nd = len(dseqs)
 
-        ids = [s.token_ids[-1] for s in dseqs]
-        pos = [s.num_tokens - 1 for s in dseqs]
-        slots = [s.block_table[p // bs] * bs + (p % bs) for s, p in zip(dseqs, pos)]
-        ctx = [s.num_tokens for s in dseqs]
-        p_ids, p_pos, p_slots, pmeta, rel_last = self._build_prefill_meta(
-            pseqs, chunks, dev
-        )
-        ids.extend(p_ids)
-        pos.extend(p_pos)
-
-        block_tables = torch.zeros(
-            nd, max(len(s.block_table) for s in dseqs), dtype=torch.int32, device=dev
-        )
-        bt_np = np.zeros(tuple(block_tables.shape), dtype=np.int32)
-        for i, s in enumerate(dseqs):
-            bt_np[i, : len(s.block_table)] = s.block_table
-        block_tables.copy_(torch.from_numpy(bt_np))
-        d_slots = torch.tensor(slots, dtype=torch.long, device=dev)
+        pos = np.array([s.num_tokens - 1 for s in dseqs], dtype=np.int64)
+        ids = np.array([s.token_ids[-1] for s in dseqs], dtype=np.int64)
+        slots = np.array([s.block_table[p // bs] * bs + (p % bs)
+                          for s, p in zip(dseqs, pos.tolist())], dtype=np.int64)
+        ctx = (pos + 1).astype(np.int32)
+        rel_last = self._final_rows(chunks, pseqs)
+        p_ids, p_pos, p_slots, pmeta, (d_ids, d_pos, d_slots, d_ctx, tables) = \
+            self._build_prefill_meta(
+                pseqs, chunks, extra=[ids, pos, slots, ctx, self._block_tables(dseqs)])
         slot_mapping = torch.cat([d_slots, p_slots])
         meta = MixedMeta(
             n_decode=nd,
             decode=DecodeMeta(
-                block_tables=block_tables,
-                context_lens=torch.tensor(ctx, dtype=torch.int32, device=dev),
+                block_tables=tables,
+                context_lens=d_ctx,
                 slot_mapping=d_slots,
             ),
             prefill=pmeta,
@@ -349,8 +377,8 @@ class ModelRunner:
                 slots=torch.cat([dr.slots, pr.slots]),
                 fresh=torch.cat([dr.fresh, pr.fresh]),
             )
-        input_ids = torch.tensor(ids, dtype=torch.long, device=dev)
-        positions = torch.tensor(pos, dtype=torch.long, device=dev)
+        input_ids = torch.cat([d_ids, p_ids])
+        positions = torch.cat([d_pos, p_pos])
         hidden = self.model.forward(input_ids, positions, self.kv_cache, meta)
         if want is not None:
             cu = [nd]

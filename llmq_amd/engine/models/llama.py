@@ -269,6 +269,25 @@ class CausalLM:
             )
         return attn.reshape(T, self.q_size)
 
+    def _prompt_layers(self, h, residual, positions, kv_cache, meta) -> torch.Tensor:
+        """The layers of a prompt step, launched from native code."""
+        s = self.spec
+        weights: List[torch.Tensor] = []
+        for i, lw in enumerate(self.layers):
+            w_next = self.layers[i + 1].input_norm if i + 1 < len(self.layers) else self.final_norm
+            weights += (lw.qkv, lw.o, lw.gate_up, lw.down, lw.pre_mlp_norm, w_next)
+            if s.post_norms:
+                weights += (lw.post_attn_norm, lw.post_mlp_norm)
+        return ops.prompt_layers(
+            h, residual, weights, [lw.qkv_bias for lw in self.layers] if s.qkv_bias else [],
+            kv_cache.k, kv_cache.v, positions, self.rope_cache, meta.slot_mapping,
+            meta.cu_seqlens, meta.block_tables, meta.cu_seqlens_k, meta.max_seqlen, s.head_dim,
+            s.scale, s.attn_softcap,
+            [s.sliding_window if s.layer_uses_sliding_window(i) else 0
+             for i in range(len(self.layers))],
+            s.rms_eps, self.norm_offset, s.gelu, s.post_norms,
+        )
+
     def _forward_few_rows(self, residual, positions, kv_cache, meta) -> torch.Tensor:
         """The layers for up to ops.FEW_ROWS rows (a decode step of few
         sequences): norms, activation and residual addition ride on the
@@ -317,6 +336,9 @@ class CausalLM:
             return self._forward_few_rows(x, positions, kv_cache, meta)
         residual = x
         h = self._norm(x, self.layers[0].input_norm)
+        if (tp is None and x.is_cuda and meta.is_prefill and meta.gather is None
+                and not _USE_SKINNY_GEMM):
+            return self._prompt_layers(h, residual, positions, kv_cache, meta)
         n_layers = len(self.layers)
         for i, lw in enumerate(self.layers):
             # ---- attention block (h = normed input, set by the previous

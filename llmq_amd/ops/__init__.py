@@ -252,6 +252,19 @@ def paged_prefill_attention(
     return out
 
 
+def prompt_layers(h, residual, weights, biases, k_caches, v_caches, positions, cos_sin, slots,
+                  cu_seqlens, block_tables, cu_seqlens_k, max_seqlen: int, head_dim: int,
+                  scale: float, softcap: float, windows, eps: float, offset: float, gelu: bool,
+                  post_norms: bool) -> torch.Tensor:
+    """All layers of a packed prompt step on the GPU in one call: the launches of
+    the per-layer code (projections, rope_and_cache, prompt attention, norms,
+    activation) without its crossings from Python. Returns the final normed rows."""
+    assert _use_hip(h)
+    return _EXT.prompt_layers(h, residual, weights, biases, k_caches, v_caches, positions, cos_sin,
+                              slots, cu_seqlens, block_tables, cu_seqlens_k, int(max_seqlen),
+                              head_dim, scale, softcap, windows, eps, offset, gelu, post_norms)
+
+
 # ---------------------------------------------------------- skinny GEMM --
 
 

@@ -605,6 +605,60 @@ void stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
   else epilogue.template operator()<false>();
 }
 
+// ------------------------------------------------------ prompt steps, whole --
+
+// All layers of a packed prompt step (no portion gathered into packed rows): the
+// same calls that the engine's per-layer code makes, in one crossing from Python.
+// A layer's weights: qkv, o, gate_up, down, pre-MLP norm, next layer's input norm
+// (or the final one), and with sandwich norms the post-attention and post-MLP
+// ones. h is the normed input of layer 0; returns the final normed rows.
+at::Tensor prompt_layers(at::Tensor h, at::Tensor residual, at::TensorList weights,
+                         at::TensorList biases, at::TensorList k_caches,
+                         at::TensorList v_caches, at::Tensor positions, at::Tensor cos_sin,
+                         at::Tensor slots, at::Tensor cu_seqlens,
+                         c10::optional<at::Tensor> block_tables,
+                         c10::optional<at::Tensor> cu_seqlens_k, long max_seqlen,
+                         long head_dim, double scale, double softcap, at::IntArrayRef windows,
+                         double eps, double offset, bool gelu, bool post_norms) {
+  CHECK_GPU(h);
+  const size_t per = post_norms ? 8 : 6, layers = k_caches.size();
+  TORCH_CHECK(weights.size() == per * layers && v_caches.size() == layers &&
+                  windows.size() == layers && (biases.empty() || biases.size() == layers),
+              "one entry per layer");
+  const long T = h.size(0);
+  for (size_t i = 0; i < layers; ++i) {
+    const at::Tensor* w = &weights[per * i];
+    const at::Tensor qkv = at::linear(
+        h, w[0], biases.empty() ? c10::optional<at::Tensor>() : c10::make_optional(biases[i]));
+    const long kv_heads = k_caches[i].size(1);
+    const long heads = qkv.size(1) / head_dim - 2 * kv_heads;
+    auto part = [&](long first, long n) {
+      return qkv.narrow(1, first * head_dim, n * head_dim).view({T, n, head_dim});
+    };
+    const at::Tensor q = part(0, heads), k = part(heads, kv_heads),
+                     v = part(heads + kv_heads, kv_heads);
+    rope_and_cache(q, k, v, k_caches[i], v_caches[i], positions, cos_sin, slots);
+    at::Tensor attn = at::empty({T, heads, head_dim}, qkv.options());
+    if (cu_seqlens_k.has_value())
+      paged_prefill_attention(attn, q, k_caches[i], v_caches[i], *block_tables, cu_seqlens,
+                              *cu_seqlens_k, max_seqlen, scale, softcap, windows[i]);
+    else
+      varlen_prefill_attention(attn, q, k, v, cu_seqlens, cu_seqlens, max_seqlen, scale, softcap,
+                               windows[i]);
+    h = at::linear(attn.view({T, heads * head_dim}), w[1]);
+    if (post_norms) norm_add_norm(h, residual, w[6], w[4], eps, offset);
+    else fused_add_rmsnorm(h, residual, w[4], eps, offset);
+    const at::Tensor gate_up = at::linear(h, w[2]);
+    at::Tensor act = at::empty({T, gate_up.size(1) / 2}, gate_up.options());
+    if (gelu) gelu_tanh_and_mul(act, gate_up);
+    else silu_and_mul(act, gate_up);
+    h = at::linear(act, w[3]);
+    if (post_norms) norm_add_norm(h, residual, w[7], w[5], eps, offset);
+    else fused_add_rmsnorm(h, residual, w[5], eps, offset);
+  }
+  return h;
+}
+
 // ------------------------------------------------------------- sampling --
 
 // Chunks of a logits row: enough workgroups to fill the chip at few rows, whole
@@ -710,6 +764,7 @@ TORCH_LIBRARY(llmq_amd, m) {
   m.def("paged_decode_attention(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor context_lens, float scale, float softcap, int window) -> ()");
   m.def("varlen_prefill_attention(Tensor(a!) out, Tensor q, Tensor k, Tensor v, Tensor cu_seqlens, Tensor cu_seqlens_k, int max_seqlen, float scale, float softcap, int window) -> ()");
   m.def("paged_prefill_attention(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor cu_seqlens, Tensor cu_seqlens_k, int max_seqlen, float scale, float softcap, int window) -> ()");
+  m.def("prompt_layers(Tensor h, Tensor(a!) residual, Tensor[] weights, Tensor[] biases, Tensor[] k_caches, Tensor[] v_caches, Tensor positions, Tensor cos_sin, Tensor slots, Tensor cu_seqlens, Tensor? block_tables, Tensor? cu_seqlens_k, int max_seqlen, int head_dim, float scale, float softcap, int[] windows, float eps, float offset, bool gelu, bool post_norms) -> Tensor");
   m.def("sample_gumbel_argmax(Tensor(a!) out, Tensor(b!) keys, Tensor logits, Tensor temps, Tensor req_seeds, Tensor req_pos, int seed, int step, Tensor? bounds=None) -> ()");
   m.def("topk_topp_bound(Tensor(a!) out_bound, Tensor logits, Tensor temps, Tensor top_ps, Tensor top_ks) -> ()");
   m.def("softcap_logits(Tensor(a!) out, Tensor input, float cap) -> ()");
@@ -729,6 +784,7 @@ TORCH_LIBRARY_IMPL(llmq_amd, CUDA, m) {
   m.impl("paged_decode_attention", &paged_decode_attention);
   m.impl("varlen_prefill_attention", &varlen_prefill_attention);
   m.impl("paged_prefill_attention", &paged_prefill_attention);
+  m.impl("prompt_layers", &prompt_layers);
   m.impl("sample_gumbel_argmax", &sample_gumbel_argmax);
   m.impl("topk_topp_bound", &topk_topp_bound);
   m.impl("softcap_logits", &softcap_logits);
