@@ -234,19 +234,21 @@ class CausalLM:
             s.attn_softcap, window, cu_seqlens_k=g.cu_seqlens_k,
         )
 
-    def _attention(self, i: int, qkv, positions, kv_cache, meta) -> torch.Tensor:
-        """Layer i between its projections: RoPE, cache write, attention of each
-        segment. qkv [T, q+2kv] -> [T, q]."""
+    def _attention(self, i: int, qkv, positions, kv_cache, meta,
+                   cached: bool = False) -> torch.Tensor:
+        """Layer i between its projections: RoPE, cache write (unless done,
+        ``cached``), attention of each segment. qkv [T, q+2kv] -> [T, q]."""
         s = self.spec
         T = qkv.shape[0]
         q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
         q = q.view(T, self.heads, s.head_dim)
         k = k.view(T, self.kv_heads, s.head_dim)
         v = v.view(T, self.kv_heads, s.head_dim)
-        ops.rope_and_cache(
-            q, k, v, kv_cache.k[i], kv_cache.v[i], positions,
-            self.rope_cache, meta.slot_mapping,
-        )
+        if not cached:
+            ops.rope_and_cache(
+                q, k, v, kv_cache.k[i], kv_cache.v[i], positions,
+                self.rope_cache, meta.slot_mapping,
+            )
         window = s.sliding_window if s.layer_uses_sliding_window(i) else 0
         if meta.is_prefill:
             attn = self._prefill_attn(q, k, v, meta, kv_cache, i, window)
@@ -268,6 +270,28 @@ class CausalLM:
                 meta.context_lens, s.scale, s.attn_softcap, window,
             )
         return attn.reshape(T, self.q_size)
+
+    def _forward_slabs(self, h, residual, positions, kv_cache, meta) -> torch.Tensor:
+        """The layers for up to ops.SLAB_ROWS rows (an ordinary decode step):
+        streaming products whose partial sums the norms and the rotation add up."""
+        s = self.spec
+        for i, lw in enumerate(self.layers):
+            w_next = self.layers[i + 1].input_norm if i + 1 < len(self.layers) else self.final_norm
+            qkv = ops.slab_rope_cache(
+                ops.slab_linear(h, lw.qkv), lw.qkv_bias, kv_cache.k[i], kv_cache.v[i], positions,
+                self.rope_cache, meta.slot_mapping,
+            )
+            attn = self._attention(i, qkv, positions, kv_cache, meta, cached=True)
+            h = ops.slab_add_norm(ops.slab_linear(attn, lw.o), residual, lw.post_attn_norm,
+                                  lw.pre_mlp_norm, s.rms_eps, self.norm_offset)
+            if ops.slab_act_ok(h, lw.gate_up):
+                act = ops.slab_act_linear(h, lw.gate_up, s.gelu)
+            else:
+                gate_up = _proj(h, lw.gate_up)
+                act = ops.gelu_tanh_and_mul(gate_up) if s.gelu else ops.silu_and_mul(gate_up)
+            h = ops.slab_add_norm(ops.slab_linear(act, lw.down), residual, lw.post_mlp_norm,
+                                  w_next, s.rms_eps, self.norm_offset)
+        return h
 
     def _prompt_layers(self, h, residual, positions, kv_cache, meta) -> torch.Tensor:
         """The layers of a prompt step, launched from native code."""
@@ -339,6 +363,10 @@ class CausalLM:
         if (tp is None and x.is_cuda and meta.is_prefill and meta.gather is None
                 and not _USE_SKINNY_GEMM):
             return self._prompt_layers(h, residual, positions, kv_cache, meta)
+        if (tp is None and kv_cache.k[0].dtype in (torch.bfloat16, torch.float8_e4m3fn)
+                and ops.slab_ok(h, (l0.qkv, l0.o, l0.gate_up, l0.down), s.hidden_size)
+                and not _USE_SKINNY_GEMM):
+            return self._forward_slabs(h, residual, positions, kv_cache, meta)
         n_layers = len(self.layers)
         for i, lw in enumerate(self.layers):
             # ---- attention block (h = normed input, set by the previous

@@ -335,6 +335,54 @@ def few_rows_linear(
     return y if residual is None else residual.add_(y)
 
 
+# --------------------------------------------- projections, 17 to 128 rows --
+# The product stays as fp32 partial sums ("slabs" [parts, M, N]) that the next
+# kernel adds up: norm and residual, or rotation and cache write.
+
+SLAB_ROWS = 128
+
+
+def slab_ok(x: torch.Tensor, weights, hidden: int) -> bool:
+    """Whether the slab kernels take these rows and weights [N, K]."""
+    return (
+        x.is_cuda and x.dim() == 2 and FEW_ROWS < x.shape[0] <= SLAB_ROWS
+        and x.dtype == torch.bfloat16 and x.is_contiguous() and hidden <= 8192
+        and all(w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] % 128 == 0
+                and w.shape[0] % 64 == 0 and w.data_ptr() % 16 == 0 for w in weights)
+    )
+
+
+def slab_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x @ w.T as fp32 slabs [parts, M, N] whose sum is the product."""
+    assert _use_hip(x)
+    return _EXT.slab_linear(x, w)
+
+
+def slab_act_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether slab_act_linear beats the library's product and an activation."""
+    return x.shape[0] <= 64 and w.numel() < 48 << 20
+
+
+def slab_act_linear(x: torch.Tensor, w: torch.Tensor, gelu: bool) -> torch.Tensor:
+    """act(x @ gate.T) * (x @ up.T), w = [gate | up] rows, SiLU or tanh-GELU."""
+    assert _use_hip(x)
+    return _EXT.slab_act_linear(x, w, bool(gelu))
+
+
+def slab_add_norm(slabs, residual, w_post, w, eps: float, offset: float) -> torch.Tensor:
+    """residual (in place) += the slabs' sum, RMS-normalised by w_post first
+    where given; returns rmsnorm(residual) by w."""
+    assert _use_hip(slabs)
+    return _EXT.slab_add_norm(slabs, residual, w_post, w, eps, offset)
+
+
+def slab_rope_cache(slabs, bias, k_cache, v_cache, positions, cos_sin, slots) -> torch.Tensor:
+    """bf16 q/k/v rows of the slabs' sum + bias, q and k rotated; k and v also
+    into the paged cache."""
+    assert _use_hip(slabs)
+    return _EXT.slab_rope_cache(slabs, bias, k_cache, v_cache, positions, cos_sin, slots)
+
+
 # ------------------------------------------------------------- sampling --
 
 

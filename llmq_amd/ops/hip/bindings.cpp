@@ -605,10 +605,155 @@ void stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
   else epilogue.template operator()<false>();
 }
 
+// ------------------------------------------- projections, 17 to 128 rows --
+
+bool slab_rows_ok(const at::Tensor& x, const at::Tensor& w) {
+  return x.dim() == 2 && w.dim() == 2 && x.size(0) > 16 && x.size(0) <= 128 &&
+         x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 &&
+         x.stride(1) == 1 && rows_start_on(x, 16) && w.is_contiguous() &&
+         reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 && x.size(1) == w.size(1) &&
+         w.size(1) % kSlabBK == 0 && w.size(1) > 0 && w.size(0) % 64 == 0;
+}
+
+// Parts of K: as many as keep 512 workgroups (two a CU) busy, two steps each at the
+// least. Measured (us): 64 rows, 2048 x 8192: 16 parts 12.7, 8 14.1, 4 20; 128 rows,
+// 3072 x 3072: 8 parts 13.9, 12 15.4, 4 14.4; 96 rows, 8192 x 3584: 4 parts 22.2,
+// 6 23.2, 3 25.3.
+int slab_parts(long N, long K) {
+  const long tiles = N / 64, steps = K / kSlabBK;
+  for (int s : {16, 12, 8, 6, 4, 3, 2})
+    if (s * tiles <= 512 && steps / s >= 2) return s;
+  return 1;
+}
+
+template <int EPI>
+void launch_slab_gemm(float* slabs, __hip_bfloat16* out, long out_stride, const at::Tensor& x,
+                      const at::Tensor& w, int parts) {
+  const int M = x.size(0), K = x.size(1), N = w.size(0);
+  const int steps = (K / kSlabBK + parts - 1) / parts;
+  auto go = [&]<int TM, int WK>() {
+    hipLaunchKernelGGL((slab_gemm_kernel<TM, WK, EPI>), dim3(N / 64, parts), dim3(256 * WK), 0,
+                       stream(), slabs, out, out_stride,
+                       reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()), x.stride(0),
+                       reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()), M, N, K, steps);
+  };
+  // Gates need whole sums: two groups of waves instead of parts (64 rows,
+  // 16384 x 2048: 20.8 us, one group 25.3).
+  constexpr int WK = EPI == kSlabSums ? 1 : 2;
+  const int tm = (M + 15) / 16;
+  if (tm <= 2) go.template operator()<2, WK>();
+  else if (tm == 3) go.template operator()<3, WK>();
+  else if (tm == 4) go.template operator()<4, WK>();
+  else if constexpr (EPI == kSlabSums) {
+    if (tm <= 6) go.template operator()<6, 1>();
+    else go.template operator()<8, 1>();
+  }
+}
+
+// x W^T as fp32 slabs [parts, M, N]; their sum is the product.
+at::Tensor slab_linear(const at::Tensor& x, const at::Tensor& w) {
+  CHECK_GPU(x);
+  TORCH_CHECK(slab_rows_ok(x, w),
+              "slab_linear: 17 to 128 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
+  const int parts = slab_parts(w.size(0), w.size(1));
+  at::Tensor slabs = at::empty({parts, x.size(0), w.size(0)}, x.options().dtype(at::kFloat));
+  launch_slab_gemm<kSlabSums>(slabs.data_ptr<float>(), nullptr, 0, x, w, parts);
+  return slabs;
+}
+
+// Whether gate and value rows are worth a product of their own with the activation
+// in it: from 48 M weights on the library's product and the activation are as fast
+// (48 rows, 28672 x 3584: 49.0 + 5.2 us against 53.5).
+bool slab_act_ok(const at::Tensor& x, const at::Tensor& w) {
+  return slab_rows_ok(x, w) && x.size(0) <= 64 && w.numel() < (48L << 20);
+}
+
+at::Tensor slab_act_linear(const at::Tensor& x, const at::Tensor& w, bool gelu) {
+  CHECK_GPU(x);
+  TORCH_CHECK(slab_rows_ok(x, w) && x.size(0) <= 64,
+              "slab_act_linear: 17 to 64 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
+  at::Tensor out = at::empty({x.size(0), w.size(0) / 2}, x.options());
+  auto* p = reinterpret_cast<__hip_bfloat16*>(out.data_ptr());
+  if (gelu) launch_slab_gemm<kSlabGelu>(nullptr, p, out.stride(0), x, w, 1);
+  else launch_slab_gemm<kSlabSilu>(nullptr, p, out.stride(0), x, w, 1);
+  return out;
+}
+
+void check_slabs(const at::Tensor& slabs) {
+  CHECK_GPU(slabs);
+  TORCH_CHECK(slabs.dim() == 3 && slabs.scalar_type() == at::kFloat && slabs.is_contiguous(),
+              "slabs must be contiguous fp32 [parts, M, N]");
+}
+
+// residual += sum of slabs (RMS-normalised by w_post first, where given); returns
+// rmsnorm(residual) by w.
+at::Tensor slab_add_norm(const at::Tensor& slabs, at::Tensor residual,
+                         c10::optional<at::Tensor> w_post, const at::Tensor& w, double eps,
+                         double offset) {
+  check_slabs(slabs);
+  const int S = slabs.size(0), M = slabs.size(1), N = slabs.size(2);
+  TORCH_CHECK(residual.is_contiguous() && residual.scalar_type() == at::kBFloat16 &&
+                  residual.numel() == (long)M * N && N % 4 == 0 && N <= 8192,
+              "residual must be contiguous bf16 [M, N], N a multiple of 4 up to 8192");
+  auto weights = [&](const at::Tensor& t) {
+    TORCH_CHECK(t.is_contiguous() && t.scalar_type() == at::kBFloat16 && t.numel() == N,
+                "norm weights must be bf16 [N]");
+    return reinterpret_cast<const __hip_bfloat16*>(t.data_ptr());
+  };
+  at::Tensor h = at::empty_like(residual);
+  auto go = [&]<bool POST>() {
+    const int threads = std::min(kSlabNT, (N / 4 + 63) / 64 * 64);
+    hipLaunchKernelGGL(slab_add_norm_kernel<POST>, dim3(M), dim3(threads), 0, stream(),
+                       reinterpret_cast<__hip_bfloat16*>(h.data_ptr()),
+                       reinterpret_cast<__hip_bfloat16*>(residual.data_ptr()),
+                       slabs.data_ptr<float>(), S, POST ? weights(*w_post) : nullptr, weights(w),
+                       M, N, (float)eps, (float)offset);
+  };
+  if (w_post.has_value() && w_post->defined()) go.template operator()<true>();
+  else go.template operator()<false>();
+  return h;
+}
+
+// bf16 rows [M, (heads + 2 kv heads) D] of the summed slabs + bias, q and k rotated;
+// k and v also into the paged cache.
+at::Tensor slab_rope_cache(const at::Tensor& slabs, c10::optional<at::Tensor> bias,
+                           at::Tensor k_cache, at::Tensor v_cache, const at::Tensor& positions,
+                           const at::Tensor& cos_sin, const at::Tensor& slots) {
+  check_slabs(slabs);
+  const int S = slabs.size(0), M = slabs.size(1), N = slabs.size(2);
+  const int kv_heads = k_cache.size(1), bs = k_cache.size(2), D = k_cache.size(3);
+  TORCH_CHECK(N % D == 0 && N / D > 2 * kv_heads && D % 8 == 0, "N must be (heads + 2 kv heads) D");
+  TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous() &&
+                  k_cache.scalar_type() == v_cache.scalar_type());
+  TORCH_CHECK(positions.scalar_type() == at::kLong && positions.numel() == M &&
+                  slots.scalar_type() == at::kLong && slots.numel() == M &&
+                  cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous() &&
+                  cos_sin.size(1) == D);
+  const __hip_bfloat16* bp = nullptr;
+  if (bias.has_value() && bias->defined()) {
+    TORCH_CHECK(bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() &&
+                bias->numel() == N, "bias must be bf16 [N]");
+    bp = reinterpret_cast<const __hip_bfloat16*>(bias->data_ptr());
+  }
+  at::Tensor qkv = at::empty({M, N}, slabs.options().dtype(at::kBFloat16));
+  auto go = [&]<typename TC>() {
+    hipLaunchKernelGGL(slab_rope_cache_kernel<TC>, dim3(M, 4), dim3(256), 0, stream(),
+                       reinterpret_cast<__hip_bfloat16*>(qkv.data_ptr()),
+                       slabs.data_ptr<float>(), S, bp, reinterpret_cast<TC*>(k_cache.data_ptr()),
+                       reinterpret_cast<TC*>(v_cache.data_ptr()), positions.data_ptr<long>(),
+                       cos_sin.data_ptr<float>(), slots.data_ptr<long>(), M,
+                       N / D - 2 * kv_heads, kv_heads, D, bs);
+  };
+  if (k_cache.scalar_type() == at::kBFloat16) go.template operator()<__hip_bfloat16>();
+  else if (k_cache.scalar_type() == at::kFloat8_e4m3fn) go.template operator()<__hip_fp8_e4m3>();
+  else TORCH_CHECK(false, "bf16 or fp8 cache");
+  return qkv;
+}
+
 // ------------------------------------------------------ prompt steps, whole --
 
 // All layers of a packed prompt step (no portion gathered into packed rows): the
-// same calls that the engine's per-layer code makes, in one crossing from Python.
+// calls that the engine's per-layer code makes, in one crossing from Python.
 // A layer's weights: qkv, o, gate_up, down, pre-MLP norm, next layer's input norm
 // (or the final one), and with sandwich norms the post-attention and post-MLP
 // ones. h is the normed input of layer 0; returns the final normed rows.
@@ -626,10 +771,23 @@ at::Tensor prompt_layers(at::Tensor h, at::Tensor residual, at::TensorList weigh
                   windows.size() == layers && (biases.empty() || biases.size() == layers),
               "one entry per layer");
   const long T = h.size(0);
+  // 17 to 128 rows of these shapes: the streaming products, whose sums the next
+  // kernel takes up
+  const bool slab = layers > 0 && k_caches[0].size(3) == head_dim && h.size(1) <= 8192 &&
+                    (k_caches[0].scalar_type() == at::kBFloat16 ||
+                     k_caches[0].scalar_type() == at::kFloat8_e4m3fn) &&
+                    slab_rows_ok(h, weights[0]) && weights[1].size(0) == h.size(1) &&
+                    weights[1].size(1) % kSlabBK == 0 && weights[1].size(0) % 64 == 0 &&
+                    weights[3].size(1) % kSlabBK == 0 && residual.is_contiguous();
+  const c10::optional<at::Tensor> none;
   for (size_t i = 0; i < layers; ++i) {
     const at::Tensor* w = &weights[per * i];
-    const at::Tensor qkv = at::linear(
-        h, w[0], biases.empty() ? c10::optional<at::Tensor>() : c10::make_optional(biases[i]));
+    const c10::optional<at::Tensor> bias =
+        biases.empty() ? none : c10::make_optional(biases[i]);
+    const at::Tensor qkv =
+        slab ? slab_rope_cache(slab_linear(h, w[0]), bias, k_caches[i], v_caches[i], positions,
+                               cos_sin, slots)
+             : at::linear(h, w[0], bias);
     const long kv_heads = k_caches[i].size(1);
     const long heads = qkv.size(1) / head_dim - 2 * kv_heads;
     auto part = [&](long first, long n) {
@@ -637,7 +795,7 @@ at::Tensor prompt_layers(at::Tensor h, at::Tensor residual, at::TensorList weigh
     };
     const at::Tensor q = part(0, heads), k = part(heads, kv_heads),
                      v = part(heads + kv_heads, kv_heads);
-    rope_and_cache(q, k, v, k_caches[i], v_caches[i], positions, cos_sin, slots);
+    if (!slab) rope_and_cache(q, k, v, k_caches[i], v_caches[i], positions, cos_sin, slots);
     at::Tensor attn = at::empty({T, heads, head_dim}, qkv.options());
     if (cu_seqlens_k.has_value())
       paged_prefill_attention(attn, q, k_caches[i], v_caches[i], *block_tables, cu_seqlens,
@@ -645,16 +803,29 @@ at::Tensor prompt_layers(at::Tensor h, at::Tensor residual, at::TensorList weigh
     else
       varlen_prefill_attention(attn, q, k, v, cu_seqlens, cu_seqlens, max_seqlen, scale, softcap,
                                windows[i]);
-    h = at::linear(attn.view({T, heads * head_dim}), w[1]);
-    if (post_norms) norm_add_norm(h, residual, w[6], w[4], eps, offset);
-    else fused_add_rmsnorm(h, residual, w[4], eps, offset);
-    const at::Tensor gate_up = at::linear(h, w[2]);
-    at::Tensor act = at::empty({T, gate_up.size(1) / 2}, gate_up.options());
-    if (gelu) gelu_tanh_and_mul(act, gate_up);
-    else silu_and_mul(act, gate_up);
-    h = at::linear(act, w[3]);
-    if (post_norms) norm_add_norm(h, residual, w[7], w[5], eps, offset);
-    else fused_add_rmsnorm(h, residual, w[5], eps, offset);
+    // the product, added to the residual (normalised first with sandwich norms), normed
+    auto project_add_norm = [&](const at::Tensor& a, const at::Tensor& wt,
+                                const at::Tensor* post, const at::Tensor& norm) {
+      if (slab)
+        return slab_add_norm(slab_linear(a, wt), residual,
+                             post ? c10::make_optional(*post) : none, norm, eps, offset);
+      at::Tensor y = at::linear(a, wt);
+      if (post) norm_add_norm(y, residual, *post, norm, eps, offset);
+      else fused_add_rmsnorm(y, residual, norm, eps, offset);
+      return y;
+    };
+    h = project_add_norm(attn.view({T, heads * head_dim}), w[1], post_norms ? &w[6] : nullptr,
+                         w[4]);
+    at::Tensor act;
+    if (slab && slab_act_ok(h, w[2])) {
+      act = slab_act_linear(h, w[2], gelu);
+    } else {
+      const at::Tensor gate_up = at::linear(h, w[2]);
+      act = at::empty({T, gate_up.size(1) / 2}, gate_up.options());
+      if (gelu) gelu_tanh_and_mul(act, gate_up);
+      else silu_and_mul(act, gate_up);
+    }
+    h = project_add_norm(act, w[3], post_norms ? &w[7] : nullptr, w[5]);
   }
   return h;
 }
@@ -764,6 +935,10 @@ TORCH_LIBRARY(llmq_amd, m) {
   m.def("paged_decode_attention(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor context_lens, float scale, float softcap, int window) -> ()");
   m.def("varlen_prefill_attention(Tensor(a!) out, Tensor q, Tensor k, Tensor v, Tensor cu_seqlens, Tensor cu_seqlens_k, int max_seqlen, float scale, float softcap, int window) -> ()");
   m.def("paged_prefill_attention(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor cu_seqlens, Tensor cu_seqlens_k, int max_seqlen, float scale, float softcap, int window) -> ()");
+  m.def("slab_linear(Tensor x, Tensor w) -> Tensor");
+  m.def("slab_act_linear(Tensor x, Tensor w, bool gelu) -> Tensor");
+  m.def("slab_add_norm(Tensor slabs, Tensor(a!) residual, Tensor? w_post, Tensor w, float eps, float offset) -> Tensor");
+  m.def("slab_rope_cache(Tensor slabs, Tensor? bias, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor positions, Tensor cos_sin, Tensor slots) -> Tensor");
   m.def("prompt_layers(Tensor h, Tensor(a!) residual, Tensor[] weights, Tensor[] biases, Tensor[] k_caches, Tensor[] v_caches, Tensor positions, Tensor cos_sin, Tensor slots, Tensor cu_seqlens, Tensor? block_tables, Tensor? cu_seqlens_k, int max_seqlen, int head_dim, float scale, float softcap, int[] windows, float eps, float offset, bool gelu, bool post_norms) -> Tensor");
   m.def("sample_gumbel_argmax(Tensor(a!) out, Tensor(b!) keys, Tensor logits, Tensor temps, Tensor req_seeds, Tensor req_pos, int seed, int step, Tensor? bounds=None) -> ()");
   m.def("topk_topp_bound(Tensor(a!) out_bound, Tensor logits, Tensor temps, Tensor top_ps, Tensor top_ks) -> ()");
@@ -784,6 +959,10 @@ TORCH_LIBRARY_IMPL(llmq_amd, CUDA, m) {
   m.impl("paged_decode_attention", &paged_decode_attention);
   m.impl("varlen_prefill_attention", &varlen_prefill_attention);
   m.impl("paged_prefill_attention", &paged_prefill_attention);
+  m.impl("slab_linear", &slab_linear);
+  m.impl("slab_act_linear", &slab_act_linear);
+  m.impl("slab_add_norm", &slab_add_norm);
+  m.impl("slab_rope_cache", &slab_rope_cache);
   m.impl("prompt_layers", &prompt_layers);
   m.impl("sample_gumbel_argmax", &sample_gumbel_argmax);
   m.impl("topk_topp_bound", &topk_topp_bound);

@@ -7,5 +7,6 @@
 #include "flash_prefill.hip"
 #include "skinny_gemm.hip"
 #include "stream_gemm.hip"
+#include "slab_gemm.hip"
 #include "sampling.hip"
 #include "bindings.cpp"

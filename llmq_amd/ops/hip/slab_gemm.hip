@@ -1,0 +1,282 @@
+// Projections of 17 to 128 rows, x[M, K] W[N, K]^T with fp32 sums: the products of
+// an ordinary decode step or a short prompt (gfx950).
+//
+// Bound by the weights' bytes. A workgroup owns 64 weight rows, all M tokens and one
+// of S parts of K. Weights go straight from memory into the matrix layout, two
+// 128-wide K steps ahead; the tokens, which every workgroup reads again, are staged
+// once per workgroup in LDS by global_load_lds (16-byte granules placed by row, so
+// operand reads meet no bank conflict), one step ahead. v_mfma_f32_16x16x32_bf16,
+// A = weights (row = lane%16, k = 8*(lane/16)..+7), B = tokens likewise, C: column =
+// token, rows = 4 weight rows.
+//
+// With S > 1 the parts are left as fp32 slabs [S, M, N] and added up by the kernel
+// that reads them anyway (norm and residual, rotation and cache write): the sum
+// costs no launch and no rounding. Gate and value rows (PAIR) are activated here.
+// Measured (us, the library's product before): 64 rows, 2048 x 8192: 22.8 -> 12.7,
+// 2048 x 2048: 8.8 -> 5.6, 3072 x 2048: 12.0 -> 8.1; 96 rows, 3584 x 14336: 50.4 ->
+// 38.6; 128 rows, 3072 x 8192: 42.8 -> 25.6; 24 rows, 1536 x 8960: 28.7 -> 11.9.
+
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(8))) short sl_s16x8;
+typedef __attribute__((ext_vector_type(4))) float sl_f32x4;
+
+enum : int { kSlabSums = 0, kSlabSilu = 1, kSlabGelu = 2 };
+
+constexpr int kSlabBK = 128;
+
+// TM: token tiles of 16; WK: groups of four waves that take the K steps in turn.
+template <int TM, int WK, int EPI>
+__global__ __launch_bounds__(256 * WK) void slab_gemm_kernel(
+    float* __restrict__ slabs, __hip_bfloat16* __restrict__ out, long out_stride,
+    const __hip_bfloat16* __restrict__ x, long x_stride,
+    const __hip_bfloat16* __restrict__ wt, int M, int N, int K, int steps_per_split) {
+  constexpr bool PAIR = EPI != kSlabSums;
+  constexpr int ROWS = TM * 16, TILE = ROWS * kSlabBK;       // one staged token tile
+  constexpr int RED = 4 * WK * TM * 256 * 2;                  // fp32 sums, in shorts
+  constexpr int STAGE = 2 * WK * TILE;
+  __shared__ __align__(16) short lds[STAGE > RED ? STAGE : RED];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nt = w & 3, kg = w >> 2;
+  const int col = lane & 15, grp = lane >> 4;
+  const int step0 = blockIdx.y * steps_per_split;
+  const int total = min(steps_per_split, K / kSlabBK - step0);
+  const int loops = (total + WK - 1) / WK;
+  const int n0 = blockIdx.x * (PAIR ? 32 : 64);
+  const int wrow = PAIR ? (nt < 2 ? n0 + nt * 16 : N / 2 + n0 + (nt - 2) * 16) : n0 + nt * 16;
+  const __hip_bfloat16* wp = wt + (long)(wrow + col) * K + (long)step0 * kSlabBK + grp * 8;
+  // staging: load j of this wave fills rows 4 (nt + 4 j) + lane/16 of its group's tile
+  const int srow = nt * 4 + (lane >> 4);
+  const int sgran = ((lane & 15) ^ (srow & 15)) << 3;
+  const __hip_bfloat16* xp[TM];
+#pragma unroll
+  for (int j = 0; j < TM; ++j)
+    xp[j] = x + (long)min(srow + j * 16, M - 1) * x_stride + (long)step0 * kSlabBK + sgran;
+  short* const mine = lds + kg * TILE;                        // + stage * WK * TILE
+  auto stage = [&](int i) {
+    const int s = i * WK + kg;
+    if (s >= total) return;
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+      glds16(xp[j] + s * kSlabBK, mine + (i & 1) * (WK * TILE) + (nt + j * 4) * 512);
+  };
+  auto fetch = [&](sl_s16x8 (&f)[4], int i) {
+    const int s = min(i * WK + kg, total - 1);                // past the end: unused
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      f[u] = __builtin_nontemporal_load(
+          reinterpret_cast<const sl_s16x8*>(wp + s * kSlabBK + u * 32));
+  };
+  sl_f32x4 acc[TM];
+#pragma unroll
+  for (int m = 0; m < TM; ++m) acc[m] = sl_f32x4{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](int i, sl_s16x8 (&f)[4]) {
+    // this step's tokens and weights have landed, the next weights may travel
+    if (i + 1 < loops) pipe_barrier_vm<4>();
+    else pipe_barrier_vm<0>();
+    if (i + 1 < loops) stage(i + 1);
+    if (i * WK + kg < total) {
+      const short* xt = mine + (i & 1) * (WK * TILE) + col * kSlabBK;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int m = 0; m < TM; ++m) {
+          const sl_s16x8 xf = *reinterpret_cast<const sl_s16x8*>(
+              xt + m * 16 * kSlabBK + (((u * 4 + grp) ^ col) << 3));
+          acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[u], xf, acc[m], 0, 0, 0);
+        }
+    }
+    if (i + 2 < loops) fetch(f, i + 2);
+  };
+  sl_s16x8 wa[4], wb[4];
+  stage(0);
+  fetch(wa, 0);
+  if (loops > 1) fetch(wb, 1);
+  for (int i = 0; i < loops; i += 2) {
+    step(i, wa);
+    if (i + 1 < loops) step(i + 1, wb);
+  }
+
+  if constexpr (!PAIR && WK == 1) {
+    float* slab = slabs + (long)blockIdx.y * M * N + wrow + grp * 4;
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+      if (m * 16 + col < M)
+        *reinterpret_cast<sl_f32x4*>(slab + (long)(m * 16 + col) * N) = acc[m];
+    return;
+  }
+  // sums of the groups, and of gate and value rows, meet in LDS
+  __syncthreads();
+  float* red = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+    *reinterpret_cast<sl_f32x4*>(red + ((w * TM + m) * 64 + lane) * 4) = acc[m];
+  __syncthreads();
+  constexpr int UNITS = TM * (PAIR ? 2 : 4);                  // (n tile, m tile) of 64 lanes
+  for (int unit = w; unit < UNITS; unit += 4 * WK) {
+    const int t = unit / TM, m = unit % TM;
+    auto sum = [&](int tile) {
+      sl_f32x4 s = *reinterpret_cast<const sl_f32x4*>(red + ((tile * TM + m) * 64 + lane) * 4);
+#pragma unroll
+      for (int g = 1; g < WK; ++g)
+        s += *reinterpret_cast<const sl_f32x4*>(
+            red + (((g * 4 + tile) * TM + m) * 64 + lane) * 4);
+      return s;
+    };
+    const int row = m * 16 + col;
+    sl_f32x4 y = sum(t);
+    if constexpr (!PAIR) {
+      if (row < M)
+        *reinterpret_cast<sl_f32x4*>(slabs + ((long)blockIdx.y * M + row) * N + n0 + t * 16 +
+                                     grp * 4) = y;
+    } else {
+      const sl_f32x4 up = sum(t + 2);
+      Vec4<__hip_bfloat16> v;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float g = y[r];
+        const float a = EPI == kSlabSilu
+            ? g / (1.0f + __expf(-g))
+            : 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
+        v.data[r] = __float2bfloat16(a * up[r]);
+      }
+      if (row < M)
+        *reinterpret_cast<int2*>(out + (long)row * out_stride + n0 + t * 16 + grp * 4) =
+            *reinterpret_cast<const int2*>(v.data);
+    }
+  }
+}
+
+// ------------------------------------------------------- readers of the slabs --
+
+// Sum of S slabs at one place, eight loads in flight: their L2 is another XCD's.
+DEVINL sl_f32x4 slab_sum(const float* __restrict__ slabs, long at, long stride, int S) {
+  sl_f32x4 y = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < S; s0 += 8) {
+    sl_f32x4 v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      v[e] = *reinterpret_cast<const sl_f32x4*>(slabs + min(s0 + e, S - 1) * stride + at);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (s0 + e < S) y += v[e];
+  }
+  return y;
+}
+
+DEVINL sl_f32x4 slab_bf4(const __hip_bfloat16* p) {
+  const Vec4<__hip_bfloat16> v = load8(p);
+  return sl_f32x4{to_f32(v.data[0]), to_f32(v.data[1]), to_f32(v.data[2]), to_f32(v.data[3])};
+}
+
+DEVINL Vec4<__hip_bfloat16> slab_store(__hip_bfloat16* p, sl_f32x4 y) {
+  Vec4<__hip_bfloat16> v;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v.data[r] = __float2bfloat16(y[r]);
+  *reinterpret_cast<int2*>(p) = *reinterpret_cast<const int2*>(v.data);
+  return v;
+}
+
+// residual += y, or with POST += rmsnorm(y) (w_post + offset), y the summed slabs;
+// h = rmsnorm(residual) (w + offset). One workgroup per row, the row in registers:
+// up to 8192 channels. Bound by latency: few rows, each behind S slabs (64 rows of
+// 2048, 16 slabs: 4.8 us; with 256 threads that added slab by slab 9.4).
+constexpr int kSlabNT = 1024;
+
+template <bool POST>
+__global__ __launch_bounds__(kSlabNT) void slab_add_norm_kernel(
+    __hip_bfloat16* __restrict__ h, __hip_bfloat16* __restrict__ residual,
+    const float* __restrict__ slabs, int S, const __hip_bfloat16* __restrict__ w_post,
+    const __hip_bfloat16* __restrict__ w, int M, int N, float eps, float offset) {
+  __shared__ float red[kSlabNT / WAVE];
+  const long row = (long)blockIdx.x * N;
+  const long stride = (long)M * N;
+  sl_f32x4 y[2], r[2];
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int i = (k * blockDim.x + threadIdx.x) * 4;
+    y[k] = r[k] = sl_f32x4{0.f, 0.f, 0.f, 0.f};
+    if (i >= N) continue;
+    r[k] = slab_bf4(residual + row + i);
+    y[k] = slab_sum(slabs, row + i, stride, S);
+    if (POST) ss += y[k][0] * y[k][0] + y[k][1] * y[k][1] + y[k][2] * y[k][2] + y[k][3] * y[k][3];
+  }
+  float inv = 1.f;
+  if (POST) inv = rsqrtf(block_reduce_sum(ss, red) / N + eps);
+  ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int i = (k * blockDim.x + threadIdx.x) * 4;
+    if (i >= N) continue;
+    if (POST) r[k] += y[k] * inv * (slab_bf4(w_post + i) + offset);
+    else r[k] += y[k];
+    const Vec4<__hip_bfloat16> v = slab_store(residual + row + i, r[k]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      r[k][e] = to_f32(v.data[e]);           // the rounded stream is what is normalised
+      ss += r[k][e] * r[k][e];
+    }
+  }
+  inv = rsqrtf(block_reduce_sum(ss, red) / N + eps);
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int i = (k * blockDim.x + threadIdx.x) * 4;
+    if (i < N) slab_store(h + row + i, r[k] * inv * (slab_bf4(w + i) + offset));
+  }
+}
+
+// The summed slabs of a q/k/v projection (+ bias): q and k rotated (halves of a head,
+// as in rope_and_cache_kernel), all written as packed bf16 rows and k, v into the
+// paged cache. Workgroups of (token, quarter of the heads), four channel pairs per
+// thread.
+template <typename TC>
+__global__ __launch_bounds__(256) void slab_rope_cache_kernel(
+    __hip_bfloat16* __restrict__ qkv, const float* __restrict__ slabs, int S,
+    const __hip_bfloat16* __restrict__ bias, TC* __restrict__ k_cache, TC* __restrict__ v_cache,
+    const long* __restrict__ positions, const float* __restrict__ cos_sin,
+    const long* __restrict__ slots, int M, int heads, int kv_heads, int D, int block_size) {
+  const int token = blockIdx.x, half = D / 2, quads = half / 4;
+  const int N = (heads + 2 * kv_heads) * D;
+  const long row = (long)token * N, stride = (long)M * N;
+  const float* cs = cos_sin + positions[token] * D;
+  const long slot = slots[token];
+  const long block = slot / block_size;
+  const int off = (int)(slot % block_size);
+  for (int t = blockIdx.y * 256 + threadIdx.x; t < (heads + 2 * kv_heads) * quads;
+       t += gridDim.y * 256) {
+    const int hd = t / quads, d = (t % quads) * 4;
+    const int i = hd * D + d;
+    sl_f32x4 a = slab_sum(slabs, row + i, stride, S);
+    sl_f32x4 b = slab_sum(slabs, row + i + half, stride, S);
+    if (bias) {
+      a += slab_bf4(bias + i);
+      b += slab_bf4(bias + i + half);
+    }
+    if (hd < heads + kv_heads) {
+      const sl_f32x4 c = *reinterpret_cast<const sl_f32x4*>(cs + d);
+      const sl_f32x4 s = *reinterpret_cast<const sl_f32x4*>(cs + half + d);
+      const sl_f32x4 ra = a * c - b * s;
+      b = b * c + a * s;
+      a = ra;
+    }
+    const Vec4<__hip_bfloat16> va = slab_store(qkv + row + i, a);
+    const Vec4<__hip_bfloat16> vb = slab_store(qkv + row + i + half, b);
+    if (hd < heads || slot < 0) continue;
+    const bool is_v = hd >= heads + kv_heads;
+    const int kh = hd - heads - (is_v ? kv_heads : 0);
+    TC* dst = (is_v ? v_cache : k_cache) +
+              ((block * kv_heads + kh) * (long)block_size + off) * D + d;
+    if constexpr (std::is_same_v<TC, __hip_bfloat16>) {
+      *reinterpret_cast<int2*>(dst) = *reinterpret_cast<const int2*>(va.data);
+      *reinterpret_cast<int2*>(dst + half) = *reinterpret_cast<const int2*>(vb.data);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {          // from the rounded rows, as the other path
+        dst[e] = from_f32<TC>(to_f32(va.data[e]));
+        dst[half + e] = from_f32<TC>(to_f32(vb.data[e]));
+      }
+    }
+  }
+}

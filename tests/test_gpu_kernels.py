@@ -337,6 +337,81 @@ class TestPrefillRanges:
         assert_close_to_f32_ref(out.cpu(), ref, 5 * 2 ** -9, 2 ** -8)
 
 
+class TestSlabProjections:
+    """Streaming products of 17 to 128 rows and the kernels that add up their
+    partial sums: each row-tile count, K that leaves parts of unequal length."""
+
+    @pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 96, 97, 128])
+    @pytest.mark.parametrize("N,K", [(64, 128), (192, 640), (2048, 2048), (3072, 8960)])
+    def test_products(self, M, N, K):
+        x = torch.randn(M, K + 8, device=DEV, dtype=torch.bfloat16)[:, :K]
+        w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) * K ** -0.5
+        ref = x.double() @ w.double().t()
+        got = ops.slab_linear(x, w).double().sum(0)
+        assert ((got - ref).abs() <= 1e-5 * (1 + ref.abs())).all()     # fp32 sums of unit size
+        if M > 64:
+            return
+        for gelu in (False, True):
+            g, u = ref.chunk(2, -1)
+            act = torch.nn.functional.gelu(g, approximate="tanh") if gelu \
+                else torch.nn.functional.silu(g)
+            y = ops.slab_act_linear(x, w, gelu).double()
+            # the output's rounding; sums' errors through a slope under 1.2
+            tol = 2 ** -8 * (act * u).abs() + 3e-5 * (1 + g.abs()) * (1 + u.abs())
+            assert ((y - act * u).abs() <= tol).all()
+
+    @pytest.mark.parametrize("S,M,N", [(1, 17, 64), (3, 20, 1000), (16, 64, 2048), (2, 128, 8192)])
+    @pytest.mark.parametrize("post", [False, True])
+    def test_add_norm(self, S, M, N, post):
+        slabs = torch.randn(S, M, N, device=DEV)
+        res = torch.randn(M, N, device=DEV, dtype=torch.bfloat16)
+        w, wp = (torch.randn(N, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+
+        def norm(t, wt):
+            return t * torch.rsqrt(t.square().mean(-1, keepdim=True) + 1e-6) * (wt.double() + 1.0)
+
+        y = slabs.double().sum(0)
+        want = res.double() + (norm(y, wp) if post else y)
+        h = ops.slab_add_norm(slabs, res, wp if post else None, w, 1e-6, 1.0).double()
+        tol = 2 ** -8 * want.abs() + 1e-5 * S                  # rounding; fp32 sums
+        assert ((res.double() - want).abs() <= tol).all()
+        ref = norm(res.double(), w)                             # of the rounded stream
+        assert ((h - ref).abs() <= 2 ** -8 * ref.abs() + 1e-5).all()
+
+    @pytest.mark.parametrize("D,H,KVH,fp8", [(64, 4, 2, False), (128, 3, 1, True), (256, 2, 2, False)])
+    @pytest.mark.parametrize("bias", [False, True])
+    def test_rope_cache(self, D, H, KVH, fp8, bias):
+        S, M, N, BS, NB = 3, 21, (H + 2 * KVH) * D, 16, 5
+        slabs = torch.randn(S, M, N, device=DEV)
+        b = torch.randn(N, device=DEV, dtype=torch.bfloat16) if bias else None
+        pos = torch.randint(0, 900, (M,), device=DEV)
+        slots = torch.randperm(NB * BS, device=DEV)[:M]
+        slots[3] = -1                                           # a padding row: no cache entry
+        cs = torch_ref.build_rope_cache(1000, D, 10000.0, DEV)
+        kind = torch.float8_e4m3fn if fp8 else torch.bfloat16
+        kc, vc = (torch.zeros(NB, KVH, BS, D, device=DEV, dtype=kind) for _ in range(2))
+        qkv = ops.slab_rope_cache(slabs, b, kc, vc, pos, cs, slots)
+        y = slabs.double().sum(0) + (b.double() if bias else 0)
+        q, k, v = (t.reshape(M, -1, D).clone() for t in y.split([H * D, KVH * D, KVH * D], -1))
+        c, s = (t[pos].double()[:, None] for t in cs.split(D // 2, -1))
+        for t in (q, k):
+            a, e = t.split(D // 2, -1)
+            t.copy_(torch.cat([a * c - e * s, e * c + a * s], -1))
+        want = torch.cat([t.reshape(M, -1) for t in (q, k, v)], -1)
+        assert ((qkv.double() - want).abs() <= 2 ** -8 * want.abs() + 3e-5).all()
+        rows = qkv.view(M, -1, D)
+        for t in range(M):
+            if t == 3:
+                continue
+            blk, off = int(slots[t]) // BS, int(slots[t]) % BS
+            assert torch.equal(kc[blk, :, off].float(), rows[t, H:H + KVH].to(kind).float())
+            assert torch.equal(vc[blk, :, off].float(), rows[t, H + KVH:].to(kind).float())
+        used = torch.zeros(NB * BS, dtype=torch.bool)
+        used[slots[slots >= 0].cpu()] = True
+        empty = (kc.float().transpose(1, 2).reshape(NB * BS, -1) == 0).all(1).cpu()
+        assert torch.equal(empty, ~used)
+
+
 class TestPagedPrefill:
     """The prompt kernel on cache blocks gives what it gives on packed rows, bit for
     bit: the same tiles, whatever the blocks' order and the rows past the end hold."""
