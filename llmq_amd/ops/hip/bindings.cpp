@@ -185,33 +185,38 @@ void rope_and_cache(at::Tensor q, at::Tensor k, at::Tensor value,
   const int bs = k_cache.size(2);
   TORCH_CHECK(q.stride(1) == d && k.stride(1) == d, "head dim must be packed");
   const bool fp8_cache = k_cache.scalar_type() == at::kFloat8_e4m3fn;
+  // 8-byte pieces of every row, 16-byte ones of the angles
+  auto pieces = [&](const at::Tensor& t, long bytes) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % bytes == 0 &&
+           t.stride(0) * (long)t.element_size() % bytes == 0;
+  };
   dispatch_dtype(q, "rope_and_cache", [&]<typename T>() {
+    constexpr int NP = 8 / sizeof(T);
+    const bool wide = d % (2 * NP) == 0 && pieces(q, 8) && pieces(k, 8) && pieces(value, 8) &&
+                      pieces(cos_sin, 4 * NP) && (d / 2 * 4) % (4 * NP) == 0 &&
+                      reinterpret_cast<uintptr_t>(k_cache.data_ptr()) % 8 == 0 &&
+                      reinterpret_cast<uintptr_t>(v_cache.data_ptr()) % 8 == 0;
+    auto go = [&]<typename TC, int N>() {
+      // few tokens: the heads over four workgroups
+      hipLaunchKernelGGL((rope_and_cache_kernel<T, TC, N>), dim3(T_, T_ < 1024 ? 4 : 1), dim3(256),
+                         0, stream(), reinterpret_cast<T*>(q.data_ptr()),
+                         reinterpret_cast<T*>(k.data_ptr()),
+                         reinterpret_cast<const T*>(value.data_ptr()),
+                         reinterpret_cast<TC*>(k_cache.data_ptr()),
+                         reinterpret_cast<TC*>(v_cache.data_ptr()), positions.data_ptr<long>(),
+                         cos_sin.data_ptr<float>(), slot_mapping.data_ptr<long>(), hq, hk, d, bs,
+                         q.stride(0), k.stride(0), value.stride(0));
+    };
+    auto pick = [&]<typename TC>() {
+      if (wide) go.template operator()<TC, NP>();
+      else go.template operator()<TC, 1>();
+    };
     if (fp8_cache) {
-      if constexpr (std::is_same_v<T, __hip_bfloat16>) {
-        hipLaunchKernelGGL((rope_and_cache_kernel<T, __hip_fp8_e4m3>),
-                           dim3(T_), dim3(256), 0, stream(),
-                           reinterpret_cast<T*>(q.data_ptr()),
-                           reinterpret_cast<T*>(k.data_ptr()),
-                           reinterpret_cast<const T*>(value.data_ptr()),
-                           reinterpret_cast<__hip_fp8_e4m3*>(k_cache.data_ptr()),
-                           reinterpret_cast<__hip_fp8_e4m3*>(v_cache.data_ptr()),
-                           positions.data_ptr<long>(), cos_sin.data_ptr<float>(),
-                           slot_mapping.data_ptr<long>(), hq, hk, d, bs,
-                           q.stride(0), k.stride(0), value.stride(0));
-      } else {
-        TORCH_CHECK(false, "fp8 KV cache requires bf16 activations");
-      }
+      if constexpr (std::is_same_v<T, __hip_bfloat16>) pick.template operator()<__hip_fp8_e4m3>();
+      else TORCH_CHECK(false, "fp8 KV cache requires bf16 activations");
       return;
     }
-    hipLaunchKernelGGL(rope_and_cache_kernel<T>, dim3(T_), dim3(256), 0,
-                       stream(), reinterpret_cast<T*>(q.data_ptr()),
-                       reinterpret_cast<T*>(k.data_ptr()),
-                       reinterpret_cast<const T*>(value.data_ptr()),
-                       reinterpret_cast<T*>(k_cache.data_ptr()),
-                       reinterpret_cast<T*>(v_cache.data_ptr()),
-                       positions.data_ptr<long>(), cos_sin.data_ptr<float>(),
-                       slot_mapping.data_ptr<long>(), hq, hk, d, bs,
-                       q.stride(0), k.stride(0), value.stride(0));
+    pick.template operator()<T>();
   });
 }
 
@@ -260,8 +265,12 @@ void launch_paged_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor&
   };
   if (softcap > 0) go.template operator()<true>();
   else go.template operator()<false>();
-  hipLaunchKernelGGL((paged_decode_merge_kernel<D, Shape::kTileShift>), dim3(B, q.size(1)),
-                     dim3(256), 0, stream(),
+  // One wave merges a (sequence, head) where there are enough of those, four else.
+  const int H = q.size(1);
+  const bool many = (long)B * H >= 1024 && H % 4 == 0;
+  hipLaunchKernelGGL((many ? paged_decode_merge_kernel<D, Shape::kTileShift, 1>
+                           : paged_decode_merge_kernel<D, Shape::kTileShift, 4>),
+                     dim3(B, many ? H / 4 : H), dim3(256), 0, stream(),
                      reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), out.stride(0),
                      part_o.data_ptr<float>(), part_ml.data_ptr<float>(), cl.data_ptr<int>(), B,
                      KVH, G, (int)window, waves);
