@@ -579,8 +579,9 @@ void stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
   }
   auto go = [&]<int KH, int NW, int KU, bool NORM, int EPI>() {
     constexpr int RO = EPI >= kSgSilu ? 8 / KH : 16 / KH;
+    const size_t lds = NORM ? sizeof(short) * (size_t)M * SgTokens<KH>::row(K) : 0;
     hipLaunchKernelGGL((stream_gemm_kernel<KH, NW, KU, NORM, EPI>), dim3(cols / RO),
-                       dim3(64 * NW), 0, stream(),
+                       dim3(64 * NW), lds, stream(),
                        reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), out.stride(0),
                        reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()), x.stride(0),
                        reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()), bp, np,
@@ -610,8 +611,16 @@ void stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
     else if (epi == kSgSilu) slices.template operator()<NORM, kSgSilu>();
     else slices.template operator()<NORM, kSgGelu>();
   };
-  if (np) epilogue.template operator()<true>();
-  else epilogue.template operator()<false>();
+  if (!np) return epilogue.template operator()<false>();
+  // Every workgroup weights all tokens: worth the launch that it saves for few of
+  // them (17920 x 1536 pairs: seven tokens 24.3 us here, 16.2 + 4 with a norm of its
+  // own; 16384 x 2048 pairs, one token 17.3 and 14.7 + 4). They have to fit beside
+  // the sums (24 KB at the most).
+  if (M <= (pair ? 4 : 8) && (long)M * (K + 512) * 2 <= (120 << 10))
+    return epilogue.template operator()<true>();
+  at::Tensor h = at::empty({M, K}, x.options());
+  rmsnorm(h, x.is_contiguous() ? x : x.contiguous(), *norm_w, eps, offset);
+  stream_gemm(out, h, w, bias, c10::nullopt, 0, 0, epi);
 }
 
 // ------------------------------------------- projections, 17 to 128 rows --

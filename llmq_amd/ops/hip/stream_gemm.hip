@@ -14,9 +14,12 @@
 //     blocks on C's diagonal. That sets a workgroup's share to 16, 8, 4, 2 or 1
 //     weight rows without a masked lane.
 //   - The workgroup's waves share out the slices in chunks and add up through LDS.
-//   - NORM: the tokens are RMS-normalised on the way in: x is multiplied by the
-//     norm's weights (and rounded, as a normalised row is), its squares are summed
-//     beside, and the row's factor meets the fp32 sums at the end.
+//   - NORM: the tokens are RMS-normalised on the way in: x times the norm's weights
+//     (rounded, as a normalised row is) goes to LDS once per workgroup, while the
+//     first weights travel, its squares are summed beside, and the row's factor
+//     meets the fp32 sums at the end. (Weighting each operand where it is used cost
+//     16384 x 2048 pairs with one token 25.3 instead of 17.3 us: more vector work than the
+//     weights' bytes leave time for.)
 //   - RES: the sums are added to the residual in place. ACT: half of the weight
 //     rows are gates, half the values that they act on (x = [gate | up]).
 
@@ -29,6 +32,15 @@ typedef __attribute__((ext_vector_type(2))) float sg_f32x2;
 typedef __attribute__((ext_vector_type(2))) __bf16 sg_bf16x2;
 
 enum : int { kSgPlain = 0, kSgResidual = 1, kSgSilu = 2, kSgGelu = 3 };
+
+// Places of weighted tokens in LDS (shorts): the 16 columns of an operand read lie in
+// 16 different 16-byte bank groups where slices are multiples of 128.
+template <int KH>
+struct SgTokens {
+  static constexpr int kPlaces = 16 / KH;
+  __host__ __device__ static int slice(int K) { return K / KH + 8 * kPlaces; }
+  __host__ __device__ static int row(int K) { return (KH * slice(K) + 127) / 128 * 128 + 8; }
+};
 
 // KH: slices of K (16 / KH >= M); NW: waves; KU: 32-wide K steps of a chunk.
 template <int KH, int NW, int KU, bool NORM, int EPI>
@@ -54,9 +66,10 @@ __global__ __launch_bounds__(64 * NW) void stream_gemm_kernel(
   const long kslice = (long)(col / R) * ks + grp * 8;
   const __hip_bfloat16* wp = wt + (long)wrow * K + kslice;
   const __hip_bfloat16* xp = x + (long)min(col % MP, M - 1) * x_stride + kslice;
-  const __hip_bfloat16* np = NORM ? norm_w + kslice : nullptr;
+  extern __shared__ __align__(16) short tokens[];
+  const short* tp = tokens + min(col % MP, M - 1) * SgTokens<KH>::row(K) +
+                    (col / R) * SgTokens<KH>::slice(K) + grp * 8;
   sg_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  float ss = 0.f;
 
   sg_s16x8 wf[KU], wn[KU];
   auto fetch = [&](sg_s16x8 (&f)[KU], int k0) {
@@ -66,30 +79,37 @@ __global__ __launch_bounds__(64 * NW) void stream_gemm_kernel(
   };
   int k0 = w * KC;
   if (k0 < ks) fetch(wf, k0);
-  for (; k0 < ks; k0 += NW * KC) {
-    sg_s16x8 xf[KU];
-#pragma unroll
-    for (int u = 0; u < KU; ++u)
-      xf[u] = *reinterpret_cast<const sg_s16x8*>(xp + k0 + u * 32);
-    const int next = k0 + NW * KC;
-    if (next < ks) fetch(wn, next);
-    if constexpr (NORM) {
-#pragma unroll
-      for (int u = 0; u < KU; ++u) {
-        const Vec8<__hip_bfloat16> nv = load16(np + k0 + u * 32);
+  if constexpr (NORM) {
+    for (int m = 0; m < M; ++m) {
+      float ss = 0.f;
+      for (int k = threadIdx.x * 8; k < K; k += 64 * NW * 8) {
+        const Vec8<__hip_bfloat16> xv = load16(x + (long)m * x_stride + k);
+        const Vec8<__hip_bfloat16> nv = load16(norm_w + k);
         sg_u32x4 y;
 #pragma unroll
         for (int e = 0; e < 8; e += 2) {
-          const float a = __uint_as_float((unsigned)(unsigned short)xf[u][e] << 16);
-          const float b = __uint_as_float((unsigned)(unsigned short)xf[u][e + 1] << 16);
+          const float a = to_f32(xv.data[e]), b = to_f32(xv.data[e + 1]);
           ss += a * a + b * b;
           y[e / 2] = __builtin_bit_cast(unsigned, __builtin_convertvector(
               (sg_f32x2{a * (to_f32(nv.data[e]) + offset), b * (to_f32(nv.data[e + 1]) + offset)}),
               sg_bf16x2));
         }
-        xf[u] = __builtin_bit_cast(sg_s16x8, y);
+        *reinterpret_cast<sg_u32x4*>(tokens + m * SgTokens<KH>::row(K) +
+                                     (k / ks) * SgTokens<KH>::slice(K) + k % ks) = y;
       }
+      ss = wave_reduce_sum(ss);
+      if (lane == 0) sums[w][m] = ss;
     }
+    __syncthreads();
+  }
+  for (; k0 < ks; k0 += NW * KC) {
+    sg_s16x8 xf[KU];
+#pragma unroll
+    for (int u = 0; u < KU; ++u)
+      xf[u] = NORM ? *reinterpret_cast<const sg_s16x8*>(tp + k0 + u * 32)
+                   : *reinterpret_cast<const sg_s16x8*>(xp + k0 + u * 32);
+    const int next = k0 + NW * KC;
+    if (next < ks) fetch(wn, next);
 #pragma unroll
     for (int u = 0; u < KU; ++u)
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], xf[u], acc, 0, 0, 0);
@@ -98,11 +118,6 @@ __global__ __launch_bounds__(64 * NW) void stream_gemm_kernel(
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) red[w][(grp * 4 + r) * RP + col] = acc[r];
-  if constexpr (NORM) {
-    ss += __shfl_xor(ss, 16, WAVE);
-    ss += __shfl_xor(ss, 32, WAVE);
-    if (grp == 0) sums[w][col] = ss;
-  }
   __syncthreads();
   // four threads per sum: each takes every fourth wave
   auto total = [&](int m, int row, int part) {
@@ -124,9 +139,7 @@ __global__ __launch_bounds__(64 * NW) void stream_gemm_kernel(
     if constexpr (NORM) {
       float q = 0.f;
 #pragma unroll
-      for (int v = 0; v < NW / 4; ++v)
-#pragma unroll
-        for (int h = 0; h < KH; ++h) q += sums[part + v * 4][h * MP + m];
+      for (int v = 0; v < NW / 4; ++v) q += sums[part + v * 4][min(m, M - 1)];
       q += __shfl_xor(q, 1, WAVE);
       q += __shfl_xor(q, 2, WAVE);
       inv = rsqrtf(q / K + eps);

@@ -454,7 +454,8 @@ class TestFewRowsLinear:
     large matrices), chunk remainders, norm, bias, activation and residual."""
 
     @pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
-    @pytest.mark.parametrize("N,K", [(32, 128), (96, 384), (1536, 640), (16384, 3072)])
+    @pytest.mark.parametrize("N,K", [(32, 128), (96, 384), (1536, 640), (16384, 3072),
+                                     (64, 14336)])
     @pytest.mark.parametrize("norm", [False, True])
     @pytest.mark.parametrize("what", ["plain", "bias", "residual", "silu", "gelu_tanh"])
     def test_vs_64_bits(self, M, N, K, norm, what):
@@ -467,6 +468,10 @@ class TestFewRowsLinear:
         if norm:   # the kernel's operands: weighted in fp32, rounded, scaled after the sum
             inv = torch.rsqrt(h.square().mean(-1, keepdim=True) + 1e-5)
             h = (x.float() * (nw.float() + 1.0)).bfloat16().double() * inv
+            act_rows = what in ("silu", "gelu_tanh")
+            if M > (4 if act_rows else 8) or M * (K + 512) * 2 > 120 << 10:
+                # a norm of its own first: normalised rows, rounded
+                h = (x.float() * inv.float() * (nw.float() + 1.0)).bfloat16().double()
         ref = h @ w.double().t()
         mag = h.norm(dim=-1, keepdim=True) * K ** -0.5       # of one sum
         act = what if what in ("silu", "gelu_tanh") else ""
