@@ -145,8 +145,7 @@ class ModelRunner:
                 # capture and warmup rows write the scratch slot only
                 self.in_rec.slots.fill_(self.recurrent.pad_slot)
                 self.in_rec.fresh.fill_(1)
-            if self.paged_prefill:
-                self.in_slots.fill_(-1)  # capture/warmup rows enter no cache slot
+            self.in_slots.fill_(-1)  # capture/warmup rows enter no cache slot
             # warmup (also materialises workspace allocations)
             out = self.model.forward(self.in_ids[:bs], self.in_pos[:bs], self.kv_cache, meta)
             torch.cuda.synchronize()
@@ -465,9 +464,9 @@ class ModelRunner:
                 self._staged_rows[i] = (s.uid, s.num_preemptions, n)
         if B < bucket:
             # pad rows: context_len 1 pointing at block 0 (defined garbage,
-            # their logits are never read)
-            # padding rows of a paged-prefill model enter no cache slot at all
-            self.h_slots[B:bucket] = -1 if self.paged_prefill else 0
+            # their logits are never read); they enter no cache slot at all
+            # (slot 0 is a live sequence's)
+            self.h_slots[B:bucket] = -1
             self.h_ids[B:bucket] = 0
             self.h_pos[B:bucket] = 0
             for i in range(B, bucket):

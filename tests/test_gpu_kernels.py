@@ -412,6 +412,24 @@ class TestSlabProjections:
         assert torch.equal(empty, ~used)
 
 
+class TestGraphPaddingRows:
+    def test_padding_rows_write_no_cache_slot(self):
+        """A decode step whose batch is under its graph's bucket pads rows; the
+        first cache slot belongs to a sequence and keeps its keys."""
+        from llmq_amd.engine.config import EngineConfig
+        from llmq_amd.engine.engine import LLMEngine
+
+        eng = LLMEngine(EngineConfig(model="tiny-llama-d128", max_num_seqs=4, max_model_len=64,
+                                     load_weights=False, num_kv_blocks=32))
+        assert eng.runner.use_graphs
+        eng.replay_step([{"id": f"s{i}", "tokens": [7 + i, 9, 11], "want": []} for i in range(3)])
+        assert 0 in eng._seqs["s0"].block_table
+        before = [c[0].clone() for c in (*eng.kv_cache.k, *eng.kv_cache.v)]
+        eng.replay_step([{"id": f"s{i}", "tokens": [5], "want": [0]} for i in range(3)])
+        for a, c in zip(before, (*eng.kv_cache.k, *eng.kv_cache.v)):
+            assert torch.equal(a[:, :3], c[0][:, :3])
+
+
 class TestPagedPrefill:
     """The prompt kernel on cache blocks gives what it gives on packed rows, bit for
     bit: the same tiles, whatever the blocks' order and the rows past the end hold."""
