@@ -314,17 +314,18 @@ class CausalLM:
 
     def _forward_few_rows(self, residual, positions, kv_cache, meta) -> torch.Tensor:
         """The layers for up to ops.FEW_ROWS rows (a decode step of few
-        sequences): norms, activation and residual addition ride on the
-        projections, which stream the weights once."""
+        sequences): norms, rotation, cache write, activation and residual addition
+        ride on the projections, which stream the weights once."""
         s = self.spec
         act = "gelu_tanh" if s.gelu else "silu"
         n_layers = len(self.layers)
         h = self._norm(residual, self.layers[0].input_norm) if s.post_norms else None
         for i, lw in enumerate(self.layers):
+            cache = (kv_cache.k[i], kv_cache.v[i], positions, self.rope_cache, meta.slot_mapping)
             if s.post_norms:
-                qkv = ops.few_rows_linear(h, lw.qkv, lw.qkv_bias)
+                qkv = ops.few_rows_qkv(h, lw.qkv, lw.qkv_bias, None, 0.0, 0.0, *cache)
                 y = ops.few_rows_linear(
-                    self._attention(i, qkv, positions, kv_cache, meta), lw.o)
+                    self._attention(i, qkv, positions, kv_cache, meta, cached=True), lw.o)
                 h, residual = ops.norm_add_norm(
                     y, residual, lw.post_attn_norm, lw.pre_mlp_norm, s.rms_eps, self.norm_offset)
                 y = ops.few_rows_linear(ops.few_rows_linear(h, lw.gate_up, act=act), lw.down)
@@ -332,10 +333,10 @@ class CausalLM:
                 h, residual = ops.norm_add_norm(
                     y, residual, lw.post_mlp_norm, w_next, s.rms_eps, self.norm_offset)
                 continue
-            qkv = ops.few_rows_linear(residual, lw.qkv, lw.qkv_bias, lw.input_norm,
-                                      s.rms_eps, self.norm_offset)
-            ops.few_rows_linear(self._attention(i, qkv, positions, kv_cache, meta), lw.o,
-                                residual=residual)
+            qkv = ops.few_rows_qkv(residual, lw.qkv, lw.qkv_bias, lw.input_norm, s.rms_eps,
+                                   self.norm_offset, *cache)
+            ops.few_rows_linear(self._attention(i, qkv, positions, kv_cache, meta, cached=True),
+                                lw.o, residual=residual)
             a = ops.few_rows_linear(residual, lw.gate_up, None, lw.pre_mlp_norm,
                                     s.rms_eps, self.norm_offset, act=act)
             ops.few_rows_linear(a, lw.down, residual=residual)

@@ -335,6 +335,27 @@ def few_rows_linear(
     return y if residual is None else residual.add_(y)
 
 
+def few_rows_qkv(
+    x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
+    norm: Optional[torch.Tensor], eps: float, offset: float,
+    k_cache: torch.Tensor, v_cache: torch.Tensor, positions: torch.Tensor,
+    cos_sin: torch.Tensor, slot_mapping: torch.Tensor,
+) -> torch.Tensor:
+    """few_rows_linear for q/k/v weights, then rope_and_cache, in one launch:
+    returns the rows [M, q+2kv] with q and k rotated."""
+    if (_use_hip(x) and k_cache.shape[3] % 16 == 0
+            and k_cache.dtype in (torch.bfloat16, torch.float8_e4m3fn)):
+        out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
+        _EXT.stream_qkv(out, x, w, bias, norm, eps, offset, k_cache, v_cache, positions,
+                        cos_sin, slot_mapping)
+        return out
+    kvh, d = k_cache.shape[1], k_cache.shape[3]
+    out = few_rows_linear(x, w, bias, norm, eps, offset)
+    q, k, v = out.view(x.shape[0], -1, d).split([w.shape[0] // d - 2 * kvh, kvh, kvh], dim=1)
+    rope_and_cache(q, k, v, k_cache, v_cache, positions, cos_sin, slot_mapping)
+    return out
+
+
 # --------------------------------------------- projections, 17 to 128 rows --
 # The product stays as fp32 partial sums ("slabs" [parts, M, N]) that the next
 # kernel adds up: norm and residual, or rotation and cache write.

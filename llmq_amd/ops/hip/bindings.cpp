@@ -546,19 +546,18 @@ void skinny_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
 // out = f(x) W^T for up to 16 rows: see stream_gemm.hip. norm_w: x is RMS-normalised
 // first; epi: 0 plain, 1 added to out in place, 2 / 3 SiLU / tanh-GELU of the first
 // half of W's rows times the second half.
-void stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
-                 c10::optional<at::Tensor> bias, c10::optional<at::Tensor> norm_w,
-                 double eps, double offset, long epi) {
+void launch_stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
+                        c10::optional<at::Tensor> bias, c10::optional<at::Tensor> norm_w,
+                        double eps, double offset, long epi, const SgRope& rope = {}) {
   CHECK_GPU(x);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2, "x, w and out must be matrices");
   const int M = x.size(0), K = x.size(1), N = w.size(0);
-  const bool pair = epi >= kSgSilu;
+  const bool pair = epi == kSgSilu || epi == kSgGelu;
   const int cols = pair ? N / 2 : N;
   auto bf16 = [](const at::Tensor& t) { return t.scalar_type() == at::kBFloat16; };
   auto start16 = [](const at::Tensor& t) {
     return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
   };
-  TORCH_CHECK(epi >= kSgPlain && epi <= kSgGelu, "unknown epilogue");
   TORCH_CHECK(bf16(x) && bf16(w) && bf16(out), "x, w and out must be bfloat16");
   TORCH_CHECK(M >= 1 && M <= 16, "1 to 16 rows");
   TORCH_CHECK(w.size(1) == K && out.size(0) == M && out.size(1) == cols, "shapes differ");
@@ -578,14 +577,14 @@ void stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
     np = reinterpret_cast<const __hip_bfloat16*>(norm_w->data_ptr());
   }
   auto go = [&]<int KH, int NW, int KU, bool NORM, int EPI>() {
-    constexpr int RO = EPI >= kSgSilu ? 8 / KH : 16 / KH;
+    constexpr int R = 16 / KH;            // weight rows of a workgroup
     const size_t lds = NORM ? sizeof(short) * (size_t)M * SgTokens<KH>::row(K) : 0;
-    hipLaunchKernelGGL((stream_gemm_kernel<KH, NW, KU, NORM, EPI>), dim3(cols / RO),
+    hipLaunchKernelGGL((stream_gemm_kernel<KH, NW, KU, NORM, EPI>), dim3(N / R),
                        dim3(64 * NW), lds, stream(),
                        reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), out.stride(0),
                        reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()), x.stride(0),
                        reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()), bp, np,
-                       (float)eps, (float)offset, M, N, K);
+                       (float)eps, (float)offset, M, N, K, rope);
   };
   // Slices: as many as the tokens leave room for, up to four (2048 x 8192, one
   // token: 13.0 us with one slice, 8.9 with four; eight gain nothing), because a
@@ -609,6 +608,7 @@ void stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
     if (epi == kSgPlain) slices.template operator()<NORM, kSgPlain>();
     else if (epi == kSgResidual) slices.template operator()<NORM, kSgResidual>();
     else if (epi == kSgSilu) slices.template operator()<NORM, kSgSilu>();
+    else if (epi == kSgRope) slices.template operator()<NORM, kSgRope>();
     else slices.template operator()<NORM, kSgGelu>();
   };
   if (!np) return epilogue.template operator()<false>();
@@ -620,7 +620,41 @@ void stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
     return epilogue.template operator()<true>();
   at::Tensor h = at::empty({M, K}, x.options());
   rmsnorm(h, x.is_contiguous() ? x : x.contiguous(), *norm_w, eps, offset);
-  stream_gemm(out, h, w, bias, c10::nullopt, 0, 0, epi);
+  launch_stream_gemm(out, h, w, bias, c10::nullopt, 0, 0, epi, rope);
+}
+
+void stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
+                 c10::optional<at::Tensor> bias, c10::optional<at::Tensor> norm_w,
+                 double eps, double offset, long epi) {
+  TORCH_CHECK(epi >= kSgPlain && epi <= kSgGelu, "unknown epilogue");
+  launch_stream_gemm(out, x, w, bias, norm_w, eps, offset, epi);
+}
+
+// out = rmsnorm(x) W^T (+ bias) as q/k/v rows [M, (heads + 2 kv heads) D], q and k
+// rotated, k and v also written into the paged cache.
+void stream_qkv(at::Tensor out, at::Tensor x, at::Tensor w, c10::optional<at::Tensor> bias,
+                c10::optional<at::Tensor> norm_w, double eps, double offset, at::Tensor k_cache,
+                at::Tensor v_cache, at::Tensor positions, at::Tensor cos_sin, at::Tensor slots) {
+  CHECK_GPU(x);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && k_cache.dim() == 4 && cos_sin.dim() == 2);
+  const int M = x.size(0), N = w.size(0), kv_heads = k_cache.size(1), D = k_cache.size(3);
+  const bool fp8 = k_cache.scalar_type() == at::kFloat8_e4m3fn;
+  TORCH_CHECK(D > 0 && D % 16 == 0 && N % D == 0 && N / D > 2 * kv_heads,
+              "w must have (heads + 2 kv heads) D rows, D a multiple of 16");
+  TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous() &&
+                  k_cache.sizes() == v_cache.sizes() &&
+                  k_cache.scalar_type() == v_cache.scalar_type() &&
+                  (fp8 || k_cache.scalar_type() == at::kBFloat16),
+              "caches must be contiguous, bfloat16 or e4m3");
+  TORCH_CHECK(positions.scalar_type() == at::kLong && positions.numel() == M &&
+                  slots.scalar_type() == at::kLong && slots.numel() == M &&
+                  positions.is_contiguous() && slots.is_contiguous() &&
+                  cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous() &&
+                  cos_sin.size(1) == D, "one int64 position and slot per row, fp32 cos_sin [*, D]");
+  launch_stream_gemm(out, x, w, bias, norm_w, eps, offset, kSgRope,
+                     SgRope{k_cache.data_ptr(), v_cache.data_ptr(), positions.data_ptr<long>(),
+                            slots.data_ptr<long>(), cos_sin.data_ptr<float>(),
+                            N / D - 2 * kv_heads, kv_heads, D, (int)k_cache.size(2), fp8});
 }
 
 // ------------------------------------------- projections, 17 to 128 rows --
@@ -953,6 +987,7 @@ TORCH_LIBRARY(llmq_amd, m) {
   m.def("paged_decode_attention(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor context_lens, float scale, float softcap, int window) -> ()");
   m.def("varlen_prefill_attention(Tensor(a!) out, Tensor q, Tensor k, Tensor v, Tensor cu_seqlens, Tensor cu_seqlens_k, int max_seqlen, float scale, float softcap, int window) -> ()");
   m.def("paged_prefill_attention(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor cu_seqlens, Tensor cu_seqlens_k, int max_seqlen, float scale, float softcap, int window) -> ()");
+  m.def("stream_qkv(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, Tensor? norm_w, float eps, float offset, Tensor(b!) k_cache, Tensor(c!) v_cache, Tensor positions, Tensor cos_sin, Tensor slots) -> ()");
   m.def("slab_linear(Tensor x, Tensor w) -> Tensor");
   m.def("slab_act_linear(Tensor x, Tensor w, bool gelu) -> Tensor");
   m.def("slab_add_norm(Tensor slabs, Tensor(a!) residual, Tensor? w_post, Tensor w, float eps, float offset) -> Tensor");
@@ -987,6 +1022,7 @@ TORCH_LIBRARY_IMPL(llmq_amd, CUDA, m) {
   m.impl("softcap_logits", &softcap_logits);
   m.impl("skinny_gemm", &skinny_gemm);
   m.impl("stream_gemm", &stream_gemm);
+  m.impl("stream_qkv", &stream_qkv);
   m.impl("norm_add_norm", &norm_add_norm);
   m.impl("rope_and_cache", &rope_and_cache);
 }

@@ -22,6 +22,10 @@
 //     weights' bytes leave time for.)
 //   - RES: the sums are added to the residual in place. ACT: half of the weight
 //     rows are gates, half the values that they act on (x = [gate | up]).
+//   - ROPE (the q/k/v projection): a workgroup takes channel pairs of one head, rotates
+//     q and k and writes k and v into the paged cache too; positions and
+//     angles are read while the weights travel. A launch of its own for that took 4.5 us
+//     a layer (a step of llama-3.2-1b, one sequence: 902 us, 873 without it).
 
 #include "common.h"
 
@@ -31,7 +35,17 @@ typedef __attribute__((ext_vector_type(4))) float sg_f32x4;
 typedef __attribute__((ext_vector_type(2))) float sg_f32x2;
 typedef __attribute__((ext_vector_type(2))) __bf16 sg_bf16x2;
 
-enum : int { kSgPlain = 0, kSgResidual = 1, kSgSilu = 2, kSgGelu = 3 };
+enum : int { kSgPlain = 0, kSgResidual = 1, kSgSilu = 2, kSgGelu = 3, kSgRope = 4 };
+
+// What kSgRope needs: the paged caches [blocks, kv_heads, bs, D] (bf16 or e4m3),
+// cos_sin [positions, D] as cosines | sines, a cache slot per row (negative: none).
+struct SgRope {
+  void *k_cache, *v_cache;
+  const long *positions, *slots;
+  const float* cos_sin;
+  int heads, kv_heads, D, bs;
+  bool fp8;
+};
 
 // Places of weighted tokens in LDS (shorts): the 16 columns of an operand read lie in
 // 16 different 16-byte bank groups where slices are multiples of 128.
@@ -49,10 +63,10 @@ __global__ __launch_bounds__(64 * NW) void stream_gemm_kernel(
     const __hip_bfloat16* __restrict__ x, long x_stride,
     const __hip_bfloat16* __restrict__ wt, const __hip_bfloat16* __restrict__ bias,
     const __hip_bfloat16* __restrict__ norm_w, float eps, float offset,
-    int M, int N, int K) {
+    int M, int N, int K, SgRope rope) {
   constexpr int R = 16 / KH, MP = 16 / KH, KC = 32 * KU;   // weight rows, token places
-  constexpr bool PAIR = EPI == kSgSilu || EPI == kSgGelu;
-  constexpr int RO = PAIR ? R / 2 : R;                     // output columns
+  constexpr bool PAIR = EPI >= kSgSilu;
+  constexpr int RO = PAIR ? R / 2 : R;                     // output columns (kSgRope: pairs)
   constexpr int RP = 17;
   __shared__ float red[NW][16 * RP];
   __shared__ float sums[NW][16];
@@ -60,9 +74,13 @@ __global__ __launch_bounds__(64 * NW) void stream_gemm_kernel(
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
   const int ks = K / KH;
-  const int n0 = blockIdx.x * RO;
+  // a pair's second row lies `apart` rows behind its first; halves of a head are pairs
+  const int half = EPI == kSgRope ? rope.D / 2 : 0;
+  const int head = EPI == kSgRope ? blockIdx.x * RO / half : 0;
+  const int n0 = blockIdx.x * RO + head * half;
+  const int apart = EPI == kSgRope ? half : N / 2;
   const int i = col % R;
-  const int wrow = PAIR ? (i < RO ? n0 + i : N / 2 + n0 + i - RO) : n0 + i;
+  const int wrow = PAIR && i >= RO ? apart + n0 + i - RO : n0 + i;
   const long kslice = (long)(col / R) * ks + grp * 8;
   const __hip_bfloat16* wp = wt + (long)wrow * K + kslice;
   const __hip_bfloat16* xp = x + (long)min(col % MP, M - 1) * x_stride + kslice;
@@ -78,7 +96,22 @@ __global__ __launch_bounds__(64 * NW) void stream_gemm_kernel(
       f[u] = __builtin_nontemporal_load(reinterpret_cast<const sg_s16x8*>(wp + k0 + u * 32));
   };
   int k0 = w * KC;
+  long slot = -1, position = 0;
+  float cosine = 1.f, sine = 0.f;
+  if constexpr (EPI == kSgRope) {      // one sum per thread: 4 RO MP <= 64 NW
+    const int m = min(((int)threadIdx.x >> 2) / RO, M - 1);
+    position = rope.positions[m];
+    slot = rope.slots[m];
+  }
   if (k0 < ks) fetch(wf, k0);
+  if constexpr (EPI == kSgRope) {
+    if (head < rope.heads + rope.kv_heads) {
+      const float* cs = rope.cos_sin + position * rope.D + (n0 - head * rope.D) +
+                        (threadIdx.x >> 2) % RO;
+      cosine = cs[0];
+      sine = cs[half];
+    }
+  }
   if constexpr (NORM) {
     for (int m = 0; m < M; ++m) {
       float ss = 0.f;
@@ -131,6 +164,7 @@ __global__ __launch_bounds__(64 * NW) void stream_gemm_kernel(
     s += __shfl_xor(s, 2, WAVE);
     return s;
   };
+  static_assert(EPI != kSgRope || 4 * RO * MP <= 64 * NW, "angles of one sum per thread");
   for (int t = threadIdx.x; t < 4 * RO * MP; t += 64 * NW) {
     const int part = t & 3, row = (t >> 2) % RO, m = (t >> 2) / RO;
     float y = total(m, row, part);
@@ -148,7 +182,32 @@ __global__ __launch_bounds__(64 * NW) void stream_gemm_kernel(
     const int n = n0 + row;
     y *= inv;
     if (bias) y += to_f32(bias[n]);
-    if constexpr (PAIR) {
+    if constexpr (EPI == kSgRope) {
+      up *= inv;
+      if (bias) up += to_f32(bias[n + half]);
+      const __hip_bfloat16 a = __float2bfloat16(y * cosine - up * sine);
+      const __hip_bfloat16 b = __float2bfloat16(up * cosine + y * sine);
+      __hip_bfloat16* o = out + (long)m * out_stride + n;
+      o[0] = a;
+      o[half] = b;
+      if (head < rope.heads || slot < 0) continue;
+      const bool is_v = head >= rope.heads + rope.kv_heads;
+      const int kh = head - rope.heads - (is_v ? rope.kv_heads : 0);
+      const long at = ((slot / rope.bs * rope.kv_heads + kh) * rope.bs + slot % rope.bs) * rope.D +
+                      n - head * rope.D;
+      void* cache = is_v ? rope.v_cache : rope.k_cache;
+      if (rope.fp8) {                      // from the rounded rows, as elsewhere
+        __hip_fp8_e4m3* c = static_cast<__hip_fp8_e4m3*>(cache) + at;
+        c[0] = from_f32<__hip_fp8_e4m3>(to_f32(a));
+        c[half] = from_f32<__hip_fp8_e4m3>(to_f32(b));
+      } else {
+        __hip_bfloat16* c = static_cast<__hip_bfloat16*>(cache) + at;
+        c[0] = a;
+        c[half] = b;
+      }
+      continue;
+    }
+    if constexpr (EPI == kSgSilu || EPI == kSgGelu) {
       up *= inv;
       if constexpr (EPI == kSgSilu) {
         y = y / (1.0f + __expf(-y)) * up;

@@ -509,6 +509,50 @@ class TestFewRowsLinear:
         tol = 2 ** -8 * ref.abs() + 1e-5 * mag + 1e-6
         assert ((got.double() - ref).abs() <= tol).all()
 
+    @pytest.mark.parametrize("M", [1, 4, 5, 9, 16])
+    @pytest.mark.parametrize("H,KVH,D,K", [(8, 2, 64, 384), (3, 1, 128, 1536), (2, 1, 256, 3584),
+                                           (4, 2, 16, 128), (192, 1, 128, 2048)])
+    @pytest.mark.parametrize("norm", [False, True])
+    @pytest.mark.parametrize("fp8", [False, True])
+    def test_rotated_rows_and_cache_vs_64_bits(self, M, H, KVH, D, K, norm, fp8):
+        """q/k/v with rotation and cache write: heads' edges, the large-matrix
+        split, a row without a slot."""
+        N = (H + 2 * KVH) * D
+        x = torch.randn(M, K, device=DEV, dtype=torch.bfloat16) * 2
+        w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) * K ** -0.5
+        nw = torch.randn(K, device=DEV, dtype=torch.bfloat16) if norm else None
+        bias = torch.randn(N, device=DEV, dtype=torch.bfloat16)
+        pos = torch.randint(0, 500, (M,), device=DEV)
+        slots = torch.randperm(48, device=DEV)[:M]
+        if M > 1:
+            slots[1] = -1
+        cs = torch_ref.build_rope_cache(512, D, 10000.0, DEV)
+        dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+        kc, vc = (torch.zeros(3, KVH, 16, D, device=DEV, dtype=dt) for _ in range(2))
+        got = ops.few_rows_qkv(x, w, bias, nw, 1e-5, 1.0, kc, vc, pos, cs, slots)
+
+        h = x.double()
+        if norm:
+            inv = torch.rsqrt(h.square().mean(-1, keepdim=True) + 1e-5)
+            h = (x.float() * (nw.float() + 1.0)).bfloat16().double() * inv
+            if M > 8 or M * (K + 512) * 2 > 120 << 10:
+                # a norm of its own first; its rows as rounded there, since an operand
+                # that rounds the other way is 2^-8 K^-0.5 of a sum: over 2e-5
+                h = ops.rmsnorm(x, nw, 1e-5, 1.0).double()
+        ref = (h @ w.double().t() + bias.double()).view(M, -1, D)
+        mag = h.norm(dim=-1).view(M, 1, 1) * K ** -0.5 + 1.0     # of one sum with its bias
+        c, s = cs.double()[pos].view(M, 1, D).chunk(2, -1)
+        a, b = ref[:, : H + KVH].chunk(2, -1)
+        ref = torch.cat([torch.cat([a * c - b * s, b * c + a * s], -1), ref[:, H + KVH:]], 1)
+        # rounding, and the fp32 sums of both halves
+        tol = 2 ** -8 * ref.abs() + 2e-5 * mag + 1e-6
+        assert ((got.view(M, -1, D).double() - ref).abs() <= tol).all()
+        for cache, heads in ((kc, slice(H, H + KVH)), (vc, slice(H + KVH, H + 2 * KVH))):
+            want = torch.zeros(48, KVH, D, device=DEV, dtype=torch.float32)
+            rows = slots >= 0
+            want[slots[rows]] = got.view(M, -1, D)[rows][:, heads].to(dt).float()
+            assert torch.equal(cache.float().transpose(1, 2).reshape(48, KVH, D), want)
+
 
 class TestEngineGPU:
     def test_engine_generates_and_graphs_match_eager(self):
