@@ -612,11 +612,15 @@ void launch_stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
     else slices.template operator()<NORM, kSgGelu>();
   };
   if (!np) return epilogue.template operator()<false>();
-  // Every workgroup weights all tokens: worth the launch that it saves for few of
-  // them (17920 x 1536 pairs: seven tokens 24.3 us here, 16.2 + 4 with a norm of its
-  // own; 16384 x 2048 pairs, one token 17.3 and 14.7 + 4). They have to fit beside
-  // the sums (24 KB at the most).
-  if (M <= (pair ? 4 : 8) && (long)M * (K + 512) * 2 <= (120 << 10))
+  // Every workgroup weights all tokens, M K elements in N / R workgroups: worth the
+  // launch that it saves up to 12 million of them, for up to six tokens. Measured (us, in
+  // the launch / a norm of its own): 16384 x 2048 pairs, 1 token (8.4 million)
+  // 18.0 / 18.6, 2 tokens 22.4 / 19.2; 16384 x 3072 pairs, 3 tokens (9.4) 28.1 / 28.9, 4
+  // 29.7 / 28.0; 5120 x 3072, 3 tokens (11.8) 12.2 / 12.6, 8 18.7 / 15.5; 2048 x 1536,
+  // 6 tokens (2.4) 6.5 / 6.4, 8 7.5 / 6.6. They have to fit beside the sums (24 KB at
+  // the most).
+  const int R = large || M > 8 ? 16 : M > 4 ? 8 : 4;
+  if (M <= 6 && (long)(N / R) * M * K <= 12'000'000 && (long)M * (K + 512) * 2 <= (120 << 10))
     return epilogue.template operator()<true>();
   at::Tensor h = at::empty({M, K}, x.options());
   rmsnorm(h, x.is_contiguous() ? x : x.contiguous(), *norm_w, eps, offset);

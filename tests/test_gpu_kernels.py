@@ -471,6 +471,12 @@ class TestFewRowsLinear:
     """Streaming projections of up to 16 rows: each split of K (rows <= 4, 8, 16;
     large matrices), chunk remainders, norm, bias, activation and residual."""
 
+    @staticmethod
+    def _normed_inside(M, N, K):
+        """Whether the projection weights its tokens itself (else a norm runs first)."""
+        rows = 16 if N * K >= 48 << 20 or M > 8 else 8 if M > 4 else 4
+        return M <= 6 and N // rows * M * K <= 12e6 and M * (K + 512) * 2 <= 120 << 10
+
     @pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
     @pytest.mark.parametrize("N,K", [(32, 128), (96, 384), (1536, 640), (16384, 3072),
                                      (64, 14336)])
@@ -486,10 +492,10 @@ class TestFewRowsLinear:
         if norm:   # the kernel's operands: weighted in fp32, rounded, scaled after the sum
             inv = torch.rsqrt(h.square().mean(-1, keepdim=True) + 1e-5)
             h = (x.float() * (nw.float() + 1.0)).bfloat16().double() * inv
-            act_rows = what in ("silu", "gelu_tanh")
-            if M > (4 if act_rows else 8) or M * (K + 512) * 2 > 120 << 10:
-                # a norm of its own first: normalised rows, rounded
-                h = (x.float() * inv.float() * (nw.float() + 1.0)).bfloat16().double()
+            if not self._normed_inside(M, N, K):
+                # a norm of its own first; its rows as rounded there, since an operand
+                # that rounds the other way is 2^-8 K^-0.5 of a sum: over 1e-5
+                h = ops.rmsnorm(x.contiguous(), nw, 1e-5, 1.0).double()
         ref = h @ w.double().t()
         mag = h.norm(dim=-1, keepdim=True) * K ** -0.5       # of one sum
         act = what if what in ("silu", "gelu_tanh") else ""
@@ -535,7 +541,7 @@ class TestFewRowsLinear:
         if norm:
             inv = torch.rsqrt(h.square().mean(-1, keepdim=True) + 1e-5)
             h = (x.float() * (nw.float() + 1.0)).bfloat16().double() * inv
-            if M > 8 or M * (K + 512) * 2 > 120 << 10:
+            if not self._normed_inside(M, N, K):
                 # a norm of its own first; its rows as rounded there, since an operand
                 # that rounds the other way is 2^-8 K^-0.5 of a sum: over 2e-5
                 h = ops.rmsnorm(x, nw, 1e-5, 1.0).double()
