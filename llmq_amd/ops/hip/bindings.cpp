@@ -260,7 +260,7 @@ void launch_paged_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor&
                        reinterpret_cast<const TC*>(vc.data_ptr()), bt.data_ptr<int>(),
                        (int)bt.stride(0), cl.data_ptr<int>(), B, KVH, G, bs_shift, (int)window,
                        (float)(scale * kLog2e), (float)(softcap * kLog2e),
-                       softcap > 0 ? (float)(2 * scale / softcap * kLog2e) : 0.f,
+                       softcap > 0 ? (float)(2 / softcap) : 0.f,
                        part_o.data_ptr<float>(), part_ml.data_ptr<float>());
   };
   if (softcap > 0) go.template operator()<true>();
@@ -376,7 +376,7 @@ void launch_flash_prefill(at::Tensor& out, const PrefillArgs& a) {
                        PAGED ? (int)a.block_tables->stride(0) : 0,
                        PAGED && a.k.size(2) == 32 ? 5 : 4, a.B, H, a.KVH, (int)a.window,
                        (float)(a.scale * kLog2e), (float)(a.softcap * kLog2e),
-                       a.softcap > 0 ? (float)(2 * a.scale / a.softcap * kLog2e) : 0.f, n_qt);
+                       a.softcap > 0 ? (float)(2 / a.softcap) : 0.f, n_qt);
   };
   if (a.block_tables) {
     if (a.softcap > 0) go.template operator()<true, true>();

@@ -251,14 +251,7 @@ __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
         s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], s[t], 0, 0, 0);
       }
     __builtin_amdgcn_s_setprio(0);
-    if constexpr (CAP) {   // cap tanh(x / cap) = cap - 2 cap / (e^(2 x / cap) + 1), log2 domain
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          s[t][r] = fmaf(-2.f * cap_log2, __builtin_amdgcn_rcpf(
-              __builtin_amdgcn_exp2f(s[t][r] * cap_in) + 1.f), cap_log2);
-    }
+    if constexpr (CAP) cap_tile<NT, 16>(s, scale_log2, cap_log2, cap_in);
     if (kt + KT - 1 > wave_first || kt < wave_all) {
       asm volatile("");                                // a branch, not selects on every tile
 #pragma unroll

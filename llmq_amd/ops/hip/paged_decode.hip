@@ -263,18 +263,14 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
         }
       if (more) fetch_k();
 
+      if constexpr (CAP) cap_tile<NK, 4>(s, scale_log2, cap_log2, cap_in);
       const bool ragged = key0 < lo || key0 + KT - 1 > pos;
       float tmax = -INFINITY;
 #pragma unroll
       for (int g = 0; g < NK; ++g)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          float x;
-          if constexpr (CAP)   // cap tanh(s / cap) = cap - 2 cap / (e^(2 s / cap) + 1)
-            x = cap_log2 - 2.f * cap_log2 *
-                    __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(s[g][r] * cap_in) + 1.f);
-          else
-            x = s[g][r] * scale_log2;
+          float x = CAP ? s[g][r] : s[g][r] * scale_log2;
           if (ragged) {
             const int key = key0 + g * 16 + grp * 4 + r;
             x = key >= lo && key <= pos ? x : -INFINITY;

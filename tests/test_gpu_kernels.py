@@ -337,6 +337,45 @@ class TestPrefillRanges:
         assert_close_to_f32_ref(out.cpu(), ref, 5 * 2 ** -9, 2 ** -8)
 
 
+class TestScoreCap:
+    """The score cap in both attention kernels, from caps that saturate (scores of
+    size 4 against 2) to caps that change nothing: tanh near zero, beyond it, and both
+    in one tile."""
+
+    @pytest.mark.parametrize("cap", [2.0, 10.0, 50.0, 1e4, 1e6, 1e8])
+    @pytest.mark.parametrize("D,H,KVH,fp8", [(64, 4, 2, False), (128, 3, 1, False),
+                                             (256, 2, 1, False), (128, 4, 2, True),
+                                             (256, 2, 2, True)])
+    def test_decode_vs_ref(self, cap, D, H, KVH, fp8):
+        lens = [1, 40, 300]
+        kc, vc, bt = _build_cache(len(lens), KVH, D, 16, max(lens), torch.bfloat16)
+        if fp8:
+            kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+        ctx = torch.tensor(lens, dtype=torch.int32, device=DEV)
+        q = 4 * torch.randn(len(lens), H, D, device=DEV, dtype=torch.bfloat16)
+        out = ops.paged_decode_attention(q, kc, vc, bt, ctx, D ** -0.5, cap)
+        ref = torch_ref.paged_decode_attention(
+            q.float().cpu(), kc.float().cpu(), vc.float().cpu(), bt.cpu(), ctx.cpu(),
+            D ** -0.5, cap)
+        # the output's rounding (2^-9, twice that allowed), fp32 scores and sums
+        assert_close_to_f32_ref(out.cpu(), ref, 2e-4, 2 ** -8)
+
+    @pytest.mark.parametrize("cap", [2.0, 10.0, 50.0, 1e4, 1e6, 1e8])
+    @pytest.mark.parametrize("D,H,KVH", [(64, 4, 2), (64, 3, 1), (128, 3, 1), (256, 2, 1),
+                                         (256, 1, 1)])
+    def test_prompt_vs_ref(self, cap, D, H, KVH):
+        lens = [1, 33, 200]
+        cu = torch.tensor([0, 1, 34, 234], dtype=torch.int32, device=DEV)
+        q, k, v = (torch.randn(234, h, D, device=DEV, dtype=torch.bfloat16)
+                   for h in (H, KVH, KVH))
+        q = 4 * q
+        out = ops.varlen_prefill_attention(q, k, v, cu, max(lens), D ** -0.5, cap)
+        ref = torch_ref.varlen_prefill_attention(q.float().cpu(), k.float().cpu(),
+                                                 v.float().cpu(), cu.cpu(), D ** -0.5, cap)
+        # weights rounded to bf16, then the output: as in TestPrefillRanges
+        assert_close_to_f32_ref(out.cpu(), ref, 5 * 2 ** -9, 2 ** -8)
+
+
 class TestSlabProjections:
     """Streaming products of 17 to 128 rows and the kernels that add up their
     partial sums: each row-tile count, K that leaves parts of unequal length."""
