@@ -389,10 +389,21 @@ void launch_flash_prefill(at::Tensor& out, const PrefillArgs& a) {
 
 void launch_flash_prefill_any(at::Tensor& out, const PrefillArgs& args) {
   const int H = args.q.size(1), D = args.q.size(2);
-  const at::Tensor qa = rows_on_16(args.q), ka = rows_on_16(args.k), va = rows_on_16(args.v);
+  at::Tensor qa = rows_on_16(args.q);
+  const at::Tensor ka = rows_on_16(args.k), va = rows_on_16(args.v);
   at::Tensor oa = rows_start_on(out, 8) ? out : out.clone(at::MemoryFormat::Contiguous);
+  // The kernel masks scores with -inf before it scales them: a negative scale goes into
+  // the queries, and zero (every visible key alike) too.
+  double scale = args.scale;
+  if ((float)scale == 0.f) {
+    qa = at::zeros_like(qa, qa.options(), at::MemoryFormat::Contiguous);
+    scale = 1;
+  } else if (scale < 0) {
+    qa = qa.neg().contiguous();
+    scale = -scale;
+  }
   const PrefillArgs a{qa, ka, va, args.cu, args.cu_k, args.block_tables, args.B, args.KVH,
-                      args.scale, args.softcap, args.window, args.max_seqlen};
+                      scale, args.softcap, args.window, args.max_seqlen};
   // Two heads of a kv head on one stream of tiles where the group is even
   // (2 x 64 rows at head size 64, 2 x 128 at 256: 138 against 147 us for
   // 8 x 1024 tokens). Tiles of 32 keys where that buys a third wave per SIMD

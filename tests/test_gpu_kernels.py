@@ -376,6 +376,40 @@ class TestScoreCap:
         assert_close_to_f32_ref(out.cpu(), ref, 5 * 2 ** -9, 2 ** -8)
 
 
+class TestScaleSigns:
+    """Scales that are negative or zero: masked keys stay masked."""
+
+    @pytest.mark.parametrize("factor", [-1.0, 0.0, 1e-30])
+    @pytest.mark.parametrize("softcap,window", [(0.0, 0), (5.0, 0), (0.0, 40)])
+    @pytest.mark.parametrize("D,H,KVH", [(64, 4, 2), (128, 3, 1), (256, 2, 1)])
+    def test_vs_ref(self, factor, softcap, window, D, H, KVH):
+        lens, scale = [1, 33, 100], factor * D ** -0.5
+        cu = torch.tensor([0, 1, 34, 134], dtype=torch.int32, device=DEV)
+        qkv = torch.randn(134, (H + 2 * KVH) * D, device=DEV, dtype=torch.bfloat16)
+        q, k, v = qkv.view(134, -1, D).split([H, KVH, KVH], dim=1)
+        out = ops.varlen_prefill_attention(q, k, v, cu, max(lens), scale, softcap, window)
+        ref = torch_ref.varlen_prefill_attention(
+            q.float().cpu(), k.float().cpu(), v.float().cpu(), cu.cpu(), scale, softcap, window)
+        assert_close_to_f32_ref(out.cpu(), ref, 5 * 2 ** -9, 2 ** -8)  # as in TestPrefillRanges
+        kc, vc, bt = _build_cache(3, KVH, D, 16, 100, torch.bfloat16)
+        ctx = torch.tensor(lens, dtype=torch.int32, device=DEV)
+        rows = q[:3]
+        out = ops.paged_decode_attention(rows, kc, vc, bt, ctx, scale, softcap, window)
+        ref = torch_ref.paged_decode_attention(rows.float().cpu(), kc.float().cpu(),
+                                               vc.float().cpu(), bt.cpu(), ctx.cpu(), scale,
+                                               softcap, window)
+        assert_close_to_f32_ref(out.cpu(), ref, 2e-4, 2 ** -8)         # as in TestDecodeRanges
+        # a portion that continues its context, on cache blocks
+        cu = torch.tensor([0, 1, 21, 51], dtype=torch.int32, device=DEV)
+        cu_k = torch.tensor([0, 1, 34, 134], dtype=torch.int32, device=DEV)
+        got = ops.paged_prefill_attention(q[:51], kc, vc, bt, cu, cu_k, 30, scale, softcap, window)
+        k, v = (torch.cat([c[bt[b].long()].transpose(1, 2).reshape(-1, KVH, D)[:n]
+                           for b, n in enumerate(lens)]).float().cpu() for c in (kc, vc))
+        ref = torch_ref.varlen_prefill_attention(q[:51].float().cpu(), k, v, cu.cpu(), scale,
+                                                 softcap, window, cu_seqlens_k=cu_k.cpu())
+        assert_close_to_f32_ref(got.cpu(), ref, 5 * 2 ** -9, 2 ** -8)
+
+
 class TestSlabProjections:
     """Streaming products of 17 to 128 rows and the kernels that add up their
     partial sums: each row-tile count, K that leaves parts of unequal length."""
