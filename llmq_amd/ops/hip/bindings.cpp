@@ -363,10 +363,12 @@ template <int D, int HP, int WR, int KT, int MINW>
 void launch_flash_prefill(at::Tensor& out, const PrefillArgs& a) {
   constexpr double kLog2e = 1.4426950408889634;
   const int H = a.q.size(1);
+  // Tiles on an axis of their own: one axis holds 2^32 threads, which 2048 sequences of
+  // up to 40000 tokens, 32 heads, would pass.
   const int n_qt = (int)((std::max<long>(a.max_seqlen, 1) + 32 * WR - 1) / (32 * WR));
   auto go = [&]<bool CAP, bool PAGED>() {
     hipLaunchKernelGGL((flash_prefill_kernel<D, HP, WR, KT, MINW, CAP, PAGED>),
-                       dim3((unsigned)(n_qt * (H / HP) * a.B)), dim3(64 * HP * WR), 0, stream(),
+                       dim3(H / HP * a.B, n_qt), dim3(64 * HP * WR), 0, stream(),
                        reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), out.stride(0),
                        reinterpret_cast<const __hip_bfloat16*>(a.q.data_ptr()), a.q.stride(0),
                        reinterpret_cast<const __hip_bfloat16*>(a.k.data_ptr()), a.k.stride(0),
@@ -374,9 +376,9 @@ void launch_flash_prefill(at::Tensor& out, const PrefillArgs& a) {
                        a.cu.data_ptr<int>(), a.cu_k.data_ptr<int>(),
                        PAGED ? a.block_tables->data_ptr<int>() : nullptr,
                        PAGED ? (int)a.block_tables->stride(0) : 0,
-                       PAGED && a.k.size(2) == 32 ? 5 : 4, a.B, H, a.KVH, (int)a.window,
+                       PAGED && a.k.size(2) == 32 ? 5 : 4, H, a.KVH, (int)a.window,
                        (float)(a.scale * kLog2e), (float)(a.softcap * kLog2e),
-                       a.softcap > 0 ? (float)(2 / a.softcap) : 0.f, n_qt);
+                       a.softcap > 0 ? (float)(2 / a.softcap) : 0.f);
   };
   if (a.block_tables) {
     if (a.softcap > 0) go.template operator()<true, true>();

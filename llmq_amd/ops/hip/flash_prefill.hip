@@ -101,19 +101,18 @@ __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
     const __hip_bfloat16* __restrict__ k, long k_stride,
     const __hip_bfloat16* __restrict__ v, long v_stride,
     const int* __restrict__ cu_q, const int* __restrict__ cu_k,
-    const int* __restrict__ block_tables, int bt_stride, int bs_shift, int B, int H, int KVH,
-    int window, float scale_log2, float cap_log2, float cap_in, int n_qt) {
+    const int* __restrict__ block_tables, int bt_stride, int bs_shift, int H, int KVH,
+    int window, float scale_log2, float cap_log2, float cap_in) {
   constexpr int NW = HP * WR, QT = 32 * WR, NT = KT / 32;
   constexpr int KS = D / 16, DT = D / 32, GPR = D / 8;
   constexpr int NI = KT * GPR / 64;                    // 1 KiB loads of a tile's K (and V)
   __shared__ __align__(16) short lds[4 * KT * D];      // [buffer][K | V][KT][D]
 
   const int hg = H / HP;                               // head groups
-  const int nb = hg * B;
-  const int id = blockIdx.x % nb;
+  const int nb = gridDim.x, id = blockIdx.x;
   const int pair = nb % 8 == 0 ? (id % 8) * (nb / 8) + id / 8 : id;
   const int b = pair / hg, h0 = (pair % hg) * HP;
-  const int r0 = (n_qt - 1 - (int)(blockIdx.x / nb)) * QT;
+  const int r0 = (int)(gridDim.y - 1 - blockIdx.y) * QT;
   const int row0 = cu_q[b];
   const int nq = cu_q[b + 1] - row0;
   if (r0 >= nq) return;

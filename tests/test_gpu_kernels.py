@@ -410,6 +410,26 @@ class TestScaleSigns:
         assert_close_to_f32_ref(got.cpu(), ref, 5 * 2 ** -9, 2 ** -8)
 
 
+class TestManyShortPrompts:
+    def test_bound_far_above_the_lengths(self):
+        """2048 prompts of 1 to 3 tokens under a length bound of 40000: 20 million
+        workgroups, more threads than one axis of a grid holds. The bound changes
+        nothing."""
+        H, KVH, D = 32, 8, 64
+        lens = torch.arange(2048) % 3 + 1
+        cu = torch.cat([torch.zeros(1), lens.cumsum(0)]).to(DEV, torch.int32)
+        T = int(lens.sum())
+        q = torch.randn(T, H, D, device=DEV, dtype=torch.bfloat16)
+        kv = torch.randn(2, T, KVH, D, device=DEV, dtype=torch.bfloat16)
+        want = ops.varlen_prefill_attention(q, kv[0], kv[1], cu, 3, D ** -0.5)
+        torch.empty_like(q).fill_(float("nan"))     # what an unwritten output would hold
+        got = ops.varlen_prefill_attention(q, kv[0], kv[1], cu, 40000, D ** -0.5)
+        assert torch.equal(got, want)
+        ref = torch_ref.varlen_prefill_attention(q.float().cpu()[:6], *kv.float().cpu()[:, :6],
+                                                 cu.cpu()[:4], D ** -0.5)
+        assert_close_to_f32_ref(got.cpu()[:6], ref, 5 * 2 ** -9, 2 ** -8)  # as in TestPrefillRanges
+
+
 class TestSlabProjections:
     """Streaming products of 17 to 128 rows and the kernels that add up their
     partial sums: each row-tile count, K that leaves parts of unequal length."""
