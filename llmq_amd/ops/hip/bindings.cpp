@@ -906,8 +906,8 @@ at::Tensor prompt_layers(at::Tensor h, at::Tensor residual, at::TensorList weigh
 bool row_chunks(const at::Tensor& logits, int B, int V, int& chunk, int& splits) {
   int n = 1;
   while (B * n < 2048 && n < 64 && (V / n) > 4096) n *= 2;
-  chunk = ((V + n - 1) / n + 3) / 4 * 4;
-  splits = (V + chunk - 1) / chunk;
+  chunk = std::max(((V + n - 1) / n + 3) / 4 * 4, 4);
+  splits = std::max((V + chunk - 1) / chunk, 1);         // an empty vocabulary launches too
   return V % 4 == 0 && logits.stride(0) % 4 == 0 &&
          reinterpret_cast<uintptr_t>(logits.data_ptr()) % 16 == 0;
 }

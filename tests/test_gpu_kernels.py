@@ -850,6 +850,17 @@ class TestFusedSampler:
             counts, expected)
 
 
+class TestEmptyVocabulary:
+    def test_returns(self):
+        """Logits without columns: a bound and index 0, no division by a chunk of zero."""
+        logits = torch.empty(3, 0, device=DEV)
+        temps, ks = torch.ones(3, device=DEV), torch.zeros(3, dtype=torch.int64, device=DEV)
+        bound = ops.topk_topp_bound(logits, temps, temps * 0.9, ks)
+        out, keys, z = torch.ones_like(ks), torch.ones_like(ks), ks.int()
+        ops.sample_gumbel_argmax(out, keys, logits, temps, z, z, 1, 1, bound)
+        assert (bound < -1e38).all() and (out == 0).all()
+
+
 class TestTruncationRanges:
     """topk_topp_bound and the sampler over chunked rows: odd row lengths (4-byte
     loads), few rows (many chunks), each way a top-k narrows the histogram (up to
