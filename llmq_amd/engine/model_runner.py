@@ -72,10 +72,11 @@ class ModelRunner:
         # layers (per-sequence state slots), get the extra step metadata.
         self.paged_prefill = bool(getattr(model, "paged_prefill", False))
         # Portions on cached context, other models: attention reads a bf16 cache
-        # in place; a cache of another type is gathered into packed rows.
-        self.paged_portions = not self.paged_prefill and device.type == "cuda" and all(
-            t is not None and t.dtype == torch.bfloat16 and model.dtype == torch.bfloat16
-            for t in kv_cache.k + kv_cache.v)
+        # of 16 or 32 tokens a block in place; any other is gathered into packed rows.
+        self.paged_portions = (
+            not self.paged_prefill and device.type == "cuda" and self.block_size in (16, 32)
+            and all(t is not None and t.dtype == torch.bfloat16 and model.dtype == torch.bfloat16
+                    for t in kv_cache.k + kv_cache.v))
         self.recurrent = kv_cache.recurrent if (
             kv_cache.recurrent is not None and kv_cache.recurrent.active) else None
         if self.use_graphs:

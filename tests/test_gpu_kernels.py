@@ -1183,6 +1183,30 @@ class TestChunkedPrefillAttention:
         assert run(4096) == run(96)
 
 
+class TestPortionBlockSizes:
+    @pytest.mark.parametrize("block", [8, 16, 32, 64])
+    def test_continued_portion_matches_whole(self, block):
+        """A replayed prompt in two portions: attention reads blocks of 16 and 32
+        tokens in place and gathers any other."""
+        from llmq_amd.engine.config import EngineConfig
+        from llmq_amd.engine.engine import LLMEngine
+
+        toks = torch.arange(150) * 37 % 500
+        out = []
+        for cuts in ((0, 150), (0, 70, 150)):
+            eng = LLMEngine(EngineConfig(
+                model="tiny-llama-d128", max_num_seqs=2, max_model_len=256, load_weights=False,
+                num_kv_blocks=512 // block, kv_block_size=block, enforce_eager=True))
+            for a, b in zip(cuts, cuts[1:]):
+                want = list(range(70 - a, b - a)) if b == 150 else []
+                logits = eng.replay_step([{"id": "r", "tokens": toks[a:b].tolist(), "want": want}])
+            out.append(logits)
+        # the packed kernel on the same keys, rows in other tiles: bf16 weights
+        # and products of other row counts, two layers
+        err = (out[0] - out[1]).norm() / out[0].norm()
+        assert torch.isfinite(out[1]).all() and err < 0.02
+
+
 class TestPreemptionGPU:
     def test_preemption_under_graphs(self):
         """KV pressure forces evict+recompute while hipGraphs replay decode:
