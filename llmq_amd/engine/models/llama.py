@@ -357,7 +357,8 @@ class CausalLM:
             x = x * math.sqrt(s.hidden_size)
             x = x.to(self.dtype)
         l0 = self.layers[0]
-        if tp is None and ops.few_rows_ok(x, (l0.qkv, l0.o, l0.gate_up, l0.down)):
+        if (tp is None and not _USE_SKINNY_GEMM
+                and ops.few_rows_ok(x, (l0.qkv, l0.o, l0.gate_up, l0.down))):
             return self._forward_few_rows(x, positions, kv_cache, meta)
         residual = x
         h = self._norm(x, self.layers[0].input_norm)

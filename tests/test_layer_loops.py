@@ -257,3 +257,20 @@ def test_loops_vs_64_bits(name, fp8, kind, rows, loops, monkeypatch):
         # its streaming products: the same launches as the slab loop's
         monkeypatch.setattr(CausalLM, "_prompt_layers", CausalLM._forward_slabs)
         assert torch.equal(_run(model, cache, batch), got) and loops[1:] == ["slabs"]
+
+
+@on_gpu
+@pytest.mark.parametrize("kind,rows", [("decode", 1), ("decode", 16), ("decode", 33),
+                                       ("prompt", 7), ("prompt", 40), ("mixed", 9)])
+def test_skinny_gemm_switch(kind, rows, loops, monkeypatch):
+    """LLMQ_SKINNY_GEMM=1 puts every projection of a step on that kernel."""
+    calls = []
+    monkeypatch.setattr(llama, "_USE_SKINNY_GEMM", True)
+    skinny = ops.skinny_gemm
+    monkeypatch.setattr(ops, "skinny_gemm", lambda *a: calls.append(a[1].shape) or skinny(*a))
+    model = _model("llama", "cuda", torch.bfloat16)
+    cache, batch = _cache(model.spec, "cuda", torch.bfloat16), _batch(kind, rows)
+    want = _oracle(model, cache, batch)
+    got = _run(model, cache, batch)
+    assert loops == [] and len(calls) == 4 * model.spec.num_layers + 1
+    assert _off(got, want) < LIMIT
