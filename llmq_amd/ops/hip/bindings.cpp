@@ -640,11 +640,32 @@ void launch_stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
   launch_stream_gemm(out, h, w, bias, c10::nullopt, 0, 0, epi, rope);
 }
 
+// Weights that the streaming kernels read: packed rows from a 16-byte boundary. Others
+// (a transposed or padded view, one inside a larger buffer) go to the library.
+bool streamable(const at::Tensor& w) {
+  return w.is_contiguous() && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0;
+}
+
+// The library's product of the rows, normalised first where weights are given.
+at::Tensor norm_linear(const at::Tensor& x, const at::Tensor& w,
+                       const c10::optional<at::Tensor>& bias,
+                       const c10::optional<at::Tensor>& norm_w, double eps, double offset) {
+  if (!norm_w.has_value() || !norm_w->defined()) return at::linear(x, w, bias);
+  at::Tensor h = at::empty({x.size(0), x.size(1)}, x.options());
+  rmsnorm(h, x.contiguous(), *norm_w, eps, offset);
+  return at::linear(h, w, bias);
+}
+
 void stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
                  c10::optional<at::Tensor> bias, c10::optional<at::Tensor> norm_w,
                  double eps, double offset, long epi) {
   TORCH_CHECK(epi >= kSgPlain && epi <= kSgGelu, "unknown epilogue");
-  launch_stream_gemm(out, x, w, bias, norm_w, eps, offset, epi);
+  if (streamable(w)) return launch_stream_gemm(out, x, w, bias, norm_w, eps, offset, epi);
+  const at::Tensor y = norm_linear(x, w, bias, norm_w, eps, offset);
+  if (epi == kSgPlain) out.copy_(y);
+  else if (epi == kSgResidual) out.add_(y);
+  else if (epi == kSgSilu) silu_and_mul(out, y);
+  else gelu_tanh_and_mul(out, y);
 }
 
 // out = rmsnorm(x) W^T (+ bias) as q/k/v rows [M, (heads + 2 kv heads) D], q and k
@@ -668,6 +689,14 @@ void stream_qkv(at::Tensor out, at::Tensor x, at::Tensor w, c10::optional<at::Te
                   positions.is_contiguous() && slots.is_contiguous() &&
                   cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous() &&
                   cos_sin.size(1) == D, "one int64 position and slot per row, fp32 cos_sin [*, D]");
+  if (!streamable(w)) {
+    out.copy_(norm_linear(x, w, bias, norm_w, eps, offset));
+    const at::Tensor heads = out.view({M, N / D, D});
+    const long q = N / D - 2 * kv_heads;
+    return rope_and_cache(heads.narrow(1, 0, q), heads.narrow(1, q, kv_heads),
+                          heads.narrow(1, q + kv_heads, kv_heads), k_cache, v_cache, positions,
+                          cos_sin, slots);
+  }
   launch_stream_gemm(out, x, w, bias, norm_w, eps, offset, kSgRope,
                      SgRope{k_cache.data_ptr(), v_cache.data_ptr(), positions.data_ptr<long>(),
                             slots.data_ptr<long>(), cos_sin.data_ptr<float>(),
@@ -679,8 +708,7 @@ void stream_qkv(at::Tensor out, at::Tensor x, at::Tensor w, c10::optional<at::Te
 bool slab_rows_ok(const at::Tensor& x, const at::Tensor& w) {
   return x.dim() == 2 && w.dim() == 2 && x.size(0) > 16 && x.size(0) <= 128 &&
          x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 &&
-         x.stride(1) == 1 && rows_start_on(x, 16) && w.is_contiguous() &&
-         reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 && x.size(1) == w.size(1) &&
+         x.stride(1) == 1 && rows_start_on(x, 16) && x.size(1) == w.size(1) &&
          w.size(1) % kSlabBK == 0 && w.size(1) > 0 && w.size(0) % 64 == 0;
 }
 
@@ -724,6 +752,7 @@ at::Tensor slab_linear(const at::Tensor& x, const at::Tensor& w) {
   CHECK_GPU(x);
   TORCH_CHECK(slab_rows_ok(x, w),
               "slab_linear: 17 to 128 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
+  if (!streamable(w)) return at::linear(x, w).to(at::kFloat).unsqueeze(0);
   const int parts = slab_parts(w.size(0), w.size(1));
   at::Tensor slabs = at::empty({parts, x.size(0), w.size(0)}, x.options().dtype(at::kFloat));
   launch_slab_gemm<kSlabSums>(slabs.data_ptr<float>(), nullptr, 0, x, w, parts);
@@ -742,6 +771,12 @@ at::Tensor slab_act_linear(const at::Tensor& x, const at::Tensor& w, bool gelu) 
   TORCH_CHECK(slab_rows_ok(x, w) && x.size(0) <= 64,
               "slab_act_linear: 17 to 64 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
   at::Tensor out = at::empty({x.size(0), w.size(0) / 2}, x.options());
+  if (!streamable(w)) {
+    const at::Tensor y = at::linear(x, w);
+    if (gelu) gelu_tanh_and_mul(out, y);
+    else silu_and_mul(out, y);
+    return out;
+  }
   auto* p = reinterpret_cast<__hip_bfloat16*>(out.data_ptr());
   if (gelu) launch_slab_gemm<kSlabGelu>(nullptr, p, out.stride(0), x, w, 1);
   else launch_slab_gemm<kSlabSilu>(nullptr, p, out.stride(0), x, w, 1);

@@ -274,3 +274,30 @@ def test_skinny_gemm_switch(kind, rows, loops, monkeypatch):
     got = _run(model, cache, batch)
     assert loops == [] and len(calls) == 4 * model.spec.num_layers + 1
     assert _off(got, want) < LIMIT
+
+
+def _layouts(w):
+    """The same weights as a transposed view, with padded rows, off a 16-byte boundary."""
+    padded = torch.zeros(w.shape[0], w.shape[1] + 8, dtype=w.dtype, device=w.device)
+    padded[:, :w.shape[1]] = w
+    moved = torch.zeros(w.numel() + 4, dtype=w.dtype, device=w.device)
+    moved[4:] = w.reshape(-1)
+    return [w.t().contiguous().t(), padded[:, :w.shape[1]], moved[4:].view(w.shape)]
+
+
+@on_gpu
+@pytest.mark.parametrize("kind,rows", [("decode", 5), ("decode", 16), ("decode", 33),
+                                       ("decode", 65), ("decode", 129), ("prompt", 16),
+                                       ("prompt", 40), ("portion", 200), ("mixed", 9)])
+@pytest.mark.parametrize("layer", [0, 1])
+@pytest.mark.parametrize("name", ["llama", "qwen2", "gemma2"])
+def test_weight_layouts(name, layer, kind, rows):
+    """Weights of one layer that are no packed, aligned matrices."""
+    model = _model(name, "cuda", torch.bfloat16)
+    cache, batch = _cache(model.spec, "cuda", torch.bfloat16), _batch(kind, rows)
+    want = _oracle(model, cache, batch)
+    lw = model.layers[layer]
+    for turn in range(3):
+        for i, which in enumerate(("qkv", "o", "gate_up", "down")):
+            setattr(lw, which, _layouts(getattr(lw, which))[(i + turn) % 3])
+        assert _off(_run(model, cache, batch), want) < LIMIT
