@@ -556,6 +556,18 @@ void skinny_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
 
 // --------------------------------------------------- projections, few rows --
 
+// Weights that the streaming kernels read: packed rows from a 16-byte boundary. Others
+// (a transposed or padded view, one inside a larger buffer) go to the library.
+bool streamable(const at::Tensor& w) {
+  return w.is_contiguous() && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0;
+}
+
+// A norm's weights or a bias as the kernels read them: a copy of any that is a strided
+// view or starts elsewhere.
+at::Tensor packed(const at::Tensor& t) {
+  return streamable(t) ? t : t.clone(at::MemoryFormat::Contiguous);
+}
+
 // out = f(x) W^T for up to 16 rows: see stream_gemm.hip. norm_w: x is RMS-normalised
 // first; epi: 0 plain, 1 added to out in place, 2 / 3 SiLU / tanh-GELU of the first
 // half of W's rows times the second half.
@@ -580,13 +592,14 @@ void launch_stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
               "w must be contiguous, x's rows start on 16 bytes, rows packed");
   const __hip_bfloat16 *bp = nullptr, *np = nullptr;
   if (bias.has_value() && bias->defined()) {
-    TORCH_CHECK(bf16(*bias) && bias->is_contiguous() && bias->numel() == N && !pair,
+    TORCH_CHECK(bf16(*bias) && bias->numel() == N && !pair,
                 "bias must be bfloat16 [N], without an activation");
+    bias = packed(*bias);
     bp = reinterpret_cast<const __hip_bfloat16*>(bias->data_ptr());
   }
   if (norm_w.has_value() && norm_w->defined()) {
-    TORCH_CHECK(bf16(*norm_w) && norm_w->is_contiguous() && norm_w->numel() == K &&
-                    start16(*norm_w), "norm weights must be bfloat16 [K]");
+    TORCH_CHECK(bf16(*norm_w) && norm_w->numel() == K, "norm weights must be bfloat16 [K]");
+    norm_w = packed(*norm_w);
     np = reinterpret_cast<const __hip_bfloat16*>(norm_w->data_ptr());
   }
   auto go = [&]<int KH, int NW, int KU, bool NORM, int EPI>() {
@@ -638,12 +651,6 @@ void launch_stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
   at::Tensor h = at::empty({M, K}, x.options());
   rmsnorm(h, x.is_contiguous() ? x : x.contiguous(), *norm_w, eps, offset);
   launch_stream_gemm(out, h, w, bias, c10::nullopt, 0, 0, epi, rope);
-}
-
-// Weights that the streaming kernels read: packed rows from a 16-byte boundary. Others
-// (a transposed or padded view, one inside a larger buffer) go to the library.
-bool streamable(const at::Tensor& w) {
-  return w.is_contiguous() && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0;
 }
 
 // The library's product of the rows, normalised first where weights are given.
@@ -800,20 +807,24 @@ at::Tensor slab_add_norm(const at::Tensor& slabs, at::Tensor residual,
                   residual.numel() == (long)M * N && N % 4 == 0 && N <= 8192,
               "residual must be contiguous bf16 [M, N], N a multiple of 4 up to 8192");
   auto weights = [&](const at::Tensor& t) {
-    TORCH_CHECK(t.is_contiguous() && t.scalar_type() == at::kBFloat16 && t.numel() == N,
+    TORCH_CHECK(t.scalar_type() == at::kBFloat16 && t.numel() == N,
                 "norm weights must be bf16 [N]");
-    return reinterpret_cast<const __hip_bfloat16*>(t.data_ptr());
+    return packed(t);
   };
+  const bool post = w_post.has_value() && w_post->defined();
+  const at::Tensor wp = post ? weights(*w_post) : at::Tensor(), wn = weights(w);
   at::Tensor h = at::empty_like(residual);
   auto go = [&]<bool POST>() {
     const int threads = std::min(kSlabNT, (N / 4 + 63) / 64 * 64);
     hipLaunchKernelGGL(slab_add_norm_kernel<POST>, dim3(M), dim3(threads), 0, stream(),
                        reinterpret_cast<__hip_bfloat16*>(h.data_ptr()),
                        reinterpret_cast<__hip_bfloat16*>(residual.data_ptr()),
-                       slabs.data_ptr<float>(), S, POST ? weights(*w_post) : nullptr, weights(w),
-                       M, N, (float)eps, (float)offset);
+                       slabs.data_ptr<float>(), S,
+                       POST ? reinterpret_cast<const __hip_bfloat16*>(wp.data_ptr()) : nullptr,
+                       reinterpret_cast<const __hip_bfloat16*>(wn.data_ptr()), M, N, (float)eps,
+                       (float)offset);
   };
-  if (w_post.has_value() && w_post->defined()) go.template operator()<true>();
+  if (post) go.template operator()<true>();
   else go.template operator()<false>();
   return h;
 }
@@ -835,8 +846,9 @@ at::Tensor slab_rope_cache(const at::Tensor& slabs, c10::optional<at::Tensor> bi
                   cos_sin.size(1) == D);
   const __hip_bfloat16* bp = nullptr;
   if (bias.has_value() && bias->defined()) {
-    TORCH_CHECK(bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() &&
-                bias->numel() == N, "bias must be bf16 [N]");
+    TORCH_CHECK(bias->scalar_type() == at::kBFloat16 && bias->numel() == N,
+                "bias must be bf16 [N]");
+    bias = packed(*bias);
     bp = reinterpret_cast<const __hip_bfloat16*>(bias->data_ptr());
   }
   at::Tensor qkv = at::empty({M, N}, slabs.options().dtype(at::kBFloat16));

@@ -301,3 +301,21 @@ def test_weight_layouts(name, layer, kind, rows):
         for i, which in enumerate(("qkv", "o", "gate_up", "down")):
             setattr(lw, which, _layouts(getattr(lw, which))[(i + turn) % 3])
         assert _off(_run(model, cache, batch), want) < LIMIT
+
+
+@on_gpu
+@pytest.mark.parametrize("kind,rows", [("decode", 1), ("decode", 12), ("decode", 33),
+                                       ("prompt", 40), ("mixed", 9)])
+@pytest.mark.parametrize("name", ["qwen2", "gemma2"])
+def test_vector_layouts(name, kind, rows):
+    """A bias that is a strided view, norm weights 8 bytes off a 16-byte boundary."""
+    model = _model(name, "cuda", torch.bfloat16)
+    cache, batch = _cache(model.spec, "cuda", torch.bfloat16), _batch(kind, rows)
+    want = _oracle(model, cache, batch)
+    lw = model.layers[1]
+    for which in ("input_norm", "pre_mlp_norm", "post_attn_norm", "post_mlp_norm"):
+        if getattr(lw, which) is not None:
+            setattr(lw, which, torch.cat([getattr(lw, which)[:4], getattr(lw, which)])[4:])
+    if lw.qkv_bias is not None:
+        lw.qkv_bias = lw.qkv_bias.repeat_interleave(2)[::2]
+    assert _off(_run(model, cache, batch), want) < LIMIT
