@@ -45,7 +45,11 @@ __global__ __launch_bounds__(256 * WK) void slab_gemm_kernel(
   const int loops = (total + WK - 1) / WK;
   const int n0 = blockIdx.x * (PAIR ? 32 : 64);
   const int wrow = PAIR ? (nt < 2 ? n0 + nt * 16 : N / 2 + n0 + (nt - 2) * 16) : n0 + nt * 16;
-  const __hip_bfloat16* wp = wt + (long)(wrow + col) * K + (long)step0 * kSlabBK + grp * 8;
+  // Through an opaque asm: as a plain kernel argument that nothing aliases, the compiler
+  // might move its loads across the barriers' memory clobbers, and step() counts them.
+  auto wp = (const __attribute__((address_space(1))) __hip_bfloat16*)(
+      wt + (long)(wrow + col) * K + (long)step0 * kSlabBK + grp * 8);
+  asm volatile("" : "+v"(wp) :: "memory");
   // staging: load j of this wave fills rows 4 (nt + 4 j) + lane/16 of its group's tile
   const int srow = nt * 4 + (lane >> 4);
   const int sgran = ((lane & 15) ^ (srow & 15)) << 3;
@@ -60,19 +64,22 @@ __global__ __launch_bounds__(256 * WK) void slab_gemm_kernel(
 #pragma unroll
     for (int j = 0; j < TM; ++j)
       glds16(xp[j] + s * kSlabBK, mine + (i & 1) * (WK * TILE) + (nt + j * 4) * 512);
+    __builtin_amdgcn_sched_barrier(0);                        // before any weights
   };
   auto fetch = [&](sl_s16x8 (&f)[4], int i) {
     const int s = min(i * WK + kg, total - 1);                // past the end: unused
 #pragma unroll
     for (int u = 0; u < 4; ++u)
       f[u] = __builtin_nontemporal_load(
-          reinterpret_cast<const sl_s16x8*>(wp + s * kSlabBK + u * 32));
+          reinterpret_cast<const __attribute__((address_space(1))) sl_s16x8*>(
+              wp + s * kSlabBK + u * 32));
   };
   sl_f32x4 acc[TM];
 #pragma unroll
   for (int m = 0; m < TM; ++m) acc[m] = sl_f32x4{0.f, 0.f, 0.f, 0.f};
   auto step = [&](int i, sl_s16x8 (&f)[4]) {
-    // this step's tokens and weights have landed, the next weights may travel
+    // this step's tokens and weights have landed, the next weights may travel: the last
+    // four loads are fetch(i + 1)'s, issued after stage(i)'s and nothing after them
     if (i + 1 < loops) pipe_barrier_vm<4>();
     else pipe_barrier_vm<0>();
     if (i + 1 < loops) stage(i + 1);
@@ -88,6 +95,7 @@ __global__ __launch_bounds__(256 * WK) void slab_gemm_kernel(
         }
     }
     if (i + 2 < loops) fetch(f, i + 2);
+    __builtin_amdgcn_sched_barrier(0);                        // not past the next barrier
   };
   sl_s16x8 wa[4], wb[4];
   stage(0);
