@@ -528,7 +528,7 @@ class ModelRunner:
             # Fused one-pass HIP sampler (gumbel-max / greedy argmax).
             # Top-k/top-p rows reduce to a per-row logit keep-bound via
             # histogram select — no full-vocab sort, no CPU round trips,
-            # seeded rows stay on-device (ADVICE r1 low #4 / weakness 6).
+            # seeded rows stay on-device.
             B = len(seqs)
             buf = self._sample_buf(buf_name, B, dev)
             th = buf["temps_h"]

@@ -278,7 +278,7 @@ def skinny_gemm(
     """Hand-written skinny-M decode-projection GEMM (out = x @ w.T + bias).
 
     256x256x64 MFMA tile, glds-staged with source-side st_16x32 swizzle,
-    counted-vmcnt pipeline; split-K slabs + fused reduce for narrow-N
+    double-buffered with one full wait per K step; split-K slabs + fused reduce for narrow-N
     shapes. Falls back to F.linear off-GPU / unsupported shapes."""
     M, K = x.shape
     N = w.shape[0]

@@ -627,8 +627,8 @@ void launch_stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
   auto slices = [&]<bool NORM, int EPI>() {
     if (large) chunk.template operator()<1, 16, NORM, EPI>();
     else if (M <= 4) chunk.template operator()<4, 8, NORM, EPI>();
-    else if (M <= 8) chunk.template operator()<2, 8, NORM, EPI>();
-    else chunk.template operator()<1, 8, NORM, EPI>();
+    else if (NORM || M <= 8) chunk.template operator()<2, 8, NORM, EPI>();  // norm: M <= 6
+    else if constexpr (!NORM) chunk.template operator()<1, 8, NORM, EPI>();
   };
   auto epilogue = [&]<bool NORM>() {
     if (epi == kSgPlain) slices.template operator()<NORM, kSgPlain>();

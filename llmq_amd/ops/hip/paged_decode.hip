@@ -1,6 +1,7 @@
 // Single-token GQA attention over the paged cache on the matrix cores (gfx950):
-// bf16 queries, bf16 or fp8 (OCP e4m3) cache, head size 64, 128 or 256, up to 16
-// query heads per kv head, optional score cap and sliding window.
+// bf16 queries; head size 128 or 256 with a bf16 or fp8 (OCP e4m3) cache and up to 16
+// query heads per kv head, head size 64 with a bf16 cache and up to 8; optional score
+// cap and sliding window.
 //
 // Bound by the cache's bytes: at 16 query columns the products take a few percent
 // of the matrix cores, so everything here serves to keep loads in flight on all
@@ -17,7 +18,10 @@
 //     the tiles of the whole batch, in order, are dealt to a fixed number of waves
 //     in equal contiguous ranges. Every wave finds its range by itself from
 //     context_lens, so lengths may differ and change under a captured graph, and
-//     neither a long sequence nor a last round of workgroups leaves CUs idle.
+//     neither a long sequence nor a last round of workgroups leaves CUs idle. Where a
+//     sequence is cut, and with it the order of its sums, depends on the lengths of the
+//     whole batch and on the table's width: its result may differ in the last bf16
+//     digit between batches, and between a captured graph and an eager call.
 //   - Waves are independent: no barrier anywhere. K operands come straight from
 //     memory in matrix layout; V rows pass through a wave-private LDS tile
 //     (row-major, 32-byte column groups swizzled by key) and are read transposed

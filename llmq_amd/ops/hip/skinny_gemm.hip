@@ -7,7 +7,8 @@
 // both operands are k-contiguous ([M,K] activations, [N,K] torch linear
 // weights), staged to LDS by global_load_lds with the st_16x32 XOR swizzle
 // on the SOURCE address (lane-linear dest, rule 21), MFMA 16x16x32_bf16,
-// counted-vmcnt software pipeline with raw barriers.
+// double-buffered: the next K step travels during the current one's products, one
+// full wait and raw barrier per step.
 //
 // Split-K: gridDim.z slices of K accumulate fp32 partial slabs
 // [SPLITK, M, N]; a separate reduce kernel folds them (+ optional bias) to

@@ -2,12 +2,16 @@
 // an ordinary decode step or a short prompt (gfx950).
 //
 // Bound by the weights' bytes. A workgroup owns 64 weight rows, all M tokens and one
-// of S parts of K. Weights go straight from memory into the matrix layout, two
-// 128-wide K steps ahead; the tokens, which every workgroup reads again, are staged
-// once per workgroup in LDS by global_load_lds (16-byte granules placed by row, so
-// operand reads meet no bank conflict), one step ahead. v_mfma_f32_16x16x32_bf16,
-// A = weights (row = lane%16, k = 8*(lane/16)..+7), B = tokens likewise, C: column =
-// token, rows = 4 weight rows.
+// of S parts of K. Weights go straight from memory into the matrix layout; the tokens,
+// which every workgroup reads again, are staged once per workgroup in LDS by
+// global_load_lds (16-byte granules placed by row, so operand reads meet no bank
+// conflict). v_mfma_f32_16x16x32_bf16, A = weights (row = lane%16, k =
+// 8*(lane/16)..+7), B = tokens likewise, C: column = token, rows = 4 weight rows.
+// A step of 128 channels asks for the next step's tokens at its start and for the
+// weights of the one after at its end, but its products wait for both: the loads sit
+// under conditions, and the compiler's count of what may still travel is the least over
+// all paths. What overlaps is the weights' way with one step's end and the next's
+// barrier: 2.6 to 2.7 TB/s, where decode attention reads 5.8.
 //
 // With S > 1 the parts are left as fp32 slabs [S, M, N] and added up by the kernel
 // that reads them anyway (norm and residual, rotation and cache write): the sum
@@ -25,17 +29,17 @@ enum : int { kSlabSums = 0, kSlabSilu = 1, kSlabGelu = 2 };
 
 constexpr int kSlabBK = 128;
 
-// TM: token tiles of 16; WK: groups of four waves that take the K steps in turn.
+// TM: token tiles of 16; WK: groups of four waves that take the K steps in turn (gate
+// and value rows, whose sums have to be whole; else parts of K do that).
 template <int TM, int WK, int EPI>
 __global__ __launch_bounds__(256 * WK) void slab_gemm_kernel(
     float* __restrict__ slabs, __hip_bfloat16* __restrict__ out, long out_stride,
     const __hip_bfloat16* __restrict__ x, long x_stride,
     const __hip_bfloat16* __restrict__ wt, int M, int N, int K, int steps_per_split) {
   constexpr bool PAIR = EPI != kSlabSums;
+  static_assert(PAIR || WK == 1, "groups' sums meet in LDS for gate and value rows only");
   constexpr int ROWS = TM * 16, TILE = ROWS * kSlabBK;       // one staged token tile
-  constexpr int RED = 4 * WK * TM * 256 * 2;                  // fp32 sums, in shorts
-  constexpr int STAGE = 2 * WK * TILE;
-  __shared__ __align__(16) short lds[STAGE > RED ? STAGE : RED];
+  __shared__ __align__(16) short lds[2 * WK * TILE];         // and fewer fp32 sums later
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nt = w & 3, kg = w >> 2;
@@ -106,7 +110,7 @@ __global__ __launch_bounds__(256 * WK) void slab_gemm_kernel(
     if (i + 1 < loops) step(i + 1, wb);
   }
 
-  if constexpr (!PAIR && WK == 1) {
+  if constexpr (!PAIR) {
     float* slab = slabs + (long)blockIdx.y * M * N + wrow + grp * 4;
 #pragma unroll
     for (int m = 0; m < TM; ++m)
@@ -121,8 +125,7 @@ __global__ __launch_bounds__(256 * WK) void slab_gemm_kernel(
   for (int m = 0; m < TM; ++m)
     *reinterpret_cast<sl_f32x4*>(red + ((w * TM + m) * 64 + lane) * 4) = acc[m];
   __syncthreads();
-  constexpr int UNITS = TM * (PAIR ? 2 : 4);                  // (n tile, m tile) of 64 lanes
-  for (int unit = w; unit < UNITS; unit += 4 * WK) {
+  for (int unit = w; unit < 2 * TM; unit += 4 * WK) {         // (n tile, m tile) of 64 lanes
     const int t = unit / TM, m = unit % TM;
     auto sum = [&](int tile) {
       sl_f32x4 s = *reinterpret_cast<const sl_f32x4*>(red + ((tile * TM + m) * 64 + lane) * 4);
@@ -133,26 +136,19 @@ __global__ __launch_bounds__(256 * WK) void slab_gemm_kernel(
       return s;
     };
     const int row = m * 16 + col;
-    sl_f32x4 y = sum(t);
-    if constexpr (!PAIR) {
-      if (row < M)
-        *reinterpret_cast<sl_f32x4*>(slabs + ((long)blockIdx.y * M + row) * N + n0 + t * 16 +
-                                     grp * 4) = y;
-    } else {
-      const sl_f32x4 up = sum(t + 2);
-      Vec4<__hip_bfloat16> v;
+    const sl_f32x4 y = sum(t), up = sum(t + 2);
+    Vec4<__hip_bfloat16> v;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float g = y[r];
-        const float a = EPI == kSlabSilu
-            ? g / (1.0f + __expf(-g))
-            : 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
-        v.data[r] = __float2bfloat16(a * up[r]);
-      }
-      if (row < M)
-        *reinterpret_cast<int2*>(out + (long)row * out_stride + n0 + t * 16 + grp * 4) =
-            *reinterpret_cast<const int2*>(v.data);
+    for (int r = 0; r < 4; ++r) {
+      const float g = y[r];
+      const float a = EPI == kSlabSilu
+          ? g / (1.0f + __expf(-g))
+          : 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
+      v.data[r] = __float2bfloat16(a * up[r]);
     }
+    if (row < M)
+      *reinterpret_cast<int2*>(out + (long)row * out_stride + n0 + t * 16 + grp * 4) =
+          *reinterpret_cast<const int2*>(v.data);
   }
 }
 

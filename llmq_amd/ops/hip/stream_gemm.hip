@@ -11,9 +11,11 @@
 //   - With M tokens only 16/KH >= M of the 16 columns are needed, so K is cut in KH
 //     slices that take the rest: A's rows are 16/KH weight rows times KH slices, B's
 //     columns 16/KH tokens times KH slices, and the result is the sum of the
-//     blocks on C's diagonal. That sets a workgroup's share to 16, 8, 4, 2 or 1
-//     weight rows without a masked lane.
-//   - The workgroup's waves share out the slices in chunks and add up through LDS.
+//     blocks on C's diagonal. That sets a workgroup's share to 16, 8 or 4 weight
+//     rows (KH = 1, 2, 4) without a masked lane.
+//   - The workgroup's waves share out the slices in chunks and add up through LDS. A
+//     wave with several chunks asks for the next one's weights ahead of a chunk's
+//     products, under a condition, so that the wait before those covers them too.
 //   - NORM: the tokens are RMS-normalised on the way in: x times the norm's weights
 //     (rounded, as a normalised row is) goes to LDS once per workgroup, while the
 //     first weights travel, its squares are summed beside, and the row's factor
