@@ -1,12 +1,12 @@
 #!/bin/bash
-# CI-style sanitizer pass over the HIP kernels.
+# CI-style sanitizer pass over the main library's HIP kernels.
 # No compute-sanitizer ships in this image; the recipe is:
 #   - AMD_SERIALIZE_KERNEL=3: every kernel launches synchronously and any
 #     fault (incl. OOB reads that leave the mapped heap) aborts AT the
 #     offending launch instead of corrupting later state;
 #   - tests/test_gpu_sanitize.py: canary-halo (guard-band) tensors around
-#     every kernel's inputs/outputs, verified bitwise after each op
-#     (catches OOB WRITES that stay inside the heap);
+#     inputs and outputs, verified bitwise after each op (catches OOB
+#     WRITES that stay inside the heap);
 #   - the full numerics suite re-run under serialization.
 set -e
 cd "$(dirname "$0")/.."

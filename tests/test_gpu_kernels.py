@@ -166,18 +166,15 @@ class TestDecodeAttention:
         atol, rtol = TOL[dtype]
         assert_close_to_f32_ref(out.cpu(), ref, atol, 5 * rtol)
 
-    @pytest.mark.parametrize("pipe", ["0", "64", "128"])
     @pytest.mark.parametrize("B,G,KVH,D,softcap,window", [
         (9, 2, 8, 256, 0.0, 0),    # headline gemma2 shape
         (9, 4, 8, 128, 0.0, 0),
         (5, 2, 8, 256, 50.0, 100), # softcap + window (start mid-chunk)
-        (2, 16, 1, 256, 0.0, 0),   # TP-rank shape: split-KV z-grid engaged
+        (2, 16, 1, 256, 0.0, 0),   # TP-rank shape: pairs cut in pieces
     ])
-    def test_pipe_variants(self, pipe, B, G, KVH, D, softcap, window, monkeypatch):
-        """The software-pipelined glds decode kernel (LLMQ_DECODE_PIPE=64/128)
-        must match the plain-staged kernel's reference across chunk-boundary
-        contexts (tail chunk short/exact/overflowing) and the split-KV path."""
-        monkeypatch.setenv("LLMQ_DECODE_PIPE", pipe)
+    def test_tile_boundaries(self, B, G, KVH, D, softcap, window):
+        """Contexts that end short of, on and past a tile's edge, whole and cut
+        pairs."""
         dtype = torch.bfloat16
         H = G * KVH
         torch.manual_seed(4)

@@ -1,13 +1,13 @@
-"""Guard-band (canary) pass over the HIP kernels.
+"""Guard-band (canary) pass over the main library's kernels.
 
 No compute-sanitizer ships in this image, so out-of-bounds WRITES are
-checked directly: every input/output tensor is carved out of an
-over-allocated buffer with canary halos on both sides, and the halos are
-verified bitwise after each op. Run under ``AMD_SERIALIZE_KERNEL=3`` (the
-CI recipe — tests/sanitize_gpu.sh) so any kernel fault aborts at the
-offending launch instead of surfacing later. Canaries do not catch OOB
-READS; those surface as faults under serialized launches or as numerics
-failures in test_gpu_kernels.
+checked directly: inputs and outputs are carved out of over-allocated
+buffers with canary halos on both sides, and the halos are verified bitwise
+after each op. Run under ``AMD_SERIALIZE_KERNEL=3`` (tests/sanitize_gpu.sh)
+so any kernel fault aborts at the offending launch instead of surfacing
+later. Not covered: OOB READS (those surface as faults under serialized
+launches or as numerics failures in test_gpu_kernels), and tensors that an
+op allocates itself (the slab products, their readers' bf16 rows, scratch).
 """
 
 from __future__ import annotations
@@ -19,6 +19,8 @@ pytestmark = pytest.mark.gpu
 
 if torch.cuda.is_available():
     from llmq_amd import ops
+
+    assert ops.has_hip_ext()  # _EXT below: ops with outputs of the caller's
 else:
     pytest.skip("no GPU", allow_module_level=True)
 
@@ -68,37 +70,102 @@ def g():
     gg.verify()
 
 
-def test_decode_attention_guarded(g, monkeypatch):
-    B, G, KVH, D, BS = 7, 2, 8, 256, 16
-    H = G * KVH
-    max_blocks = 70
+@pytest.mark.parametrize("D,G,KVH,BS,fp8", [(64, 4, 3, 16, False), (128, 6, 2, 32, False),
+                                             (256, 2, 8, 16, False), (128, 4, 2, 16, True),
+                                             (256, 2, 2, 32, True)])
+@pytest.mark.parametrize("softcap,window", [(0.0, 0), (50.0, 70)])
+def test_decode_attention_guarded(g, D, G, KVH, BS, fp8, softcap, window):
+    B, H, max_blocks = 7, G * KVH, 70
     NB = B * max_blocks + 1
-    kc = g.tensor(NB, KVH, BS, D)
-    vc = g.tensor(NB, KVH, BS, D)
-    q = g.tensor(B, H, D)
+    kc, vc = (g.tensor(NB, KVH, BS, D, dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16)
+              for _ in range(2))
+    q, out = g.tensor(B, H, D), g.tensor(B, H, D)
     bt = g.from_values(
         torch.arange(1, 1 + B * max_blocks).reshape(B, max_blocks), torch.int32)
     ctx = g.from_values(torch.tensor([1, 63, 64, 65, 129, 1000, 1025]), torch.int32)
-    for pipe in ("0", "64", "128"):
-        monkeypatch.setenv("LLMQ_DECODE_PIPE", pipe)
-        out = ops.paged_decode_attention(q, kc, vc, bt, ctx, D ** -0.5, 0.0, 0)
-        assert out.isfinite().all()
-    # split-KV path (scratch + merge kernels)
-    out = ops.paged_decode_attention(q[:2], kc, vc, bt[:2], ctx[:2], D ** -0.5, 0.0, 0)
+    for n in (7, 2):                         # pairs within a wave's range, cut in pieces
+        ops._EXT.paged_decode_attention(out[:n], q[:n], kc, vc, bt[:n], ctx[:n], D ** -0.5,
+                                        softcap, window)
+        assert out[:n].isfinite().all()
+
+
+@pytest.mark.parametrize("D,H,KVH", [(64, 4, 2), (64, 3, 1), (128, 6, 2), (256, 16, 8),
+                                     (256, 3, 3)])
+@pytest.mark.parametrize("softcap,window", [(0.0, 0), (50.0, 70)])
+def test_prefill_attention_guarded(g, D, H, KVH, softcap, window):
+    lens, past, BS = [1, 33, 129, 300], [0, 20, 64, 5], 16
+    lens_k = [n + p for n, p in zip(lens, past)]
+    T, Tk = sum(lens), sum(lens_k)
+    q, out = g.tensor(T, H, D), g.tensor(T, H, D)
+    k, v = g.tensor(Tk, KVH, D), g.tensor(Tk, KVH, D)
+    cu, cu_k = (g.from_values(torch.tensor([0] + list(torch.tensor(x).cumsum(0))), torch.int32)
+                for x in (lens, lens_k))
+    args = (max(lens), D ** -0.5, softcap, window)
+    ops._EXT.varlen_prefill_attention(out, q, k, v, cu, cu_k, *args)
+    assert out.isfinite().all()
+    width = -(-max(lens_k) // BS)
+    kc, vc = (g.tensor(len(lens) * width, KVH, BS, D) for _ in range(2))
+    bt = g.from_values(torch.arange(len(lens) * width).reshape(len(lens), width), torch.int32)
+    ops._EXT.paged_prefill_attention(out, q, kc, vc, bt, cu, cu_k, *args)
     assert out.isfinite().all()
 
 
-def test_prefill_attention_guarded(g, monkeypatch):
-    B, H, KVH, D, L = 3, 16, 8, 256, 300
-    T = B * L
-    q = g.tensor(T, H, D)
-    k = g.tensor(T, KVH, D)
-    v = g.tensor(T, KVH, D)
-    cu = g.from_values(torch.arange(0, T + 1, L), torch.int32)
-    for pipe in ("0", "1"):
-        monkeypatch.setenv("LLMQ_PREFILL_PIPE", pipe)
-        out = ops.varlen_prefill_attention(q, k, v, cu, L, D ** -0.5)
+@pytest.mark.parametrize("M", [1, 5, 16])
+@pytest.mark.parametrize("N,K", [(32, 128), (96, 384), (64, 14336)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_few_row_products_guarded(g, M, N, K, norm):
+    x, w = g.tensor(M, K), g.tensor(N, K)
+    nw = g.tensor(K) if norm else None
+    for epi in range(4):                     # plain, residual, SiLU and GELU pairs
+        out = g.tensor(M, N if epi < 2 else N // 2)
+        bias = g.tensor(N) if epi == 0 else None
+        ops._EXT.stream_gemm(out, x, w, bias, nw, 1e-5, 0.0, epi)
         assert out.isfinite().all()
+
+
+@pytest.mark.parametrize("M", [1, 5, 16])
+@pytest.mark.parametrize("D,H,KVH,fp8", [(64, 3, 1, False), (128, 2, 2, True), (16, 4, 2, False)])
+def test_few_row_qkv_guarded(g, M, D, H, KVH, fp8):
+    from llmq_amd.ops import torch_ref
+
+    N, K = (H + 2 * KVH) * D, 128
+    kc, vc = (g.tensor(2, KVH, 16, D, dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16)
+              for _ in range(2))
+    cs = g.from_values(torch_ref.build_rope_cache(64, D, 10000.0, DEV), torch.float32)
+    slots = torch.randperm(32)[:M]
+    slots[0] = -1
+    out = g.tensor(M, N)
+    ops._EXT.stream_qkv(out, g.tensor(M, K), g.tensor(N, K), g.tensor(N), g.tensor(K), 1e-5, 0.0,
+                        kc, vc, g.from_values(torch.arange(M), torch.int64), cs,
+                        g.from_values(slots, torch.int64))
+    assert out.isfinite().all()
+
+
+@pytest.mark.parametrize("M", [17, 33, 64, 97, 128])
+@pytest.mark.parametrize("D,H,KVH,fp8", [(64, 2, 1, False), (128, 2, 2, True)])
+def test_slab_products_guarded(g, M, D, H, KVH, fp8):
+    from llmq_amd.ops import torch_ref
+
+    N, K = (H + 2 * KVH) * D, 384
+    x = g.tensor(M, K)
+    slabs = ops.slab_linear(x, g.tensor(N, K))
+    kc, vc = (g.tensor(9, KVH, 16, D, dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16)
+              for _ in range(2))
+    cs = g.from_values(torch_ref.build_rope_cache(128, D, 10000.0, DEV), torch.float32)
+    slots = torch.randperm(144)[:M]
+    slots[3] = -1
+    held = g.tensor(*slabs.shape, dtype=torch.float32)
+    held.copy_(slabs)
+    rows = ops.slab_rope_cache(held, g.tensor(N), kc, vc,
+                               g.from_values(torch.arange(M), torch.int64), cs,
+                               g.from_values(slots, torch.int64))
+    residual = g.tensor(M, N)
+    assert rows.isfinite().all()
+    for post in (None, g.tensor(N)):
+        assert ops.slab_add_norm(held, residual, post, g.tensor(N), 1e-5, 1.0).isfinite().all()
+    if M <= 64:
+        for gelu in (False, True):
+            assert ops.slab_act_linear(x, g.tensor(128, K), gelu).isfinite().all()
 
 
 def test_elementwise_and_cache_guarded(g):
@@ -126,9 +193,13 @@ def test_elementwise_and_cache_guarded(g):
     ops.rope_and_cache(qkv_q, qkv_k, vval, kc, vc, pos, cs, slots)
 
 
-def test_sampler_guarded(g):
-    B, V = 64, 50257
+@pytest.mark.parametrize("B,V", [(64, 50257), (3, 1003), (1, 50000), (2, 1)])
+def test_sampler_guarded(g, B, V):
+    half = g.tensor(B, V)
     logits = g.tensor(B, V, dtype=torch.float32)
+    if half.data_ptr() % 16 == 0 and logits.data_ptr() % 16 == 0:
+        ops._EXT.softcap_logits(logits, half, 30.0)
+        assert logits.isfinite().all()
     temps = g.tensor(B, dtype=torch.float32, fill="zeros")
     temps.fill_(0.8)
     tps = g.tensor(B, dtype=torch.float32, fill="zeros")
@@ -137,6 +208,7 @@ def test_sampler_guarded(g):
     out = g.from_values(torch.zeros(B), torch.int64)
     keys = g.from_values(torch.zeros(B), torch.int64)
     zs = g.from_values(torch.zeros(B), torch.int32)
-    bound = ops.topk_topp_bound(logits, temps, tps, tks)
+    bound = g.tensor(B, dtype=torch.float32)
+    ops._EXT.topk_topp_bound(bound, logits, temps, tps, tks)
     ops.sample_gumbel_argmax(out, keys, logits, temps, zs, zs, 3, 1, bound)
     assert bool((out >= 0).all()) and bool((out < V).all())
