@@ -643,8 +643,8 @@ void launch_stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
   // the launch / a norm of its own): 16384 x 2048 pairs, 1 token (8.4 million)
   // 18.0 / 18.6, 2 tokens 22.4 / 19.2; 16384 x 3072 pairs, 3 tokens (9.4) 28.1 / 28.9, 4
   // 29.7 / 28.0; 5120 x 3072, 3 tokens (11.8) 12.2 / 12.6, 8 18.7 / 15.5; 2048 x 1536,
-  // 6 tokens (2.4) 6.5 / 6.4, 8 7.5 / 6.6. They have to fit beside the sums (24 KB at
-  // the most).
+  // 6 tokens (2.4) 6.5 / 6.4, 8 7.5 / 6.6; on the wrong side 17920 x 1536 pairs, 1 token
+  // (6.9), 16.9 / 16.1. They have to fit beside the sums (24 KB at the most).
   const int R = large || M > 8 ? 16 : M > 4 ? 8 : 4;
   if (M <= 6 && (long)(N / R) * M * K <= 12'000'000 && (long)M * (K + 512) * 2 <= (120 << 10))
     return epilogue.template operator()<true>();

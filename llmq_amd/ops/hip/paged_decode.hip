@@ -31,8 +31,12 @@
 //     lane%16, k = 8*(lane/16)..+7; B: column = lane%16; C: column = lane%16, rows
 //     4*(lane/16)+r), so a lane's scores belong to one query and its weights are
 //     already the second product's operand: slot 8h+4b+i = key 16b+4h+i.
-//   - Weights enter as two bf16 planes (p = hi + lo, 16 mantissa bits): fp32
-//     weights for the price of a second product that is not the bound.
+//   - Weights enter as bf16 planes, a product each, which is not the bound. Head sizes
+//     128 and 256: two, 16 mantissa bits. Head size 64: three, all 24 bits, as the fp32
+//     kernel that still serves fp32 caches has them: 64 x 1040 keys, queries of size 3,
+//     outputs other than the 64-bit result's nearest bf16: that kernel 4.3e-4, three
+//     planes 3.8e-4, two 1.5e-3; 1b decode step of 64 sequences 1726 and 1708 us with
+//     two and three.
 //   - A pair that lies in one wave's range is written at once; the pieces of the
 //     others go to `part` (output, maximum in the log2 domain, sum) and are merged
 //     by paged_decode_merge_kernel.
@@ -116,13 +120,19 @@ DEVINL pd_s16x8 pd_widen(unsigned lo, unsigned hi) {
   return __builtin_bit_cast(pd_s16x8, r);
 }
 
-// two weights -> their bf16 planes: hi cut off, lo the rounded rest
-DEVINL void pd_planes(float p0, float p1, unsigned& hi, unsigned& lo) {
-  const unsigned b0 = __float_as_uint(p0), b1 = __float_as_uint(p1);
-  hi = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
-  const pd_f32x2 rest = {p0 - __uint_as_float(b0 & 0xffff0000u),
-                         p1 - __uint_as_float(b1 & 0xffff0000u)};
-  lo = __builtin_bit_cast(unsigned, __builtin_convertvector(rest, pd_bf16x2));
+// Two weights -> their bf16 planes: hi cut off, lo the rounded rest (16 mantissa bits),
+// or with three planes the rest cut off and rounded again, exact: 24 bits.
+template <int PL>
+DEVINL void pd_planes(float p0, float p1, unsigned (&w)[PL]) {
+#pragma unroll
+  for (int i = 0; i + 1 < PL; ++i) {
+    const unsigned b0 = __float_as_uint(p0), b1 = __float_as_uint(p1);
+    w[i] = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+    p0 -= __uint_as_float(b0 & 0xffff0000u);
+    p1 -= __uint_as_float(b1 & 0xffff0000u);
+  }
+  w[PL - 1] = __builtin_bit_cast(
+      unsigned, __builtin_convertvector((pd_f32x2{p0, p1}), pd_bf16x2));
 }
 
 // Swizzle of the V tile's 16-byte granules: the 8 keys that one transposing read
@@ -150,6 +160,7 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
   constexpr bool F8 = sizeof(TC) == 1;
   constexpr int TS = PdShape<D, TC, NK>::kTileShift, KT = 16 * NK;
   constexpr int KS = D / 32, DT = D / 16;
+  constexpr int PL = D == 64 ? 3 : 2;                // bf16 planes of a weight
   constexpr int KL = F8 ? KS / 2 : KS;               // 16-byte loads of a K operand row
   constexpr int GPR = D * (int)sizeof(TC) / 16;      // 16-byte granules of a V row
   constexpr int RPI = WAVE / GPR;                    // V rows per load
@@ -319,39 +330,40 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
       __builtin_amdgcn_wave_barrier();
 
       if constexpr (NK == 1) {
-        unsigned hi[2], lw[2];
+        pd_u32x2 pw[PL];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           const float p0 = __builtin_amdgcn_exp2f(s[0][2 * e] - mb);
           const float p1 = __builtin_amdgcn_exp2f(s[0][2 * e + 1] - mb);
           l += p0 + p1;
-          pd_planes(p0, p1, hi[e], lw[e]);
+          unsigned w2[PL];
+          pd_planes(p0, p1, w2);
+#pragma unroll
+          for (int pl = 0; pl < PL; ++pl) pw[pl][e] = w2[pl];
         }
-        const pd_s16x4 ph = __builtin_bit_cast(pd_s16x4, pd_u32x2{hi[0], hi[1]});
-        const pd_s16x4 pl = __builtin_bit_cast(pd_s16x4, pd_u32x2{lw[0], lw[1]});
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
           const pd_s16x4 va = __builtin_bit_cast(pd_s16x4, __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
               (pd_lds_bf16x4*)(Vt + tbase + (((dt * 2 + tg) ^ tsw) << 3))));
-          o[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va, ph, o[dt], 0, 0, 0);
-          o[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va, pl, o[dt], 0, 0, 0);
+#pragma unroll
+          for (int pl = 0; pl < PL; ++pl)
+            o[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                va, __builtin_bit_cast(pd_s16x4, pw[pl]), o[dt], 0, 0, 0);
         }
       } else {
 #pragma unroll
         for (int j = 0; j < NK / 2; ++j) {
-          pd_u32x4 hi, lw;
+          pd_u32x4 pw[PL];
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const float p0 = __builtin_amdgcn_exp2f(s[2 * j + e / 2][(e & 1) * 2] - mb);
             const float p1 = __builtin_amdgcn_exp2f(s[2 * j + e / 2][(e & 1) * 2 + 1] - mb);
             l += p0 + p1;
-            unsigned h, lo_;
-            pd_planes(p0, p1, h, lo_);
-            hi[e] = h;
-            lw[e] = lo_;
+            unsigned w2[PL];
+            pd_planes(p0, p1, w2);
+#pragma unroll
+            for (int pl = 0; pl < PL; ++pl) pw[pl][e] = w2[pl];
           }
-          const pd_s16x8 ph = __builtin_bit_cast(pd_s16x8, hi);
-          const pd_s16x8 pl = __builtin_bit_cast(pd_s16x8, lw);
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt) {
             short* at = Vt + j * 32 * D + tbase + (((dt * 2 + tg) ^ tsw) << 3);
@@ -360,8 +372,10 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
             const pd_s16x4 v1 = __builtin_bit_cast(pd_s16x4,
                 __builtin_amdgcn_ds_read_tr16_b64_v4bf16((pd_lds_bf16x4*)(at + 16 * D)));
             const pd_s16x8 va = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-            o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, ph, o[dt], 0, 0, 0);
-            o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pl, o[dt], 0, 0, 0);
+#pragma unroll
+            for (int pl = 0; pl < PL; ++pl)
+              o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  va, __builtin_bit_cast(pd_s16x8, pw[pl]), o[dt], 0, 0, 0);
           }
         }
       }
