@@ -272,7 +272,8 @@ class CausalLM:
         return attn.reshape(T, self.q_size)
 
     def _forward_slabs(self, h, residual, positions, kv_cache, meta) -> torch.Tensor:
-        """The layers for up to ops.SLAB_ROWS rows (an ordinary decode step):
+        """The layers for up to ops.SLAB_ROWS rows (an ordinary decode step, few
+        rows of large layers):
         streaming products whose partial sums the norms and the rotation add up."""
         s = self.spec
         for i, lw in enumerate(self.layers):
@@ -314,7 +315,7 @@ class CausalLM:
 
     def _forward_few_rows(self, residual, positions, kv_cache, meta) -> torch.Tensor:
         """The layers for up to ops.FEW_ROWS rows (a decode step of few
-        sequences): norms, rotation, cache write, activation and residual addition
+        sequences; fewer rows of large layers): norms, rotation, cache write, activation and residual addition
         ride on the projections, which stream the weights once."""
         s = self.spec
         act = "gelu_tanh" if s.gelu else "silu"

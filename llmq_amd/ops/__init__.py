@@ -300,13 +300,27 @@ _FEW_ACTS = {"silu": 2, "gelu_tanh": 3}
 
 
 def few_rows_ok(x: torch.Tensor, weights) -> bool:
-    """Whether few_rows_linear's kernel takes these rows and weights [N, K]."""
+    """Whether few_rows_linear's kernel takes these rows and weights [N, K]: those
+    of a layer, and is worth it."""
     return (
         x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= FEW_ROWS
         and x.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0
         and all(w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] % 128 == 0
                 and w.shape[0] % 32 == 0 and w.data_ptr() % 16 == 0 for w in weights)
+        and x.shape[0] <= few_rows_limit(sum(w.numel() for w in weights))
     )
+
+
+def few_rows_limit(layer_weights: int) -> int:
+    """Rows up to which few_rows_linear serves a layer of that many weights. Its
+    workgroups own 4 to 16 weight rows and each reads all tokens again, at 16 rows as
+    many bytes as weights: the larger the matrices, the sooner that is more than the
+    launches that it saves. Beyond, the slab kernels (64 weight rows a workgroup).
+    Measured, us for six layers, few-row / slab loop: 61 M weights a layer, 8 rows 416 /
+    414, 14 rows 478 / 432; 101 M, 6 rows 581 / 580, 8 rows 625 / 588; 218 M, 4 rows
+    860 / 878, 8 rows 937 / 908; 487 M, 1 row 1648 / 1396, 4 rows 1845 / 1479; 877 M,
+    1 row 2302 / 2448, 2 rows 2368 / 2460, 16 rows 3220 / 2490 (the library's 2592)."""
+    return max(2, 800_000_000 // max(layer_weights, 1))
 
 
 def few_rows_linear(
@@ -356,7 +370,7 @@ def few_rows_qkv(
     return out
 
 
-# --------------------------------------------- projections, 17 to 128 rows --
+# --------------------------------------------- projections, up to 128 rows --
 # The product stays as fp32 partial sums ("slabs" [parts, M, N]) that the next
 # kernel adds up: norm and residual, or rotation and cache write.
 
@@ -366,7 +380,7 @@ SLAB_ROWS = 128
 def slab_ok(x: torch.Tensor, weights, hidden: int) -> bool:
     """Whether the slab kernels take these rows and weights [N, K]."""
     return (
-        x.is_cuda and x.dim() == 2 and FEW_ROWS < x.shape[0] <= SLAB_ROWS
+        x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= SLAB_ROWS
         and x.dtype == torch.bfloat16 and x.is_contiguous() and hidden <= 8192
         and all(w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] % 128 == 0
                 and w.shape[0] % 64 == 0 and w.data_ptr() % 16 == 0 for w in weights)
@@ -381,7 +395,7 @@ def slab_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def slab_act_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether slab_act_linear beats the library's product and an activation."""
-    return x.shape[0] <= 64 and w.numel() < 48 << 20
+    return x.shape[0] <= 64 and w.numel() < (128 if x.shape[0] <= 16 else 48) << 20
 
 
 def slab_act_linear(x: torch.Tensor, w: torch.Tensor, gelu: bool) -> torch.Tensor:

@@ -710,10 +710,10 @@ void stream_qkv(at::Tensor out, at::Tensor x, at::Tensor w, c10::optional<at::Te
                             N / D - 2 * kv_heads, kv_heads, D, (int)k_cache.size(2), fp8});
 }
 
-// ------------------------------------------- projections, 17 to 128 rows --
+// ------------------------------------------- projections, up to 128 rows --
 
 bool slab_rows_ok(const at::Tensor& x, const at::Tensor& w) {
-  return x.dim() == 2 && w.dim() == 2 && x.size(0) > 16 && x.size(0) <= 128 &&
+  return x.dim() == 2 && w.dim() == 2 && x.size(0) > 0 && x.size(0) <= 128 &&
          x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 &&
          x.stride(1) == 1 && rows_start_on(x, 16) && x.size(1) == w.size(1) &&
          w.size(1) % kSlabBK == 0 && w.size(1) > 0 && w.size(0) % 64 == 0;
@@ -745,7 +745,8 @@ void launch_slab_gemm(float* slabs, __hip_bfloat16* out, long out_stride, const 
   // 16384 x 2048: 20.8 us, one group 25.3).
   constexpr int WK = EPI == kSlabSums ? 1 : 2;
   const int tm = (M + 15) / 16;
-  if (tm <= 2) go.template operator()<2, WK>();
+  if (tm == 1) go.template operator()<1, WK>();
+  else if (tm == 2) go.template operator()<2, WK>();
   else if (tm == 3) go.template operator()<3, WK>();
   else if (tm == 4) go.template operator()<4, WK>();
   else if constexpr (EPI == kSlabSums) {
@@ -758,7 +759,7 @@ void launch_slab_gemm(float* slabs, __hip_bfloat16* out, long out_stride, const 
 at::Tensor slab_linear(const at::Tensor& x, const at::Tensor& w) {
   CHECK_GPU(x);
   TORCH_CHECK(slab_rows_ok(x, w),
-              "slab_linear: 17 to 128 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
+              "slab_linear: 1 to 128 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
   if (!streamable(w)) return at::linear(x, w).to(at::kFloat).unsqueeze(0);
   const int parts = slab_parts(w.size(0), w.size(1));
   at::Tensor slabs = at::empty({parts, x.size(0), w.size(0)}, x.options().dtype(at::kFloat));
@@ -768,15 +769,18 @@ at::Tensor slab_linear(const at::Tensor& x, const at::Tensor& w) {
 
 // Whether gate and value rows are worth a product of their own with the activation
 // in it: from 48 M weights on the library's product and the activation are as fast
-// (48 rows, 28672 x 3584: 49.0 + 5.2 us against 53.5).
+// (48 rows, 28672 x 3584: 49.0 + 5.2 us against 53.5), up to 16 rows from 128 M on (8
+// rows, 28672 x 4096: 61.5 against 51.3, 28672 x 3584: 45.8 / 47.5, 37888 x 3584: 56.1 /
+// 66.1, 55296 x 5120: 98 / 144).
 bool slab_act_ok(const at::Tensor& x, const at::Tensor& w) {
-  return slab_rows_ok(x, w) && x.size(0) <= 64 && w.numel() < (48L << 20);
+  return slab_rows_ok(x, w) && x.size(0) <= 64 &&
+         w.numel() < ((x.size(0) <= 16 ? 128L : 48L) << 20);
 }
 
 at::Tensor slab_act_linear(const at::Tensor& x, const at::Tensor& w, bool gelu) {
   CHECK_GPU(x);
   TORCH_CHECK(slab_rows_ok(x, w) && x.size(0) <= 64,
-              "slab_act_linear: 17 to 64 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
+              "slab_act_linear: 1 to 64 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
   at::Tensor out = at::empty({x.size(0), w.size(0) / 2}, x.options());
   if (!streamable(w)) {
     const at::Tensor y = at::linear(x, w);
@@ -887,7 +891,7 @@ at::Tensor prompt_layers(at::Tensor h, at::Tensor residual, at::TensorList weigh
                   windows.size() == layers && (biases.empty() || biases.size() == layers),
               "one entry per layer");
   const long T = h.size(0);
-  // 17 to 128 rows of these shapes: the streaming products, whose sums the next
+  // up to 128 rows of these shapes: the streaming products, whose sums the next
   // kernel takes up
   const bool slab = layers > 0 && k_caches[0].size(3) == head_dim && h.size(1) <= 8192 &&
                     (k_caches[0].scalar_type() == at::kBFloat16 ||

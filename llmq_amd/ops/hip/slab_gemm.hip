@@ -1,5 +1,6 @@
-// Projections of 17 to 128 rows, x[M, K] W[N, K]^T with fp32 sums: the products of
-// an ordinary decode step or a short prompt (gfx950).
+// Projections of up to 128 rows, x[M, K] W[N, K]^T with fp32 sums: the products of
+// an ordinary decode step or a short prompt, and of few rows through large layers
+// (gfx950).
 //
 // Bound by the weights' bytes. A workgroup owns 64 weight rows, all M tokens and one
 // of S parts of K. Weights go straight from memory into the matrix layout; the tokens,

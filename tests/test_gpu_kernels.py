@@ -444,10 +444,10 @@ class TestManyShortPrompts:
 
 
 class TestSlabProjections:
-    """Streaming products of 17 to 128 rows and the kernels that add up their
+    """Streaming products of up to 128 rows and the kernels that add up their
     partial sums: each row-tile count, K that leaves parts of unequal length."""
 
-    @pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 96, 97, 128])
+    @pytest.mark.parametrize("M", [1, 5, 16, 17, 32, 33, 64, 65, 96, 97, 128])
     @pytest.mark.parametrize("N,K", [(64, 128), (192, 640), (2048, 2048), (3072, 8960)])
     def test_products(self, M, N, K):
         x = torch.randn(M, K + 8, device=DEV, dtype=torch.bfloat16)[:, :K]
@@ -466,7 +466,7 @@ class TestSlabProjections:
             tol = 2 ** -8 * (act * u).abs() + 3e-5 * (1 + g.abs()) * (1 + u.abs())
             assert ((y - act * u).abs() <= tol).all()
 
-    @pytest.mark.parametrize("S,M,N", [(1, 17, 64), (3, 20, 1000), (16, 64, 2048), (2, 128, 8192)])
+    @pytest.mark.parametrize("S,M,N", [(1, 1, 64), (16, 5, 8192), (1, 17, 64), (3, 20, 1000), (16, 64, 2048), (2, 128, 8192)])
     @pytest.mark.parametrize("post", [False, True])
     def test_add_norm(self, S, M, N, post):
         slabs = torch.randn(S, M, N, device=DEV)

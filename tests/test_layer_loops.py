@@ -1,5 +1,5 @@
 """The layer loops of the Llama, Qwen2 and Gemma-2 families against a 64-bit
-forward pass: up to 16 rows (few_rows), 17 to 128 (slabs), prompts launched from
+forward pass: few rows (few_rows), up to 128 (slabs), prompts launched from
 native code (prompt_layers) and the per-operation loop, for decode steps, whole
 prompts, portions that continue a cached context and mixed steps. Three layers of
 sizes that the streaming kernels take, norm weights and biases that differ
@@ -319,3 +319,26 @@ def test_vector_layouts(name, kind, rows):
     if lw.qkv_bias is not None:
         lw.qkv_bias = lw.qkv_bias.repeat_interleave(2)[::2]
     assert _off(_run(model, cache, batch), want) < LIMIT
+
+
+def test_few_rows_limit():
+    """Fewer rows of larger layers, two at the least; the layers of llama-3.2-1b (61 M
+    weights), -3b (101 M) and qwen2.5-72b (877 M)."""
+    assert [ops.few_rows_limit(n) for n in (61_000_000, 101_000_000, 877_000_000, 1)] == [
+        13, 7, 2, 800_000_000]
+
+
+@on_gpu
+@pytest.mark.parametrize("rows", [3, 4, 16])
+@pytest.mark.parametrize("kind", ["decode", "prompt", "portion", "mixed"])
+@pytest.mark.parametrize("name,fp8", [("llama", False), ("qwen2", True), ("gemma2", False)])
+def test_few_rows_of_large_layers(name, fp8, kind, rows, loops, monkeypatch):
+    """Rows over a layer's limit: the slab kernels' loops, here with a limit of three."""
+    monkeypatch.setattr(ops, "few_rows_limit", lambda n: 3)
+    model = _model(name, "cuda", torch.bfloat16)
+    cache = _cache(model.spec, "cuda", torch.float8_e4m3fn if fp8 else torch.bfloat16)
+    batch = _batch(kind, rows)
+    want = _oracle(model, cache, batch)
+    got = _run(model, cache, batch)
+    assert loops == (["few"] if rows == 3 else _expected(kind, 17, fp8))
+    assert _off(got, want) < LIMIT

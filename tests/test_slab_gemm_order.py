@@ -15,8 +15,8 @@ import pytest
 from llmq_amd.ops.build import HERE, HIPCC_FLAGS
 
 HIPCC = shutil.which("hipcc") or shutil.which("/opt/rocm/bin/hipcc")
-VARIANTS = [(2, 1, 0), (3, 1, 0), (4, 1, 0), (6, 1, 0), (8, 1, 0),      # TM, WK, EPI
-            (2, 2, 1), (3, 2, 1), (4, 2, 1), (2, 2, 2), (3, 2, 2), (4, 2, 2)]
+VARIANTS = [(tm, 1, 0) for tm in (1, 2, 3, 4, 6, 8)] + [       # TM, WK, EPI
+    (tm, 2, epi) for tm in (1, 2, 3, 4) for epi in (1, 2)]
 SOURCE = '#include "flash_prefill.hip"\n#include "slab_gemm.hip"\n' + "".join(
     f"template __global__ void slab_gemm_kernel<{tm}, {wk}, {epi}>(float*, __hip_bfloat16*, long, "
     "const __hip_bfloat16*, long, const __hip_bfloat16*, int, int, int, int);\n"
