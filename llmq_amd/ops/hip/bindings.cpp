@@ -411,9 +411,22 @@ void launch_flash_prefill_any(at::Tensor& out, const PrefillArgs& args) {
   // 8 x 1024 tokens). Tiles of 32 keys where that buys a third wave per SIMD
   // (head size 128: 160 against 187 us for 16 x 1024) or the registers (256).
   const bool even = (H / args.KVH) % 2 == 0;
+  // Head size 256: four waves a workgroup instead of eight where the wide ones would not
+  // fill the CUs (a wave then has its SIMD to itself) or where a prompt fits in one narrow
+  // tile. Measured, us, 16 heads of 8 kv heads, wide / narrow: 1 x 100 21.0 / 15.6, 1 x 500
+  // 50.0 / 41.8, 8 x 300 (192 wide workgroups) 37.8 / 33.0, 16 x 200 (256) 35.3 / 41.0,
+  // 1 x 5000 (320) 363 / 470, 300 x 33 111 / 99, 64 x 65 (512) 42.7 / 51.1.
+  const int wide_rows = even ? 128 : 256;
+  const long wide = (args.max_seqlen + wide_rows - 1) / wide_rows * (H / (even ? 2 : 1)) * args.B;
+  int cus = 0;
+  TORCH_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
+                                    args.q.get_device()) == hipSuccess);
+  const bool narrow = args.max_seqlen <= wide_rows / 2 || wide < cus;
   if (D == 64 && even) launch_flash_prefill<64, 2, 2, 64, 3>(oa, a);
   else if (D == 64) launch_flash_prefill<64, 1, 4, 64, 3>(oa, a);
   else if (D == 128) launch_flash_prefill<128, 1, 4, 32, 3>(oa, a);
+  else if (narrow && even) launch_flash_prefill<256, 2, 2, 32, 1>(oa, a);
+  else if (narrow) launch_flash_prefill<256, 1, 4, 32, 1>(oa, a);
   else if (even) launch_flash_prefill<256, 2, 4, 32, 1>(oa, a);
   else launch_flash_prefill<256, 1, 8, 32, 1>(oa, a);
   if (!oa.is_same(out)) out.copy_(oa);

@@ -148,17 +148,23 @@ __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
   const bool idle = wr * 32 >= rows;
 
   // Staging: load i = w + j NW of a tile (K rows, then V rows) is 1 KiB = KPL key
-  // rows. A wave's loads lie a multiple of 16 keys apart, so its lanes' place in a
-  // row and their offset from the load's first row are the same for all of them.
-  constexpr int KPL = 64 / GPR, STEP = NW * KPL;
-  static_assert(NI % NW == 0 && STEP % 16 == 0, "a wave's loads share their swizzle");
+  // rows. A wave's loads lie STEP keys apart: its lanes' place in a row and their offset
+  // from the load's first row are the same for all of them, K's at STEP = 8 for every
+  // second one.
+  constexpr int KPL = 64 / GPR, STEP = NW * KPL, PH = STEP % 16 == 0 ? 1 : 2;
+  static_assert(NI % NW == 0 && STEP % 8 == 0, "a wave's loads share their swizzle");
   const int skey = w * KPL + lane / GPR;
-  const int kgran = ((lane % GPR) ^ fp_kswz<D>(skey)) << 3;
   const int vgran = ((lane % GPR) ^ fp_vswz<D>(skey)) << 3;
   constexpr int NJ = NI / NW;                          // a wave's K loads per tile
   const int lrow = PAGED ? lane / GPR : skey;          // row that the lane's offset counts
   const unsigned krow = PAGED ? D : (unsigned)k_stride, vrow = PAGED ? D : (unsigned)v_stride;
-  const unsigned koff = ((unsigned)lrow * krow + kgran) * 2;
+  int kgran[PH];
+  unsigned koff[PH];
+#pragma unroll
+  for (int ph = 0; ph < PH; ++ph) {
+    kgran[ph] = ((lane % GPR) ^ fp_kswz<D>(skey + ph * STEP)) << 3;
+    koff[ph] = ((unsigned)lrow * krow + kgran[ph]) * 2;
+  }
   const unsigned voff = ((unsigned)lrow * vrow + vgran) * 2;
   const __hip_bfloat16* kb = PAGED ? k : k + (long)k0 * k_stride + (long)kvh * D;
   const __hip_bfloat16* vb = PAGED ? v : v + (long)k0 * v_stride + (long)kvh * D;
@@ -179,13 +185,14 @@ __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       short* const to = dst + (w + j * NW) * 512;
-      const int gran = is_v ? vgran : kgran;
+      const int gran = is_v ? vgran : kgran[j % PH];
+      const unsigned off = is_v ? voff : koff[j % PH];
       if constexpr (PAGED) {
         const int first = kt + j * STEP + w * KPL;
         const __hip_bfloat16* base =
             (is_v ? vb : kb) + (((long)bid[j] * KVH + kvh) << bs_shift) * D;
         if (whole)
-          glds16_at(base + (first & bs_mask) * D, is_v ? voff : koff, to);
+          glds16_at(base + (first & bs_mask) * D, off, to);
         else
           glds16(base + (min(first + lrow, nk - 1) & bs_mask) * D + gran, to);
       } else {
@@ -193,7 +200,7 @@ __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
         const long stride = is_v ? v_stride : k_stride;
         const __hip_bfloat16* base = (is_v ? vb : kb) + (long)first * stride;
         if (whole)
-          glds16_at(base, is_v ? voff : koff, to);
+          glds16_at(base, off, to);
         else
           glds16(base + (long)(min(first + skey, nk - 1) - first) * stride + gran, to);
       }

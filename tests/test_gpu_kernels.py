@@ -325,7 +325,8 @@ class TestPrefillRanges:
     windows that open inside a tile, and rows inside a wider projection."""
 
     @pytest.mark.parametrize("D,H,KVH", [(64, 6, 3), (64, 3, 1), (128, 3, 1), (128, 4, 2),
-                                         (256, 4, 2), (256, 3, 3)])
+                                         (256, 4, 2), (256, 3, 3),
+                                         (256, 32, 16), (256, 33, 33)])   # eight waves
     @pytest.mark.parametrize("window,softcap", [(0, 0.0), (40, 0.0), (130, 30.0)])
     @pytest.mark.parametrize("past", [0, 1, 100])
     def test_vs_ref(self, D, H, KVH, window, softcap, past):
@@ -541,7 +542,8 @@ class TestPagedPrefill:
     bit: the same tiles, whatever the blocks' order and the rows past the end hold."""
 
     @pytest.mark.parametrize("D,H,KVH,BS", [(64, 4, 2, 16), (64, 3, 3, 32), (128, 6, 2, 16),
-                                            (128, 2, 2, 32), (256, 4, 2, 16), (256, 3, 1, 32)])
+                                            (128, 2, 2, 32), (256, 4, 2, 16), (256, 3, 1, 32),
+                                            (256, 64, 32, 16), (256, 57, 19, 32)])
     @pytest.mark.parametrize("window,softcap", [(0, 0.0), (70, 30.0)])
     def test_equals_packed(self, D, H, KVH, BS, window, softcap):
         lens = [1, 33, 128, 200, 16]
