@@ -273,24 +273,28 @@ class CausalLM:
 
     def _forward_slabs(self, h, residual, positions, kv_cache, meta) -> torch.Tensor:
         """The layers for up to ops.SLAB_ROWS rows (an ordinary decode step, few
-        rows of large layers):
-        streaming products whose partial sums the norms and the rotation add up."""
+        rows of large layers)."""
+        return self._ring_layers(h, residual, positions, kv_cache, meta)
+
+    def _ring_layers(self, h, residual, positions, kv_cache, meta) -> torch.Tensor:
+        """The layers for up to ops.RING_ROWS rows: streaming products whose partial
+        sums the norms and the rotation add up."""
         s = self.spec
         for i, lw in enumerate(self.layers):
             w_next = self.layers[i + 1].input_norm if i + 1 < len(self.layers) else self.final_norm
             qkv = ops.slab_rope_cache(
-                ops.slab_linear(h, lw.qkv), lw.qkv_bias, kv_cache.k[i], kv_cache.v[i], positions,
+                ops.ring_linear(h, lw.qkv), lw.qkv_bias, kv_cache.k[i], kv_cache.v[i], positions,
                 self.rope_cache, meta.slot_mapping,
             )
             attn = self._attention(i, qkv, positions, kv_cache, meta, cached=True)
-            h = ops.slab_add_norm(ops.slab_linear(attn, lw.o), residual, lw.post_attn_norm,
+            h = ops.slab_add_norm(ops.ring_linear(attn, lw.o), residual, lw.post_attn_norm,
                                   lw.pre_mlp_norm, s.rms_eps, self.norm_offset)
-            if ops.slab_act_ok(h, lw.gate_up):
-                act = ops.slab_act_linear(h, lw.gate_up, s.gelu)
+            if ops.ring_act_ok(h, lw.gate_up):
+                act = ops.ring_act_linear(h, lw.gate_up, s.gelu)
             else:
                 gate_up = _proj(h, lw.gate_up)
                 act = ops.gelu_tanh_and_mul(gate_up) if s.gelu else ops.silu_and_mul(gate_up)
-            h = ops.slab_add_norm(ops.slab_linear(act, lw.down), residual, lw.post_mlp_norm,
+            h = ops.slab_add_norm(ops.ring_linear(act, lw.down), residual, lw.post_mlp_norm,
                                   w_next, s.rms_eps, self.norm_offset)
         return h
 
@@ -367,9 +371,11 @@ class CausalLM:
                 and not _USE_SKINNY_GEMM):
             return self._prompt_layers(h, residual, positions, kv_cache, meta)
         if (tp is None and kv_cache.k[0].dtype in (torch.bfloat16, torch.float8_e4m3fn)
-                and ops.slab_ok(h, (l0.qkv, l0.o, l0.gate_up, l0.down), s.hidden_size)
+                and ops.slab_ok(h, (l0.qkv, l0.o, l0.gate_up, l0.down), s.hidden_size,
+                                ops.RING_ROWS)
                 and not _USE_SKINNY_GEMM):
-            return self._forward_slabs(h, residual, positions, kv_cache, meta)
+            layers = self._forward_slabs if len(h) <= ops.SLAB_ROWS else self._ring_layers
+            return layers(h, residual, positions, kv_cache, meta)
         n_layers = len(self.layers)
         for i, lw in enumerate(self.layers):
             # ---- attention block (h = normed input, set by the previous

@@ -370,36 +370,55 @@ def few_rows_qkv(
     return out
 
 
-# --------------------------------------------- projections, up to 128 rows --
+# --------------------------------------------- projections, up to 256 rows --
 # The product stays as fp32 partial sums ("slabs" [parts, M, N]) that the next
 # kernel adds up: norm and residual, or rotation and cache write.
 
 SLAB_ROWS = 128
+RING_ROWS = 256
 
 
-def slab_ok(x: torch.Tensor, weights, hidden: int) -> bool:
-    """Whether the slab kernels take these rows and weights [N, K]."""
+def slab_ok(x: torch.Tensor, weights, hidden: int, rows: int = SLAB_ROWS) -> bool:
+    """Whether the slab kernels take these rows (up to ``rows``) and weights [N, K]."""
     return (
-        x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= SLAB_ROWS
+        x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= rows
         and x.dtype == torch.bfloat16 and x.is_contiguous() and hidden <= 8192
         and all(w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] % 128 == 0
                 and w.shape[0] % 64 == 0 and w.data_ptr() % 16 == 0 for w in weights)
     )
 
 
+def ring_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x @ w.T as fp32 slabs [parts, M, N] whose sum is the product, up to RING_ROWS rows."""
+    assert _use_hip(x)
+    return _EXT.ring_linear(x, w)
+
+
+def ring_act_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ring_act_linear beats the library's product and an activation."""
+    return x.shape[0] <= 192 or w.shape[0] <= 32768
+
+
+def ring_act_linear(x: torch.Tensor, w: torch.Tensor, gelu: bool) -> torch.Tensor:
+    """act(x @ gate.T) * (x @ up.T), w = [gate | up] rows, SiLU or tanh-GELU, up to
+    RING_ROWS rows."""
+    assert _use_hip(x)
+    return _EXT.ring_act_linear(x, w, bool(gelu))
+
+
 def slab_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """x @ w.T as fp32 slabs [parts, M, N] whose sum is the product."""
+    """ring_linear for up to SLAB_ROWS rows."""
     assert _use_hip(x)
     return _EXT.slab_linear(x, w)
 
 
 def slab_act_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether slab_act_linear beats the library's product and an activation."""
-    return x.shape[0] <= 64 and w.numel() < (128 if x.shape[0] <= 16 else 48) << 20
+    return x.shape[0] <= 64
 
 
 def slab_act_linear(x: torch.Tensor, w: torch.Tensor, gelu: bool) -> torch.Tensor:
-    """act(x @ gate.T) * (x @ up.T), w = [gate | up] rows, SiLU or tanh-GELU."""
+    """ring_act_linear for up to 64 rows."""
     assert _use_hip(x)
     return _EXT.slab_act_linear(x, w, bool(gelu))
 

@@ -723,39 +723,115 @@ void stream_qkv(at::Tensor out, at::Tensor x, at::Tensor w, c10::optional<at::Te
                             N / D - 2 * kv_heads, kv_heads, D, (int)k_cache.size(2), fp8});
 }
 
-// ------------------------------------------- projections, up to 128 rows --
+// ------------------------------------------- projections, up to 256 rows --
 
-bool slab_rows_ok(const at::Tensor& x, const at::Tensor& w) {
-  return x.dim() == 2 && w.dim() == 2 && x.size(0) > 0 && x.size(0) <= 128 &&
+constexpr long kSlabRows = 128, kRingRows = 256;
+
+bool slab_rows_ok(const at::Tensor& x, const at::Tensor& w, long rows) {
+  return x.dim() == 2 && w.dim() == 2 && x.size(0) > 0 && x.size(0) <= rows &&
          x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 &&
          x.stride(1) == 1 && rows_start_on(x, 16) && x.size(1) == w.size(1) &&
          w.size(1) % kSlabBK == 0 && w.size(1) > 0 && w.size(0) % 64 == 0;
 }
 
-// Parts of K: as many as keep 512 workgroups (two a CU) busy, two steps each at the
-// least. Measured (us): 64 rows, 2048 x 8192: 16 parts 12.7, 8 14.1, 4 20; 128 rows,
-// 3072 x 3072: 8 parts 13.9, 12 15.4, 4 14.4; 96 rows, 8192 x 3584: 4 parts 22.2,
-// 6 23.2, 3 25.3.
-int slab_parts(long N, long K) {
-  const long tiles = N / 64, steps = K / kSlabBK;
-  for (int s : {16, 12, 8, 6, 4, 3, 2})
-    if (s * tiles <= 512 && steps / s >= 2) return s;
-  return 1;
+int compute_units(const at::Tensor& x) {
+  int cus = 0;
+  TORCH_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
+                                    x.get_device()) == hipSuccess);
+  return cus;
 }
 
-template <int EPI>
-void launch_slab_gemm(float* slabs, __hip_bfloat16* out, long out_stride, const at::Tensor& x,
-                      const at::Tensor& w, int parts) {
+// Token tiles of 16 that ring_gemm.hip is built for.
+int ring_token_tiles(long M) {
+  const int tt = (int)(M + 15) / 16;
+  for (int t : {1, 2, 3, 4, 6, 8, 12, 16})
+    if (tt <= t) return t;
+  return 16;
+}
+
+// ring_gemm.hip counts bytes from a workgroup's first row in 32 bits.
+bool ring_reaches(const at::Tensor& x, const at::Tensor& w) {
+  return w.numel() * 2 < (1L << 32) && x.size(0) * x.stride(0) * 2 < (1L << 32);
+}
+
+// Weight rows of a workgroup (64 or 128) and parts of K: what takes least, a CU taking in
+// (weight + token rows) x 128 bytes a stage at 46 KB/us and the slabs being written at
+// 3.3 and read at 10 MB/us, with no more workgroups than CUs while K has parts. Measured
+// (us, R x parts): 64 rows, 3584 x 14336: 64 x 4 22.6, 128 x 8 20.6, 128 x 9 19.9; 64 rows,
+// 3072 x 2048: 64 x 4 6.2, 64 x 5 5.9, 64 x 8 6.4, 128 x 8 6.5; 96 rows, 8192 x 3584: 64 x 2
+// 16.0, 128 x 4 14.7, 128 x 8 18; 189 rows, 3072 x 3072: 64 x 5 11.7, 128 x 10 12.1.
+struct RingPlan { int rows, parts, steps; };
+
+RingPlan ring_plan(long M, long N, long K, int cus) {
+  RingPlan best{64, 1, (int)(K / kRingBK)};
+  double least = 0;
+  const int tokens = 16 * ring_token_tiles(M), stages = (int)(K / kRingBK);
+  for (int R : {64, 128}) {
+    if (N % R) continue;
+    const long tiles = N / R;
+    for (int p = 1; p <= std::max<long>(1, cus / tiles) && p <= stages; ++p) {
+      const int steps = (stages + p - 1) / p, parts = (stages + steps - 1) / steps;
+      const long rounds = (tiles * parts + cus - 1) / cus;
+      const double us = rounds * (R + tokens) * steps * (128 / 46e3) +
+                        parts * M * N * 4 * (1 / 3.3e6 + 1 / 10e6);
+      if (least == 0 || us < least) least = us, best = RingPlan{R, parts, steps};
+    }
+  }
+  return best;
+}
+
+template <int TT, int RT, int WN, int WT, int WK, int ST, int EPI, bool ROT>
+void launch_ring(float* slabs, __hip_bfloat16* out, long out_stride, const at::Tensor& x,
+                 const at::Tensor& w, int parts, int steps) {
+  using Shape = RingShape<TT, RT, WN, WT, WK, ST>;
   const int M = x.size(0), K = x.size(1), N = w.size(0);
-  const int steps = (K / kSlabBK + parts - 1) / parts;
+  hipLaunchKernelGGL((ring_gemm_kernel<TT, RT, WN, WT, WK, ST, EPI, ROT>),
+                     dim3(N / Shape::kRows * parts), dim3(64 * Shape::kWaves), Shape::kLds,
+                     stream(), slabs, out, out_stride,
+                     reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()), x.stride(0),
+                     reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()), M, N, K, parts, steps);
+}
+
+template <typename F>
+void ring_tiles(long M, F&& go) {
+  switch (ring_token_tiles(M)) {
+    case 1: return go.template operator()<1>();
+    case 2: return go.template operator()<2>();
+    case 3: return go.template operator()<3>();
+    case 4: return go.template operator()<4>();
+    case 6: return go.template operator()<6>();
+    case 8: return go.template operator()<8>();
+    case 12: return go.template operator()<12>();
+    default: return go.template operator()<16>();
+  }
+}
+
+// Two weight tiles and one wave column suit few tokens, four and two (four from 129 rows
+// on) the others, whose operand reads from LDS count (128 rows, 3584 x 14336: 25.7 and 26.3).
+template <int TT, int EPI>
+void launch_ring_128(float* slabs, __hip_bfloat16* out, long out_stride, const at::Tensor& x,
+                     const at::Tensor& w, int parts, int steps) {
+  if constexpr (TT <= 3)
+    launch_ring<TT, 2, 4, 1, 1, 4, EPI, false>(slabs, out, out_stride, x, w, parts, steps);
+  else if constexpr (TT <= 8)
+    launch_ring<TT, 4, 2, 2, 1, 3, EPI, false>(slabs, out, out_stride, x, w, parts, steps);
+  else
+    launch_ring<TT, 4, 2, 4, 1, 3, EPI, false>(slabs, out, out_stride, x, w, parts, steps);
+}
+
+// slab_gemm.hip: operands out of the ring kernels' reach.
+template <int EPI>
+void launch_slab_gemm(float* slab, __hip_bfloat16* out, long out_stride, const at::Tensor& x,
+                      const at::Tensor& w) {
+  const int M = x.size(0), K = x.size(1), N = w.size(0);
   auto go = [&]<int TM, int WK>() {
-    hipLaunchKernelGGL((slab_gemm_kernel<TM, WK, EPI>), dim3(N / 64, parts), dim3(256 * WK), 0,
-                       stream(), slabs, out, out_stride,
+    hipLaunchKernelGGL((slab_gemm_kernel<TM, WK, EPI>), dim3(N / 64), dim3(256 * WK), 0, stream(),
+                       slab, out, out_stride,
                        reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()), x.stride(0),
-                       reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()), M, N, K, steps);
+                       reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()), M, N, K,
+                       K / kSlabBK);
   };
-  // Gates need whole sums: two groups of waves instead of parts (64 rows,
-  // 16384 x 2048: 20.8 us, one group 25.3).
+  // Gates need whole sums: two groups of waves instead of parts of K.
   constexpr int WK = EPI == kSlabSums ? 1 : 2;
   const int tm = (M + 15) / 16;
   if (tm == 1) go.template operator()<1, WK>();
@@ -769,42 +845,104 @@ void launch_slab_gemm(float* slabs, __hip_bfloat16* out, long out_stride, const 
 }
 
 // x W^T as fp32 slabs [parts, M, N]; their sum is the product.
-at::Tensor slab_linear(const at::Tensor& x, const at::Tensor& w) {
+at::Tensor ring_linear(const at::Tensor& x, const at::Tensor& w) {
   CHECK_GPU(x);
-  TORCH_CHECK(slab_rows_ok(x, w),
-              "slab_linear: 1 to 128 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
+  TORCH_CHECK(slab_rows_ok(x, w, kRingRows),
+              "ring_linear: 1 to 256 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
   if (!streamable(w)) return at::linear(x, w).to(at::kFloat).unsqueeze(0);
-  const int parts = slab_parts(w.size(0), w.size(1));
-  at::Tensor slabs = at::empty({parts, x.size(0), w.size(0)}, x.options().dtype(at::kFloat));
-  launch_slab_gemm<kSlabSums>(slabs.data_ptr<float>(), nullptr, 0, x, w, parts);
+  const long M = x.size(0), N = w.size(0), K = w.size(1);
+  const auto opts = x.options().dtype(at::kFloat);
+  if (!ring_reaches(x, w)) {
+    if (M > kSlabRows) return at::linear(x, w).to(at::kFloat).unsqueeze(0);
+    at::Tensor slab = at::empty({1, M, N}, opts);
+    launch_slab_gemm<kSlabSums>(slab.data_ptr<float>(), nullptr, 0, x, w);
+    return slab;
+  }
+  const RingPlan plan = ring_plan(M, N, K, compute_units(x));
+  at::Tensor slabs = at::empty({plan.parts, M, N}, opts);
+  float* p = slabs.data_ptr<float>();
+  ring_tiles(M, [&]<int TT>() {
+    if (plan.rows == 128)
+      launch_ring_128<TT, kSlabSums>(p, nullptr, 0, x, w, plan.parts, plan.steps);
+    else if constexpr (TT <= 8)
+      launch_ring<TT, 1, 4, 1, 1, 4, kSlabSums, false>(p, nullptr, 0, x, w, plan.parts, plan.steps);
+    else
+      launch_ring<TT, 2, 2, 4, 1, 4, kSlabSums, false>(p, nullptr, 0, x, w, plan.parts, plan.steps);
+  });
   return slabs;
 }
 
-// Whether gate and value rows are worth a product of their own with the activation
-// in it: from 48 M weights on the library's product and the activation are as fast
-// (48 rows, 28672 x 3584: 49.0 + 5.2 us against 53.5), up to 16 rows from 128 M on (8
-// rows, 28672 x 4096: 61.5 against 51.3, 28672 x 3584: 45.8 / 47.5, 37888 x 3584: 56.1 /
-// 66.1, 55296 x 5120: 98 / 144).
-bool slab_act_ok(const at::Tensor& x, const at::Tensor& w) {
-  return slab_rows_ok(x, w) && x.size(0) <= 64 &&
-         w.numel() < ((x.size(0) <= 16 ? 128L : 48L) << 20);
+// Gate and value rows: as many weight rows a workgroup as make one round of workgroups.
+// Measured (us, 64 / 128 / 256 rows): 64 tokens, 28672 x 3584 42.6 / 35.8 / -; 48 tokens,
+// 37888 x 3584 60 / 60 / 51.5; 128, 55296 x 5120 177 / 132 / 107; 128, 16384 x 3072 28.2 / 38 / -.
+template <int EPI>
+void launch_ring_act(__hip_bfloat16* out, long out_stride, const at::Tensor& x,
+                     const at::Tensor& w) {
+  const long N = w.size(0), cus = compute_units(x);
+  const int steps = (int)(w.size(1) / kRingBK);
+  const bool r128 = N / 64 > cus && N % 128 == 0;
+  const bool r256 = N / 128 > cus && N % 256 == 0;
+  ring_tiles(x.size(0), [&]<int TT>() {
+    auto go = [&]<int RT, int WN, int WT, int WK, int ST, bool ROT>() {
+      launch_ring<TT, RT, WN, WT, WK, ST, EPI, ROT>(nullptr, out, out_stride, x, w, 1, steps);
+    };
+    if (r256) {
+      if constexpr (TT <= 3) go.template operator()<2, 8, 1, 1, 3, false>();
+      else if constexpr (TT <= 8) go.template operator()<4, 4, 2, 1, 3, false>();
+      else go.template operator()<4, 4, 2, 1, 2, false>();
+    } else if (r128) {
+      launch_ring_128<TT, EPI>(nullptr, out, out_stride, x, w, 1, steps);
+    } else {
+      // eight waves where two groups, or four columns, have work for them (64 rows of 16384 x
+      // 2048: one group 14.0, two 14.6; 96 rows 17.1 and 16.5; 45 rows 16.1 and 14.1)
+      if constexpr (TT == 1 || TT == 3) go.template operator()<2, 2, 1, 2, 4, true>();
+      else if constexpr (TT <= 4) go.template operator()<2, 2, 2, 1, 4, true>();
+      else if constexpr (TT == 6) go.template operator()<2, 2, 2, 2, 3, true>();
+      else go.template operator()<2, 2, 4, 1, 4, true>();
+    }
+  });
+}
+
+// Whether gate and value rows are worth a product of their own with the activation in
+// it: up to 192 rows always, up to 256 while 128 weight rows a workgroup make one round
+// (256 rows, the library's product + activation: 28672 x 3584 63.2 + 6 against 62.6,
+// 37888 x 3584 79 + 7 / 106; 189 rows, 55296 x 5120 146 + 8 / 138; 96 rows, 28672 x 3584
+// 46.8 + 5 / 39.6).
+bool ring_act_ok(const at::Tensor& x, const at::Tensor& w) {
+  return slab_rows_ok(x, w, kRingRows) && (x.size(0) <= 192 || w.size(0) <= 32768);
+}
+
+at::Tensor ring_act_linear(const at::Tensor& x, const at::Tensor& w, bool gelu) {
+  CHECK_GPU(x);
+  TORCH_CHECK(slab_rows_ok(x, w, kRingRows),
+              "ring_act_linear: 1 to 256 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
+  at::Tensor out = at::empty({x.size(0), w.size(0) / 2}, x.options());
+  auto* p = reinterpret_cast<__hip_bfloat16*>(out.data_ptr());
+  if (!streamable(w) || (!ring_reaches(x, w) && x.size(0) > 64)) {
+    const at::Tensor y = at::linear(x, w);
+    if (gelu) gelu_tanh_and_mul(out, y);
+    else silu_and_mul(out, y);
+  } else if (!ring_reaches(x, w)) {
+    if (gelu) launch_slab_gemm<kSlabGelu>(nullptr, p, out.stride(0), x, w);
+    else launch_slab_gemm<kSlabSilu>(nullptr, p, out.stride(0), x, w);
+  } else if (gelu) launch_ring_act<kSlabGelu>(p, out.stride(0), x, w);
+  else launch_ring_act<kSlabSilu>(p, out.stride(0), x, w);
+  return out;
+}
+
+// The two for up to 128 and 64 rows.
+at::Tensor slab_linear(const at::Tensor& x, const at::Tensor& w) {
+  CHECK_GPU(x);
+  TORCH_CHECK(slab_rows_ok(x, w, kSlabRows),
+              "slab_linear: 1 to 128 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
+  return ring_linear(x, w);
 }
 
 at::Tensor slab_act_linear(const at::Tensor& x, const at::Tensor& w, bool gelu) {
   CHECK_GPU(x);
-  TORCH_CHECK(slab_rows_ok(x, w) && x.size(0) <= 64,
+  TORCH_CHECK(slab_rows_ok(x, w, 64),
               "slab_act_linear: 1 to 64 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
-  at::Tensor out = at::empty({x.size(0), w.size(0) / 2}, x.options());
-  if (!streamable(w)) {
-    const at::Tensor y = at::linear(x, w);
-    if (gelu) gelu_tanh_and_mul(out, y);
-    else silu_and_mul(out, y);
-    return out;
-  }
-  auto* p = reinterpret_cast<__hip_bfloat16*>(out.data_ptr());
-  if (gelu) launch_slab_gemm<kSlabGelu>(nullptr, p, out.stride(0), x, w, 1);
-  else launch_slab_gemm<kSlabSilu>(nullptr, p, out.stride(0), x, w, 1);
-  return out;
+  return ring_act_linear(x, w, gelu);
 }
 
 void check_slabs(const at::Tensor& slabs) {
@@ -904,12 +1042,12 @@ at::Tensor prompt_layers(at::Tensor h, at::Tensor residual, at::TensorList weigh
                   windows.size() == layers && (biases.empty() || biases.size() == layers),
               "one entry per layer");
   const long T = h.size(0);
-  // up to 128 rows of these shapes: the streaming products, whose sums the next
+  // up to 256 rows of these shapes: the streaming products, whose sums the next
   // kernel takes up
   const bool slab = layers > 0 && k_caches[0].size(3) == head_dim && h.size(1) <= 8192 &&
                     (k_caches[0].scalar_type() == at::kBFloat16 ||
                      k_caches[0].scalar_type() == at::kFloat8_e4m3fn) &&
-                    slab_rows_ok(h, weights[0]) && weights[1].size(0) == h.size(1) &&
+                    slab_rows_ok(h, weights[0], kRingRows) && weights[1].size(0) == h.size(1) &&
                     weights[1].size(1) % kSlabBK == 0 && weights[1].size(0) % 64 == 0 &&
                     weights[3].size(1) % kSlabBK == 0 && residual.is_contiguous();
   const c10::optional<at::Tensor> none;
@@ -918,7 +1056,7 @@ at::Tensor prompt_layers(at::Tensor h, at::Tensor residual, at::TensorList weigh
     const c10::optional<at::Tensor> bias =
         biases.empty() ? none : c10::make_optional(biases[i]);
     const at::Tensor qkv =
-        slab ? slab_rope_cache(slab_linear(h, w[0]), bias, k_caches[i], v_caches[i], positions,
+        slab ? slab_rope_cache(ring_linear(h, w[0]), bias, k_caches[i], v_caches[i], positions,
                                cos_sin, slots)
              : at::linear(h, w[0], bias);
     const long kv_heads = k_caches[i].size(1);
@@ -940,7 +1078,7 @@ at::Tensor prompt_layers(at::Tensor h, at::Tensor residual, at::TensorList weigh
     auto project_add_norm = [&](const at::Tensor& a, const at::Tensor& wt,
                                 const at::Tensor* post, const at::Tensor& norm) {
       if (slab)
-        return slab_add_norm(slab_linear(a, wt), residual,
+        return slab_add_norm(ring_linear(a, wt), residual,
                              post ? c10::make_optional(*post) : none, norm, eps, offset);
       at::Tensor y = at::linear(a, wt);
       if (post) norm_add_norm(y, residual, *post, norm, eps, offset);
@@ -950,8 +1088,8 @@ at::Tensor prompt_layers(at::Tensor h, at::Tensor residual, at::TensorList weigh
     h = project_add_norm(attn.view({T, heads * head_dim}), w[1], post_norms ? &w[6] : nullptr,
                          w[4]);
     at::Tensor act;
-    if (slab && slab_act_ok(h, w[2])) {
-      act = slab_act_linear(h, w[2], gelu);
+    if (slab && ring_act_ok(h, w[2])) {
+      act = ring_act_linear(h, w[2], gelu);
     } else {
       const at::Tensor gate_up = at::linear(h, w[2]);
       act = at::empty({T, gate_up.size(1) / 2}, gate_up.options());
@@ -1070,6 +1208,8 @@ TORCH_LIBRARY(llmq_amd, m) {
   m.def("paged_prefill_attention(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor cu_seqlens, Tensor cu_seqlens_k, int max_seqlen, float scale, float softcap, int window) -> ()");
   m.def("stream_qkv(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, Tensor? norm_w, float eps, float offset, Tensor(b!) k_cache, Tensor(c!) v_cache, Tensor positions, Tensor cos_sin, Tensor slots) -> ()");
   m.def("slab_linear(Tensor x, Tensor w) -> Tensor");
+  m.def("ring_linear(Tensor x, Tensor w) -> Tensor");
+  m.def("ring_act_linear(Tensor x, Tensor w, bool gelu) -> Tensor");
   m.def("slab_act_linear(Tensor x, Tensor w, bool gelu) -> Tensor");
   m.def("slab_add_norm(Tensor slabs, Tensor(a!) residual, Tensor? w_post, Tensor w, float eps, float offset) -> Tensor");
   m.def("slab_rope_cache(Tensor slabs, Tensor? bias, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor positions, Tensor cos_sin, Tensor slots) -> Tensor");
@@ -1094,6 +1234,8 @@ TORCH_LIBRARY_IMPL(llmq_amd, CUDA, m) {
   m.impl("varlen_prefill_attention", &varlen_prefill_attention);
   m.impl("paged_prefill_attention", &paged_prefill_attention);
   m.impl("slab_linear", &slab_linear);
+  m.impl("ring_linear", &ring_linear);
+  m.impl("ring_act_linear", &ring_act_linear);
   m.impl("slab_act_linear", &slab_act_linear);
   m.impl("slab_add_norm", &slab_add_norm);
   m.impl("slab_rope_cache", &slab_rope_cache);

@@ -8,5 +8,6 @@
 #include "skinny_gemm.hip"
 #include "stream_gemm.hip"
 #include "slab_gemm.hip"
+#include "ring_gemm.hip"
 #include "sampling.hip"
 #include "bindings.cpp"

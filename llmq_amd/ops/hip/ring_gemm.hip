@@ -1,0 +1,214 @@
+// Projections of up to 256 rows, x[M, K] W[N, K]^T with fp32 sums: the products of an
+// ordinary decode step, a short prompt, or few rows through large layers (gfx950).
+//
+// Bound by the weights' bytes up to some 64 rows, beyond by what a CU takes from its L2:
+// every workgroup reads the tokens again, and 45 to 47 KB/us a CU is the most that was
+// seen. So weights and tokens alike go to LDS by global_load_lds, without passing
+// registers, through a ring of ST stages of 64 channels whose loads are counted by hand:
+// ST - 1 stages travel while one is multiplied. (With weights in registers and tokens in
+// LDS the compiler's own wait covered both: 2.6 to 2.7 TB/s at all sizes.)
+//
+//   - A workgroup owns R = 16 RT WN weight rows, all token rows and one of S parts of K;
+//     its waves stand WN x WT over them, each with RT x TT/WT tiles of
+//     v_mfma_f32_16x16x32_bf16 (A = weights: row = lane%16, k = 8*(lane/16)..+7;
+//     B = tokens likewise; C: column = token, rows = 4 weight rows).
+//   - A stage's rows are 128 bytes in 16-byte granules, placed by row so that the 16
+//     rows of an operand read lie in 16 different bank groups.
+//   - S > 1 leaves the parts as fp32 slabs [S, M, N], added up by the kernel that reads
+//     them anyway (norm and residual, rotation and cache write): the sum costs no launch
+//     and no rounding. Parts of the same K lie on the same XCDs, whose L2 then holds
+//     that part of the tokens only.
+//   - Gate and value rows (EPI kSlabSilu, kSlabGelu) are activated here: a wave's first
+//     RT/2 tiles are gates, the others the values of the same columns. They need whole
+//     sums, so no parts of K: WK groups of waves take the stages in turn instead.
+//   - ROT: workgroups start at different stages. Rows of 4096 bytes start on the same
+//     memory channel, which all workgroups would ask at once (64 rows, 16384 x 2048:
+//     16.2 us, 14.0 with it).
+//
+// Measured (us; before = slab_gemm_kernel, from 129 rows on the library's product):
+// 64 rows, 2048 x 8192: 12.4 -> 9.0, 16384 x 2048 pairs 20.3 -> 14.0; 96 rows, 3584 x 14336:
+// 37.9 -> 23.3, 8192 x 3584 21.5 -> 14.7; 45 rows, 28672 x 3584 pairs 52.8 -> 34.1 (206 MB,
+// 6.0 TB/s); 128 rows, 3072 x 8192 23.8 -> 16.8; 189 rows, 3072 x 8192 58 -> 20.1, 3072 x 3072
+// 26.5 -> 12.5; 256 rows, 3584 x 14336 59.4 -> 36.5.
+
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(8))) short rg_s16x8;
+typedef __attribute__((ext_vector_type(4))) float rg_f32x4;
+
+constexpr int kRingBK = 64;
+
+// 16 bytes per lane from base + off to LDS, lane-linear from lds_off (uniform).
+template <bool NT>
+DEVINL void ring_load(const void* base, unsigned off, unsigned lds_off) {
+  unsigned keep;
+  if constexpr (NT)
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %3\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %2 nt\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_off) : "memory");
+  else
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %3\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %2\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_off) : "memory");
+}
+
+// The wave's loads have landed but those of the last min(left, N) stages, NL each;
+// everyone's LDS reads are done.
+template <int N, int NL>
+DEVINL void ring_wait(int left) {
+  if constexpr (N == 0) pipe_barrier_vm<0>();
+  else if (left >= N) pipe_barrier_vm<N * NL>();
+  else ring_wait<N - 1, NL>(left);
+}
+
+template <int TT, int RT, int WN, int WT, int WK, int ST>
+struct RingShape {
+  static constexpr int kRows = 16 * RT * WN, kTokens = 16 * TT, kWaves = WN * WT * WK;
+  static constexpr size_t kLds = sizeof(short) * (size_t)WK * ST * (kRows + kTokens) * kRingBK;
+  static_assert(kLds <= (160 << 10));
+};
+
+// parts: of K, none of them empty; steps: stages of a part (the last may have fewer).
+template <int TT, int RT, int WN, int WT, int WK, int ST, int EPI, bool ROT>
+__global__ __launch_bounds__(64 * WN * WT * WK) void ring_gemm_kernel(
+    float* __restrict__ slabs, __hip_bfloat16* __restrict__ out, long out_stride,
+    const __hip_bfloat16* __restrict__ x, long x_stride,
+    const __hip_bfloat16* __restrict__ wt, int M, int N, int K, int parts, int steps) {
+  constexpr bool PAIR = EPI != kSlabSums;
+  static_assert(PAIR || WK == 1, "groups' sums meet in LDS for gate and value rows only");
+  static_assert(!PAIR || RT % 2 == 0, "a wave holds gates and their values");
+  constexpr int BK = kRingBK, R = 16 * RT * WN, T = 16 * TT, TW = TT / WT, G = WN * WT;
+  constexpr int UW = R / 8, UT = T / 8;                  // loads of a stage: 8 rows each
+  constexpr int NW = UW / G, NT = (UT + G - 1) / G, NL = NW + NT;   // a wave's
+  static_assert(UW % G == 0 && TT % WT == 0 && (ST - 2) * NL < 64);
+  constexpr int STAGE = (R + T) * BK;
+  extern __shared__ __align__(16) short ring_lds[];      // [WK][ST][R weight | T token rows][BK]
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int w = wave % G, kg = wave / G;
+  const int wn = w % WN, wc = w / WN;
+  const int col = lane & 15, grp = lane >> 4;
+  const int part = blockIdx.x % parts, tile = blockIdx.x / parts;
+  const int step0 = part * steps, total = min(steps, K / BK - step0);
+  const int loops = (total + WK - 1) / WK;
+  const int n0 = tile * (PAIR ? R / 2 : R);
+  const int rot = ROT ? tile % loops : 0;
+
+  // Staging: load u of a stage is rows 8 u + lane/8, the weights' first; a wave takes
+  // every G-th. Loads past the last token row repeat it.
+  auto place = [&](int row) { return ((lane & 7) ^ ((row >> 1) & 7)) << 3; };
+  unsigned woff[NW], xoff[NT];
+#pragma unroll
+  for (int j = 0; j < NW; ++j) {
+    const int lr = (w + j * G) * 8 + (lane >> 3);
+    int row = lr;                                        // from n0
+    if constexpr (PAIR) {
+      const int t = (lr / 16) % RT;
+      row = lr / (16 * RT) * (RT * 8) + t % (RT / 2) * 16 + lr % 16 + (t < RT / 2 ? 0 : N / 2);
+    }
+    woff[j] = ((unsigned)row * (unsigned)K + place(lr)) * 2u;
+  }
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int lr = min(w + j * G, UT - 1) * 8 + (lane >> 3);
+    xoff[j] = ((unsigned)min(lr, M - 1) * (unsigned)x_stride + place(lr)) * 2u;
+  }
+  const __hip_bfloat16* wb = wt + (long)n0 * K + (long)step0 * BK;
+  const __hip_bfloat16* xb = x + (long)step0 * BK;
+  short* const ring = ring_lds + kg * (ST * STAGE);
+  const unsigned ring_off = (unsigned)(unsigned long)(
+      (__attribute__((address_space(3))) char*)ring);
+  auto step_of = [&](int i) {                            // stage i's 64 channels
+    int s = i + rot;
+    if (s >= loops) s -= loops;
+    return s * WK + kg;
+  };
+  auto stage = [&](int i) {
+    const long k = (long)min(step_of(i), total - 1) * BK;
+    const unsigned to = __builtin_amdgcn_readfirstlane(ring_off + (unsigned)(i % ST) * (STAGE * 2));
+#pragma unroll
+    for (int j = 0; j < NW; ++j) ring_load<true>(wb + k, woff[j], to + (w + j * G) * 1024);
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+      ring_load<false>(xb + k, xoff[j], to + (UW + min(w + j * G, UT - 1)) * 1024);
+  };
+  rg_f32x4 acc[RT][TW];
+#pragma unroll
+  for (int a = 0; a < RT; ++a)
+#pragma unroll
+    for (int m = 0; m < TW; ++m) acc[a][m] = rg_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < ST - 1; ++i)
+    if (i < loops) stage(i);
+  for (int i = 0; i < loops; ++i) {
+    ring_wait<ST - 2, NL>(loops - 1 - i);                // stage i is here, i - 1 is read
+    if (i + ST - 1 < loops) stage(i + ST - 1);
+    if (WK > 1 && step_of(i) >= total) continue;
+    const short* at = ring + (i % ST) * STAGE;
+    const short* wa = at + (wn * RT * 16 + col) * BK;
+    const short* xa = at + (R + wc * TW * 16 + col) * BK;
+#pragma unroll
+    for (int u = 0; u < BK / 32; ++u) {
+      const int g = ((u * 4 + grp) ^ ((col >> 1) & 7)) << 3;
+      rg_s16x8 wf[RT];
+#pragma unroll
+      for (int a = 0; a < RT; ++a) wf[a] = *reinterpret_cast<const rg_s16x8*>(wa + a * 16 * BK + g);
+#pragma unroll
+      for (int m = 0; m < TW; ++m) {
+        const rg_s16x8 xf = *reinterpret_cast<const rg_s16x8*>(xa + m * 16 * BK + g);
+#pragma unroll
+        for (int a = 0; a < RT; ++a)
+          acc[a][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[a], xf, acc[a][m], 0, 0, 0);
+      }
+    }
+  }
+  if constexpr (WK > 1) {                                // the groups' sums
+    constexpr int NA = RT * TW;
+    static_assert((size_t)(WK - 1) * G * NA * 1024 <= RingShape<TT, RT, WN, WT, WK, ST>::kLds);
+    rg_f32x4* red = reinterpret_cast<rg_f32x4*>(ring_lds) + lane;
+    __syncthreads();
+    if (kg > 0)
+#pragma unroll
+      for (int e = 0; e < NA; ++e)
+        red[(((kg - 1) * G + w) * NA + e) * 64] = acc[e / TW][e % TW];
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int g = 0; g < WK - 1; ++g)
+#pragma unroll
+      for (int e = 0; e < NA; ++e) acc[e / TW][e % TW] += red[((g * G + w) * NA + e) * 64];
+  }
+#pragma unroll
+  for (int m = 0; m < TW; ++m) {
+    const int row = (wc * TW + m) * 16 + col;
+    if (row >= M) continue;
+    if constexpr (!PAIR) {
+      float* slab = slabs + ((long)part * M + row) * N + n0 + wn * RT * 16 + grp * 4;
+#pragma unroll
+      for (int a = 0; a < RT; ++a) *reinterpret_cast<rg_f32x4*>(slab + a * 16) = acc[a][m];
+    } else {
+#pragma unroll
+      for (int a = 0; a < RT / 2; ++a) {
+        Vec4<__hip_bfloat16> v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float g = acc[a][m][r];
+          const float y = EPI == kSlabSilu
+              ? g / (1.0f + __expf(-g))
+              : 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
+          v.data[r] = __float2bfloat16(y * acc[a + RT / 2][m][r]);
+        }
+        *reinterpret_cast<int2*>(out + (long)row * out_stride + n0 + (wn * (RT / 2) + a) * 16 +
+                                 grp * 4) = *reinterpret_cast<const int2*>(v.data);
+      }
+    }
+  }
+}

@@ -1,8 +1,8 @@
-// Projections of up to 128 rows, x[M, K] W[N, K]^T with fp32 sums: the products of
-// an ordinary decode step or a short prompt, and of few rows through large layers
-// (gfx950).
+// Projections of up to 128 rows, x[M, K] W[N, K]^T with fp32 sums, by 64-bit addresses:
+// for operands that ring_gemm.hip cannot reach with 32-bit offsets (rows spread over
+// 4 GiB). And the kernels that add up the slabs of either.
 //
-// Bound by the weights' bytes. A workgroup owns 64 weight rows, all M tokens and one
+// A workgroup owns 64 weight rows, all M tokens and one
 // of S parts of K. Weights go straight from memory into the matrix layout; the tokens,
 // which every workgroup reads again, are staged once per workgroup in LDS by
 // global_load_lds (16-byte granules placed by row, so operand reads meet no bank
@@ -11,15 +11,8 @@
 // A step of 128 channels asks for the next step's tokens at its start and for the
 // weights of the one after at its end, but its products wait for both: the loads sit
 // under conditions, and the compiler's count of what may still travel is the least over
-// all paths. What overlaps is the weights' way with one step's end and the next's
-// barrier: 2.6 to 2.7 TB/s, where decode attention reads 5.8.
-//
-// With S > 1 the parts are left as fp32 slabs [S, M, N] and added up by the kernel
-// that reads them anyway (norm and residual, rotation and cache write): the sum
-// costs no launch and no rounding. Gate and value rows (PAIR) are activated here.
-// Measured (us, the library's product before): 64 rows, 2048 x 8192: 22.8 -> 12.7,
-// 2048 x 2048: 8.8 -> 5.6, 3072 x 2048: 12.0 -> 8.1; 96 rows, 3584 x 14336: 50.4 ->
-// 38.6; 128 rows, 3072 x 8192: 42.8 -> 25.6; 24 rows, 1536 x 8960: 28.7 -> 11.9.
+// all paths: 2.6 to 2.7 TB/s, where the ring kernel reads 3.7 to 6 (64 rows, 2048 x 8192:
+// 12.4 us against 9.0). Gate and value rows (PAIR) are activated here.
 
 #include "common.h"
 

@@ -467,6 +467,45 @@ class TestSlabProjections:
             tol = 2 ** -8 * (act * u).abs() + 3e-5 * (1 + g.abs()) * (1 + u.abs())
             assert ((y - act * u).abs() <= tol).all()
 
+    @pytest.mark.parametrize("M", [1, 16, 17, 48, 64, 96, 128, 129, 192, 193, 256])
+    @pytest.mark.parametrize("N,K", [(64, 128), (192, 640), (384, 1152), (2048, 8192)])
+    def test_ring_products(self, M, N, K):
+        """Every token-tile count and both widths of a workgroup, up to 256 rows; fewer
+        stages than the ring holds, and parts of unequal length."""
+        x = torch.randn(M, K + 8, device=DEV, dtype=torch.bfloat16)[:, :K]
+        w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) * K ** -0.5
+        ref = x.double() @ w.double().t()
+        got = ops.ring_linear(x, w).double().sum(0)
+        assert ((got - ref).abs() <= 1e-5 * (1 + ref.abs())).all()     # fp32 sums of unit size
+
+    @pytest.mark.parametrize("M", [1, 16, 17, 48, 64, 96, 128, 129, 192, 193, 256])
+    @pytest.mark.parametrize("N,K", [(64, 128), (16384, 192 * 2), (16448, 128), (16512, 640),
+                                     (33024, 256), (65792, 128)])
+    def test_ring_activated(self, M, N, K):
+        """64, 128 and 256 weight rows a workgroup, one round of them and more."""
+        x = torch.randn(M, K, device=DEV, dtype=torch.bfloat16)
+        w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) * K ** -0.5
+        g, u = (x.double() @ w.double().t()).chunk(2, -1)
+        for gelu in (False, True):
+            act = torch.nn.functional.gelu(g, approximate="tanh") if gelu \
+                else torch.nn.functional.silu(g)
+            y = ops.ring_act_linear(x, w, gelu).double()
+            tol = 2 ** -8 * (act * u).abs() + 3e-5 * (1 + g.abs()) * (1 + u.abs())
+            assert ((y - act * u).abs() <= tol).all()
+
+    def test_rows_far_apart(self):
+        """Rows over 4 GiB from the first: the kernels with 64-bit addresses."""
+        flat = torch.zeros((1 << 31) + 256, device=DEV, dtype=torch.bfloat16)
+        x = flat.as_strided((3, 256), (1 << 30, 1))
+        x.normal_()
+        w = torch.randn(64, 256, device=DEV, dtype=torch.bfloat16) / 16
+        ref = x.double() @ w.double().t()
+        got = ops.slab_linear(x, w).double().sum(0)
+        assert ((got - ref).abs() <= 1e-5 * (1 + ref.abs())).all()
+        g, u = ref.chunk(2, -1)
+        y, want = ops.slab_act_linear(x, w, False).double(), torch.nn.functional.silu(g) * u
+        assert ((y - want).abs() <= 2 ** -8 * want.abs() + 3e-5 * (1 + g.abs()) * (1 + u.abs())).all()
+
     @pytest.mark.parametrize("S,M,N", [(1, 1, 64), (16, 5, 8192), (1, 17, 64), (3, 20, 1000), (16, 64, 2048), (2, 128, 8192)])
     @pytest.mark.parametrize("post", [False, True])
     def test_add_norm(self, S, M, N, post):
