@@ -318,34 +318,36 @@ class CausalLM:
         )
 
     def _forward_few_rows(self, residual, positions, kv_cache, meta) -> torch.Tensor:
-        """The layers for up to ops.FEW_ROWS rows (a decode step of few
-        sequences; fewer rows of large layers): norms, rotation, cache write, activation and residual addition
-        ride on the projections, which stream the weights once."""
+        """The layers for up to ops.FEW_ROWS rows (a decode step of few sequences; fewer
+        rows of large layers): norms, rotation, cache write, activation and residual
+        addition ride on the projections, which stream the weights once."""
         s = self.spec
         act = "gelu_tanh" if s.gelu else "silu"
         n_layers = len(self.layers)
-        h = self._norm(residual, self.layers[0].input_norm) if s.post_norms else None
+        if not s.post_norms:
+            rows = ops.FewRows(residual, s.rms_eps, self.norm_offset)
+            rows.start(self.layers[0].input_norm)
+            for i, lw in enumerate(self.layers):
+                qkv = rows.qkv(lw.qkv, lw.qkv_bias, kv_cache.k[i], kv_cache.v[i], positions,
+                               self.rope_cache, meta.slot_mapping)
+                rows.add(self._attention(i, qkv, positions, kv_cache, meta, cached=True), lw.o,
+                         lw.pre_mlp_norm)
+                rows.add(rows.act(lw.gate_up, s.gelu), lw.down,
+                         self.layers[i + 1].input_norm if i + 1 < n_layers else None)
+            return self._norm(residual, self.final_norm)
+        h = self._norm(residual, self.layers[0].input_norm)
         for i, lw in enumerate(self.layers):
-            cache = (kv_cache.k[i], kv_cache.v[i], positions, self.rope_cache, meta.slot_mapping)
-            if s.post_norms:
-                qkv = ops.few_rows_qkv(h, lw.qkv, lw.qkv_bias, None, 0.0, 0.0, *cache)
-                y = ops.few_rows_linear(
-                    self._attention(i, qkv, positions, kv_cache, meta, cached=True), lw.o)
-                h, residual = ops.norm_add_norm(
-                    y, residual, lw.post_attn_norm, lw.pre_mlp_norm, s.rms_eps, self.norm_offset)
-                y = ops.few_rows_linear(ops.few_rows_linear(h, lw.gate_up, act=act), lw.down)
-                w_next = self.layers[i + 1].input_norm if i + 1 < n_layers else self.final_norm
-                h, residual = ops.norm_add_norm(
-                    y, residual, lw.post_mlp_norm, w_next, s.rms_eps, self.norm_offset)
-                continue
-            qkv = ops.few_rows_qkv(residual, lw.qkv, lw.qkv_bias, lw.input_norm, s.rms_eps,
-                                   self.norm_offset, *cache)
-            ops.few_rows_linear(self._attention(i, qkv, positions, kv_cache, meta, cached=True),
-                                lw.o, residual=residual)
-            a = ops.few_rows_linear(residual, lw.gate_up, None, lw.pre_mlp_norm,
-                                    s.rms_eps, self.norm_offset, act=act)
-            ops.few_rows_linear(a, lw.down, residual=residual)
-        return h if s.post_norms else self._norm(residual, self.final_norm)
+            qkv = ops.few_rows_qkv(h, lw.qkv, lw.qkv_bias, None, 0.0, 0.0, kv_cache.k[i],
+                                   kv_cache.v[i], positions, self.rope_cache, meta.slot_mapping)
+            y = ops.few_rows_linear(
+                self._attention(i, qkv, positions, kv_cache, meta, cached=True), lw.o)
+            h, residual = ops.norm_add_norm(
+                y, residual, lw.post_attn_norm, lw.pre_mlp_norm, s.rms_eps, self.norm_offset)
+            y = ops.few_rows_linear(ops.few_rows_linear(h, lw.gate_up, act=act), lw.down)
+            w_next = self.layers[i + 1].input_norm if i + 1 < n_layers else self.final_norm
+            h, residual = ops.norm_add_norm(
+                y, residual, lw.post_mlp_norm, w_next, s.rms_eps, self.norm_offset)
+        return h
 
     @torch.no_grad()
     def forward(

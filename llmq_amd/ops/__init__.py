@@ -370,6 +370,41 @@ def few_rows_qkv(
     return out
 
 
+class FewRows:
+    """The rows of a step of few sequences between its products: the norms ride on
+    these. ``add`` and ``start`` leave the residual rows times the next norm's weights
+    and their squares' sums; ``qkv`` and ``act`` take them."""
+
+    def __init__(self, residual: torch.Tensor, eps: float, offset: float):
+        assert _use_hip(residual)
+        m, k = residual.shape
+        self.residual, self.eps, self.offset, self.n = residual, eps, offset, 0
+        self.g = torch.empty(m, k, dtype=residual.dtype, device=residual.device)
+        self.sq = torch.empty(m * (k // 4 + 4), dtype=torch.float32, device=residual.device)
+
+    def start(self, norm: torch.Tensor) -> None:
+        self.norm = norm
+        self.n = _EXT.few_prep(self.residual, norm, self.offset, self.g, self.sq)
+
+    def add(self, x: torch.Tensor, w: torch.Tensor, norm: Optional[torch.Tensor]) -> None:
+        """residual += x @ w.T; norm: the next one's weights."""
+        self.norm = norm
+        self.n = _EXT.few_add(x, w, self.residual, norm, self.offset, self.g, self.sq)
+
+    def qkv(self, w, bias, k_cache, v_cache, positions, cos_sin, slot_mapping) -> torch.Tensor:
+        """few_rows_qkv of the normalised rows."""
+        if k_cache.shape[3] % 16 or k_cache.dtype not in (torch.bfloat16, torch.float8_e4m3fn):
+            h = rmsnorm(self.residual, self.norm, self.eps, self.offset)
+            return few_rows_qkv(h, w, bias, None, 0.0, 0.0, k_cache, v_cache, positions, cos_sin,
+                                slot_mapping)
+        return _EXT.few_qkv(self.g, self.sq, self.n, self.eps, w, bias, k_cache, v_cache,
+                            positions, cos_sin, slot_mapping)
+
+    def act(self, w: torch.Tensor, gelu: bool) -> torch.Tensor:
+        """few_rows_linear with act of the normalised rows."""
+        return _EXT.few_act(self.g, self.sq, self.n, self.eps, w, bool(gelu))
+
+
 # --------------------------------------------- projections, up to 256 rows --
 # The product stays as fp32 partial sums ("slabs" [parts, M, N]) that the next
 # kernel adds up: norm and residual, or rotation and cache write.

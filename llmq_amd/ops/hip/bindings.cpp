@@ -567,8 +567,6 @@ void skinny_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
                      slabs.data_ptr<float>(), bias_ptr, z, MN, N);
 }
 
-// --------------------------------------------------- projections, few rows --
-
 // Weights that the streaming kernels read: packed rows from a 16-byte boundary. Others
 // (a transposed or padded view, one inside a larger buffer) go to the library.
 bool streamable(const at::Tensor& w) {
@@ -579,148 +577,6 @@ bool streamable(const at::Tensor& w) {
 // view or starts elsewhere.
 at::Tensor packed(const at::Tensor& t) {
   return streamable(t) ? t : t.clone(at::MemoryFormat::Contiguous);
-}
-
-// out = f(x) W^T for up to 16 rows: see stream_gemm.hip. norm_w: x is RMS-normalised
-// first; epi: 0 plain, 1 added to out in place, 2 / 3 SiLU / tanh-GELU of the first
-// half of W's rows times the second half.
-void launch_stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
-                        c10::optional<at::Tensor> bias, c10::optional<at::Tensor> norm_w,
-                        double eps, double offset, long epi, const SgRope& rope = {}) {
-  CHECK_GPU(x);
-  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2, "x, w and out must be matrices");
-  const int M = x.size(0), K = x.size(1), N = w.size(0);
-  const bool pair = epi == kSgSilu || epi == kSgGelu;
-  const int cols = pair ? N / 2 : N;
-  auto bf16 = [](const at::Tensor& t) { return t.scalar_type() == at::kBFloat16; };
-  auto start16 = [](const at::Tensor& t) {
-    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
-  };
-  TORCH_CHECK(bf16(x) && bf16(w) && bf16(out), "x, w and out must be bfloat16");
-  TORCH_CHECK(M >= 1 && M <= 16, "1 to 16 rows");
-  TORCH_CHECK(w.size(1) == K && out.size(0) == M && out.size(1) == cols, "shapes differ");
-  TORCH_CHECK(K > 0 && K % 128 == 0 && N % 32 == 0, "K must be a multiple of 128, N of 32");
-  TORCH_CHECK(w.is_contiguous() && x.stride(1) == 1 && x.stride(0) % 8 == 0 &&
-                  out.stride(1) == 1 && start16(x) && start16(w),
-              "w must be contiguous, x's rows start on 16 bytes, rows packed");
-  const __hip_bfloat16 *bp = nullptr, *np = nullptr;
-  if (bias.has_value() && bias->defined()) {
-    TORCH_CHECK(bf16(*bias) && bias->numel() == N && !pair,
-                "bias must be bfloat16 [N], without an activation");
-    bias = packed(*bias);
-    bp = reinterpret_cast<const __hip_bfloat16*>(bias->data_ptr());
-  }
-  if (norm_w.has_value() && norm_w->defined()) {
-    TORCH_CHECK(bf16(*norm_w) && norm_w->numel() == K, "norm weights must be bfloat16 [K]");
-    norm_w = packed(*norm_w);
-    np = reinterpret_cast<const __hip_bfloat16*>(norm_w->data_ptr());
-  }
-  auto go = [&]<int KH, int NW, int KU, bool NORM, int EPI>() {
-    constexpr int R = 16 / KH;            // weight rows of a workgroup
-    const size_t lds = NORM ? sizeof(short) * (size_t)M * SgTokens<KH>::row(K) : 0;
-    hipLaunchKernelGGL((stream_gemm_kernel<KH, NW, KU, NORM, EPI>), dim3(N / R),
-                       dim3(64 * NW), lds, stream(),
-                       reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), out.stride(0),
-                       reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()), x.stride(0),
-                       reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()), bp, np,
-                       (float)eps, (float)offset, M, N, K, rope);
-  };
-  // Slices: as many as the tokens leave room for, up to four (2048 x 8192, one
-  // token: 13.0 us with one slice, 8.9 with four; eight gain nothing), because a
-  // small matrix then has more workgroups; a large one has enough of them anyway
-  // and saves the second reading of x (16384 x 3072, three tokens: 22.2 us with
-  // one slice and 16 waves, 23.3 with two, 23.8 with four).
-  const bool large = (long)N * K >= (48L << 20);
-  auto chunk = [&]<int KH, int NW, bool NORM, int EPI>() {
-    const int ks = K / KH;
-    if (ks % 128 == 0) go.template operator()<KH, NW, 4, NORM, EPI>();
-    else if (ks % 64 == 0) go.template operator()<KH, NW, 2, NORM, EPI>();
-    else go.template operator()<KH, NW, 1, NORM, EPI>();
-  };
-  auto slices = [&]<bool NORM, int EPI>() {
-    if (large) chunk.template operator()<1, 16, NORM, EPI>();
-    else if (M <= 4) chunk.template operator()<4, 8, NORM, EPI>();
-    else if (NORM || M <= 8) chunk.template operator()<2, 8, NORM, EPI>();  // norm: M <= 6
-    else if constexpr (!NORM) chunk.template operator()<1, 8, NORM, EPI>();
-  };
-  auto epilogue = [&]<bool NORM>() {
-    if (epi == kSgPlain) slices.template operator()<NORM, kSgPlain>();
-    else if (epi == kSgResidual) slices.template operator()<NORM, kSgResidual>();
-    else if (epi == kSgSilu) slices.template operator()<NORM, kSgSilu>();
-    else if (epi == kSgRope) slices.template operator()<NORM, kSgRope>();
-    else slices.template operator()<NORM, kSgGelu>();
-  };
-  if (!np) return epilogue.template operator()<false>();
-  // Every workgroup weights all tokens, M K elements in N / R workgroups: worth the
-  // launch that it saves up to 12 million of them, for up to six tokens. Measured (us, in
-  // the launch / a norm of its own): 16384 x 2048 pairs, 1 token (8.4 million)
-  // 18.0 / 18.6, 2 tokens 22.4 / 19.2; 16384 x 3072 pairs, 3 tokens (9.4) 28.1 / 28.9, 4
-  // 29.7 / 28.0; 5120 x 3072, 3 tokens (11.8) 12.2 / 12.6, 8 18.7 / 15.5; 2048 x 1536,
-  // 6 tokens (2.4) 6.5 / 6.4, 8 7.5 / 6.6; on the wrong side 17920 x 1536 pairs, 1 token
-  // (6.9), 16.9 / 16.1. They have to fit beside the sums (24 KB at the most).
-  const int R = large || M > 8 ? 16 : M > 4 ? 8 : 4;
-  if (M <= 6 && (long)(N / R) * M * K <= 12'000'000 && (long)M * (K + 512) * 2 <= (120 << 10))
-    return epilogue.template operator()<true>();
-  at::Tensor h = at::empty({M, K}, x.options());
-  rmsnorm(h, x.is_contiguous() ? x : x.contiguous(), *norm_w, eps, offset);
-  launch_stream_gemm(out, h, w, bias, c10::nullopt, 0, 0, epi, rope);
-}
-
-// The library's product of the rows, normalised first where weights are given.
-at::Tensor norm_linear(const at::Tensor& x, const at::Tensor& w,
-                       const c10::optional<at::Tensor>& bias,
-                       const c10::optional<at::Tensor>& norm_w, double eps, double offset) {
-  if (!norm_w.has_value() || !norm_w->defined()) return at::linear(x, w, bias);
-  at::Tensor h = at::empty({x.size(0), x.size(1)}, x.options());
-  rmsnorm(h, x.contiguous(), *norm_w, eps, offset);
-  return at::linear(h, w, bias);
-}
-
-void stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
-                 c10::optional<at::Tensor> bias, c10::optional<at::Tensor> norm_w,
-                 double eps, double offset, long epi) {
-  TORCH_CHECK(epi >= kSgPlain && epi <= kSgGelu, "unknown epilogue");
-  if (streamable(w)) return launch_stream_gemm(out, x, w, bias, norm_w, eps, offset, epi);
-  const at::Tensor y = norm_linear(x, w, bias, norm_w, eps, offset);
-  if (epi == kSgPlain) out.copy_(y);
-  else if (epi == kSgResidual) out.add_(y);
-  else if (epi == kSgSilu) silu_and_mul(out, y);
-  else gelu_tanh_and_mul(out, y);
-}
-
-// out = rmsnorm(x) W^T (+ bias) as q/k/v rows [M, (heads + 2 kv heads) D], q and k
-// rotated, k and v also written into the paged cache.
-void stream_qkv(at::Tensor out, at::Tensor x, at::Tensor w, c10::optional<at::Tensor> bias,
-                c10::optional<at::Tensor> norm_w, double eps, double offset, at::Tensor k_cache,
-                at::Tensor v_cache, at::Tensor positions, at::Tensor cos_sin, at::Tensor slots) {
-  CHECK_GPU(x);
-  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && k_cache.dim() == 4 && cos_sin.dim() == 2);
-  const int M = x.size(0), N = w.size(0), kv_heads = k_cache.size(1), D = k_cache.size(3);
-  const bool fp8 = k_cache.scalar_type() == at::kFloat8_e4m3fn;
-  TORCH_CHECK(D > 0 && D % 16 == 0 && N % D == 0 && N / D > 2 * kv_heads,
-              "w must have (heads + 2 kv heads) D rows, D a multiple of 16");
-  TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous() &&
-                  k_cache.sizes() == v_cache.sizes() &&
-                  k_cache.scalar_type() == v_cache.scalar_type() &&
-                  (fp8 || k_cache.scalar_type() == at::kBFloat16),
-              "caches must be contiguous, bfloat16 or e4m3");
-  TORCH_CHECK(positions.scalar_type() == at::kLong && positions.numel() == M &&
-                  slots.scalar_type() == at::kLong && slots.numel() == M &&
-                  positions.is_contiguous() && slots.is_contiguous() &&
-                  cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous() &&
-                  cos_sin.size(1) == D, "one int64 position and slot per row, fp32 cos_sin [*, D]");
-  if (!streamable(w)) {
-    out.copy_(norm_linear(x, w, bias, norm_w, eps, offset));
-    const at::Tensor heads = out.view({M, N / D, D});
-    const long q = N / D - 2 * kv_heads;
-    return rope_and_cache(heads.narrow(1, 0, q), heads.narrow(1, q, kv_heads),
-                          heads.narrow(1, q + kv_heads, kv_heads), k_cache, v_cache, positions,
-                          cos_sin, slots);
-  }
-  launch_stream_gemm(out, x, w, bias, norm_w, eps, offset, kSgRope,
-                     SgRope{k_cache.data_ptr(), v_cache.data_ptr(), positions.data_ptr<long>(),
-                            slots.data_ptr<long>(), cos_sin.data_ptr<float>(),
-                            N / D - 2 * kv_heads, kv_heads, D, (int)k_cache.size(2), fp8});
 }
 
 // ------------------------------------------- projections, up to 256 rows --
@@ -751,7 +607,7 @@ int ring_token_tiles(long M) {
 
 // ring_gemm.hip counts bytes from a workgroup's first row in 32 bits.
 bool ring_reaches(const at::Tensor& x, const at::Tensor& w) {
-  return w.numel() * 2 < (1L << 32) && x.size(0) * x.stride(0) * 2 < (1L << 32);
+  return w.numel() * 2 < (1L << 32) && (x.size(0) - 1) * x.stride(0) * 2 < (1L << 32) - (1 << 20);
 }
 
 // Weight rows of a workgroup (64 or 128) and parts of K: what takes least, a CU taking in
@@ -780,16 +636,22 @@ RingPlan ring_plan(long M, long N, long K, int cus) {
   return best;
 }
 
+size_t sums_bytes(long M, const SgScale& scale) {
+  return sizeof(float) * (size_t)M * sg_sums_stride(scale);
+}
+
 template <int TT, int RT, int WN, int WT, int WK, int ST, int EPI, bool ROT>
 void launch_ring(float* slabs, __hip_bfloat16* out, long out_stride, const at::Tensor& x,
-                 const at::Tensor& w, int parts, int steps) {
+                 const at::Tensor& w, int parts, int steps, const SgScale& scale = {}) {
   using Shape = RingShape<TT, RT, WN, WT, WK, ST>;
   const int M = x.size(0), K = x.size(1), N = w.size(0);
   hipLaunchKernelGGL((ring_gemm_kernel<TT, RT, WN, WT, WK, ST, EPI, ROT>),
-                     dim3(N / Shape::kRows * parts), dim3(64 * Shape::kWaves), Shape::kLds,
+                     dim3(N / Shape::kRows * parts), dim3(64 * Shape::kWaves),
+                     Shape::kLds + (scale.sq ? sums_bytes(M, scale) : 0),
                      stream(), slabs, out, out_stride,
                      reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()), x.stride(0),
-                     reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()), M, N, K, parts, steps);
+                     reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()), M, N, K, parts, steps,
+                     scale);
 }
 
 template <typename F>
@@ -810,13 +672,13 @@ void ring_tiles(long M, F&& go) {
 // on) the others, whose operand reads from LDS count (128 rows, 3584 x 14336: 25.7 and 26.3).
 template <int TT, int EPI>
 void launch_ring_128(float* slabs, __hip_bfloat16* out, long out_stride, const at::Tensor& x,
-                     const at::Tensor& w, int parts, int steps) {
+                     const at::Tensor& w, int parts, int steps, const SgScale& scale = {}) {
   if constexpr (TT <= 3)
-    launch_ring<TT, 2, 4, 1, 1, 4, EPI, false>(slabs, out, out_stride, x, w, parts, steps);
+    launch_ring<TT, 2, 4, 1, 1, 4, EPI, false>(slabs, out, out_stride, x, w, parts, steps, scale);
   else if constexpr (TT <= 8)
-    launch_ring<TT, 4, 2, 2, 1, 3, EPI, false>(slabs, out, out_stride, x, w, parts, steps);
+    launch_ring<TT, 4, 2, 2, 1, 3, EPI, false>(slabs, out, out_stride, x, w, parts, steps, scale);
   else
-    launch_ring<TT, 4, 2, 4, 1, 3, EPI, false>(slabs, out, out_stride, x, w, parts, steps);
+    launch_ring<TT, 4, 2, 4, 1, 3, EPI, false>(slabs, out, out_stride, x, w, parts, steps, scale);
 }
 
 // slab_gemm.hip: operands out of the ring kernels' reach.
@@ -877,21 +739,21 @@ at::Tensor ring_linear(const at::Tensor& x, const at::Tensor& w) {
 // 37888 x 3584 60 / 60 / 51.5; 128, 55296 x 5120 177 / 132 / 107; 128, 16384 x 3072 28.2 / 38 / -.
 template <int EPI>
 void launch_ring_act(__hip_bfloat16* out, long out_stride, const at::Tensor& x,
-                     const at::Tensor& w) {
+                     const at::Tensor& w, const SgScale& scale = {}) {
   const long N = w.size(0), cus = compute_units(x);
   const int steps = (int)(w.size(1) / kRingBK);
   const bool r128 = N / 64 > cus && N % 128 == 0;
   const bool r256 = N / 128 > cus && N % 256 == 0;
   ring_tiles(x.size(0), [&]<int TT>() {
     auto go = [&]<int RT, int WN, int WT, int WK, int ST, bool ROT>() {
-      launch_ring<TT, RT, WN, WT, WK, ST, EPI, ROT>(nullptr, out, out_stride, x, w, 1, steps);
+      launch_ring<TT, RT, WN, WT, WK, ST, EPI, ROT>(nullptr, out, out_stride, x, w, 1, steps, scale);
     };
     if (r256) {
       if constexpr (TT <= 3) go.template operator()<2, 8, 1, 1, 3, false>();
       else if constexpr (TT <= 8) go.template operator()<4, 4, 2, 1, 3, false>();
       else go.template operator()<4, 4, 2, 1, 2, false>();
     } else if (r128) {
-      launch_ring_128<TT, EPI>(nullptr, out, out_stride, x, w, 1, steps);
+      launch_ring_128<TT, EPI>(nullptr, out, out_stride, x, w, 1, steps, scale);
     } else {
       // eight waves where two groups, or four columns, have work for them (64 rows of 16384 x
       // 2048: one group 14.0, two 14.6; 96 rows 17.1 and 16.5; 45 rows 16.1 and 14.1)
@@ -944,6 +806,284 @@ at::Tensor slab_act_linear(const at::Tensor& x, const at::Tensor& w, bool gelu) 
               "slab_act_linear: 1 to 64 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
   return ring_act_linear(x, w, gelu);
 }
+
+// --------------------------------------------------- projections, few rows --
+
+// Weights that stream_gemm.hip takes: it counts bytes from a workgroup's first row in 32
+// bits.
+bool few_streams(const at::Tensor& w) { return streamable(w) && w.numel() * 2 < (1L << 32); }
+
+// Slices of K in stream_gemm.hip, 16 / slices weight rows a workgroup: two where that makes
+// workgroups for CUs without one and the tokens leave room. Measured (us, one / two slices):
+// 3 rows, 2048 x 2048 4.2 / 3.9, 3072 x 2048 4.6 / 4.6, 3072 x 8192 11.1 / 10.5, 5120 x 3072
+// 7.6 / 8.2; 7 rows, 1536 x 8960 10.7 / 8.1, 3072 x 3072 5.7 / 7.3. Four were never better.
+int stream_slices(long M, long N) {
+  return M <= 8 && N / 16 <= (M <= 4 ? 256 : 128) ? 2 : 1;
+}
+
+void launch_stream_prep(at::Tensor& g, at::Tensor& sq, const at::Tensor& x, const at::Tensor& w,
+                        double offset) {
+  hipLaunchKernelGGL(stream_prep_kernel, dim3(x.size(0)), dim3(256), 0, stream(),
+                     reinterpret_cast<__hip_bfloat16*>(g.data_ptr()), sq.data_ptr<float>(),
+                     reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()), x.stride(0),
+                     reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()), (float)offset,
+                     (int)x.size(1));
+}
+
+// The library's product of the rows, normalised first where weights are given.
+at::Tensor norm_linear(const at::Tensor& x, const at::Tensor& w,
+                       const c10::optional<at::Tensor>& bias,
+                       const c10::optional<at::Tensor>& norm_w, double eps, double offset) {
+  if (!norm_w.has_value() || !norm_w->defined()) return at::linear(x, w, bias);
+  at::Tensor h = at::empty({x.size(0), x.size(1)}, x.options());
+  rmsnorm(h, x.contiguous(), *norm_w, eps, offset);
+  return at::linear(h, w, bias);
+}
+
+// out = f(y) of a product y = x W^T.
+void finish_product(at::Tensor out, const at::Tensor& y, long epi) {
+  if (epi == kSgPlain) out.copy_(y);
+  else if (epi == kSgResidual) out.add_(y);
+  else if (epi == kSgSilu) silu_and_mul(out, y);
+  else gelu_tanh_and_mul(out, y);
+}
+
+// out = f(x) W^T for up to 16 rows: see stream_gemm.hip. norm_w: x is RMS-normalised
+// first; epi: 0 plain, 1 added to out in place, 2 / 3 SiLU / tanh-GELU of the first
+// half of W's rows times the second half. scale: x's rows await their factors; next:
+// what kSgResidual leaves for the next norm.
+void launch_stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
+                        c10::optional<at::Tensor> bias, c10::optional<at::Tensor> norm_w,
+                        double eps, double offset, long epi, const SgRope& rope = {},
+                        const SgScale& scale = {}, const SgNext& next = {}) {
+  CHECK_GPU(x);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2, "x, w and out must be matrices");
+  const int M = x.size(0), K = x.size(1), N = w.size(0);
+  const bool pair = epi == kSgSilu || epi == kSgGelu;
+  const int cols = pair ? N / 2 : N;
+  auto bf16 = [](const at::Tensor& t) { return t.scalar_type() == at::kBFloat16; };
+  auto start16 = [](const at::Tensor& t) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  TORCH_CHECK(bf16(x) && bf16(w) && bf16(out), "x, w and out must be bfloat16");
+  TORCH_CHECK(M >= 1 && M <= 16, "1 to 16 rows");
+  TORCH_CHECK(w.size(1) == K && out.size(0) == M && out.size(1) == cols, "shapes differ");
+  TORCH_CHECK(K > 0 && K % 128 == 0 && N % 32 == 0, "K must be a multiple of 128, N of 32");
+  TORCH_CHECK(w.is_contiguous() && x.stride(1) == 1 && x.stride(0) % 8 == 0 &&
+                  out.stride(1) == 1 && start16(x) && start16(w),
+              "w must be contiguous, x's rows start on 16 bytes, rows packed");
+  const __hip_bfloat16* bp = nullptr;
+  if (bias.has_value() && bias->defined()) {
+    TORCH_CHECK(bf16(*bias) && bias->numel() == N && !pair,
+                "bias must be bfloat16 [N], without an activation");
+    bias = packed(*bias);
+    bp = reinterpret_cast<const __hip_bfloat16*>(bias->data_ptr());
+  }
+  if (!ring_reaches(x, w))                               // rows far apart
+    return launch_stream_gemm(out, x.contiguous(), w, bias, norm_w, eps, offset, epi, rope, scale,
+                              next);
+  if (norm_w.has_value() && norm_w->defined()) {
+    TORCH_CHECK(bf16(*norm_w) && norm_w->numel() == K, "norm weights must be bfloat16 [K]");
+    norm_w = packed(*norm_w);
+    // Either way a launch before the product. Up to six rows of not too much work for the
+    // workgroups the rows' factors meet the sums (operands rounded before their scaling),
+    // else the rows are normalised: the roundings that each size has had.
+    const int R = (long)N * K >= (48L << 20) || M > 8 ? 16 : M > 4 ? 8 : 4;
+    at::Tensor h = at::empty({M, K}, x.options());
+    if (M <= 6 && (long)(N / R) * M * K <= 12'000'000 && (long)M * (K + 512) * 2 <= (120 << 10)) {
+      at::Tensor sq = at::empty({4L * M}, x.options().dtype(at::kFloat));
+      launch_stream_prep(h, sq, x, *norm_w, offset);
+      launch_stream_gemm(out, h, w, bias, c10::nullopt, 0, 0, epi, rope,
+                         SgScale{sq.data_ptr<float>(), 1, (float)eps});
+    } else {
+      rmsnorm(h, x.is_contiguous() ? x : x.contiguous(), *norm_w, eps, offset);
+      launch_stream_gemm(out, h, w, bias, c10::nullopt, 0, 0, epi, rope);
+    }
+    return;
+  }
+  if (pair && N % 64 == 0 && out.stride(0) % 4 == 0 &&
+      reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0) {
+    auto* p = reinterpret_cast<__hip_bfloat16*>(out.data_ptr());
+    if (epi == kSgSilu) launch_ring_act<kSlabSilu>(p, out.stride(0), x, w, scale);
+    else launch_ring_act<kSlabGelu>(p, out.stride(0), x, w, scale);
+    return;
+  }
+  auto go = [&]<int KH, int ST, int NX, bool SCALE, int EPI>() {
+    using Shape = StreamShape<KH, ST, NX>;
+    hipLaunchKernelGGL((stream_gemm_kernel<KH, ST, NX, SCALE, EPI>), dim3(N / Shape::kRows),
+                       dim3(stream_threads(EPI)), Shape::kLds + (SCALE ? sums_bytes(M, scale) : 0), stream(),
+                       reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
+                       out.stride(0), reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()),
+                       x.stride(0), reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()), bp,
+                       scale, next, M, N, K, rope);
+  };
+  // Rings of four stages while each workgroup has a CU to itself; two, and two or three
+  // workgroups a CU, where there are more (us, two / four stages: 3 rows, 5120 x 3072
+  // 7.6 / 9.1, 3072 x 8192 in slices 10.5 / 11.6, 2048 x 8192 in slices 8.7 / 7.4).
+  const bool sliced = stream_slices(M, N) == 2, many = N / (sliced ? 8 : 16) > 256;
+  auto shape = [&]<bool SCALE, int EPI>() {
+    constexpr int FOUR = SCALE ? 3 : 4;                  // beside the rows' sums in LDS
+    if (M > 8) go.template operator()<1, FOUR, 2, SCALE, EPI>();
+    else if (!sliced && many) go.template operator()<1, 2, 1, SCALE, EPI>();
+    else if (!sliced) go.template operator()<1, 4, 1, SCALE, EPI>();
+    else if (M > 4) go.template operator()<2, FOUR, 2, SCALE, EPI>();
+    else if (many) go.template operator()<2, 2, 1, SCALE, EPI>();
+    else go.template operator()<2, 4, 1, SCALE, EPI>();
+  };
+  auto epilogue = [&]<bool SCALE>() {
+    if (epi == kSgPlain) shape.template operator()<SCALE, kSgPlain>();
+    else if (epi == kSgResidual) shape.template operator()<SCALE, kSgResidual>();
+    else if (epi == kSgSilu) shape.template operator()<SCALE, kSgSilu>();
+    else if (epi == kSgRope) shape.template operator()<SCALE, kSgRope>();
+    else shape.template operator()<SCALE, kSgGelu>();
+  };
+  if (scale.sq) epilogue.template operator()<true>();
+  else epilogue.template operator()<false>();
+}
+
+void stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
+                 c10::optional<at::Tensor> bias, c10::optional<at::Tensor> norm_w,
+                 double eps, double offset, long epi) {
+  TORCH_CHECK(epi >= kSgPlain && epi <= kSgGelu, "unknown epilogue");
+  if (few_streams(w)) return launch_stream_gemm(out, x, w, bias, norm_w, eps, offset, epi);
+  finish_product(out, norm_linear(x, w, bias, norm_w, eps, offset), epi);
+}
+
+// out = rmsnorm(x) W^T (+ bias) as q/k/v rows [M, (heads + 2 kv heads) D], q and k
+// rotated, k and v also written into the paged cache. scale: in the norm's place.
+void launch_stream_qkv(at::Tensor out, at::Tensor x, at::Tensor w, c10::optional<at::Tensor> bias,
+                       c10::optional<at::Tensor> norm_w, double eps, double offset,
+                       at::Tensor k_cache, at::Tensor v_cache, at::Tensor positions,
+                       at::Tensor cos_sin, at::Tensor slots, const SgScale& scale = {}) {
+  CHECK_GPU(x);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && k_cache.dim() == 4 && cos_sin.dim() == 2);
+  const int M = x.size(0), N = w.size(0), kv_heads = k_cache.size(1), D = k_cache.size(3);
+  const bool fp8 = k_cache.scalar_type() == at::kFloat8_e4m3fn;
+  TORCH_CHECK(D > 0 && D % 16 == 0 && N % D == 0 && N / D > 2 * kv_heads,
+              "w must have (heads + 2 kv heads) D rows, D a multiple of 16");
+  TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous() &&
+                  k_cache.sizes() == v_cache.sizes() &&
+                  k_cache.scalar_type() == v_cache.scalar_type() &&
+                  (fp8 || k_cache.scalar_type() == at::kBFloat16),
+              "caches must be contiguous, bfloat16 or e4m3");
+  TORCH_CHECK(positions.scalar_type() == at::kLong && positions.numel() == M &&
+                  slots.scalar_type() == at::kLong && slots.numel() == M &&
+                  positions.is_contiguous() && slots.is_contiguous() &&
+                  cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous() &&
+                  cos_sin.size(1) == D, "one int64 position and slot per row, fp32 cos_sin [*, D]");
+  if (!few_streams(w)) {
+    out.copy_(norm_linear(x, w, bias, norm_w, eps, offset));
+    const at::Tensor heads = out.view({M, N / D, D});
+    const long q = N / D - 2 * kv_heads;
+    return rope_and_cache(heads.narrow(1, 0, q), heads.narrow(1, q, kv_heads),
+                          heads.narrow(1, q + kv_heads, kv_heads), k_cache, v_cache, positions,
+                          cos_sin, slots);
+  }
+  launch_stream_gemm(out, x, w, bias, norm_w, eps, offset, kSgRope,
+                     SgRope{k_cache.data_ptr(), v_cache.data_ptr(), positions.data_ptr<long>(),
+                            slots.data_ptr<long>(), cos_sin.data_ptr<float>(),
+                            N / D - 2 * kv_heads, kv_heads, D, (int)k_cache.size(2), fp8},
+                     scale);
+}
+
+void stream_qkv(at::Tensor out, at::Tensor x, at::Tensor w, c10::optional<at::Tensor> bias,
+                c10::optional<at::Tensor> norm_w, double eps, double offset, at::Tensor k_cache,
+                at::Tensor v_cache, at::Tensor positions, at::Tensor cos_sin, at::Tensor slots) {
+  launch_stream_qkv(out, x, w, bias, norm_w, eps, offset, k_cache, v_cache, positions, cos_sin,
+                    slots);
+}
+
+// The steps of a layer of few rows whose norms ride on its products. Between them go
+// g [M, K], the residual rows times the next norm's weights, and sq, n sums of squares a
+// row (rounded up to 4): few_prep and few_add leave them and return n, few_qkv and few_act
+// take them.
+
+void check_scaled(const at::Tensor& g, const at::Tensor& sq, long n) {
+  CHECK_GPU(g);
+  TORCH_CHECK(g.dim() == 2 && g.scalar_type() == at::kBFloat16 && g.is_contiguous() &&
+                  streamable(g) && g.size(1) % 8 == 0 && g.size(0) >= 1 && g.size(0) <= 16,
+              "g must be 1 to 16 packed bf16 rows from a 16-byte boundary");
+  TORCH_CHECK(sq.scalar_type() == at::kFloat && sq.is_contiguous() && n >= 1 &&
+                  sq.numel() >= g.size(0) * ((n + 3) / 4 * 4) && streamable(sq),
+              "sq must hold n fp32 sums a row, rounded up to 4");
+}
+
+at::Tensor scaled_rows(const at::Tensor& g, const at::Tensor& sq, long n, double eps) {
+  const long M = g.size(0);
+  const long ns = (n + 3) / 4 * 4;
+  const at::Tensor ms =
+      sq.flatten().narrow(0, 0, M * ns).view({M, ns}).narrow(1, 0, n).sum(1, true) / g.size(1);
+  return (g.to(at::kFloat) * at::rsqrt(ms + eps)).to(at::kBFloat16);
+}
+
+long few_prep(const at::Tensor& x, const at::Tensor& w, double offset, at::Tensor g,
+              at::Tensor sq) {
+  check_scaled(g, sq, 1);
+  TORCH_CHECK(x.sizes() == g.sizes() && x.scalar_type() == at::kBFloat16 && x.stride(1) == 1 &&
+                  rows_start_on(x, 16) && w.scalar_type() == at::kBFloat16 &&
+                  w.numel() == x.size(1), "x must be bf16 rows on 16 bytes, w bf16 [K]");
+  launch_stream_prep(g, sq, x, packed(w), offset);
+  return 1;
+}
+
+// residual += x W^T, and with next_w what the next norm by next_w + offset needs.
+long few_add(const at::Tensor& x, const at::Tensor& w, at::Tensor residual,
+             c10::optional<at::Tensor> next_w, double offset, at::Tensor g, at::Tensor sq) {
+  const bool more = next_w.has_value() && next_w->defined();
+  if (!few_streams(w)) {
+    residual.add_(at::linear(x, w));
+    return more ? few_prep(residual, *next_w, offset, g, sq) : 0;
+  }
+  SgNext next{};
+  long n = 0;
+  at::Tensor wn;
+  if (more) {
+    TORCH_CHECK(residual.is_contiguous() && g.sizes() == residual.sizes() &&
+                    next_w->scalar_type() == at::kBFloat16 && next_w->numel() == w.size(0),
+                "residual must be packed, next_w bf16 [N]");
+    n = w.size(0) / (16 / stream_slices(x.size(0), w.size(0)));
+    check_scaled(g, sq, n);
+    wn = packed(*next_w);
+    next = SgNext{reinterpret_cast<__hip_bfloat16*>(g.data_ptr()), sq.data_ptr<float>(),
+                  reinterpret_cast<const __hip_bfloat16*>(wn.data_ptr()), (float)offset};
+  }
+  launch_stream_gemm(residual, x, w, c10::nullopt, c10::nullopt, 0, 0, kSgResidual, SgRope{},
+                     SgScale{}, next);
+  return n;
+}
+
+// Whether a product scales the rows itself: their sums beside its other LDS.
+bool scales(const at::Tensor& w, const at::Tensor& g, long n) {
+  return few_streams(w) && sums_bytes(g.size(0), SgScale{nullptr, (int)n, 0}) <= (48 << 10);
+}
+
+at::Tensor few_qkv(const at::Tensor& g, const at::Tensor& sq, long n, double eps,
+                   const at::Tensor& w, c10::optional<at::Tensor> bias, at::Tensor k_cache,
+                   at::Tensor v_cache, at::Tensor positions, at::Tensor cos_sin,
+                   at::Tensor slots) {
+  check_scaled(g, sq, n);
+  at::Tensor out = at::empty({g.size(0), w.size(0)}, g.options());
+  const bool ok = scales(w, g, n);
+  launch_stream_qkv(out, ok ? g : scaled_rows(g, sq, n, eps), w, bias, c10::nullopt, 0, 0, k_cache,
+                    v_cache, positions, cos_sin, slots,
+                    ok ? SgScale{sq.data_ptr<float>(), (int)n, (float)eps} : SgScale{});
+  return out;
+}
+
+at::Tensor few_act(const at::Tensor& g, const at::Tensor& sq, long n, double eps,
+                   const at::Tensor& w, bool gelu) {
+  check_scaled(g, sq, n);
+  at::Tensor out = at::empty({g.size(0), w.size(0) / 2}, g.options());
+  if (!scales(w, g, n))
+    stream_gemm(out, scaled_rows(g, sq, n, eps), w, c10::nullopt, c10::nullopt, 0, 0,
+                gelu ? kSgGelu : kSgSilu);
+  else
+    launch_stream_gemm(out, g, w, c10::nullopt, c10::nullopt, 0, 0, gelu ? kSgGelu : kSgSilu,
+                       SgRope{}, SgScale{sq.data_ptr<float>(), (int)n, (float)eps});
+  return out;
+}
+
+// ------------------------------------- readers of the ring products' slabs --
 
 void check_slabs(const at::Tensor& slabs) {
   CHECK_GPU(slabs);
@@ -1207,6 +1347,10 @@ TORCH_LIBRARY(llmq_amd, m) {
   m.def("varlen_prefill_attention(Tensor(a!) out, Tensor q, Tensor k, Tensor v, Tensor cu_seqlens, Tensor cu_seqlens_k, int max_seqlen, float scale, float softcap, int window) -> ()");
   m.def("paged_prefill_attention(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor cu_seqlens, Tensor cu_seqlens_k, int max_seqlen, float scale, float softcap, int window) -> ()");
   m.def("stream_qkv(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, Tensor? norm_w, float eps, float offset, Tensor(b!) k_cache, Tensor(c!) v_cache, Tensor positions, Tensor cos_sin, Tensor slots) -> ()");
+  m.def("few_prep(Tensor x, Tensor w, float offset, Tensor(a!) g, Tensor(b!) sq) -> int");
+  m.def("few_add(Tensor x, Tensor w, Tensor(a!) residual, Tensor? next_w, float offset, Tensor(b!) g, Tensor(c!) sq) -> int");
+  m.def("few_qkv(Tensor g, Tensor sq, int n, float eps, Tensor w, Tensor? bias, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor positions, Tensor cos_sin, Tensor slots) -> Tensor");
+  m.def("few_act(Tensor g, Tensor sq, int n, float eps, Tensor w, bool gelu) -> Tensor");
   m.def("slab_linear(Tensor x, Tensor w) -> Tensor");
   m.def("ring_linear(Tensor x, Tensor w) -> Tensor");
   m.def("ring_act_linear(Tensor x, Tensor w, bool gelu) -> Tensor");
@@ -1233,6 +1377,10 @@ TORCH_LIBRARY_IMPL(llmq_amd, CUDA, m) {
   m.impl("paged_decode_attention", &paged_decode_attention);
   m.impl("varlen_prefill_attention", &varlen_prefill_attention);
   m.impl("paged_prefill_attention", &paged_prefill_attention);
+  m.impl("few_prep", &few_prep);
+  m.impl("few_add", &few_add);
+  m.impl("few_qkv", &few_qkv);
+  m.impl("few_act", &few_act);
   m.impl("slab_linear", &slab_linear);
   m.impl("ring_linear", &ring_linear);
   m.impl("ring_act_linear", &ring_act_linear);

@@ -31,34 +31,12 @@
 // 6.0 TB/s); 128 rows, 3072 x 8192 23.8 -> 16.8; 189 rows, 3072 x 8192 58 -> 20.1, 3072 x 3072
 // 26.5 -> 12.5; 256 rows, 3584 x 14336 59.4 -> 36.5.
 
-#include "common.h"
+#include "common.h"   // and ring_load, SgScale of stream_gemm.hip
 
 typedef __attribute__((ext_vector_type(8))) short rg_s16x8;
 typedef __attribute__((ext_vector_type(4))) float rg_f32x4;
 
 constexpr int kRingBK = 64;
-
-// 16 bytes per lane from base + off to LDS, lane-linear from lds_off (uniform).
-template <bool NT>
-DEVINL void ring_load(const void* base, unsigned off, unsigned lds_off) {
-  unsigned keep;
-  if constexpr (NT)
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %3\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, %2 nt\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_off) : "memory");
-  else
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %3\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, %2\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_off) : "memory");
-}
 
 // The wave's loads have landed but those of the last min(left, N) stages, NL each;
 // everyone's LDS reads are done.
@@ -81,7 +59,8 @@ template <int TT, int RT, int WN, int WT, int WK, int ST, int EPI, bool ROT>
 __global__ __launch_bounds__(64 * WN * WT * WK) void ring_gemm_kernel(
     float* __restrict__ slabs, __hip_bfloat16* __restrict__ out, long out_stride,
     const __hip_bfloat16* __restrict__ x, long x_stride,
-    const __hip_bfloat16* __restrict__ wt, int M, int N, int K, int parts, int steps) {
+    const __hip_bfloat16* __restrict__ wt, int M, int N, int K, int parts, int steps,
+    SgScale scale) {
   constexpr bool PAIR = EPI != kSlabSums;
   static_assert(PAIR || WK == 1, "groups' sums meet in LDS for gate and value rows only");
   static_assert(!PAIR || RT % 2 == 0, "a wave holds gates and their values");
@@ -145,12 +124,28 @@ __global__ __launch_bounds__(64 * WN * WT * WK) void ring_gemm_kernel(
   for (int a = 0; a < RT; ++a)
 #pragma unroll
     for (int m = 0; m < TW; ++m) acc[a][m] = rg_f32x4{0.f, 0.f, 0.f, 0.f};
+  // the sums behind the factors of rows that stream_gemm.hip left unscaled, ahead of all
+  constexpr bool SCALE = PAIR && TT == 1;
+  constexpr int WAVES = WN * WT * WK;
+  float* const sums = reinterpret_cast<float*>(ring_lds + WK * ST * STAGE);
+  if (SCALE && scale.sq)
+    for (int m = wave; m < M; m += WAVES)
+      sg_fetch_sums(scale, m, lane, sums + m * sg_sums_stride(scale));
 #pragma unroll
   for (int i = 0; i < ST - 1; ++i)
     if (i < loops) stage(i);
+  __shared__ float invs[SCALE ? 16 : 1];
+  auto factors = [&]() {
+    for (int m = wave; m < M; m += WAVES) {
+      const float inv = sg_inv(scale, lane, K, sums + m * sg_sums_stride(scale));
+      if (lane == 0) invs[m] = inv;
+    }
+  };
   for (int i = 0; i < loops; ++i) {
     ring_wait<ST - 2, NL>(loops - 1 - i);                // stage i is here, i - 1 is read
     if (i + ST - 1 < loops) stage(i + ST - 1);
+    if constexpr (SCALE)
+      if (i == 1 && scale.sq && loops >= 3) factors();   // while the weights travel
     if (WK > 1 && step_of(i) >= total) continue;
     const short* at = ring + (i % ST) * STAGE;
     const short* wa = at + (wn * RT * 16 + col) * BK;
@@ -170,6 +165,11 @@ __global__ __launch_bounds__(64 * WN * WT * WK) void ring_gemm_kernel(
       }
     }
   }
+  if constexpr (SCALE)
+    if (scale.sq && loops < 3) {
+      factors();
+      __syncthreads();
+    }
   if constexpr (WK > 1) {                                // the groups' sums
     constexpr int NA = RT * TW;
     static_assert((size_t)(WK - 1) * G * NA * 1024 <= RingShape<TT, RT, WN, WT, WK, ST>::kLds);
@@ -190,6 +190,7 @@ __global__ __launch_bounds__(64 * WN * WT * WK) void ring_gemm_kernel(
   for (int m = 0; m < TW; ++m) {
     const int row = (wc * TW + m) * 16 + col;
     if (row >= M) continue;
+    const float inv = SCALE && scale.sq ? invs[row] : 1.f;
     if constexpr (!PAIR) {
       float* slab = slabs + ((long)part * M + row) * N + n0 + wn * RT * 16 + grp * 4;
 #pragma unroll
@@ -200,11 +201,11 @@ __global__ __launch_bounds__(64 * WN * WT * WK) void ring_gemm_kernel(
         Vec4<__hip_bfloat16> v;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float g = acc[a][m][r];
+          const float g = acc[a][m][r] * inv;
           const float y = EPI == kSlabSilu
               ? g / (1.0f + __expf(-g))
               : 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
-          v.data[r] = __float2bfloat16(y * acc[a + RT / 2][m][r]);
+          v.data[r] = __float2bfloat16(y * (acc[a + RT / 2][m][r] * inv));
         }
         *reinterpret_cast<int2*>(out + (long)row * out_stride + n0 + (wn * (RT / 2) + a) * 16 +
                                  grp * 4) = *reinterpret_cast<const int2*>(v.data);

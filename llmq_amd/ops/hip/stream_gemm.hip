@@ -2,40 +2,61 @@
 // sums: the products of a decode step of few sequences (gfx950).
 //
 // Bound by the weights' bytes, each needed once, and below about 30 MB by the fixed
-// costs of a launch; so one launch does what surrounds the product too, and even a
-// matrix of a few MB is in flight on the whole chip at once.
+// costs of a launch; so one launch does what surrounds the product too.
 //
-//   - Operands go straight from memory into the layout of
-//     v_mfma_f32_16x16x32_bf16 (A = weights: row = lane%16, k = 8*(lane/16)..+7;
-//     B = tokens: column = lane%16; C: column = lane%16, rows 4*(lane/16)+r).
-//   - With M tokens only 16/KH >= M of the 16 columns are needed, so K is cut in KH
-//     slices that take the rest: A's rows are 16/KH weight rows times KH slices, B's
-//     columns 16/KH tokens times KH slices, and the result is the sum of the
-//     blocks on C's diagonal. That sets a workgroup's share to 16, 8 or 4 weight
-//     rows (KH = 1, 2, 4) without a masked lane.
-//   - The workgroup's waves share out the slices in chunks and add up through LDS. A
-//     wave with several chunks asks for the next one's weights ahead of a chunk's
-//     products, under a condition, so that the wait before those covers them too.
-//   - NORM: the tokens are RMS-normalised on the way in: x times the norm's weights
-//     (rounded, as a normalised row is) goes to LDS once per workgroup, while the
-//     first weights travel, its squares are summed beside, and the row's factor
-//     meets the fp32 sums at the end. (Weighting each operand where it is used cost
-//     16384 x 2048 pairs with one token 25.3 instead of 17.3 us: more vector work than the
-//     weights' bytes leave time for.)
-//   - RES: the sums are added to the residual in place. ACT: half of the weight
-//     rows are gates, half the values that they act on (x = [gate | up]).
+//   - v_mfma_f32_16x16x32_bf16 (A = weights: row = lane%16, k = 8*(lane/16)..+7;
+//     B = tokens: column = lane%16; C: column = lane%16, rows 4*(lane/16)+r). With up to
+//     eight tokens only 8 of the 16 columns are needed, so K may be cut in KH = 2 slices
+//     that take the rest: A's rows are 8 weight rows times 2 slices, B's columns 8 tokens
+//     times 2 slices, and the result is the sum of the blocks on C's diagonal. A
+//     workgroup then owns 8 weight rows instead of 16 without a masked lane.
+//   - The workgroup's eight waves take steps of 64 channels in turn and add up through LDS.
+//     Each has a ring of ST stages in LDS of its own, filled by global_load_lds (a load: 8
+//     rows of 128 bytes, 16-byte granules placed by row against bank conflicts): loads are
+//     counted by hand and there is no barrier before the sums. (Operands straight to
+//     registers: segments of 64 bytes, and tokens as many loads as weights. us, before ->
+//     now: 1 row, 2048 x 8192 9.0 -> 7.3; 3 rows, 3072 x 8192 14.2 -> 10.5, 5120 x 3072 9.8 ->
+//     7.6; 7 rows, 1536 x 8960 11.3 -> 8.1, 3584 x 14336 30.4 -> 18.9; 13 rows, 2048 x 2048 6.2
+//     -> 4.7.)
+//   - RMS norms ride on both sides of a product. Who adds to the residual (kSgResidual)
+//     also leaves the row times the next norm's weights (rounded, as a normalised row
+//     is) and its squares' sum over the workgroup's columns; who reads those rows (SCALE)
+//     adds up the squares, which came to LDS ahead of the first weights, and the row's
+//     factor meets the fp32 sums at the end. (Before, every workgroup of the reader weighted
+//     all tokens by itself, up to six, and more took a launch of 4 us.)
+//   - ACT: half of the weight rows are gates, half the values that they act on (x = [gate |
+//     up]): pairs of widths that ring_gemm.hip does not take.
 //   - ROPE (the q/k/v projection): a workgroup takes channel pairs of one head, rotates
 //     q and k and writes k and v into the paged cache too; positions and
-//     angles are read while the weights travel. A launch of its own for that took 4.5 us
+//     angles are read by the ninth wave while the weights travel. A launch of its own for that took 4.5 us
 //     a layer (a step of llama-3.2-1b, one sequence: 902 us, 873 without it).
 
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(8))) short sg_s16x8;
-typedef __attribute__((ext_vector_type(4))) unsigned sg_u32x4;
 typedef __attribute__((ext_vector_type(4))) float sg_f32x4;
-typedef __attribute__((ext_vector_type(2))) float sg_f32x2;
-typedef __attribute__((ext_vector_type(2))) __bf16 sg_bf16x2;
+
+// 16 bytes per lane from base + off to LDS, lane-linear from lds_off (uniform).
+template <bool NT>
+DEVINL void ring_load(const void* base, unsigned off, unsigned lds_off) {
+  unsigned keep;
+  if constexpr (NT)
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %3\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %2 nt\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_off) : "memory");
+  else
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %3\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %2\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_off) : "memory");
+}
 
 enum : int { kSgPlain = 0, kSgResidual = 1, kSgSilu = 2, kSgGelu = 3, kSgRope = 4 };
 
@@ -49,29 +70,77 @@ struct SgRope {
   bool fp8;
 };
 
-// Places of weighted tokens in LDS (shorts): the 16 columns of an operand read lie in
-// 16 different 16-byte bank groups where slices are multiples of 128.
-template <int KH>
-struct SgTokens {
-  static constexpr int kPlaces = 16 / KH;
-  __host__ __device__ static int slice(int K) { return K / KH + 8 * kPlaces; }
-  __host__ __device__ static int row(int K) { return (KH * slice(K) + 127) / 128 * 128 + 8; }
+// The wave's loads have landed but those of the last min(left, N) stages, NL each, and its
+// LDS reads are done.
+template <int N, int NL>
+DEVINL void stream_wait(int left) {
+  if constexpr (N == 0) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  else if (left >= N) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "i"(N * NL) : "memory");
+  else stream_wait<N - 1, NL>(left);
+}
+
+// What SCALE needs: n sums of squares a row, sq[row][n rounded up to 4], of the rows that
+// x holds before their scaling, each over a share of the columns.
+struct SgScale {
+  const float* sq;
+  int n;
+  float eps;
+  __host__ __device__ int stride() const { return (n + 3) & ~3; }
 };
 
-// KH: slices of K (16 / KH >= M); NW: waves; KU: 32-wide K steps of a chunk.
-template <int KH, int NW, int KU, bool NORM, int EPI>
-__global__ __launch_bounds__(64 * NW) void stream_gemm_kernel(
+// What kSgResidual leaves for the next norm: g = rows times (w + offset), and squares' sums
+// sq[row][workgroups rounded up to 4]. g null: nothing.
+struct SgNext {
+  __hip_bfloat16* g;
+  float* sq;
+  const __hip_bfloat16* w;
+  float offset;
+};
+
+// A row's factor 1 / rms: a wave sends its sums to LDS ahead of all its other loads, ...
+DEVINL void sg_fetch_sums(const SgScale& scale, int row, int lane, float* to) {
+  const float* from = scale.sq + (long)row * scale.stride();
+  for (int i = 0; i < scale.n; i += 4 * WAVE)
+    glds16(from + min(i + lane * 4, scale.stride() - 4), to + i);
+}
+// ... and has the factor of them once they have landed.
+DEVINL float sg_inv(const SgScale& scale, int lane, int K, const float* sums) {
+  float s = 0.f;
+  for (int i = lane; i < scale.n; i += WAVE) s += sums[i];
+  return rsqrtf(wave_reduce_sum(s) / K + scale.eps);
+}
+// LDS of M rows of sums, each in whole loads of a wave.
+__host__ __device__ inline int sg_sums_stride(const SgScale& scale) {
+  return (scale.n + 4 * WAVE - 1) / (4 * WAVE) * (4 * WAVE);
+}
+
+// KH: slices of K (16 / KH >= M); ST: stages of a wave's ring; NX: loads of a stage's tokens,
+// 8 NX / KH >= M token places a slice.
+template <int KH, int ST, int NX>
+struct StreamShape {
+  static constexpr int kRows = 16 / KH;
+  static constexpr size_t kLds = (size_t)8 * ST * (2 + NX) * 1024;
+};
+
+// Eight waves, and for kSgRope one more that reads angles and cache slots: their loads depend
+// on each other, and in the others' order that would be a wait for the weights first.
+constexpr int stream_threads(int epi) { return epi == kSgRope ? 576 : 512; }
+
+template <int KH, int ST, int NX, bool SCALE, int EPI>
+__global__ __launch_bounds__(stream_threads(EPI)) void stream_gemm_kernel(
     __hip_bfloat16* __restrict__ out, long out_stride,
     const __hip_bfloat16* __restrict__ x, long x_stride,
     const __hip_bfloat16* __restrict__ wt, const __hip_bfloat16* __restrict__ bias,
-    const __hip_bfloat16* __restrict__ norm_w, float eps, float offset,
-    int M, int N, int K, SgRope rope) {
-  constexpr int R = 16 / KH, MP = 16 / KH, KC = 32 * KU;   // weight rows, token places
+    SgScale scale, SgNext next, int M, int N, int K, SgRope rope) {
+  constexpr int NW = 8, R = 16 / KH, MP = 16 / KH;         // weight rows, token columns
+  constexpr int XP = 8 * NX / KH, NL = 2 + NX;             // token places, loads of a stage
   constexpr bool PAIR = EPI >= kSgSilu;
   constexpr int RO = PAIR ? R / 2 : R;                     // output columns (kSgRope: pairs)
   constexpr int RP = 17;
+  static_assert(XP <= MP && (ST - 2) * NL < 64);
+  extern __shared__ __align__(16) short sg_lds[];          // [wave][ST][16 weight | 8 NX token rows][64]
   __shared__ float red[NW][16 * RP];
-  __shared__ float sums[NW][16];
+  __shared__ float invs[16];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
@@ -81,79 +150,115 @@ __global__ __launch_bounds__(64 * NW) void stream_gemm_kernel(
   const int head = EPI == kSgRope ? blockIdx.x * RO / half : 0;
   const int n0 = blockIdx.x * RO + head * half;
   const int apart = EPI == kSgRope ? half : N / 2;
-  const int i = col % R;
-  const int wrow = PAIR && i >= RO ? apart + n0 + i - RO : n0 + i;
-  const long kslice = (long)(col / R) * ks + grp * 8;
-  const __hip_bfloat16* wp = wt + (long)wrow * K + kslice;
-  const __hip_bfloat16* xp = x + (long)min(col % MP, M - 1) * x_stride + kslice;
-  extern __shared__ __align__(16) short tokens[];
-  const short* tp = tokens + min(col % MP, M - 1) * SgTokens<KH>::row(K) +
-                    (col / R) * SgTokens<KH>::slice(K) + grp * 8;
-  sg_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 
-  sg_s16x8 wf[KU], wn[KU];
-  auto fetch = [&](sg_s16x8 (&f)[KU], int k0) {
-#pragma unroll
-    for (int u = 0; u < KU; ++u)
-      f[u] = __builtin_nontemporal_load(reinterpret_cast<const sg_s16x8*>(wp + k0 + u * 32));
+  // kSgRope, by the ninth wave: cosines, sines, rows of the cache (negative: none)
+  __shared__ float turned[2][EPI == kSgRope ? RO * MP : 1];
+  __shared__ long cached[EPI == kSgRope ? MP : 1];
+  float* const sums = reinterpret_cast<float*>(sg_lds + StreamShape<KH, ST, NX>::kLds / 2);
+  if (SCALE && w < NW)
+    for (int m = w; m < M; m += NW)
+      sg_fetch_sums(scale, m, lane, sums + m * sg_sums_stride(scale));
+  auto factors = [&]() {
+    for (int m = w; m < M; m += NW) {
+      const float inv = sg_inv(scale, lane, K, sums + m * sg_sums_stride(scale));
+      if (lane == 0) invs[m] = inv;
+    }
   };
-  int k0 = w * KC;
-  long slot = -1, position = 0;
-  float cosine = 1.f, sine = 0.f;
-  if constexpr (EPI == kSgRope) {      // one sum per thread: 4 RO MP <= 64 NW
-    const int m = min(((int)threadIdx.x >> 2) / RO, M - 1);
-    position = rope.positions[m];
-    slot = rope.slots[m];
-  }
-  if (k0 < ks) fetch(wf, k0);
-  if constexpr (EPI == kSgRope) {
-    if (head < rope.heads + rope.kv_heads) {
-      const float* cs = rope.cos_sin + position * rope.D + (n0 - head * rope.D) +
-                        (threadIdx.x >> 2) % RO;
-      cosine = cs[0];
-      sine = cs[half];
-    }
-  }
-  if constexpr (NORM) {
-    for (int m = 0; m < M; ++m) {
-      float ss = 0.f;
-      for (int k = threadIdx.x * 8; k < K; k += 64 * NW * 8) {
-        const Vec8<__hip_bfloat16> xv = load16(x + (long)m * x_stride + k);
-        const Vec8<__hip_bfloat16> nv = load16(norm_w + k);
-        sg_u32x4 y;
+
+  // Staging: rows 8 j + lane/8 of the operand, a slice's rows together; tokens past the
+  // last repeat it.
+  auto place = [&](int row) { return ((lane & 7) ^ ((row >> 1) & 7)) << 3; };
+  unsigned woff[2], xoff[NX];
 #pragma unroll
-        for (int e = 0; e < 8; e += 2) {
-          const float a = to_f32(xv.data[e]), b = to_f32(xv.data[e + 1]);
-          ss += a * a + b * b;
-          y[e / 2] = __builtin_bit_cast(unsigned, __builtin_convertvector(
-              (sg_f32x2{a * (to_f32(nv.data[e]) + offset), b * (to_f32(nv.data[e + 1]) + offset)}),
-              sg_bf16x2));
-        }
-        *reinterpret_cast<sg_u32x4*>(tokens + m * SgTokens<KH>::row(K) +
-                                     (k / ks) * SgTokens<KH>::slice(K) + k % ks) = y;
+  for (int j = 0; j < 2; ++j) {
+    const int r = j * 8 + (lane >> 3), i = r % R;
+    const int row = PAIR && i >= RO ? apart + i - RO : i;  // from n0
+    woff[j] = ((unsigned)row * (unsigned)K + r / R * ks + place(r)) * 2u;
+  }
+#pragma unroll
+  for (int j = 0; j < NX; ++j) {
+    const int r = j * 8 + (lane >> 3);
+    xoff[j] = ((unsigned)min(r % XP, M - 1) * (unsigned)x_stride + r / XP * ks + place(r)) * 2u;
+  }
+  const int steps = ks / 64;                               // this wave's: w, w + NW, ..
+  const int mine = w < NW && steps > w ? (steps - 1 - w) / NW + 1 : 0;
+  const __hip_bfloat16* wb = wt + (long)n0 * K + w * 64;
+  const __hip_bfloat16* xb = x + w * 64;
+  short* const ring = sg_lds + w * (ST * NL * 512);
+  const unsigned ring_off = (unsigned)(unsigned long)(
+      (__attribute__((address_space(3))) char*)ring);
+  auto stage = [&](int i) {
+    const unsigned to = __builtin_amdgcn_readfirstlane(ring_off + (unsigned)(i % ST) * (NL * 1024));
+    const long k = (long)i * (NW * 64);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) ring_load<true>(wb + k, woff[j], to + j * 1024);
+#pragma unroll
+    for (int j = 0; j < NX; ++j) ring_load<false>(xb + k, xoff[j], to + (2 + j) * 1024);
+  };
+#pragma unroll
+  for (int i = 0; i < ST - 1; ++i)
+    if (i < mine) stage(i);
+
+  // What the epilogue adds and weights, read while the weights travel: as bits, since a
+  // conversion here would wait for them. A sum is the work of four threads.
+  constexpr int TURNS = (4 * RO * MP + 64 * NW - 1) / (64 * NW);
+  static_assert(EPI != kSgRope || TURNS == 1);
+  unsigned short was[TURNS] = {}, next_w[TURNS] = {}, plus[TURNS] = {}, plus_up = 0;
+  auto bits = [](const __hip_bfloat16* p) { return *reinterpret_cast<const unsigned short*>(p); };
+  auto value = [](unsigned short b) { return __uint_as_float((unsigned)b << 16); };
+  if (w < NW)
+#pragma unroll
+    for (int i = 0; i < TURNS; ++i) {
+      const int t = (i * 64 * NW + threadIdx.x) >> 2, n = n0 + t % RO;
+      if constexpr (EPI == kSgResidual) {
+        was[i] = bits(out + (long)min(t / RO, M - 1) * out_stride + n);
+        if (next.g) next_w[i] = bits(next.w + n);
       }
-      ss = wave_reduce_sum(ss);
-      if (lane == 0) sums[w][m] = ss;
+      if (bias) plus[i] = bits(bias + n);
+      if (EPI == kSgRope && bias) plus_up = bits(bias + n + half);
     }
-    __syncthreads();
+  if constexpr (EPI == kSgRope)
+    if (w == NW) {
+      if (head < rope.heads + rope.kv_heads)
+        for (int t = lane; t < RO * M; t += WAVE) {
+          const float* cs = rope.cos_sin + rope.positions[t / RO] * rope.D +
+                            (n0 - head * rope.D) + t % RO;
+          turned[0][t] = cs[0];
+          turned[1][t] = cs[half];
+        }
+      if (head >= rope.heads && lane < M) {
+        const long slot = rope.slots[lane];
+        const int kh = (head - rope.heads) % rope.kv_heads;
+        cached[lane] = slot < 0 ? -1
+            : (slot / rope.bs * rope.kv_heads + kh) * rope.bs + slot % rope.bs;
+      }
+    }
+
+  sg_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  const int xrow = col / MP * XP + min(col % MP, XP - 1);
+  for (int i = 0; i < mine; ++i) {
+    stream_wait<ST - 2, NL>(mine - 1 - i);                 // stage i is here, i - 1 is read
+    if (i + ST - 1 < mine) stage(i + ST - 1);
+    if (SCALE && i == 0) factors();                        // while the weights travel
+    const short* at = ring + (i % ST) * (NL * 512);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const sg_s16x8 wf = *reinterpret_cast<const sg_s16x8*>(
+          at + col * 64 + (((u * 4 + grp) ^ ((col >> 1) & 7)) << 3));
+      const sg_s16x8 xf = *reinterpret_cast<const sg_s16x8*>(
+          at + (16 + xrow) * 64 + (((u * 4 + grp) ^ ((xrow >> 1) & 7)) << 3));
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf, acc, 0, 0, 0);
+    }
   }
-  for (; k0 < ks; k0 += NW * KC) {
-    sg_s16x8 xf[KU];
-#pragma unroll
-    for (int u = 0; u < KU; ++u)
-      xf[u] = NORM ? *reinterpret_cast<const sg_s16x8*>(tp + k0 + u * 32)
-                   : *reinterpret_cast<const sg_s16x8*>(xp + k0 + u * 32);
-    const int next = k0 + NW * KC;
-    if (next < ks) fetch(wn, next);
-#pragma unroll
-    for (int u = 0; u < KU; ++u)
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], xf[u], acc, 0, 0, 0);
-#pragma unroll
-    for (int u = 0; u < KU; ++u) wf[u] = wn[u];
+  if (SCALE && mine == 0 && w < NW) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    factors();
   }
+  if (w < NW)
 #pragma unroll
-  for (int r = 0; r < 4; ++r) red[w][(grp * 4 + r) * RP + col] = acc[r];
+    for (int r = 0; r < 4; ++r) red[w][(grp * 4 + r) * RP + col] = acc[r];
   __syncthreads();
+  if (w == NW) return;
   // four threads per sum: each takes every fourth wave
   auto total = [&](int m, int row, int part) {
     float s = 0.f;
@@ -166,37 +271,45 @@ __global__ __launch_bounds__(64 * NW) void stream_gemm_kernel(
     s += __shfl_xor(s, 2, WAVE);
     return s;
   };
-  static_assert(EPI != kSgRope || 4 * RO * MP <= 64 * NW, "angles of one sum per thread");
-  for (int t = threadIdx.x; t < 4 * RO * MP; t += 64 * NW) {
+#pragma unroll
+  for (int turn = 0; turn < TURNS; ++turn) {
+    const int t = turn * 64 * NW + threadIdx.x;
+    if (t >= 4 * RO * M) break;                            // whole rows
     const int part = t & 3, row = (t >> 2) % RO, m = (t >> 2) / RO;
     float y = total(m, row, part);
     float up = 0.f, inv = 1.f;
     if constexpr (PAIR) up = total(m, row + RO, part);
-    if constexpr (NORM) {
-      float q = 0.f;
-#pragma unroll
-      for (int v = 0; v < NW / 4; ++v) q += sums[part + v * 4][min(m, M - 1)];
-      q += __shfl_xor(q, 1, WAVE);
-      q += __shfl_xor(q, 2, WAVE);
-      inv = rsqrtf(q / K + eps);
-    }
-    if (part != 0 || m >= M) continue;
+    if constexpr (SCALE) inv = invs[m];
     const int n = n0 + row;
+    const bool live = part == 0;
     y *= inv;
-    if (bias) y += to_f32(bias[n]);
+    y += value(plus[turn]);
+    if constexpr (EPI == kSgResidual) {
+      const __hip_bfloat16 v = __float2bfloat16(y + value(was[turn]));
+      if (live) out[(long)m * out_stride + n] = v;
+      if (!next.g) continue;
+      const float f = to_f32(v);
+      float ss = live ? f * f : 0.f;                       // 4 RO lanes hold a row's columns
+#pragma unroll
+      for (int off = 4; off < 4 * RO; off <<= 1) ss += __shfl_xor(ss, off, WAVE);
+      if (live) next.g[(long)m * N + n] = __float2bfloat16(f * (value(next_w[turn]) + next.offset));
+      if (live && row == 0) next.sq[(long)m * ((gridDim.x + 3) & ~3) + blockIdx.x] = ss;
+      continue;
+    }
+    if (!live) continue;
     if constexpr (EPI == kSgRope) {
       up *= inv;
-      if (bias) up += to_f32(bias[n + half]);
+      up += value(plus_up);
+      const bool turns = head < rope.heads + rope.kv_heads;
+      const float cosine = turns ? turned[0][t >> 2] : 1.f, sine = turns ? turned[1][t >> 2] : 0.f;
       const __hip_bfloat16 a = __float2bfloat16(y * cosine - up * sine);
       const __hip_bfloat16 b = __float2bfloat16(up * cosine + y * sine);
       __hip_bfloat16* o = out + (long)m * out_stride + n;
       o[0] = a;
       o[half] = b;
-      if (head < rope.heads || slot < 0) continue;
+      if (head < rope.heads || cached[m] < 0) continue;
       const bool is_v = head >= rope.heads + rope.kv_heads;
-      const int kh = head - rope.heads - (is_v ? rope.kv_heads : 0);
-      const long at = ((slot / rope.bs * rope.kv_heads + kh) * rope.bs + slot % rope.bs) * rope.D +
-                      n - head * rope.D;
+      const long at = cached[m] * rope.D + n - head * rope.D;
       void* cache = is_v ? rope.v_cache : rope.k_cache;
       if (rope.fp8) {                      // from the rounded rows, as elsewhere
         __hip_fp8_e4m3* c = static_cast<__hip_fp8_e4m3*>(cache) + at;
@@ -217,8 +330,29 @@ __global__ __launch_bounds__(64 * NW) void stream_gemm_kernel(
         y = 0.5f * y * (1.0f + tanhf(0.7978845608028654f * (y + 0.044715f * y * y * y))) * up;
       }
     }
-    __hip_bfloat16* o = out + (long)m * out_stride + n;
-    if constexpr (EPI == kSgResidual) y += to_f32(*o);
-    *o = __float2bfloat16(y);
+    out[(long)m * out_stride + n] = __float2bfloat16(y);
   }
+}
+
+// The rows that the first product of a SCALE chain reads: g = x (w + offset), sq[row][0 of 4].
+__global__ __launch_bounds__(256) void stream_prep_kernel(
+    __hip_bfloat16* __restrict__ g, float* __restrict__ sq,
+    const __hip_bfloat16* __restrict__ x, long x_stride, const __hip_bfloat16* __restrict__ w,
+    float offset, int K) {
+  __shared__ float red[4];
+  const __hip_bfloat16* xr = x + (long)blockIdx.x * x_stride;
+  float ss = 0.f;
+  for (int k = threadIdx.x * 8; k < K; k += 256 * 8) {
+    const Vec8<__hip_bfloat16> xv = load16(xr + k), nv = load16(w + k);
+    Vec8<__hip_bfloat16> y;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float a = to_f32(xv.data[e]);
+      ss += a * a;
+      y.data[e] = __float2bfloat16(a * (to_f32(nv.data[e]) + offset));
+    }
+    store16(g + (long)blockIdx.x * K + k, y);
+  }
+  ss = block_reduce_sum(ss, red);
+  if (threadIdx.x == 0) sq[blockIdx.x * 4] = ss;           // one sum a row, rounded up to 4
 }

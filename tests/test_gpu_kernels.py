@@ -707,6 +707,54 @@ class TestFewRowsLinear:
             assert torch.equal(cache.float().transpose(1, 2).reshape(48, KVH, D), want)
 
 
+class TestFewRowsChain:
+    """A layer of few rows whose norms ride on its products: what an addition to the
+    residual leaves for the next norm, and who reads it."""
+
+    @pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
+    @pytest.mark.parametrize("H,K", [(128, 128), (1152, 640), (2048, 8192), (4352, 256)])
+    def test_vs_64_bits(self, M, H, K):
+        bf = dict(device=DEV, dtype=torch.bfloat16)
+        res, x = torch.randn(M, H, **bf), torch.randn(M, K, **bf)
+        w, nw = torch.randn(H, K, **bf) * K ** -0.5, torch.randn(H, **bf)
+        rows = ops.FewRows(res.clone(), 1e-5, 1.0)
+        for first in (True, False):
+            if first:
+                rows.start(nw)
+            else:
+                rows.add(x, w, nw)
+                want = res.double() + x.double() @ w.double().t()
+                assert ((rows.residual.double() - want).abs() <= 2 ** -8 * want.abs() + 2e-5).all()
+            r = rows.residual
+            assert torch.equal(rows.g, (r.float() * (nw.float() + 1.0)).bfloat16())
+            sums = rows.sq[: M * -(-rows.n // 4) * 4].view(M, -1)[:, : rows.n].double().sum(1)
+            square = r.double().square().sum(1)
+            assert ((sums - square).abs() <= 1e-5 * square).all()
+            h = rows.g.double() * torch.rsqrt(square / H + 1e-5)[:, None]
+            mag = h.norm(dim=-1, keepdim=True) * H ** -0.5
+            for N, gelu in ((96, False), (128, True), (16512, False)):
+                gu = torch.randn(N, H, **bf) * H ** -0.5
+                g, u = (h @ gu.double().t()).chunk(2, -1)
+                want = (torch.nn.functional.gelu(g, approximate="tanh") if gelu
+                        else torch.nn.functional.silu(g)) * u
+                tol = 2 ** -8 * want.abs() + 1e-5 * mag * (u.abs() + 1.2 * g.abs()) + 1e-6
+                assert ((rows.act(gu, gelu).double() - want).abs() <= tol).all()
+            D, bias = 64, torch.randn(5 * 64, **bf)
+            wq = torch.randn(5 * D, H, **bf) * H ** -0.5
+            kc, vc = (torch.zeros(2, 1, 16, D, **bf) for _ in range(2))
+            pos, slots = torch.randint(0, 500, (M,), device=DEV), torch.arange(M, device=DEV) + 7
+            cs = torch_ref.build_rope_cache(512, D, 10000.0, DEV)
+            got = rows.qkv(wq, bias, kc, vc, pos, cs, slots).view(M, 5, D).double()
+            y = (h @ wq.double().t() + bias.double()).view(M, 5, D)
+            c, s = cs.double()[pos].view(M, 1, D).chunk(2, -1)
+            a, b = y[:, :4].chunk(2, -1)
+            want = torch.cat([torch.cat([a * c - b * s, b * c + a * s], -1), y[:, 4:]], 1)
+            tol = 2 ** -8 * want.abs() + 2e-5 * (mag.view(M, 1, 1) + 1.0)
+            assert ((got - want).abs() <= tol).all()
+            assert torch.equal(kc.view(32, D)[slots], got[:, 3].bfloat16())
+            assert torch.equal(vc.view(32, D)[slots], got[:, 4].bfloat16())
+
+
 class TestEngineGPU:
     def test_engine_generates_and_graphs_match_eager(self):
         from llmq_amd.engine.config import EngineConfig
