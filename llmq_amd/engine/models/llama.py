@@ -422,4 +422,6 @@ class CausalLM:
     @torch.no_grad()
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
         """hidden [N, hidden] → logits [N, vocab] (fp32)."""
-        return ops.softcap_logits(_proj(hidden, self.lm_head), self.spec.final_softcap)
+        if _USE_SKINNY_GEMM:
+            return ops.softcap_logits(_proj(hidden, self.lm_head), self.spec.final_softcap)
+        return ops.head_logits(hidden, self.lm_head, self.spec.final_softcap)

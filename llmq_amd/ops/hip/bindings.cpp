@@ -642,7 +642,8 @@ size_t sums_bytes(long M, const SgScale& scale) {
 
 template <int TT, int RT, int WN, int WT, int WK, int ST, int EPI, bool ROT>
 void launch_ring(float* slabs, __hip_bfloat16* out, long out_stride, const at::Tensor& x,
-                 const at::Tensor& w, int parts, int steps, const SgScale& scale = {}) {
+                 const at::Tensor& w, int parts, int steps, const SgScale& scale = {},
+                 float cap = 0) {
   using Shape = RingShape<TT, RT, WN, WT, WK, ST>;
   const int M = x.size(0), K = x.size(1), N = w.size(0);
   hipLaunchKernelGGL((ring_gemm_kernel<TT, RT, WN, WT, WK, ST, EPI, ROT>),
@@ -651,7 +652,7 @@ void launch_ring(float* slabs, __hip_bfloat16* out, long out_stride, const at::T
                      stream(), slabs, out, out_stride,
                      reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()), x.stride(0),
                      reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()), M, N, K, parts, steps,
-                     scale);
+                     scale, cap);
 }
 
 template <typename F>
@@ -789,6 +790,44 @@ at::Tensor ring_act_linear(const at::Tensor& x, const at::Tensor& w, bool gelu) 
     else launch_slab_gemm<kSlabSilu>(nullptr, p, out.stride(0), x, w);
   } else if (gelu) launch_ring_act<kSlabGelu>(p, out.stride(0), x, w);
   else launch_ring_act<kSlabSilu>(p, out.stride(0), x, w);
+  return out;
+}
+
+// The head: fp32 logits x W^T, capped where cap > 0. Weight rows a workgroup as for gates;
+// measured (us, 64 / 128 / 256 rows a workgroup, the library's product and conversion): 1 row,
+// 128256 x 2048 81 / 84 / 80, 114 + 5; 7 rows, 131072 x 1536 61 / 62 / 62, 78 + 5; 96 rows, 256000
+// x 3584 434 / 385 / 335, 350 + 27; 189 rows, 128256 x 3072 - / 204 / 191, 253 + 24; 256 rows,
+// 128256 x 3072 - / 245 / 210, 255 + 24.
+bool ring_head_ok(const at::Tensor& x, const at::Tensor& w) {
+  return slab_rows_ok(x, w, kRingRows) && streamable(w) && w.size(1) < (1 << 22) &&
+         (x.size(0) - 1) * x.stride(0) < (1L << 30);
+}
+
+at::Tensor ring_head(const at::Tensor& x, const at::Tensor& w, double cap) {
+  CHECK_GPU(x);
+  TORCH_CHECK(ring_head_ok(x, w), "ring_head: 1 to 256 bf16 rows on 16 bytes, packed weights, "
+                                  "K a multiple of 128, N of 64");
+  const long N = w.size(0), cus = compute_units(x);
+  at::Tensor out = at::empty({x.size(0), N}, x.options().dtype(at::kFloat));
+  ring_tiles(x.size(0), [&]<int TT>() {
+    auto go = [&]<int RT, int WN, int WT, int ST>() {
+      launch_ring<TT, RT, WN, WT, 1, ST, kRingHead, true>(
+          out.data_ptr<float>(), nullptr, 0, x, w, 1, (int)(w.size(1) / kRingBK), {}, (float)cap);
+    };
+    if (N / 128 > cus && N % 256 == 0) {
+      if constexpr (TT <= 3) go.template operator()<2, 8, 1, 3>();
+      else if constexpr (TT <= 8) go.template operator()<4, 4, 2, 3>();
+      else if constexpr (TT == 12) go.template operator()<4, 4, 2, 2>();
+      else go.template operator()<8, 2, 4, 2>();
+    } else if (N / 64 > cus && N % 128 == 0) {
+      if constexpr (TT <= 3) go.template operator()<2, 4, 1, 4>();
+      else if constexpr (TT <= 8) go.template operator()<4, 2, 2, 3>();
+      else go.template operator()<4, 2, 4, 3>();
+    } else {
+      if constexpr (TT <= 8) go.template operator()<1, 4, 1, 4>();
+      else go.template operator()<2, 2, 4, 4>();
+    }
+  });
   return out;
 }
 
@@ -1353,6 +1392,7 @@ TORCH_LIBRARY(llmq_amd, m) {
   m.def("few_act(Tensor g, Tensor sq, int n, float eps, Tensor w, bool gelu) -> Tensor");
   m.def("slab_linear(Tensor x, Tensor w) -> Tensor");
   m.def("ring_linear(Tensor x, Tensor w) -> Tensor");
+  m.def("ring_head(Tensor x, Tensor w, float cap) -> Tensor");
   m.def("ring_act_linear(Tensor x, Tensor w, bool gelu) -> Tensor");
   m.def("slab_act_linear(Tensor x, Tensor w, bool gelu) -> Tensor");
   m.def("slab_add_norm(Tensor slabs, Tensor(a!) residual, Tensor? w_post, Tensor w, float eps, float offset) -> Tensor");
@@ -1383,6 +1423,7 @@ TORCH_LIBRARY_IMPL(llmq_amd, CUDA, m) {
   m.impl("few_act", &few_act);
   m.impl("slab_linear", &slab_linear);
   m.impl("ring_linear", &ring_linear);
+  m.impl("ring_head", &ring_head);
   m.impl("ring_act_linear", &ring_act_linear);
   m.impl("slab_act_linear", &slab_act_linear);
   m.impl("slab_add_norm", &slab_add_norm);

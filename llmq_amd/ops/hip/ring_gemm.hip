@@ -21,6 +21,9 @@
 //   - Gate and value rows (EPI kSlabSilu, kSlabGelu) are activated here: a wave's first
 //     RT/2 tiles are gates, the others the values of the same columns. They need whole
 //     sums, so no parts of K: WK groups of waves take the stages in turn instead.
+//   - The model's head (kRingHead) leaves fp32 logits, capped here: no product rounded to
+//     bf16, no pass that converts and caps (7 rows of 151936 x 1536: 163 + 5 us, now 73; 96 rows
+//     of 256000 x 3584: 350 + 27, now 335).
 //   - ROT: workgroups start at different stages. Rows of 4096 bytes start on the same
 //     memory channel, which all workgroups would ask at once (64 rows, 16384 x 2048:
 //     16.2 us, 14.0 with it).
@@ -35,6 +38,8 @@
 
 typedef __attribute__((ext_vector_type(8))) short rg_s16x8;
 typedef __attribute__((ext_vector_type(4))) float rg_f32x4;
+
+enum : int { kRingHead = 3 };   // beside slab_gemm.hip's
 
 constexpr int kRingBK = 64;
 
@@ -60,8 +65,8 @@ __global__ __launch_bounds__(64 * WN * WT * WK) void ring_gemm_kernel(
     float* __restrict__ slabs, __hip_bfloat16* __restrict__ out, long out_stride,
     const __hip_bfloat16* __restrict__ x, long x_stride,
     const __hip_bfloat16* __restrict__ wt, int M, int N, int K, int parts, int steps,
-    SgScale scale) {
-  constexpr bool PAIR = EPI != kSlabSums;
+    SgScale scale, float cap) {
+  constexpr bool PAIR = EPI == kSlabSilu || EPI == kSlabGelu;
   static_assert(PAIR || WK == 1, "groups' sums meet in LDS for gate and value rows only");
   static_assert(!PAIR || RT % 2 == 0, "a wave holds gates and their values");
   constexpr int BK = kRingBK, R = 16 * RT * WN, T = 16 * TT, TW = TT / WT, G = WN * WT;
@@ -186,6 +191,10 @@ __global__ __launch_bounds__(64 * WN * WT * WK) void ring_gemm_kernel(
 #pragma unroll
       for (int e = 0; e < NA; ++e) acc[e / TW][e % TW] += red[((g * G + w) * NA + e) * 64];
   }
+  if (EPI == kRingHead && cap > 0.f)
+#pragma unroll
+    for (int a = 0; a < RT; ++a)
+      cap_tile<TW, 4>(acc[a], 1.f, cap, 2.8853900817779268f / cap);
 #pragma unroll
   for (int m = 0; m < TW; ++m) {
     const int row = (wc * TW + m) * 16 + col;

@@ -493,6 +493,20 @@ class TestSlabProjections:
             tol = 2 ** -8 * (act * u).abs() + 3e-5 * (1 + g.abs()) * (1 + u.abs())
             assert ((y - act * u).abs() <= tol).all()
 
+    @pytest.mark.parametrize("M", [1, 17, 48, 64, 128, 129, 193, 256])
+    @pytest.mark.parametrize("N,K", [(64, 128), (16512, 256), (65792, 128), (128256, 256)])
+    @pytest.mark.parametrize("cap", [0.0, 1.5])
+    def test_head(self, M, N, K, cap):
+        """fp32 logits, both forms of the cap, one round of workgroups and more."""
+        x = torch.randn(M, K, device=DEV, dtype=torch.bfloat16)
+        w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) * K ** -0.5
+        ref = x.double() @ w.double().t()
+        want = torch.tanh(ref / cap) * cap if cap else ref
+        got = ops.head_logits(x, w, cap)
+        assert got.dtype == torch.float32
+        # fp32 sums of unit size; the cap's slope is at most one
+        assert ((got.double() - want).abs() <= 1e-5 * (1 + ref.abs())).all()
+
     def test_rows_far_apart(self):
         """Rows over 4 GiB from the first: the kernels with 64-bit addresses."""
         flat = torch.zeros((1 << 31) + 256, device=DEV, dtype=torch.bfloat16)
