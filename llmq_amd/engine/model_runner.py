@@ -58,6 +58,7 @@ class ModelRunner:
             and device.type == "cuda"
         )
         self._graphs: Dict[int, torch.cuda.CUDAGraph] = {}
+        self._hidden: Dict[int, torch.Tensor] = {}  # what a graph leaves, [bucket, hidden]
         self._graph_pool = None
         self.sampling_generator = torch.Generator(device=device if device.type == "cuda" else "cpu")
         self.sampling_generator.manual_seed(config.seed)
@@ -88,13 +89,19 @@ class ModelRunner:
         B = min(self.config.max_num_seqs, self.config.hipgraph_max_batch)
         dev = self.device
         self.graph_max_bs = B
-        self.in_ids = torch.zeros(B, dtype=torch.long, device=dev)
-        self.in_pos = torch.zeros(B, dtype=torch.long, device=dev)
-        self.in_slots = torch.zeros(B, dtype=torch.long, device=dev)
+        # ids, positions, slots and context lengths travel in ONE copy (a copy is a
+        # launch of some 4 us, whatever its size)
+        def rows(**kw):
+            buf = torch.zeros(3 * B + (B + 1) // 2, dtype=torch.long, **kw)
+            lens = buf[3 * B:].view(torch.int32)[:B]
+            lens.fill_(1)
+            return buf, buf[:B], buf[B:2 * B], buf[2 * B:3 * B], lens
+
+        self.in_rows, self.in_ids, self.in_pos, self.in_slots, self.in_context_lens = rows(
+            device=dev)
         self.in_block_tables = torch.zeros(
             B, self.max_blocks_per_seq, dtype=torch.int32, device=dev
         )
-        self.in_context_lens = torch.ones(B, dtype=torch.int32, device=dev)
         self.in_rec = None
         if self.recurrent is not None:
             # one row per sequence; slots are staged per step, rows never
@@ -106,17 +113,12 @@ class ModelRunner:
             )
             self.h_rec_slots = torch.zeros(B, dtype=torch.int32, pin_memory=True)
             self.h_rec_fresh = torch.zeros(B, dtype=torch.int32, pin_memory=True)
-        self.out_hidden = torch.zeros(
-            B, self.model.spec.hidden_size, dtype=self.model.dtype, device=dev
-        )
         # pinned host staging for fast H2D of the per-step metadata
-        self.h_ids = torch.zeros(B, dtype=torch.long, pin_memory=True)
-        self.h_pos = torch.zeros(B, dtype=torch.long, pin_memory=True)
-        self.h_slots = torch.zeros(B, dtype=torch.long, pin_memory=True)
+        self.h_rows, self.h_ids, self.h_pos, self.h_slots, self.h_context_lens = rows(
+            pin_memory=True)
         self.h_block_tables = torch.zeros(
             B, self.max_blocks_per_seq, dtype=torch.int32, pin_memory=True
         )
-        self.h_context_lens = torch.ones(B, dtype=torch.int32, pin_memory=True)
         # (seq uid, preemption count, staged_len) per row — incremental
         # block-table staging. Keyed on Sequence.uid (monotonic, never
         # reused), NOT request_id: callers may reuse request ids across
@@ -155,10 +157,10 @@ class ModelRunner:
                 out = self.model.forward(
                     self.in_ids[:bs], self.in_pos[:bs], self.kv_cache, meta
                 )
-                self.out_hidden[:bs].copy_(out)
             if self._graph_pool is None:
                 self._graph_pool = graph.pool()
             self._graphs[bs] = graph
+            self._hidden[bs] = out  # held: later captures may not reuse its memory
         torch.cuda.synchronize()
         logger.info(
             "captured %d decode hipGraphs (max_bs=%d) in %.1fs",
@@ -443,7 +445,7 @@ class ModelRunner:
         # that wants no logits does not.
         if self._staging_done is not None:
             self._staging_done.synchronize()
-        # Stage metadata through pinned host buffers, one async copy each.
+        # Stage metadata through pinned host buffers.
         self.h_ids[:B] = torch.tensor(ids, dtype=torch.long)
         self.h_pos[:B] = torch.tensor(pos, dtype=torch.long)
         self.h_slots[:B] = torch.tensor(slots, dtype=torch.long)
@@ -474,10 +476,7 @@ class ModelRunner:
                 if self._staged_rows[i] != (-1, -1, 0):
                     bt_np[i, :1] = 0
                     self._staged_rows[i] = (-1, -1, 0)
-        self.in_ids[:bucket].copy_(self.h_ids[:bucket], non_blocking=True)
-        self.in_pos[:bucket].copy_(self.h_pos[:bucket], non_blocking=True)
-        self.in_slots[:bucket].copy_(self.h_slots[:bucket], non_blocking=True)
-        self.in_context_lens[:bucket].copy_(self.h_context_lens[:bucket], non_blocking=True)
+        self.in_rows.copy_(self.h_rows, non_blocking=True)
         self.in_block_tables[:bucket, :max_w].copy_(
             self.h_block_tables[:bucket, :max_w], non_blocking=True
         )
@@ -493,9 +492,10 @@ class ModelRunner:
             self._staging_done = torch.cuda.Event()
         self._staging_done.record()
         self._graphs[bucket].replay()
+        hidden = self._hidden[bucket][:B]
         if want is not None:
-            return self._logits_at(self.out_hidden[:B], [b for b, ws in enumerate(want) if ws])
-        logits = self.model.compute_logits(self.out_hidden[:B])
+            return self._logits_at(hidden, [b for b, ws in enumerate(want) if ws])
+        logits = self.model.compute_logits(hidden)
         return self._sample(logits, seqs)
 
     # -- sampling --------------------------------------------------------
