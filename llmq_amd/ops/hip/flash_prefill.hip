@@ -3,13 +3,14 @@
 // window; a portion may continue cached context (more keys than queries).
 //
 // Bound by the matrix cores and by the softmax beside them: at head size 128 the
-// products take 40% of the SIMD cycles and the vector work 50%, at the 1.9 GHz that
-// the clock falls to. Measured (us; before = 64-row workgroups whose softmax went
-// through lane exchanges and whose weights went through LDS): 8192 tokens, 24 heads
-// of 128: 1717 -> 510 (807 TFLOP/s); 16 x 1024, 32 heads of 64: 322 -> 123;
-// 8 x 1024, 16 heads of 256, capped: 273 -> 131; 7000, the same: 1483 -> 546;
-// 40 ragged up to 170, 12 heads of 128: 34 -> 18.
-//
+// products take half of the SIMD cycles and the vector work as many, at the 1.7 to 1.9
+// GHz that the clock falls to. What is between them is the wait for operands from LDS,
+// so these are read several products ahead. Measured (us; before = each read just ahead
+// of its product, V's granules with a bank conflict a read, references that follow every
+// maximum, halves' maxima exchanged through LDS): 8192 tokens, 24 heads of 128: 558 -> 440
+// (930 TFLOP/s); 2000, the same: 69 -> 52; 8 x 1024, the same: 89 -> 73; 8192, 32 heads of
+// 64: 364 -> 315; 8 x 1024, 16 heads of 256, capped: 137 -> 104; 7000, the same: 606 -> 463;
+// 40 x 170, 12 heads of 128: 25.3 -> 22.4.
 //
 //   - Both products run TRANSPOSED on v_mfma_f32_32x32x16_bf16, S^T = K Q^T and
 //     O^T = V^T P^T (A: row = lane%32, k = 8*(lane/32)..+7; B: column = lane%32;
@@ -69,11 +70,8 @@ DEVINL void pipe_barrier_vm() {
   asm volatile("" ::: "memory");
 }
 
-// glds16 with a uniform base and a 32-bit byte offset per lane.
-DEVINL void glds16_at(const void* base, unsigned off, void* lds_dst_uniform) {
-  unsigned lds_off = (unsigned)(unsigned long)(
-      (__attribute__((address_space(3))) char*)lds_dst_uniform);
-  lds_off = __builtin_amdgcn_readfirstlane(lds_off);
+// glds16 with a uniform base, a 32-bit byte offset per lane and an LDS offset.
+DEVINL void glds16_at(const void* base, unsigned off, unsigned lds_off) {
   unsigned keep;
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
@@ -90,9 +88,17 @@ DEVINL void glds16_at(const void* base, unsigned off, void* lds_dst_uniform) {
 // different 16-byte bank groups (K) ...
 template <int D>
 DEVINL int fp_kswz(int key) { return D >= 128 ? key & 15 : (key >> 1) & 7; }
-// ... and 8 consecutive keys' 32-byte groups in 8 different ones (V).
+// ... and 4 consecutive keys' equal 64-byte groups, what half a wave's transposing read
+// takes, in 4 different ones (V).
 template <int D>
-DEVINL int fp_vswz(int key) { return D >= 128 ? (key & 7) << 1 : ((key >> 1) & 3) << 1; }
+DEVINL int fp_vswz(int key) { return D >= 128 ? (key & 3) << 2 : ((key >> 1) & 1) << 2; }
+
+// The larger of the values of lanes l and l ^ 32, without LDS: a register's halves swapped
+// with a copy's leave the lower lanes' values in one and the upper lanes' in the other.
+DEVINL float fp_max_halves(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
 
 template <int D, int HP, int WR, int KT, int MINW, bool CAP, bool PAGED>
 __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
@@ -148,24 +154,21 @@ __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
   const bool idle = wr * 32 >= rows;
 
   // Staging: load i = w + j NW of a tile (K rows, then V rows) is 1 KiB = KPL key
-  // rows. A wave's loads lie STEP keys apart: its lanes' place in a row and their offset
-  // from the load's first row are the same for all of them, K's at STEP = 8 for every
-  // second one.
-  constexpr int KPL = 64 / GPR, STEP = NW * KPL, PH = STEP % 16 == 0 ? 1 : 2;
-  static_assert(NI % NW == 0 && STEP % 8 == 0, "a wave's loads share their swizzle");
+  // rows. A wave's loads lie STEP keys apart.
+  constexpr int KPL = 64 / GPR, STEP = NW * KPL, NJ = NI / NW;   // NJ: a wave's K loads per tile
+  static_assert(NI % NW == 0 && STEP % 8 == 0, "a wave's V loads share their swizzle");
   const int skey = w * KPL + lane / GPR;
   const int vgran = ((lane % GPR) ^ fp_vswz<D>(skey)) << 3;
-  constexpr int NJ = NI / NW;                          // a wave's K loads per tile
   const int lrow = PAGED ? lane / GPR : skey;          // row that the lane's offset counts
   const unsigned krow = PAGED ? D : (unsigned)k_stride, vrow = PAGED ? D : (unsigned)v_stride;
-  int kgran[PH];
-  unsigned koff[PH];
+  auto kgran = [&](int j) { return ((lane % GPR) ^ fp_kswz<D>(skey + j * STEP)) << 3; };
+  unsigned koff[NJ], voff[NJ];                         // of a whole tile's loads
 #pragma unroll
-  for (int ph = 0; ph < PH; ++ph) {
-    kgran[ph] = ((lane % GPR) ^ fp_kswz<D>(skey + ph * STEP)) << 3;
-    koff[ph] = ((unsigned)lrow * krow + kgran[ph]) * 2;
+  for (int j = 0; j < NJ; ++j) {
+    const unsigned row = PAGED ? lrow : lrow + j * STEP;
+    koff[j] = (row * krow + kgran(j)) * 2;
+    voff[j] = (row * vrow + vgran) * 2;
   }
-  const unsigned voff = ((unsigned)lrow * vrow + vgran) * 2;
   const __hip_bfloat16* kb = PAGED ? k : k + (long)k0 * k_stride + (long)kvh * D;
   const __hip_bfloat16* vb = PAGED ? v : v + (long)k0 * v_stride + (long)kvh * D;
   // Paged: a load's rows lie in one cache block (blocks hold 16 or 32 keys); its id
@@ -180,38 +183,49 @@ __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
         bid[j] = bt[__builtin_amdgcn_readfirstlane(
             min(kt + j * STEP + w * KPL, nk - 1) >> bs_shift)];
   };
-  auto fetch = [&](int kt, bool is_v, short* dst) {
+  const unsigned lds_at = (unsigned)(unsigned long)(
+      (__attribute__((address_space(3))) char*)lds) + w * 1024;
+  // A tile's loads, K's to lds_at + to and V's behind them.
+  auto fetch = [&](int kt, unsigned to) {
+    const unsigned at = __builtin_amdgcn_readfirstlane(lds_at + to);
     const bool whole = kt + KT <= nk;
+    const __hip_bfloat16* const kp = PAGED ? kb : kb + (long)kt * k_stride;
+    const __hip_bfloat16* const vp = PAGED ? vb : vb + (long)kt * v_stride;
+    auto load = [&](int j, const __hip_bfloat16* kj, unsigned ko, const __hip_bfloat16* vj,
+                    unsigned vo) {
+      glds16_at(kj, ko, at + j * NW * 1024);
+      glds16_at(vj, vo, at + j * NW * 1024 + KT * D * 2);
+    };
+    auto block = [&](int j) { return (((long)bid[j] * KVH + kvh) << bs_shift) * D; };
+    if (whole) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        if constexpr (PAGED) {
+          const long from = block(j) + ((kt + j * STEP + w * KPL) & bs_mask) * D;
+          load(j, kp + from, koff[j], vp + from, voff[j]);
+        } else {
+          load(j, kp, koff[j], vp, voff[j]);
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-      short* const to = dst + (w + j * NW) * 512;
-      const int gran = is_v ? vgran : kgran[j % PH];
-      const unsigned off = is_v ? voff : koff[j % PH];
       if constexpr (PAGED) {
-        const int first = kt + j * STEP + w * KPL;
-        const __hip_bfloat16* base =
-            (is_v ? vb : kb) + (((long)bid[j] * KVH + kvh) << bs_shift) * D;
-        if (whole)
-          glds16_at(base + (first & bs_mask) * D, off, to);
-        else
-          glds16(base + (min(first + lrow, nk - 1) & bs_mask) * D + gran, to);
+        const unsigned row = (min(kt + j * STEP + w * KPL + lrow, nk - 1) & bs_mask) * D;
+        load(j, kp + block(j), (row + kgran(j)) * 2, vp + block(j), (row + vgran) * 2);
       } else {
-        const int first = kt + j * STEP;               // row of the workgroup's key 0
-        const long stride = is_v ? v_stride : k_stride;
-        const __hip_bfloat16* base = (is_v ? vb : kb) + (long)first * stride;
-        if (whole)
-          glds16_at(base, off, to);
-        else
-          glds16(base + (long)(min(first + skey, nk - 1) - first) * stride + gran, to);
+        const unsigned row = min(skey + j * STEP, nk - 1 - kt);
+        load(j, kp, (row * krow + kgran(j)) * 2, vp, (row * vrow + vgran) * 2);
       }
     }
   };
 
   // this lane's part of the operand reads
-  const int kbase = col * D, ksw = fp_kswz<D>(col);
+  int kat = col * D + ((half ^ fp_kswz<D>(col)) << 3);
   const int vkey = half * 4 + ((lane & 15) >> 2);
-  const int vbase = vkey * D + (lane & 1) * 4;
   const int vg = ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1);
+  int vat = vkey * D + (lane & 1) * 4 + ((vg ^ fp_vswz<D>(vkey)) << 3);
 
   float m = -INFINITY, l = 0.f;                        // log2 domain
   fp_f32x16 o[DT];
@@ -223,8 +237,7 @@ __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
   const int kt0 = window > 0 ? max(0, pos0 - window + 1) / KT * KT : 0;
   if (kt0 <= pos_last) {
     blocks(kt0);
-    fetch(kt0, false, lds);
-    fetch(kt0, true, lds + KT * D);
+    fetch(kt0, 0);
     blocks(kt0 + KT);
   }
   int cur = 0;
@@ -233,9 +246,7 @@ __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
     short* const Vt = Kt + KT * D;
     pipe_barrier_vm<0>();                              // tile landed, the other buffer is read
     if (kt + KT <= pos_last) {
-      short* const next = lds + (cur ^ 1) * (2 * KT * D);
-      fetch(kt + KT, false, next);
-      fetch(kt + KT, true, next + KT * D);
+      fetch(kt + KT, (cur ^ 1) * (4 * KT * D));
       blocks(kt + 2 * KT);
     }
     if (idle || kt > wave_last || kt + KT - 1 < wave_lo) continue;
@@ -248,15 +259,44 @@ __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[t][r] = 0.f;
+    // Operands are asked for KP (V: VP) products ahead: the compiler by itself reads each one
+    // just before its product, a wait for LDS every time. Eight waves of head size 256 have no
+    // registers for the places of all operands either: what the compiler spills it reads back
+    // from scratch memory behind the next tile's loads (7000 tokens: 625 us, 465 without).
+    constexpr bool TIGHT = D == 256 && NW == 8;
+    constexpr int NK = KS * NT, KP = TIGHT ? 2 : 4, NV = DT * KT / 16, VP = TIGHT ? 2 : 3;
+    if constexpr (TIGHT) asm volatile("" : "+v"(kat), "+v"(vat));
+    auto read_k = [&](int x) {
+      return *reinterpret_cast<const fp_s16x8*>(
+          Kt + (x % NT) * 32 * D + (kat ^ (x / NT << 4)));
+    };
+    fp_s16x8 kf[KP];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
+    for (int x = 0; x < KP; ++x) kf[x] = read_k(x);
+    __builtin_amdgcn_sched_group_barrier(0x100, KP, 0);      // LDS reads
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const fp_s16x8 kf = *reinterpret_cast<const fp_s16x8*>(
-            Kt + t * 32 * D + kbase + (((ks * 2 + half) ^ ksw) << 3));
-        s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], s[t], 0, 0, 0);
+    for (int x = 0; x < NK; ++x) {
+      s[x % NT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[x % KP], qf[x / NT], s[x % NT], 0, 0, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);     // a product
+      if (x + KP < NK) {
+        kf[x % KP] = read_k(x + KP);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       }
+    }
     __builtin_amdgcn_s_setprio(0);
+    fp_s16x8 vf[VP];                                   // values, likewise
+    auto read_v = [&](int y) {
+      const int j = y / DT, dt = y % DT;
+      const short* at = Vt + j * 16 * D + (vat ^ (dt << 5));
+      const fp_s16x4 v0 = __builtin_bit_cast(fp_s16x4,
+          __builtin_amdgcn_ds_read_tr16_b64_v4bf16((fp_lds_bf16x4*)at));
+      const fp_s16x4 v1 = __builtin_bit_cast(fp_s16x4,
+          __builtin_amdgcn_ds_read_tr16_b64_v4bf16((fp_lds_bf16x4*)(at + 8 * D)));
+      return fp_s16x8(__builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+#pragma unroll
+    for (int y = 0; y < VP; ++y) vf[y] = read_v(y);
+    __builtin_amdgcn_sched_barrier(0);
     if constexpr (CAP) cap_tile<NT, 16>(s, scale_log2, cap_log2, cap_in);
     if (kt + KT - 1 > wave_first || kt < wave_all) {
       asm volatile("");                                // a branch, not selects on every tile
@@ -273,19 +313,21 @@ __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[t][r]);
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
+    tmax = fp_max_halves(tmax);
     const float sc = CAP ? 1.f : scale_log2;           // > 0
+    // The weights' reference follows the maximum only when that is 2^8 past it: they are as
+    // precise above one as below, and most tiles then rescale nothing.
     const float m_new = fmaxf(m, tmax * sc);
-    const float mb = m_new > -INFINITY ? m_new : 0.f;
-    if (__any(m_new > m)) {
-      const float alpha = __builtin_amdgcn_exp2f(m - mb);    // m = -inf -> 0
+    if (__any(m_new > m + 8.f)) {
+      const float alpha =
+          __builtin_amdgcn_exp2f(m - (m_new > -INFINITY ? m_new : 0.f));  // m = -inf -> 0
       l *= alpha;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
       m = m_new;
     }
-#pragma unroll
-    for (int j = 0; j < KT / 16; ++j) {                // 16 keys per step
+    const float mb = m > -INFINITY ? m : 0.f;
+    auto weights = [&](int j) {                        // of 16 keys
       const int t = j >> 1, u = (j & 1) * 8;
       fp_u32x4 pw;
 #pragma unroll
@@ -296,17 +338,19 @@ __global__ __launch_bounds__(64 * HP * WR, MINW) void flash_prefill_kernel(
         pw[e / 2] = __builtin_bit_cast(
             unsigned, __builtin_convertvector((fp_f32x2{p0, p1}), fp_bf16x2));
       }
-      const fp_s16x8 pf = __builtin_bit_cast(fp_s16x8, pw);
+      return __builtin_bit_cast(fp_s16x8, pw);
+    };
+    fp_s16x8 pf = weights(0);
+#pragma unroll
+    for (int j = 0; j < KT / 16; ++j) {
+      const fp_s16x8 p = pf;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
-        const short* at = Vt + j * 16 * D + vbase + (((dt * 4 + vg) ^ fp_vswz<D>(vkey)) << 3);
-        const fp_s16x4 v0 = __builtin_bit_cast(fp_s16x4,
-            __builtin_amdgcn_ds_read_tr16_b64_v4bf16((fp_lds_bf16x4*)at));
-        const fp_s16x4 v1 = __builtin_bit_cast(fp_s16x4,
-            __builtin_amdgcn_ds_read_tr16_b64_v4bf16((fp_lds_bf16x4*)(at + 8 * D)));
-        const fp_s16x8 vf = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf, o[dt], 0, 0, 0);
+        const int y = j * DT + dt;
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[y % VP], p, o[dt], 0, 0, 0);
+        if (y + VP < NV) vf[y % VP] = read_v(y + VP);
       }
+      if (j + 1 < KT / 16) pf = weights(j + 1);
     }
   }
   l += __shfl_xor(l, 32, WAVE);
