@@ -398,8 +398,11 @@ class CausalLM:
                     attn_out, residual, lw.pre_mlp_norm, s.rms_eps, self.norm_offset
                 )
             # ---- MLP block
-            gate_up = _proj(h, lw.gate_up)
-            act = ops.gelu_tanh_and_mul(gate_up) if s.gelu else ops.silu_and_mul(gate_up)
+            if not _USE_SKINNY_GEMM and ops.tile_act_ok(h, lw.gate_up):
+                act = ops.tile_act_linear(h, lw.gate_up, s.gelu)
+            else:
+                gate_up = _proj(h, lw.gate_up)
+                act = ops.gelu_tanh_and_mul(gate_up) if s.gelu else ops.silu_and_mul(gate_up)
             mlp_out = _proj(act, lw.down)
             if tp is not None:
                 mlp_out = tp.all_reduce(mlp_out)

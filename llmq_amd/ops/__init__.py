@@ -441,6 +441,18 @@ def ring_act_linear(x: torch.Tensor, w: torch.Tensor, gelu: bool) -> torch.Tenso
     return _EXT.ring_act_linear(x, w, bool(gelu))
 
 
+def tile_act_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether tile_act_linear takes these rows and beats the library's product and an
+    activation: over RING_ROWS bf16 rows whose tiles fill the chip."""
+    return _use_hip(x) and x.dtype == torch.bfloat16 and _EXT.tile_act_ok(x, w)
+
+
+def tile_act_linear(x: torch.Tensor, w: torch.Tensor, gelu: bool) -> torch.Tensor:
+    """ring_act_linear for any number of rows."""
+    assert _use_hip(x)
+    return _EXT.tile_act_linear(x, w, bool(gelu))
+
+
 def head_logits(x: torch.Tensor, w: torch.Tensor, cap: float) -> torch.Tensor:
     """fp32 logits x @ w.T, capped (cap * tanh(logits / cap)) where cap > 0. Over 192 rows
     of a large head the library's product and a pass over it take less: its own kernel

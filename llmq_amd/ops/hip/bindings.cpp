@@ -831,6 +831,71 @@ at::Tensor ring_head(const at::Tensor& x, const at::Tensor& w, double cap) {
   return out;
 }
 
+// ------------------------------------------- gate and value rows, many tokens --
+
+// Tokens of a tile / 64 for tile_gemm.hip, and whether it is worth it. A stage of 64
+// channels takes 0.93, 1.18 or 1.5 us with tiles of 128, 192 or 256 tokens, a tile 2.5 more;
+// all CUs take a tile a round. The library's product and activation take about what
+// 1.45 PFLOP/s, a pass at 4.5 TB/s and 5 us come to, up to 1.25 times that where its own
+// tiles do not fill the chip. Measured (us, tiles of 128 / 192 / 256 tokens, library +
+// activation): 300 rows, 16384 x 3072 44 / 52 / 59, 39 (refused); 28672 x 3584 99 / 66 / 83, 64
+// (refused); 512, 16384 x 3072 49 / 57 / 64, 51; 700, 28672 x 3584 148 / 129 / 158, 142; 1000,
+// 17920 x 1536 65 / 60 / 67, 77; 2000, 16384 x 2048 121 / 115 / 99, 117.
+struct TilePlan { int tw; bool worth; };
+
+TilePlan tile_plan(long M, long N, long K, int cus) {
+  TilePlan best{0, false};
+  double least = 0;
+  const double stage_us[] = {0.93, 1.18, 1.5};
+  for (int tw = 2; tw <= 4; ++tw) {
+    const long tiles = N / kTileRows * ((M + 64 * tw - 1) / (64 * tw));
+    const double us = (tiles + cus - 1) / cus * (K / kTileBK * stage_us[tw - 2] + 2.5);
+    if (best.tw == 0 || us < least) least = us, best.tw = tw;
+  }
+  best.worth = least <= 1.25 * (2e-9 / 1.45 * M * N * K + M * N * 3 / 4.5e6 + 5);
+  return best;
+}
+
+// What tile_gemm.hip takes: it counts bytes from a tile's first row in 32 bits.
+bool tile_takes(const at::Tensor& x, const at::Tensor& w) {
+  return x.dim() == 2 && w.dim() == 2 && x.size(0) > 0 && x.size(0) < (1L << 30) &&
+         x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 &&
+         x.size(1) == w.size(1) && w.size(1) > 0 && w.size(1) % kTileBK == 0 &&
+         w.size(0) > 0 && w.size(0) % kTileRows == 0 && x.stride(1) == 1 &&
+         rows_start_on(x, 16) && streamable(w) && x.is_cuda() && w.get_device() == x.get_device() &&
+         w.numel() * 2 < (1L << 32) && x.stride(0) >= 0 && x.stride(0) < (1L << 22);
+}
+
+// Whether tile_act_linear beats the library's product and an activation. Up to 256 rows
+// are ring_gemm.hip's.
+bool tile_act_ok(const at::Tensor& x, const at::Tensor& w) {
+  return tile_takes(x, w) && x.size(0) > kRingRows &&
+         tile_plan(x.size(0), w.size(0), w.size(1), compute_units(x)).worth;
+}
+
+at::Tensor tile_act_linear(const at::Tensor& x, const at::Tensor& w, bool gelu) {
+  CHECK_GPU(x);
+  TORCH_CHECK(tile_takes(x, w), "tile_act_linear: bf16 rows on 16 bytes, packed weights, K a "
+                                "multiple of 64, N of 256");
+  const int M = x.size(0), K = x.size(1), N = w.size(0), cus = compute_units(x);
+  at::Tensor out = at::empty({M, N / 2}, x.options());
+  auto go = [&]<int TW>() {
+    const int wtiles = N / kTileRows, ttiles = (M + 64 * TW - 1) / (64 * TW);
+    auto kernel = gelu ? &tile_gemm_kernel<TW, kSlabGelu> : &tile_gemm_kernel<TW, kSlabSilu>;
+    hipLaunchKernelGGL(kernel, dim3(std::min<long>(cus, (long)wtiles * ttiles)), dim3(512),
+                       tile_lds<TW>(), stream(), reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
+                       out.stride(0), reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()),
+                       x.stride(0), reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()), M, N, K,
+                       wtiles, ttiles);
+  };
+  switch (tile_plan(M, N, K, cus).tw) {
+    case 2: go.template operator()<2>(); break;
+    case 3: go.template operator()<3>(); break;
+    default: go.template operator()<4>();
+  }
+  return out;
+}
+
 // The two for up to 128 and 64 rows.
 at::Tensor slab_linear(const at::Tensor& x, const at::Tensor& w) {
   CHECK_GPU(x);
@@ -1269,6 +1334,8 @@ at::Tensor prompt_layers(at::Tensor h, at::Tensor residual, at::TensorList weigh
     at::Tensor act;
     if (slab && ring_act_ok(h, w[2])) {
       act = ring_act_linear(h, w[2], gelu);
+    } else if (tile_act_ok(h, w[2])) {
+      act = tile_act_linear(h, w[2], gelu);
     } else {
       const at::Tensor gate_up = at::linear(h, w[2]);
       act = at::empty({T, gate_up.size(1) / 2}, gate_up.options());
@@ -1397,6 +1464,8 @@ TORCH_LIBRARY(llmq_amd, m) {
   m.def("slab_act_linear(Tensor x, Tensor w, bool gelu) -> Tensor");
   m.def("slab_add_norm(Tensor slabs, Tensor(a!) residual, Tensor? w_post, Tensor w, float eps, float offset) -> Tensor");
   m.def("slab_rope_cache(Tensor slabs, Tensor? bias, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor positions, Tensor cos_sin, Tensor slots) -> Tensor");
+  m.def("tile_act_ok(Tensor x, Tensor w) -> bool");
+  m.def("tile_act_linear(Tensor x, Tensor w, bool gelu) -> Tensor");
   m.def("prompt_layers(Tensor h, Tensor(a!) residual, Tensor[] weights, Tensor[] biases, Tensor[] k_caches, Tensor[] v_caches, Tensor positions, Tensor cos_sin, Tensor slots, Tensor cu_seqlens, Tensor? block_tables, Tensor? cu_seqlens_k, int max_seqlen, int head_dim, float scale, float softcap, int[] windows, float eps, float offset, bool gelu, bool post_norms) -> Tensor");
   m.def("sample_gumbel_argmax(Tensor(a!) out, Tensor(b!) keys, Tensor logits, Tensor temps, Tensor req_seeds, Tensor req_pos, int seed, int step, Tensor? bounds=None) -> ()");
   m.def("topk_topp_bound(Tensor(a!) out_bound, Tensor logits, Tensor temps, Tensor top_ps, Tensor top_ks) -> ()");
@@ -1422,6 +1491,8 @@ TORCH_LIBRARY_IMPL(llmq_amd, CUDA, m) {
   m.impl("few_qkv", &few_qkv);
   m.impl("few_act", &few_act);
   m.impl("slab_linear", &slab_linear);
+  m.impl("tile_act_ok", &tile_act_ok);
+  m.impl("tile_act_linear", &tile_act_linear);
   m.impl("ring_linear", &ring_linear);
   m.impl("ring_head", &ring_head);
   m.impl("ring_act_linear", &ring_act_linear);

@@ -9,5 +9,6 @@
 #include "stream_gemm.hip"
 #include "slab_gemm.hip"
 #include "ring_gemm.hip"
+#include "tile_gemm.hip"
 #include "sampling.hip"
 #include "bindings.cpp"

@@ -493,6 +493,35 @@ class TestSlabProjections:
             tol = 2 ** -8 * (act * u).abs() + 3e-5 * (1 + g.abs()) * (1 + u.abs())
             assert ((y - act * u).abs() <= tol).all()
 
+    @pytest.mark.parametrize("M", [1, 127, 257, 700, 1153])
+    @pytest.mark.parametrize("N,K", [(256, 64), (768, 192), (17920, 128), (4096, 1536)])
+    def test_tile_activated(self, M, N, K):
+        """One stage and more, whole and cut tiles of 128 to 256 tokens, one round and more;
+        rows packed and padded."""
+        x = torch.randn(M, K + 8, device=DEV, dtype=torch.bfloat16)
+        w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) * K ** -0.5
+        for x in (x[:, :K], x[:, :K].contiguous()):
+            g, u = (x.double() @ w.double().t()).chunk(2, -1)
+            for gelu in (False, True):
+                act = torch.nn.functional.gelu(g, approximate="tanh") if gelu \
+                    else torch.nn.functional.silu(g)
+                y = ops.tile_act_linear(x, w, gelu).double()
+                tol = 2 ** -8 * (act * u).abs() + 3e-5 * (1 + g.abs()) * (1 + u.abs())
+                assert ((y - act * u).abs() <= tol).all()
+
+    def test_tile_refuses(self):
+        """What the tiles cannot take is left to the library."""
+        x = torch.randn(1024, 256, device=DEV, dtype=torch.bfloat16)
+        w = torch.randn(16384, 256, device=DEV, dtype=torch.bfloat16)
+        assert ops.tile_act_ok(x, w)
+        for a, b in ((x[:256], w), (x.half(), w.half()), (x, w[:16384 - 128]),
+                     (x[:, :248], w[:, :248].contiguous()), (x, w.t().contiguous().t()),
+                     (x.t().contiguous().t(), w), (x.float(), w.float())):
+            assert not ops.tile_act_ok(a, b)
+            if a.dtype == torch.bfloat16 and a.shape[0] > 256:
+                with pytest.raises(RuntimeError):
+                    ops.tile_act_linear(a, b, False)
+
     @pytest.mark.parametrize("M", [1, 17, 48, 64, 128, 129, 193, 256])
     @pytest.mark.parametrize("N,K", [(64, 128), (16512, 256), (65792, 128), (128256, 256)])
     @pytest.mark.parametrize("cap", [0.0, 1.5])
