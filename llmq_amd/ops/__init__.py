@@ -454,12 +454,10 @@ def tile_act_linear(x: torch.Tensor, w: torch.Tensor, gelu: bool) -> torch.Tenso
 
 
 def head_logits(x: torch.Tensor, w: torch.Tensor, cap: float) -> torch.Tensor:
-    """fp32 logits x @ w.T, capped (cap * tanh(logits / cap)) where cap > 0. Over 192 rows
-    of a large head the library's product and a pass over it take less: its own kernel
-    writes a tile's logits while it multiplies nothing (256 rows of 256000 x 3584: 526 us
-    against 428 + 81; of 128256 x 3072: 210 against 255 + 24)."""
-    if (_use_hip(x) and slab_ok(x, (w,), 0, RING_ROWS) and w.shape[1] < 1 << 22
-            and (x.shape[0] <= 192 or w.numel() < 512 << 20)):
+    """fp32 logits x @ w.T, capped (cap * tanh(logits / cap)) where cap > 0. Its own kernel
+    up to RING_ROWS rows (256 rows, the library's product and a pass over it: 256000 x 3584
+    470 us against 503, 128256 x 3072 205 against 310)."""
+    if _use_hip(x) and slab_ok(x, (w,), 0, RING_ROWS) and w.shape[1] < 1 << 22:
         return _EXT.ring_head(x, w, float(cap or 0.0))
     return softcap_logits(torch.nn.functional.linear(x, w), cap)
 
