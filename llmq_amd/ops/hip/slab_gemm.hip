@@ -148,17 +148,29 @@ __global__ __launch_bounds__(256 * WK) void slab_gemm_kernel(
 
 // ------------------------------------------------------- readers of the slabs --
 
-// Sum of S slabs at one place, eight loads in flight: their L2 is another XCD's.
+// The first S of NE slabs (one at the least) added to y, all loads in flight together:
+// their L2 is another XCD's.
+template <int NE>
+DEVINL void slab_add(sl_f32x4& y, const float* __restrict__ from, long stride, int S) {
+  sl_f32x4 v[NE];
+#pragma unroll
+  for (int e = 0; e < NE; ++e)
+    v[e] = *reinterpret_cast<const sl_f32x4*>(from + min(e, S - 1) * stride);
+#pragma unroll
+  for (int e = 0; e < NE; ++e)
+    if (e < S) y += v[e];
+}
+
+// Sum of S slabs at one place.
 DEVINL sl_f32x4 slab_sum(const float* __restrict__ slabs, long at, long stride, int S) {
   sl_f32x4 y = {0.f, 0.f, 0.f, 0.f};
-  for (int s0 = 0; s0 < S; s0 += 8) {
-    sl_f32x4 v[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      v[e] = *reinterpret_cast<const sl_f32x4*>(slabs + min(s0 + e, S - 1) * stride + at);
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      if (s0 + e < S) y += v[e];
+  for (int s0 = 0; s0 < S; s0 += 16) {
+    const float* from = slabs + s0 * stride + at;
+    const int n = S - s0;
+    if (n <= 4) slab_add<4>(y, from, stride, n);
+    else if (n <= 8) slab_add<8>(y, from, stride, n);
+    else if (n <= 12) slab_add<12>(y, from, stride, n);
+    else slab_add<16>(y, from, stride, min(n, 16));
   }
   return y;
 }
@@ -178,37 +190,74 @@ DEVINL Vec4<__hip_bfloat16> slab_store(__hip_bfloat16* p, sl_f32x4 y) {
 
 // residual += y, or with POST += rmsnorm(y) (w_post + offset), y the summed slabs;
 // h = rmsnorm(residual) (w + offset). One workgroup per row, the row in registers:
-// up to 8192 channels. Bound by latency: few rows, each behind S slabs (64 rows of
-// 2048, 16 slabs: 4.8 us; with 256 threads that added slab by slab 9.4).
+// up to 8192 channels. Bound by latency: few rows, each behind S slabs; so everything is
+// asked for at once, norm weights too, and a sum over the row takes one barrier.
+// Measured (us, with weights read behind the sums, three barriers a sum and rounds of eight
+// slabs -> now; a sequence of such launches): 96 rows of 3584, 9 slabs, two norms 6.8 -> 5.7;
+// 48 rows 6.4 -> 5.5; 189 rows of 3072, 10 slabs 7.5 -> 6.9; 64 rows of 2048, 8 slabs 3.8,
+// as before (with 512 channels a wave instead of 256 4.5).
 constexpr int kSlabNT = 1024;
+
+// x plus the x of the lane that DPP control `CTRL` names, in the rows of 16 that ROWS has.
+template <int CTRL, int ROWS>
+DEVINL float slab_dpp_add(float x) {
+  return x + __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), CTRL, ROWS, 0xf,
+                                                         false));
+}
+
+// The workgroup's sum, in all threads; `red` is not used again. Sums go up within rows of 16
+// lanes, from row to row and through LDS once, without the LDS crossbar.
+DEVINL float slab_block_sum(float x, float (&red)[kSlabNT / WAVE]) {
+  x = slab_dpp_add<0x111, 0xf>(x);                         // row_shr 1, 2, 4, 8
+  x = slab_dpp_add<0x112, 0xf>(x);
+  x = slab_dpp_add<0x114, 0xf>(x);
+  x = slab_dpp_add<0x118, 0xf>(x);
+  x = slab_dpp_add<0x142, 0xa>(x);                         // row_bcast 15, 31
+  x = slab_dpp_add<0x143, 0xc>(x);
+  if ((threadIdx.x & (WAVE - 1)) == WAVE - 1) red[threadIdx.x / WAVE] = x;
+  __syncthreads();
+  const int waves = blockDim.x / WAVE;
+  x = 0.f;
+#pragma unroll
+  for (int i = 0; i < kSlabNT / WAVE; ++i) {
+    const float v = red[i];
+    x += i < waves ? v : 0.f;
+  }
+  return x;
+}
 
 template <bool POST>
 __global__ __launch_bounds__(kSlabNT) void slab_add_norm_kernel(
     __hip_bfloat16* __restrict__ h, __hip_bfloat16* __restrict__ residual,
     const float* __restrict__ slabs, int S, const __hip_bfloat16* __restrict__ w_post,
     const __hip_bfloat16* __restrict__ w, int M, int N, float eps, float offset) {
-  __shared__ float red[kSlabNT / WAVE];
+  __shared__ float red[2][kSlabNT / WAVE];
   const long row = (long)blockIdx.x * N;
   const long stride = (long)M * N;
   sl_f32x4 y[2], r[2];
+  int2 was[2], wn[2], wp[2];               // bf16 as read
   float ss = 0.f;
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
     const int i = (k * blockDim.x + threadIdx.x) * 4;
     y[k] = r[k] = sl_f32x4{0.f, 0.f, 0.f, 0.f};
     if (i >= N) continue;
-    r[k] = slab_bf4(residual + row + i);
+    was[k] = *reinterpret_cast<const int2*>(residual + row + i);
+    wn[k] = *reinterpret_cast<const int2*>(w + i);
+    if (POST) wp[k] = *reinterpret_cast<const int2*>(w_post + i);
     y[k] = slab_sum(slabs, row + i, stride, S);
     if (POST) ss += y[k][0] * y[k][0] + y[k][1] * y[k][1] + y[k][2] * y[k][2] + y[k][3] * y[k][3];
   }
   float inv = 1.f;
-  if (POST) inv = rsqrtf(block_reduce_sum(ss, red) / N + eps);
+  if (POST) inv = rsqrtf(slab_block_sum(ss, red[0]) / N + eps);
   ss = 0.f;
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
     const int i = (k * blockDim.x + threadIdx.x) * 4;
     if (i >= N) continue;
-    if (POST) r[k] += y[k] * inv * (slab_bf4(w_post + i) + offset);
+    r[k] = slab_bf4(reinterpret_cast<const __hip_bfloat16*>(&was[k]));
+    if (POST)
+      r[k] += y[k] * inv * (slab_bf4(reinterpret_cast<const __hip_bfloat16*>(&wp[k])) + offset);
     else r[k] += y[k];
     const Vec4<__hip_bfloat16> v = slab_store(residual + row + i, r[k]);
 #pragma unroll
@@ -217,11 +266,13 @@ __global__ __launch_bounds__(kSlabNT) void slab_add_norm_kernel(
       ss += r[k][e] * r[k][e];
     }
   }
-  inv = rsqrtf(block_reduce_sum(ss, red) / N + eps);
+  inv = rsqrtf(slab_block_sum(ss, red[1]) / N + eps);
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
     const int i = (k * blockDim.x + threadIdx.x) * 4;
-    if (i < N) slab_store(h + row + i, r[k] * inv * (slab_bf4(w + i) + offset));
+    if (i < N)
+      slab_store(h + row + i,
+                 r[k] * inv * (slab_bf4(reinterpret_cast<const __hip_bfloat16*>(&wn[k])) + offset));
   }
 }
 
@@ -240,8 +291,6 @@ __global__ __launch_bounds__(256) void slab_rope_cache_kernel(
   const long row = (long)token * N, stride = (long)M * N;
   const float* cs = cos_sin + positions[token] * D;
   const long slot = slots[token];
-  const long block = slot / block_size;
-  const int off = (int)(slot % block_size);
   for (int t = blockIdx.y * 256 + threadIdx.x; t < (heads + 2 * kv_heads) * quads;
        t += gridDim.y * 256) {
     const int hd = t / quads, d = (t % quads) * 4;
@@ -264,6 +313,8 @@ __global__ __launch_bounds__(256) void slab_rope_cache_kernel(
     if (hd < heads || slot < 0) continue;
     const bool is_v = hd >= heads + kv_heads;
     const int kh = hd - heads - (is_v ? kv_heads : 0);
+    const long block = slot / block_size;
+    const int off = (int)(slot - block * block_size);
     TC* dst = (is_v ? v_cache : k_cache) +
               ((block * kv_heads + kh) * (long)block_size + off) * D + d;
     if constexpr (std::is_same_v<TC, __hip_bfloat16>) {
