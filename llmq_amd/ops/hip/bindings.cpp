@@ -303,7 +303,11 @@ void launch_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor& kc,
     };
     using BF = __hip_bfloat16;
     using F8 = __hip_fp8_e4m3;
-    if (D == 64) go.template operator()<64, BF, 4, 3>();
+    // 32 keys a tile at head size 64 (us, with the merge, 64 / 32: 1 x 200 keys, 8 kv heads 9.3
+    // / 8.1; 1 x 3000 11.2 / 10.4; 8 ragged up to 1000 10.2 / 10.4; 64 x 1040 35.2 / 34.1; 6
+    // ragged up to 15000 34.8 / 33.6). At 128 64 keys and one workgroup a CU gain on 3 ragged up
+    // to 16000 (34.4 / 32.2) what they lose on 60 up to 800 (31.9 / 32.5).
+    if (D == 64) go.template operator()<64, BF, 2, 3>();
     else if (D == 128 && !fp8) go.template operator()<128, BF, 2, 2>();
     else if (D == 256 && !fp8) go.template operator()<256, BF, 1, 1>();
     else if (D == 128) go.template operator()<128, F8, 2, 3>();

@@ -7,7 +7,7 @@
 // of the matrix cores, so everything here serves to keep loads in flight on all
 // CUs until the last byte has come. Measured (us, with the merge; before = one
 // workgroup per pair, VALU at head size 64, K and V through one shared LDS
-// pipeline else): 64 x 1040 keys, 8 kv heads of 64: 391 -> 38 (136 MB);
+// pipeline else): 64 x 1040 keys, 8 kv heads of 64: 391 -> 34 (136 MB);
 // 189 ragged up to 1100, 8 of 128: 152 -> 108 (473 MB); 3 ragged up to 16000,
 // 8 of 128: 83 -> 40 (147 MB); 96 x 1064, 8 of 256, capped: 197 -> 161 (837 MB);
 // 512 x 1064: 889 -> 772 (4.46 GB, 5.8 TB/s); 48 ragged up to 2000, 8 of 256,
@@ -73,9 +73,12 @@ DEVINL int pd_total(const int* __restrict__ lens, int B, int window, int lane, i
 }
 
 // Tiles per wave: an equal share. One tile while that leaves CUs without work
-// (latency); two from there on, so that short pairs are not cut needlessly.
+// (latency); two from there on, so that short pairs are not cut needlessly; four of
+// head size 64's, which are half as many keys and bytes, beyond that.
+template <int D>
 DEVINL int pd_share(int total, int waves) {
-  return max((total + waves - 1) / waves, total > 1024 ? 2 : 1);
+  const int least = D == 64 ? (total > 2048 ? 4 : total > 512 ? 2 : 1) : total > 1024 ? 2 : 1;
+  return max((total + waves - 1) / waves, least);
 }
 
 // The first sequence whose tiles reach past `t` (all pairs counted, kv heads
@@ -144,7 +147,7 @@ DEVINL int pd_swz(int key) {
 
 template <int D, typename TC, int NK>
 struct PdShape {
-  static constexpr int kTileShift = NK == 4 ? 6 : NK == 2 ? 5 : 4;
+  static constexpr int kTileShift = NK == 2 ? 5 : 4;
   static constexpr int kKeys = 16 * NK;
   static constexpr size_t kLds = 4 * sizeof(short) * (size_t)kKeys * D;
 };
@@ -177,7 +180,7 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
   const int wave = w * gridDim.x + blockIdx.x;
   const int first = lens[min(lane, B - 1)];
   const int total = pd_total<TS>(lens, B, window, lane, first) * KVH;
-  const int share = pd_share(total, waves);
+  const int share = pd_share<D>(total, waves);
   int t = wave * share;
   const int t_end = min(total, t + share);
   if (t >= t_end) return;
@@ -442,7 +445,7 @@ __global__ __launch_bounds__(256) void paged_decode_merge_kernel(
     all += __shfl_xor(all, off, WAVE);
     before += __shfl_xor(before, off, WAVE);
   }
-  const int share = pd_share(all * KVH, waves);
+  const int share = pd_share<D>(all * KVH, waves);
   const int first_tile = before * KVH + (h / G) * nt;
   const int first = first_tile / share, last = (first_tile + nt - 1) / share;
   if (first == last) return;                 // written by its wave
