@@ -509,7 +509,7 @@ def softcap_logits(x: torch.Tensor, cap: float) -> torch.Tensor:
 
 def sample_gumbel_argmax(
     out: torch.Tensor,        # [B] int64
-    keys: torch.Tensor,       # [B] int64 scratch (packed value|~index)
+    keys: torch.Tensor,       # [B] int64, the packed value|~index of each token
     logits: torch.Tensor,     # [B, V] fp32
     temps: torch.Tensor,      # [B] fp32 (<= 0 → greedy row)
     req_seeds: torch.Tensor,  # [B] int32 (0 = unseeded)
@@ -525,7 +525,6 @@ def sample_gumbel_argmax(
     draw from (request_seed, output_position) — reproducible for a given
     request regardless of batch placement."""
     assert _use_hip(logits)
-    keys.zero_()
     _EXT.sample_gumbel_argmax(out, keys, logits, temps, req_seeds, req_pos,
                               seed, step, bounds)
 

@@ -1431,17 +1431,18 @@ void sample_gumbel_argmax(at::Tensor out, at::Tensor keys, at::Tensor logits,
   TORCH_CHECK(logits.is_contiguous(), "logits must be contiguous");
   int chunk, splits;
   const bool vec = row_chunks(logits, B, V, chunk, splits);
+  at::Tensor parts = at::empty({(long)B, (long)splits}, keys.options());
+  auto words = [](const at::Tensor& t) {
+    return reinterpret_cast<unsigned long long*>(t.data_ptr());
+  };
   hipLaunchKernelGGL(sample_argmax_kernel, dim3(B, splits), dim3(256), 0,
-                     stream(),
-                     reinterpret_cast<unsigned long long*>(keys.data_ptr()),
+                     stream(), words(parts),
                      logits.data_ptr<float>(), temps.data_ptr<float>(),
                      reinterpret_cast<const unsigned int*>(req_seeds.data_ptr()),
                      reinterpret_cast<const unsigned int*>(req_pos.data_ptr()),
                      bounds_ptr, V, (unsigned int)seed, (unsigned int)step, chunk, vec);
-  hipLaunchKernelGGL(unpack_keys_kernel, dim3((B + 255) / 256), dim3(256), 0,
-                     stream(), out.data_ptr<long>(),
-                     reinterpret_cast<const unsigned long long*>(keys.data_ptr()),
-                     B);
+  hipLaunchKernelGGL(unpack_keys_kernel, dim3((B + 3) / 4), dim3(256), 0, stream(),
+                     out.data_ptr<long>(), words(keys), words(parts), splits, B);
 }
 
 }  // namespace

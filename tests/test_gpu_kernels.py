@@ -855,6 +855,17 @@ class TestFusedSampler:
                                  seed, step)
         return out
 
+    @pytest.mark.parametrize("B,V", [(1, 1), (1, 4097), (5, 128256), (3, 262147), (260, 5000)])
+    def test_chunks_meet(self, B, V):
+        """One chunk of a row and up to 64, ties between chunks, keys as they were left."""
+        logits = torch.randn(B, V, device=DEV)
+        logits[:, [V // 3, V - 1]] = 9.0
+        out = torch.empty(B, dtype=torch.int64, device=DEV)
+        keys = torch.full((B,), -1, dtype=torch.int64, device=DEV)
+        zeros = torch.zeros(B, dtype=torch.int32, device=DEV)
+        ops.sample_gumbel_argmax(out, keys, logits, torch.zeros(B, device=DEV), zeros, zeros, 1, 1)
+        assert (out == V // 3).all()
+
     def test_greedy_matches_argmax(self):
         torch.manual_seed(0)
         logits = torch.randn(16, 50000, device=DEV, dtype=torch.float32)
