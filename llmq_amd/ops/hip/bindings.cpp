@@ -837,26 +837,30 @@ at::Tensor ring_head(const at::Tensor& x, const at::Tensor& w, double cap) {
 
 // ------------------------------------------- gate and value rows, many tokens --
 
-// Tokens of a tile / 64 for tile_gemm.hip, and whether it is worth it. A stage of 64
-// channels takes 0.93, 1.18 or 1.5 us with tiles of 128, 192 or 256 tokens, a tile 2.5 more;
-// all CUs take a tile a round. The library's product and activation take about what
-// 1.45 PFLOP/s, a pass at 4.5 TB/s and 5 us come to, up to 1.25 times that where its own
-// tiles do not fill the chip. Measured (us, tiles of 128 / 192 / 256 tokens, library +
-// activation): 300 rows, 16384 x 3072 44 / 52 / 59, 39 (refused); 28672 x 3584 99 / 66 / 83, 64
-// (refused); 512, 16384 x 3072 49 / 57 / 64, 51; 700, 28672 x 3584 148 / 129 / 158, 142; 1000,
-// 17920 x 1536 65 / 60 / 67, 77; 2000, 16384 x 2048 121 / 115 / 99, 117.
+// Tokens of a tile / 64 for tile_gemm.hip, and whether it is worth it. With weights that
+// come from memory, as a model's layers do, a stage of 64 channels takes 1.27, 1.45 or 1.68 us
+// with tiles of 128, 192 or 256 tokens (0.93, 1.18 and 1.5 from the caches), a tile 2.5 more;
+// all CUs take a tile a round. Against that stand 1.45 PFLOP/s, a pass at 4.5 TB/s and 5 us, what
+// the library's product and an activation come to at their best: up to 1.4 times that over
+// 2048 rows, which hide the weights' way, and below 2048 channels, where the library's tiles
+// fill and drain every few stages; up to 1.05 times else. Measured (us, weights from memory, library + activation / tiles): 1000 rows, 17920 x
+// 1536 82 / 69; 2000, the same 133 / 122; 512, 16384 x 3072 59 / 67 (refused); 1000, the same
+// 92 / 85; 1300, the same 130 / 137 (refused); 768, 16384 x 2048 53 / 50; 2000, the same 121 /
+// 110; 512, 28672 x 3584 96 / 100 (refused); 2000, the same 341 / 370 (refused); 2250, the same
+// 409 / 379; 4096, the same 619 / 623; 2250, 16384 x 3072 201 / 204; 2808, the same 339 / 222.
 struct TilePlan { int tw; bool worth; };
 
 TilePlan tile_plan(long M, long N, long K, int cus) {
   TilePlan best{0, false};
   double least = 0;
-  const double stage_us[] = {0.93, 1.18, 1.5};
+  const double stage_us[] = {1.27, 1.45, 1.68};
   for (int tw = 2; tw <= 4; ++tw) {
     const long tiles = N / kTileRows * ((M + 64 * tw - 1) / (64 * tw));
     const double us = (tiles + cus - 1) / cus * (K / kTileBK * stage_us[tw - 2] + 2.5);
     if (best.tw == 0 || us < least) least = us, best.tw = tw;
   }
-  best.worth = least <= 1.25 * (2e-9 / 1.45 * M * N * K + M * N * 3 / 4.5e6 + 5);
+  best.worth = least <= (M > 2048 || K < 2048 ? 1.4 : 1.05) *
+                            (2e-9 / 1.45 * M * N * K + M * N * 3 / 4.5e6 + 5);
   return best;
 }
 

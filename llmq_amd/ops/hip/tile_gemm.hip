@@ -3,8 +3,10 @@
 // decode batch (gfx950).
 //
 // Bound by the matrix cores at the clock that they leave, 1.1 to 1.4 PFLOP/s; the
-// activation costs no pass over the product and its rounding to bf16 is gone. Measured (us;
-// before = the library's product and act_and_mul_kernel): 512 rows, 17920 x 1536 40.6 -> 32.4;
+// activation costs no pass over the product and its rounding to bf16 is gone. With few
+// tokens the weights come from memory too late for two stages: the rule at the launch says
+// where. Measured (us, weights in the caches; before = the library's product and
+// act_and_mul_kernel): 512 rows, 17920 x 1536 40.6 -> 32.4;
 // 1000, 16384 x 3072 84 -> 74; 1000, 28672 x 3584 179 -> 165; 3953, 17920 x 1536 207 -> 176;
 // 8192, 16384 x 2048 454 -> 384, 16384 x 3072 630 -> 577 (1.43 PFLOP/s), 28672 x 3584 1224 ->
 // 1208. (Plain products on these tiles lose to the library by 3 to 10 % where they fill
