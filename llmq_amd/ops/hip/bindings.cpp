@@ -393,10 +393,19 @@ void launch_flash_prefill(at::Tensor& out, const PrefillArgs& a) {
   }
 }
 
+// flash_prefill.hip counts bytes from a tile's first key, up to 63 rows of k or v on, in 32
+// bits: packed copies of rows farther apart (2^25 elements, 64 MiB).
+at::Tensor rows_in_reach(const at::Tensor& t) {
+  const at::Tensor r = rows_on_16(t);
+  return r.size(0) <= 1 || r.stride(0) < (1L << 25) ? r : r.clone(at::MemoryFormat::Contiguous);
+}
+
 void launch_flash_prefill_any(at::Tensor& out, const PrefillArgs& args) {
   const int H = args.q.size(1), D = args.q.size(2);
   at::Tensor qa = rows_on_16(args.q);
-  const at::Tensor ka = rows_on_16(args.k), va = rows_on_16(args.v);
+  const bool paged = args.block_tables != nullptr;       // contiguous caches, 64-bit addresses
+  const at::Tensor ka = paged ? args.k : rows_in_reach(args.k);
+  const at::Tensor va = paged ? args.v : rows_in_reach(args.v);
   at::Tensor oa = rows_start_on(out, 8) ? out : out.clone(at::MemoryFormat::Contiguous);
   // The kernel masks scores with -inf before it scales them: a negative scale goes into
   // the queries, and zero (every visible key alike) too.

@@ -350,6 +350,24 @@ class TestPrefillRanges:
         # unit normals); the output's own rounding 2^-9 of it, twice that allowed
         assert_close_to_f32_ref(out.cpu(), ref, 5 * 2 ** -9, 2 ** -8)
 
+    @pytest.mark.parametrize("D", [64, 128, 256])
+    @pytest.mark.parametrize("stride,n", [(1 << 30, 3), (1 << 28, 9), (1 << 25, 64),
+                                          ((1 << 25) - 8, 65)])
+    def test_rows_far_apart(self, D, stride, n):
+        """Key and value rows spread over 4 GiB, in part of a tile and whole ones: the same
+        as packed."""
+        H, KVH = 4, 2
+        flat = torch.zeros((n - 1) * stride + 2 * KVH * D, device=DEV, dtype=torch.bfloat16)
+        k, v = (flat[i * KVH * D:].as_strided((n, KVH, D), (stride, D, 1)) for i in (0, 1))
+        k.normal_()
+        v.normal_()
+        q = torch.randn(n, H, D, device=DEV, dtype=torch.bfloat16)
+        cu = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+        packed = ops.varlen_prefill_attention(q, k.clone(memory_format=torch.contiguous_format),
+                                              v.clone(memory_format=torch.contiguous_format), cu,
+                                              n, D ** -0.5)
+        assert torch.equal(ops.varlen_prefill_attention(q, k, v, cu, n, D ** -0.5), packed)
+
 
 class TestScoreCap:
     """The score cap in both attention kernels, from caps that saturate (scores of
