@@ -751,22 +751,25 @@ at::Tensor ring_linear(const at::Tensor& x, const at::Tensor& w) {
 // Gate and value rows: as many weight rows a workgroup as make one round of workgroups.
 // Measured (us, 64 / 128 / 256 rows): 64 tokens, 28672 x 3584 42.6 / 35.8 / -; 48 tokens,
 // 37888 x 3584 60 / 60 / 51.5; 128, 55296 x 5120 177 / 132 / 107; 128, 16384 x 3072 28.2 / 38 / -.
+long ring_act_rows(long N, long cus) {
+  if (N / 128 > cus && N % 256 == 0) return 256;
+  return N / 64 > cus && N % 128 == 0 ? 128 : 64;
+}
+
 template <int EPI>
 void launch_ring_act(__hip_bfloat16* out, long out_stride, const at::Tensor& x,
                      const at::Tensor& w, const SgScale& scale = {}) {
-  const long N = w.size(0), cus = compute_units(x);
+  const long rows = ring_act_rows(w.size(0), compute_units(x));
   const int steps = (int)(w.size(1) / kRingBK);
-  const bool r128 = N / 64 > cus && N % 128 == 0;
-  const bool r256 = N / 128 > cus && N % 256 == 0;
   ring_tiles(x.size(0), [&]<int TT>() {
     auto go = [&]<int RT, int WN, int WT, int WK, int ST, bool ROT>() {
       launch_ring<TT, RT, WN, WT, WK, ST, EPI, ROT>(nullptr, out, out_stride, x, w, 1, steps, scale);
     };
-    if (r256) {
+    if (rows == 256) {
       if constexpr (TT <= 3) go.template operator()<2, 8, 1, 1, 3, false>();
       else if constexpr (TT <= 8) go.template operator()<4, 4, 2, 1, 3, false>();
       else go.template operator()<4, 4, 2, 1, 2, false>();
-    } else if (r128) {
+    } else if (rows == 128) {
       launch_ring_128<TT, EPI>(nullptr, out, out_stride, x, w, 1, steps, scale);
     } else {
       // eight waves where two groups, or four columns, have work for them (64 rows of 16384 x
@@ -969,6 +972,27 @@ void finish_product(at::Tensor out, const at::Tensor& y, long epi) {
   else gelu_tanh_and_mul(out, y);
 }
 
+// Whether gate and value rows of up to 16 tokens go to ring_gemm.hip, whose workgroups own 64
+// rows and more and all of K, or to stream_gemm.hip's pairs, 8 or 16 rows each. The ring wants
+// many workgroups, a last round that is no small one, and rows whose starts spread over the
+// memory channels: multiples of 1 KiB do so badly without the start of its own that a
+// workgroup of 64 rows takes, of 4 KiB worse, of 16 KiB in any form. From nine tokens on,
+// which the pairs read again for every 16 rows, it wins more. Measured (us, ring / pairs): 1 token, 2048 x
+// 2048 8.2 / 3.8, 2048 x 8192 25.3 / 8.0, 8192 x 3072 13.8 / 10.2, 9728 x 896 6.0 / 6.3, 12288 x
+// 4096 19.7 / 20.5, 16384 x 2048 13.7 / 14.4, 16384 x 8192 62 / 48, 16448 x 3072 26.9 / 21.4,
+// 17920 x 1536 14.2 / 12.9, 18432 x 2304 17.9 / 18.2, 24576 x 896 10.1 / 11.2, 28672 x 2048 26.6 / 23.3,
+// 28672 x 3584 36.0 / 37.3, 37888 x 3584 53 / 46; 9 tokens, 4096 x 896 5.2 / 3.7, 6144 x 896 5.4 /
+// 5.7, 8192 x 3072 14.9 / 12.2, 9728 x 3072 14.4 / 15.7, 16448 x 3072 26.9 / 24.5, 24640 x 2048
+// 21.8 / 24.9, 17920 x 1536 14.5 / 16.1, 28672 x 3584 35.7 / 42.4, 57344 x 8192 187 / 150.
+bool pairs_in_ring(long M, long N, long K, long cus) {
+  const bool many = M > 8;
+  if (N % 64 != 0 || N <= (many && K < 1536 ? 20 : 32) * cus || K >= 8192) return false;
+  const long rows = ring_act_rows(N, cus), tiles = N / rows;
+  if (rows == 64) return tiles <= cus || (many && tiles * 4 >= cus * 5);
+  if (many || K < 1536 || (rows == 128 && K % 512 != 0)) return true;
+  return tiles <= cus && tiles * 5 >= cus * 4 && K % 2048 != 0;
+}
+
 // out = f(x) W^T for up to 16 rows: see stream_gemm.hip. norm_w: x is RMS-normalised
 // first; epi: 0 plain, 1 added to out in place, 2 / 3 SiLU / tanh-GELU of the first
 // half of W's rows times the second half. scale: x's rows await their factors; next:
@@ -1022,7 +1046,7 @@ void launch_stream_gemm(at::Tensor out, at::Tensor x, at::Tensor w,
     }
     return;
   }
-  if (pair && N % 64 == 0 && out.stride(0) % 4 == 0 &&
+  if (pair && pairs_in_ring(M, N, K, compute_units(x)) && out.stride(0) % 4 == 0 &&
       reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0) {
     auto* p = reinterpret_cast<__hip_bfloat16*>(out.data_ptr());
     if (epi == kSgSilu) launch_ring_act<kSlabSilu>(p, out.stride(0), x, w, scale);

@@ -25,7 +25,8 @@
 //     factor meets the fp32 sums at the end. (Before, every workgroup of the reader weighted
 //     all tokens by itself, up to six, and more took a launch of 4 us.)
 //   - ACT: half of the weight rows are gates, half the values that they act on (x = [gate |
-//     up]): pairs of widths that ring_gemm.hip does not take.
+//     up]): pairs that ring_gemm.hip does not take, or takes longer over (the rule stands at
+//     the launch).
 //   - ROPE (the q/k/v projection): a workgroup takes channel pairs of one head, rotates
 //     q and k and writes k and v into the paged cache too; positions and
 //     angles are read by the ninth wave while the weights travel. A launch of its own for that took 4.5 us

@@ -815,6 +815,29 @@ class TestFewRowsChain:
             assert torch.equal(kc.view(32, D)[slots], got[:, 3].bfloat16())
             assert torch.equal(vc.view(32, D)[slots], got[:, 4].bfloat16())
 
+    @pytest.mark.parametrize("M", [1, 8, 9, 16])
+    @pytest.mark.parametrize("N,K", [(5120, 128), (5184, 128), (8192, 1536), (8256, 1536),
+                                     (16384, 640), (16448, 128), (20544, 256), (16640, 1408),
+                                     (16640, 1536), (16640, 1664), (26240, 1536), (26240, 2048),
+                                     (33024, 256), (33024, 1536), (8256, 8192)])
+    def test_pairs(self, M, N, K):
+        """Gate and value rows on both sides of the lines between the two kernels that take
+        them, of normalised rows and of rows whose scale is still to come."""
+        bf = dict(device=DEV, dtype=torch.bfloat16)
+        x, nw = torch.randn(M, K, **bf), torch.ones(K, **bf)
+        gu = torch.randn(N, K, **bf) * K ** -0.5
+        g, u = (x.double() @ gu.double().t()).chunk(2, -1)
+        want = torch.nn.functional.silu(g) * u
+        tol = 2 ** -8 * want.abs() + 3e-5 * (1 + g.abs()) * (1 + u.abs())
+        assert ((ops.few_rows_linear(x, gu, act="silu").double() - want).abs() <= tol).all()
+        rows = ops.FewRows(x, 1e-5, 0.0)
+        rows.start(nw)
+        s = torch.rsqrt(x.double().square().mean(-1, keepdim=True) + 1e-5)
+        g, u = g * s, u * s
+        want = torch.nn.functional.gelu(g, approximate="tanh") * u
+        tol = 2 ** -8 * want.abs() + 3e-5 * (1 + g.abs()) * (1 + u.abs())
+        assert ((rows.act(gu, True).double() - want).abs() <= tol).all()
+
 
 class TestEngineGPU:
     def test_engine_generates_and_graphs_match_eager(self):
