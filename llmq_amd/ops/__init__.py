@@ -455,8 +455,9 @@ def tile_act_linear(x: torch.Tensor, w: torch.Tensor, gelu: bool) -> torch.Tenso
 
 def head_logits(x: torch.Tensor, w: torch.Tensor, cap: float) -> torch.Tensor:
     """fp32 logits x @ w.T, capped (cap * tanh(logits / cap)) where cap > 0. Its own kernel
-    up to RING_ROWS rows (256 rows, the library's product and a pass over it: 256000 x 3584
-    470 us against 503, 128256 x 3072 205 against 310)."""
+    up to RING_ROWS rows. Measured, us, weights from memory, against the library's product
+    and a pass over it: 256 rows, 256000 x 3584 468 and 493, 128256 x 4096 256 and 354; 129
+    rows, 256000 x 3584 419 and 412 (rounded to bf16 on the way, error 1.7e-3; here 4e-7)."""
     if _use_hip(x) and slab_ok(x, (w,), 0, RING_ROWS) and w.shape[1] < 1 << 22:
         return _EXT.ring_head(x, w, float(cap or 0.0))
     return softcap_logits(torch.nn.functional.linear(x, w), cap)

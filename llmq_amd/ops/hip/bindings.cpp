@@ -660,7 +660,7 @@ void launch_ring(float* slabs, __hip_bfloat16* out, long out_stride, const at::T
   using Shape = RingShape<TT, RT, WN, WT, WK, ST>;
   const int M = x.size(0), K = x.size(1), N = w.size(0);
   hipLaunchKernelGGL((ring_gemm_kernel<TT, RT, WN, WT, WK, ST, EPI, ROT>),
-                     dim3(N / Shape::kRows * parts), dim3(64 * Shape::kWaves),
+                     dim3((N + Shape::kRows - 1) / Shape::kRows * parts), dim3(64 * Shape::kWaves),
                      Shape::kLds + (scale.sq ? sums_bytes(M, scale) : 0),
                      stream(), slabs, out, out_stride,
                      reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()), x.stride(0),
@@ -809,11 +809,15 @@ at::Tensor ring_act_linear(const at::Tensor& x, const at::Tensor& w, bool gelu) 
   return out;
 }
 
-// The head: fp32 logits x W^T, capped where cap > 0. Weight rows a workgroup as for gates;
-// measured (us, 64 / 128 / 256 rows a workgroup, the library's product and conversion): 1 row,
-// 128256 x 2048 81 / 84 / 80, 114 + 5; 7 rows, 131072 x 1536 61 / 62 / 62, 78 + 5; 96 rows, 256000
-// x 3584 434 / 385 / 335, 350 + 27; 189 rows, 128256 x 3072 - / 204 / 191, 253 + 24; 256 rows,
-// 128256 x 3072 - / 245 / 210, 255 + 24.
+// The head: fp32 logits x W^T, capped where cap > 0. Weight rows a workgroup as for gates, but
+// any multiple of 64 in all: the last workgroup may have fewer. Token tiles of 160 and 224 too
+// where 256 rows a workgroup take most of what a CU takes in. Measured (us, 64 / 128 / 256 rows
+// a workgroup, the library's product and conversion): 1 row, 128256 x 2048 81 / 84 / 80, 114 + 5; 7
+// rows, 131072 x 1536 61 / 62 / 62, 78 + 5; 96 rows, 256000 x 3584 434 / 385 / 335, 350 + 27; 256
+// rows, 32064 x 4096 106 / 75 / -, 86 with its conversion; 49216 x 2048 108 / - / 63, 75; 65600 x
+// 3072 189 / - / 157, 149 (257 workgroups, two rounds). Tokens rounded up to 192 or 256 / to 160 or
+// 224: 256000 x 4608, 129 rows 526 / 519, library 513; 208 rows 583 / 557, 608; 152064 x 5120, 144
+// rows 406 / 405, 372.
 bool ring_head_ok(const at::Tensor& x, const at::Tensor& w) {
   return slab_rows_ok(x, w, kRingRows) && streamable(w) && w.size(1) < (1 << 22) &&
          (x.size(0) - 1) * x.stride(0) < (1L << 30);
@@ -825,23 +829,27 @@ at::Tensor ring_head(const at::Tensor& x, const at::Tensor& w, double cap) {
                                   "K a multiple of 128, N of 64");
   const long N = w.size(0), cus = compute_units(x);
   at::Tensor out = at::empty({x.size(0), N}, x.options().dtype(at::kFloat));
-  ring_tiles(x.size(0), [&]<int TT>() {
-    auto go = [&]<int RT, int WN, int WT, int ST>() {
-      launch_ring<TT, RT, WN, WT, 1, ST, kRingHead, true>(
-          out.data_ptr<float>(), nullptr, 0, x, w, 1, (int)(w.size(1) / kRingBK), {}, (float)cap);
-    };
-    if (N / 128 > cus && N % 256 == 0) {
-      if constexpr (TT <= 3) go.template operator()<2, 8, 1, 3>();
-      else if constexpr (TT <= 8) go.template operator()<4, 4, 2, 3>();
-      else if constexpr (TT == 12) go.template operator()<4, 4, 2, 2>();
-      else go.template operator()<8, 2, 4, 2>();
-    } else if (N / 64 > cus && N % 128 == 0) {
-      if constexpr (TT <= 3) go.template operator()<2, 4, 1, 4>();
-      else if constexpr (TT <= 8) go.template operator()<4, 2, 2, 3>();
-      else go.template operator()<4, 2, 4, 3>();
+  auto go = [&]<int TT, int RT, int WN, int WT, int ST>() {
+    launch_ring<TT, RT, WN, WT, 1, ST, kRingHead, true>(
+        out.data_ptr<float>(), nullptr, 0, x, w, 1, (int)(w.size(1) / kRingBK), {}, (float)cap);
+  };
+  const int tt = (int)(x.size(0) + 15) / 16;
+  const bool wide = N / 128 > cus && (N % 256 == 0 || N % 128 != 0);
+  if (wide && (tt == 9 || tt == 10)) go.template operator()<10, 4, 4, 2, 2>();
+  else if (wide && (tt == 13 || tt == 14)) go.template operator()<14, 4, 4, 2, 2>();
+  else ring_tiles(x.size(0), [&]<int TT>() {
+    if (wide) {
+      if constexpr (TT <= 3) go.template operator()<TT, 2, 8, 1, 3>();
+      else if constexpr (TT <= 8) go.template operator()<TT, 4, 4, 2, 3>();
+      else if constexpr (TT == 12) go.template operator()<TT, 4, 4, 2, 2>();
+      else go.template operator()<TT, 8, 2, 4, 2>();
+    } else if (N / 64 > cus) {
+      if constexpr (TT <= 3) go.template operator()<TT, 2, 4, 1, 4>();
+      else if constexpr (TT <= 8) go.template operator()<TT, 4, 2, 2, 3>();
+      else go.template operator()<TT, 4, 2, 4, 3>();
     } else {
-      if constexpr (TT <= 8) go.template operator()<1, 4, 1, 4>();
-      else go.template operator()<2, 2, 4, 4>();
+      if constexpr (TT <= 8) go.template operator()<TT, 1, 4, 1, 4>();
+      else go.template operator()<TT, 2, 2, 4, 4>();
     }
   });
   return out;

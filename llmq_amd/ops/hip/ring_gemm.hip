@@ -98,6 +98,7 @@ __global__ __launch_bounds__(64 * WN * WT * WK) void ring_gemm_kernel(
       const int t = (lr / 16) % RT;
       row = lr / (16 * RT) * (RT * 8) + t % (RT / 2) * 16 + lr % 16 + (t < RT / 2 ? 0 : N / 2);
     }
+    if constexpr (EPI == kRingHead) row = min(row, N - 1 - n0);   // repeat the last row
     woff[j] = ((unsigned)row * (unsigned)K + place(lr)) * 2u;
   }
 #pragma unroll
@@ -203,7 +204,9 @@ __global__ __launch_bounds__(64 * WN * WT * WK) void ring_gemm_kernel(
     if constexpr (!PAIR) {
       float* slab = slabs + ((long)part * M + row) * N + n0 + wn * RT * 16 + grp * 4;
 #pragma unroll
-      for (int a = 0; a < RT; ++a) *reinterpret_cast<rg_f32x4*>(slab + a * 16) = acc[a][m];
+      for (int a = 0; a < RT; ++a)
+        if (EPI != kRingHead || n0 + (wn * RT + a) * 16 < N)   // N is a multiple of 16
+          *reinterpret_cast<rg_f32x4*>(slab + a * 16) = acc[a][m];
     } else {
 #pragma unroll
       for (int a = 0; a < RT / 2; ++a) {

@@ -554,6 +554,17 @@ class TestSlabProjections:
         # fp32 sums of unit size; the cap's slope is at most one
         assert ((got.double() - want).abs() <= 1e-5 * (1 + ref.abs())).all()
 
+    @pytest.mark.parametrize("M", [1, 33, 64, 128, 144, 145, 160, 161, 208, 209, 224, 225])
+    @pytest.mark.parametrize("N", [16448, 32832, 33088, 33152, 33280])
+    def test_head_parts(self, M, N):
+        """Workgroups of 128 and 256 weight rows of which the last has 64, 128 or all; the
+        token counts that only the head has tiles for."""
+        K = 128
+        x = torch.randn(M, K, device=DEV, dtype=torch.bfloat16)
+        w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) * K ** -0.5
+        ref = x.double() @ w.double().t()
+        assert ((ops.head_logits(x, w, 0.0).double() - ref).abs() <= 1e-5 * (1 + ref.abs())).all()
+
     def test_rows_far_apart(self):
         """Rows over 4 GiB from the first: the kernels with 64-bit addresses."""
         flat = torch.zeros((1 << 31) + 256, device=DEV, dtype=torch.bfloat16)
