@@ -861,13 +861,20 @@ at::Tensor ring_head(const at::Tensor& x, const at::Tensor& w, double cap) {
 // come from memory, as a model's layers do, a stage of 64 channels takes 1.27, 1.45 or 1.68 us
 // with tiles of 128, 192 or 256 tokens (0.93, 1.18 and 1.5 from the caches), a tile 2.5 more;
 // all CUs take a tile a round. Against that stand 1.45 PFLOP/s, a pass at 4.5 TB/s and 5 us, what
-// the library's product and an activation come to at their best: up to 1.4 times that over
-// 2048 rows, which hide the weights' way, and below 2048 channels, where the library's tiles
-// fill and drain every few stages; up to 1.05 times else. Measured (us, weights from memory, library + activation / tiles): 1000 rows, 17920 x
-// 1536 82 / 69; 2000, the same 133 / 122; 512, 16384 x 3072 59 / 67 (refused); 1000, the same
-// 92 / 85; 1300, the same 130 / 137 (refused); 768, 16384 x 2048 53 / 50; 2000, the same 121 /
-// 110; 512, 28672 x 3584 96 / 100 (refused); 2000, the same 341 / 370 (refused); 2250, the same
-// 409 / 379; 4096, the same 619 / 623; 2250, 16384 x 3072 201 / 204; 2808, the same 339 / 222.
+// the library's product and an activation come to at their best. They are seldom there: over
+// 2048 rows they reach 800 to 1500 TFLOP/s, from one row count to the next 30 % apart, so that
+// up to 1.4 times that estimate pays up to 6144 channels (27 shapes of 4096 to 73728 rows, 896
+// to 5120 channels, 25 row counts each from 2049 to 8192: 13 % less time on average, at worst
+// 7 % more). At 8192 channels the tiles take 1.5 % more on average. Below 2048 channels the
+// library's tiles fill and drain every few stages: 1.4 at any row count. Else, up to 2048 rows, only where the
+// estimate is near: 1.05, up to 3072 channels. Measured (us, weights from memory, library +
+// activation / tiles): 512 rows, 17920 x 1536 43 / 36; 1000, the same 83 / 69; 768, 16384 x 2048
+// 53 / 51; 1152, the same 86 / 92 (refused); 512, 16384 x 3072 58 / 68 (refused); 1000, the
+// same 91 / 85; 2048, 16384 x 4096 and 73728 x 4608 the library by 4 and 5 % (refused); 2305, 16384
+// x 3072 297 / 213; 28672 x 3584 404 / 419; 57344 x 8192 1646 / 1720 (refused); 2560, 28672 x
+// 3584 418 / 437, 28672 x 4096 459 / 492; 3073, 17920 x 1536 202 / 151, 28672 x 3584 619 / 504;
+// 4200, 16384 x 3072 401 / 350, 28672 x 3584 673 / 682, 59136 x 8192 2886 / 3000 (refused); 8192,
+// 16384 x 3072 629 / 605, 28672 x 3584 1223 / 1229, 57344 x 8192 5139 / 5379 (refused).
 struct TilePlan { int tw; bool worth; };
 
 TilePlan tile_plan(long M, long N, long K, int cus) {
@@ -879,8 +886,9 @@ TilePlan tile_plan(long M, long N, long K, int cus) {
     const double us = (tiles + cus - 1) / cus * (K / kTileBK * stage_us[tw - 2] + 2.5);
     if (best.tw == 0 || us < least) least = us, best.tw = tw;
   }
-  best.worth = least <= (M > 2048 || K < 2048 ? 1.4 : 1.05) *
-                            (2e-9 / 1.45 * M * N * K + M * N * 3 / 4.5e6 + 5);
+  const double library = 2e-9 / 1.45 * M * N * K + M * N * 3 / 4.5e6 + 5;
+  best.worth = M > 2048 || K < 2048 ? K <= 6144 && least <= 1.4 * library
+                                    : K <= 3072 && least <= 1.05 * library;
   return best;
 }
 

@@ -540,6 +540,17 @@ class TestSlabProjections:
                 with pytest.raises(RuntimeError):
                     ops.tile_act_linear(a, b, False)
 
+    def test_tile_rule(self):
+        """Row and channel counts on both sides of the lines."""
+        for M, N, K, ok in ((768, 16384, 2048, True), (2000, 16384, 3072, True),
+                            (2048, 16384, 3136, False), (2049, 16384, 3136, True),
+                            (4096, 16384, 6144, True), (4096, 16384, 6208, False),
+                            (2049, 16384, 8192, False), (512, 16384, 2048, False),
+                            (512, 17920, 1536, True)):
+            x = torch.empty(M, K, device=DEV, dtype=torch.bfloat16)
+            w = torch.empty(N, K, device=DEV, dtype=torch.bfloat16)
+            assert ops.tile_act_ok(x, w) == ok, (M, N, K)
+
     @pytest.mark.parametrize("M", [1, 17, 48, 64, 128, 129, 193, 256])
     @pytest.mark.parametrize("N,K", [(64, 128), (16512, 256), (65792, 128), (128256, 256)])
     @pytest.mark.parametrize("cap", [0.0, 1.5])
