@@ -73,11 +73,19 @@ DEVINL int pd_total(const int* __restrict__ lens, int B, int window, int lane, i
 }
 
 // Tiles per wave: an equal share. One tile while that leaves CUs without work
-// (latency); two from there on, so that short pairs are not cut needlessly; four of
-// head size 64's, which are half as many keys and bytes, beyond that.
+// (latency); two from there on, so that short pairs are not cut needlessly. Head size 64's
+// tiles are half as many keys and bytes: two where pairs of one or two tiles would be cut for
+// nothing and where one would make over 64 pieces of a pair; four beyond 2048 tiles, unless
+// pairs are short and two make one round. Measured (us, with the merge, least share of 1 / 2): 1 x 20 keys, 8 kv
+// heads 6.5 / 7.6, 8 x 60 8.3 / 7.4, 32 ragged up to 50 8.3 / 7.7, 1 x 200 8.6 / 9.4, 1 x 4000, 2 kv heads
+// 12.0 / 10.1; of 2 / 4: 200 ragged up to 100 14.7 / 16.3, 512 x 60 (three, by count) 29.4 / 24.7.
 template <int D>
-DEVINL int pd_share(int total, int waves) {
-  const int least = D == 64 ? (total > 2048 ? 4 : total > 512 ? 2 : 1) : total > 1024 ? 2 : 1;
+DEVINL int pd_share(int total, int waves, int pairs) {
+  int least = total > 1024 ? 2 : 1;
+  if constexpr (D == 64) {
+    if (total > 2048) least = total > 3 * pairs || total > 2 * waves ? 4 : 2;
+    else least = total > 512 || (total > pairs && total <= 2 * pairs) || total > 64 * pairs ? 2 : 1;
+  }
   return max((total + waves - 1) / waves, least);
 }
 
@@ -180,7 +188,7 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
   const int wave = w * gridDim.x + blockIdx.x;
   const int first = lens[min(lane, B - 1)];
   const int total = pd_total<TS>(lens, B, window, lane, first) * KVH;
-  const int share = pd_share<D>(total, waves);
+  const int share = pd_share<D>(total, waves, B * KVH);
   int t = wave * share;
   const int t_end = min(total, t + share);
   if (t >= t_end) return;
@@ -445,7 +453,7 @@ __global__ __launch_bounds__(256) void paged_decode_merge_kernel(
     all += __shfl_xor(all, off, WAVE);
     before += __shfl_xor(before, off, WAVE);
   }
-  const int share = pd_share<D>(all * KVH, waves);
+  const int share = pd_share<D>(all * KVH, waves, B * KVH);
   const int first_tile = before * KVH + (h / G) * nt;
   const int first = first_tile / share, last = (first_tile + nt - 1) / share;
   if (first == last) return;                 // written by its wave

@@ -241,6 +241,25 @@ class TestDecodeRanges:
         # fp32 sums over up to 4000 keys of unit values
         assert_close_to_f32_ref(out.cpu()[live], ref, 2e-4, 2 ** -8)
 
+    @pytest.mark.parametrize("KVH,lens", [
+        (1, [4000]), (1, [2048, 2049]), (3, [33] * 40), (2, [(i * 7) % 64 + 1 for i in range(20)]),
+        (8, [(i * 7) % 100 + 1 for i in range(200)]), (32, [60] * 100), (32, [90] * 100),
+    ])
+    @pytest.mark.parametrize("window", [0, 50])
+    def test_shares_at_head_size_64(self, KVH, lens, window):
+        """Every least share of head size 64: long pairs, pairs of one and two tiles, few and
+        many."""
+        B, G, D = len(lens), 2, 64
+        kc, vc, bt = _build_cache(B, KVH, D, 16, max(lens), torch.bfloat16)
+        ctx = torch.tensor(lens, dtype=torch.int32, device=DEV)
+        q = torch.randn(B, G * KVH, D, device=DEV, dtype=torch.bfloat16)
+        out = ops.paged_decode_attention(q, kc, vc, bt, ctx, D ** -0.5, 0.0, window)
+        ref = torch_ref.paged_decode_attention(
+            q.float().cpu(), kc.float().cpu(), vc.float().cpu(), bt.cpu(), ctx.cpu(), D ** -0.5,
+            0.0, window)
+        # the output's bf16 rounding and fp32 sums of up to 4000 unit values, as above
+        assert_close_to_f32_ref(out.cpu(), ref, 2e-4, 2 ** -8)
+
 
 class TestDecodeWeightBits:
     def test_head_size_64_keeps_fp32_weights(self):
