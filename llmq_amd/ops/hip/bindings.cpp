@@ -684,15 +684,15 @@ void ring_tiles(long M, F&& go) {
 
 // Two weight tiles and one wave column suit few tokens, four and two (four from 129 rows
 // on) the others, whose operand reads from LDS count (128 rows, 3584 x 14336: 25.7 and 26.3).
-template <int TT, int EPI>
+template <int TT, int EPI, bool ROT = false>
 void launch_ring_128(float* slabs, __hip_bfloat16* out, long out_stride, const at::Tensor& x,
                      const at::Tensor& w, int parts, int steps, const SgScale& scale = {}) {
   if constexpr (TT <= 3)
-    launch_ring<TT, 2, 4, 1, 1, 4, EPI, false>(slabs, out, out_stride, x, w, parts, steps, scale);
+    launch_ring<TT, 2, 4, 1, 1, 4, EPI, ROT>(slabs, out, out_stride, x, w, parts, steps, scale);
   else if constexpr (TT <= 8)
-    launch_ring<TT, 4, 2, 2, 1, 3, EPI, false>(slabs, out, out_stride, x, w, parts, steps, scale);
+    launch_ring<TT, 4, 2, 2, 1, 3, EPI, ROT>(slabs, out, out_stride, x, w, parts, steps, scale);
   else
-    launch_ring<TT, 4, 2, 4, 1, 3, EPI, false>(slabs, out, out_stride, x, w, parts, steps, scale);
+    launch_ring<TT, 4, 2, 4, 1, 3, EPI, ROT>(slabs, out, out_stride, x, w, parts, steps, scale);
 }
 
 // slab_gemm.hip: operands out of the ring kernels' reach.
@@ -737,13 +737,18 @@ at::Tensor ring_linear(const at::Tensor& x, const at::Tensor& w) {
   const RingPlan plan = ring_plan(M, N, K, compute_units(x));
   at::Tensor slabs = at::empty({plan.parts, M, N}, opts);
   float* p = slabs.data_ptr<float>();
-  ring_tiles(M, [&]<int TT>() {
+  auto go = [&]<int TT, bool ROT>() {
     if (plan.rows == 128)
-      launch_ring_128<TT, kSlabSums>(p, nullptr, 0, x, w, plan.parts, plan.steps);
+      launch_ring_128<TT, kSlabSums, ROT>(p, nullptr, 0, x, w, plan.parts, plan.steps);
     else if constexpr (TT <= 8)
-      launch_ring<TT, 1, 4, 1, 1, 4, kSlabSums, false>(p, nullptr, 0, x, w, plan.parts, plan.steps);
+      launch_ring<TT, 1, 4, 1, 1, 4, kSlabSums, ROT>(p, nullptr, 0, x, w, plan.parts, plan.steps);
     else
-      launch_ring<TT, 2, 2, 4, 1, 4, kSlabSums, false>(p, nullptr, 0, x, w, plan.parts, plan.steps);
+      launch_ring<TT, 2, 2, 4, 1, 4, kSlabSums, ROT>(p, nullptr, 0, x, w, plan.parts, plan.steps);
+  };
+  const bool rotate = K % 8192 == 0 && N >= 5120 && (M <= 160 || N % 8192 == 0);
+  ring_tiles(M, [&]<int TT>() {
+    if (rotate) go.template operator()<TT, true>();
+    else go.template operator()<TT, false>();
   });
   return slabs;
 }

@@ -26,7 +26,11 @@
 //     of 256000 x 3584: 350 + 27, now 335).
 //   - ROT: workgroups start at different stages. Rows of 4096 bytes start on the same
 //     memory channel, which all workgroups would ask at once (64 rows, 16384 x 2048:
-//     16.2 us, 14.0 with it).
+//     16.2 us, 14.0 with it). Sums take it for many rows of 16 KiB multiples (1 / 192 rows, us,
+//     without / with: 8192 x 8192 39.0 / 30.6 and 45.2 / 39.4, 10240 x 8192 33.2 / 29.6 and 47.8 /
+//     47.9, 8192 x 16384 69.6 / 44.2 and 74.0 / 65.4); for others it is slower, as far as it is
+//     anything: tokens' stages then meet in the L2 no more (4096 x 8192, 48 rows 15.5 / 16.0;
+//     3584 x 14336, 192 rows 33.3 / 41.6; 10240 x 8192, 256 rows 56.7 / 58.3).
 //
 // Measured (us; before = slab_gemm_kernel, from 129 rows on the library's product):
 // 64 rows, 2048 x 8192: 12.4 -> 9.0, 16384 x 2048 pairs 20.3 -> 14.0; 96 rows, 3584 x 14336:

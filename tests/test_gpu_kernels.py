@@ -515,6 +515,17 @@ class TestSlabProjections:
         got = ops.ring_linear(x, w).double().sum(0)
         assert ((got - ref).abs() <= 1e-5 * (1 + ref.abs())).all()     # fp32 sums of unit size
 
+    @pytest.mark.parametrize("M", [1, 17, 33, 96, 128, 160, 161, 256])
+    @pytest.mark.parametrize("N", [5056, 5120, 8192])
+    def test_ring_products_rotated(self, M, N):
+        """Rows of 16 KiB: workgroups that start at different stages, and those that do not."""
+        K = 8192
+        x = torch.randn(M, K, device=DEV, dtype=torch.bfloat16)
+        w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) * K ** -0.5
+        ref = x.double() @ w.double().t()
+        got = ops.ring_linear(x, w).double().sum(0)
+        assert ((got - ref).abs() <= 1e-5 * (1 + ref.abs())).all()     # fp32 sums of unit size
+
     @pytest.mark.parametrize("M", [1, 16, 17, 48, 64, 96, 128, 129, 192, 193, 256])
     @pytest.mark.parametrize("N,K", [(64, 128), (16384, 192 * 2), (16448, 128), (16512, 640),
                                      (33024, 256), (65792, 128)])
