@@ -417,7 +417,8 @@ def slab_ok(x: torch.Tensor, weights, hidden: int, rows: int = SLAB_ROWS) -> boo
     """Whether the slab kernels take these rows (up to ``rows``) and weights [N, K]."""
     return (
         x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= rows
-        and x.dtype == torch.bfloat16 and x.is_contiguous() and hidden <= 8192
+        and x.dtype == torch.bfloat16 and x.is_contiguous() and x.data_ptr() % 16 == 0
+        and hidden <= 8192
         and all(w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] % 128 == 0
                 and w.shape[0] % 64 == 0 and w.data_ptr() % 16 == 0 for w in weights)
     )

@@ -606,6 +606,28 @@ class TestSlabProjections:
         ref = x.double() @ w.double().t()
         assert ((ops.head_logits(x, w, 0.0).double() - ref).abs() <= 1e-5 * (1 + ref.abs())).all()
 
+    @pytest.mark.parametrize("cap", [0.0, 1.5])
+    def test_head_layouts(self, cap):
+        """Rows and weights off a 16-byte boundary, padded, strided or transposed."""
+        M, N, K = 5, 192, 256
+        x = torch.randn(M, K, device=DEV, dtype=torch.bfloat16)
+        w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) * K ** -0.5
+        ref = x.double() @ w.double().t()
+        want = torch.tanh(ref / cap) * cap if cap else ref
+
+        def layouts(t):
+            moved = torch.empty(t.numel() + 4, device=DEV, dtype=t.dtype)[4:].view(t.shape)
+            padded = torch.empty(t.shape[0], K + 8, device=DEV, dtype=t.dtype)[:, :K]
+            strided = torch.empty(t.shape[0], 2 * K, device=DEV, dtype=t.dtype)[:, ::2]
+            turned = torch.empty(K, t.shape[0], device=DEV, dtype=t.dtype).t()
+            return [t] + [v.copy_(t) for v in (moved, padded, strided, turned)]
+
+        for a in layouts(x):
+            for b in layouts(w):
+                got = ops.head_logits(a, b, cap).double()
+                # the library's product is rounded to bf16; the cap's slope is at most one
+                assert ((got - want).abs() <= 2 ** -8 * ref.abs() + 1e-5).all()
+
     def test_rows_far_apart(self):
         """Rows over 4 GiB from the first: the kernels with 64-bit addresses."""
         flat = torch.zeros((1 << 31) + 256, device=DEV, dtype=torch.bfloat16)
