@@ -272,13 +272,9 @@ class CausalLM:
         return attn.reshape(T, self.q_size)
 
     def _forward_slabs(self, h, residual, positions, kv_cache, meta) -> torch.Tensor:
-        """The layers for up to ops.SLAB_ROWS rows (an ordinary decode step, few
-        rows of large layers)."""
-        return self._ring_layers(h, residual, positions, kv_cache, meta)
-
-    def _ring_layers(self, h, residual, positions, kv_cache, meta) -> torch.Tensor:
-        """The layers for up to ops.RING_ROWS rows: streaming products whose partial
-        sums the norms and the rotation add up."""
+        """The layers for up to ops.RING_ROWS rows (an ordinary decode step, few rows of
+        large layers): streaming products whose partial sums the norms and the rotation
+        add up."""
         s = self.spec
         for i, lw in enumerate(self.layers):
             w_next = self.layers[i + 1].input_norm if i + 1 < len(self.layers) else self.final_norm
@@ -373,11 +369,15 @@ class CausalLM:
                 and not _USE_SKINNY_GEMM):
             return self._prompt_layers(h, residual, positions, kv_cache, meta)
         if (tp is None and kv_cache.k[0].dtype in (torch.bfloat16, torch.float8_e4m3fn)
-                and ops.slab_ok(h, (l0.qkv, l0.o, l0.gate_up, l0.down), s.hidden_size,
-                                ops.RING_ROWS)
+                and ops.slab_ok(h, (l0.qkv, l0.o, l0.gate_up, l0.down), s.hidden_size)
                 and not _USE_SKINNY_GEMM):
-            layers = self._forward_slabs if len(h) <= ops.SLAB_ROWS else self._ring_layers
-            return layers(h, residual, positions, kv_cache, meta)
+            return self._forward_slabs(h, residual, positions, kv_cache, meta)
+        return self._forward_general(h, residual, positions, kv_cache, meta)
+
+    def _forward_general(self, h, residual, positions, kv_cache, meta) -> torch.Tensor:
+        """The layers for any number of rows, weights and ranks, operation by operation."""
+        s = self.spec
+        tp = get_tp_group() if self.tp_size > 1 else None
         n_layers = len(self.layers)
         for i, lw in enumerate(self.layers):
             # ---- attention block (h = normed input, set by the previous

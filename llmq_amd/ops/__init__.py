@@ -409,14 +409,13 @@ class FewRows:
 # The product stays as fp32 partial sums ("slabs" [parts, M, N]) that the next
 # kernel adds up: norm and residual, or rotation and cache write.
 
-SLAB_ROWS = 128
 RING_ROWS = 256
 
 
-def slab_ok(x: torch.Tensor, weights, hidden: int, rows: int = SLAB_ROWS) -> bool:
-    """Whether the slab kernels take these rows (up to ``rows``) and weights [N, K]."""
+def slab_ok(x: torch.Tensor, weights, hidden: int) -> bool:
+    """Whether the slab kernels take these rows (up to RING_ROWS) and weights [N, K]."""
     return (
-        x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= rows
+        x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= RING_ROWS
         and x.dtype == torch.bfloat16 and x.is_contiguous() and x.data_ptr() % 16 == 0
         and hidden <= 8192
         and all(w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] % 128 == 0
@@ -431,8 +430,9 @@ def ring_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 def ring_act_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether ring_act_linear beats the library's product and an activation."""
-    return x.shape[0] <= 192 or w.shape[0] <= 32768
+    """Whether ring_act_linear takes these rows and beats the library's product and an
+    activation."""
+    return _use_hip(x) and _EXT.ring_act_ok(x, w)
 
 
 def ring_act_linear(x: torch.Tensor, w: torch.Tensor, gelu: bool) -> torch.Tensor:
@@ -459,20 +459,15 @@ def head_logits(x: torch.Tensor, w: torch.Tensor, cap: float) -> torch.Tensor:
     up to RING_ROWS rows. Measured, us, weights from memory, against the library's product
     and a pass over it: 256 rows, 256000 x 3584 468 and 493, 128256 x 4096 256 and 354; 129
     rows, 256000 x 3584 419 and 412 (rounded to bf16 on the way, error 1.7e-3; here 4e-7)."""
-    if _use_hip(x) and slab_ok(x, (w,), 0, RING_ROWS) and w.shape[1] < 1 << 22:
+    if _use_hip(x) and slab_ok(x, (w,), 0) and w.shape[1] < 1 << 22:
         return _EXT.ring_head(x, w, float(cap or 0.0))
     return softcap_logits(torch.nn.functional.linear(x, w), cap)
 
 
 def slab_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """ring_linear for up to SLAB_ROWS rows."""
+    """ring_linear for up to 128 rows."""
     assert _use_hip(x)
     return _EXT.slab_linear(x, w)
-
-
-def slab_act_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether slab_act_linear beats the library's product and an activation."""
-    return x.shape[0] <= 64
 
 
 def slab_act_linear(x: torch.Tensor, w: torch.Tensor, gelu: bool) -> torch.Tensor:

@@ -1523,6 +1523,7 @@ TORCH_LIBRARY(llmq_amd, m) {
   m.def("slab_linear(Tensor x, Tensor w) -> Tensor");
   m.def("ring_linear(Tensor x, Tensor w) -> Tensor");
   m.def("ring_head(Tensor x, Tensor w, float cap) -> Tensor");
+  m.def("ring_act_ok(Tensor x, Tensor w) -> bool");
   m.def("ring_act_linear(Tensor x, Tensor w, bool gelu) -> Tensor");
   m.def("slab_act_linear(Tensor x, Tensor w, bool gelu) -> Tensor");
   m.def("slab_add_norm(Tensor slabs, Tensor(a!) residual, Tensor? w_post, Tensor w, float eps, float offset) -> Tensor");
@@ -1558,6 +1559,7 @@ TORCH_LIBRARY_IMPL(llmq_amd, CUDA, m) {
   m.impl("tile_act_linear", &tile_act_linear);
   m.impl("ring_linear", &ring_linear);
   m.impl("ring_head", &ring_head);
+  m.impl("ring_act_ok", &ring_act_ok);
   m.impl("ring_act_linear", &ring_act_linear);
   m.impl("slab_act_linear", &slab_act_linear);
   m.impl("slab_add_norm", &slab_add_norm);

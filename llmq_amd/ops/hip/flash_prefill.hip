@@ -45,7 +45,7 @@ typedef __attribute__((address_space(3))) fp_bf16x4 fp_lds_bf16x4;
 // 16 bytes per lane from memory to LDS (lane-linear from a uniform LDS address, in
 // M0), in inline asm: with the builtin the compiler waits for all of them before
 // the first LDS read that may alias, which would drain the next tile's loads.
-// pipe_barrier_vm is the only wait for them.
+// The waits that count them (pipe_barrier_vm, stream_wait) are the only ones.
 DEVINL void glds16(const void* src, void* lds_dst_uniform) {
   unsigned lds_off = (unsigned)(unsigned long)(
       (__attribute__((address_space(3))) char*)lds_dst_uniform);

@@ -2,11 +2,11 @@
 // for operands that ring_gemm.hip cannot reach with 32-bit offsets (rows spread over
 // 4 GiB). And the kernels that add up the slabs of either.
 //
-// A workgroup owns 64 weight rows, all M tokens and one
-// of S parts of K. Weights go straight from memory into the matrix layout; the tokens,
-// which every workgroup reads again, are staged once per workgroup in LDS by
-// global_load_lds (16-byte granules placed by row, so operand reads meet no bank
-// conflict). v_mfma_f32_16x16x32_bf16, A = weights (row = lane%16, k =
+// A workgroup owns 64 weight rows, all M tokens and, as it is launched, all of K (a grid
+// of several parts in y would leave a slab each). Weights go straight from memory into the
+// matrix layout; the tokens, which every workgroup reads again, are staged once per
+// workgroup in LDS by global_load_lds (16-byte granules placed by row, so operand reads
+// meet no bank conflict). v_mfma_f32_16x16x32_bf16, A = weights (row = lane%16, k =
 // 8*(lane/16)..+7), B = tokens likewise, C: column = token, rows = 4 weight rows.
 // A step of 128 channels asks for the next step's tokens at its start and for the
 // weights of the one after at its end, but its products wait for both: the loads sit
@@ -24,7 +24,7 @@ enum : int { kSlabSums = 0, kSlabSilu = 1, kSlabGelu = 2 };
 constexpr int kSlabBK = 128;
 
 // TM: token tiles of 16; WK: groups of four waves that take the K steps in turn (gate
-// and value rows, whose sums have to be whole; else parts of K do that).
+// and value rows).
 template <int TM, int WK, int EPI>
 __global__ __launch_bounds__(256 * WK) void slab_gemm_kernel(
     float* __restrict__ slabs, __hip_bfloat16* __restrict__ out, long out_stride,

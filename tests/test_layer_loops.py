@@ -1,7 +1,7 @@
 """The layer loops of the Llama, Qwen2 and Gemma-2 families against a 64-bit
-forward pass: few rows (few_rows), up to 128 (slabs), prompts launched from
-native code (prompt_layers) and the per-operation loop, for decode steps, whole
-prompts, portions that continue a cached context and mixed steps. Three layers of
+forward pass: few rows (few_rows), up to 256 (slabs), prompts launched from
+native code (prompt_layers) and the per-operation loop, with tiles and without, for
+decode steps, whole prompts, portions that continue a cached context and mixed steps. Three layers of
 sizes that the streaming kernels take, norm weights and biases that differ
 everywhere, so that a swapped or missing one shows.
 """
@@ -235,15 +235,36 @@ def _expected(kind, rows, fp8):
         return ["few"]
     if kind == "prompt" or (kind == "portion" and not fp8):   # fp8 portions are gathered
         return ["native"]
-    return ["slabs"] if rows <= 128 else []
+    return ["slabs"] if rows <= 256 else []
+
+
+@pytest.fixture()
+def products(monkeypatch):
+    """The streaming and tile products that the Python loops call."""
+    taken = []
+    for op, short in (("ring_linear", "ring"), ("ring_act_linear", "ring_act"),
+                      ("tile_act_linear", "tile")):
+        def spy(*args, _f=getattr(ops, op), _short=short):
+            taken.append(_short)
+            return _f(*args)
+        monkeypatch.setattr(ops, op, spy)
+    return taken
+
+
+def _expected_products(name, rows):
+    """Over 16 rows, three layers. Tiles pay from some 540 rows of llama's and gemma2's 768
+    gate and value rows on, from 1440 of qwen2's 1280."""
+    if rows <= 256:
+        return ["ring", "ring", "ring_act", "ring"] * 3
+    return ["tile"] * 3 if rows >= 600 and name != "qwen2" else []
 
 
 @on_gpu
-@pytest.mark.parametrize("rows", [1, 5, 16, 17, 65, 128, 129])
+@pytest.mark.parametrize("rows", [1, 5, 16, 17, 65, 128, 129, 192, 256, 257, 600])
 @pytest.mark.parametrize("kind", ["decode", "prompt", "portion", "mixed"])
 @pytest.mark.parametrize("name,fp8", [("llama", False), ("qwen2", False), ("gemma2", False),
                                       ("qwen2", True), ("gemma2", True)])
-def test_loops_vs_64_bits(name, fp8, kind, rows, loops, monkeypatch):
+def test_loops_vs_64_bits(name, fp8, kind, rows, loops, products, monkeypatch):
     if kind == "mixed":
         rows = max(rows, 2)
     model = _model(name, "cuda", torch.bfloat16)
@@ -253,10 +274,13 @@ def test_loops_vs_64_bits(name, fp8, kind, rows, loops, monkeypatch):
     got = _run(model, cache, batch)
     assert loops == _expected(kind, rows, fp8)
     assert _off(got, want) < LIMIT
-    if loops == ["native"] and rows <= 128:
-        # its streaming products: the same launches as the slab loop's
-        monkeypatch.setattr(CausalLM, "_prompt_layers", CausalLM._forward_slabs)
-        assert torch.equal(_run(model, cache, batch), got) and loops[1:] == ["slabs"]
+    if loops == ["native"]:
+        # the same launches as the slab loop's, or as the per-operation loop's
+        monkeypatch.setattr(CausalLM, "_prompt_layers", CausalLM._forward_slabs if rows <= 256
+                            else CausalLM._forward_general)
+        assert torch.equal(_run(model, cache, batch), got)
+        assert loops[1:] == (["slabs"] if rows <= 256 else [])
+    assert products == ([] if rows <= 16 else _expected_products(name, rows))
 
 
 @on_gpu
