@@ -557,6 +557,20 @@ class TestSlabProjections:
                 tol = 2 ** -8 * (act * u).abs() + 3e-5 * (1 + g.abs()) * (1 + u.abs())
                 assert ((y - act * u).abs() <= tol).all()
 
+    @pytest.mark.parametrize("M,N,K", [(1153, 17920, 640), (2000, 16384, 1088), (1025, 33024, 576),
+                                       (5000, 4096, 768)])
+    def test_tile_rounds(self, M, N, K):
+        """Several tiles a workgroup, from whose first stage each XCD keeps a distance of its
+        own: nine stages and more."""
+        x = torch.randn(M, K, device=DEV, dtype=torch.bfloat16)
+        w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) * K ** -0.5
+        y = ops.tile_act_linear(x, w, False)
+        for rows in range(0, M, 512):                    # the reference in pieces
+            g, u = (x[rows:rows + 512].double() @ w.double().t()).chunk(2, -1)
+            want = torch.nn.functional.silu(g) * u
+            tol = 2 ** -8 * want.abs() + 3e-5 * (1 + g.abs()) * (1 + u.abs())
+            assert ((y[rows:rows + 512].double() - want).abs() <= tol).all()
+
     def test_tile_refuses(self):
         """What the tiles cannot take is left to the library."""
         x = torch.randn(1024, 256, device=DEV, dtype=torch.bfloat16)
@@ -640,6 +654,31 @@ class TestSlabProjections:
         g, u = ref.chunk(2, -1)
         y, want = ops.slab_act_linear(x, w, False).double(), torch.nn.functional.silu(g) * u
         assert ((y - want).abs() <= 2 ** -8 * want.abs() + 3e-5 * (1 + g.abs()) * (1 + u.abs())).all()
+
+    @pytest.mark.parametrize("M", [2, 16, 17, 33, 49, 64, 65, 97, 128, 129])
+    def test_rows_far_apart_tiles(self, M):
+        """Every token-tile count of the kernels with 64-bit addresses; the library's product
+        beyond their rows."""
+        N, K = 192, 384
+        stride = -(-(1 << 31) // (M - 1) // 8) * 8
+        x = torch.zeros((M - 1) * stride + K, device=DEV, dtype=torch.bfloat16).as_strided(
+            (M, K), (stride, 1))
+        x.normal_()
+        w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) * K ** -0.5
+        ref = x.double() @ w.double().t()
+        got = ops.ring_linear(x, w)
+        assert got.shape[0] == 1
+        tol = 1e-5 if M <= 128 else 2 ** -8              # the library's is rounded to bf16
+        assert ((got.double().sum(0) - ref).abs() <= tol * (1 + ref.abs())).all()
+        g, u = ref.chunk(2, -1)
+        for gelu in (False, True):
+            act = torch.nn.functional.gelu(g, approximate="tanh") if gelu \
+                else torch.nn.functional.silu(g)
+            # over 64 rows gates and values are rounded to bf16 before the activation
+            own = 3e-5 * (1 + g.abs()) * (1 + u.abs()) if M <= 64 else \
+                2 ** -8 * (1 + g.abs()) * (1 + u.abs())
+            y = ops.ring_act_linear(x, w, gelu).double()
+            assert ((y - act * u).abs() <= 2 ** -8 * (act * u).abs() + own).all()
 
     @pytest.mark.parametrize("S,M,N", [(1, 1, 64), (16, 5, 8192), (1, 17, 64), (3, 20, 1000), (16, 64, 2048), (2, 128, 8192)])
     @pytest.mark.parametrize("post", [False, True])
@@ -888,6 +927,24 @@ class TestFewRowsChain:
             assert ((got - want).abs() <= tol).all()
             assert torch.equal(kc.view(32, D)[slots], got[:, 3].bfloat16())
             assert torch.equal(vc.view(32, D)[slots], got[:, 4].bfloat16())
+
+    @pytest.mark.parametrize("M", [1, 8, 12, 16])
+    def test_many_sums(self, M):
+        """Rows of 16384 channels: from 13 rows on more sums than a workgroup holds beside
+        its operands, which scales them ahead of the product."""
+        H, N = 16384, 192
+        bf = dict(device=DEV, dtype=torch.bfloat16)
+        rows = ops.FewRows(torch.randn(M, H, **bf), 1e-5, 0.0)
+        rows.add(torch.randn(M, 128, **bf), torch.randn(H, 128, **bf) / 12, torch.ones(H, **bf))
+        r = rows.residual.double()
+        h = r * torch.rsqrt(r.square().mean(-1, keepdim=True) + 1e-5)
+        gu = torch.randn(N, H, **bf) * H ** -0.5
+        g, u = (h @ gu.double().t()).chunk(2, -1)
+        want = torch.nn.functional.silu(g) * u
+        # scaled ahead, rows are rounded to bf16: 2^-9 3^-0.5 rms of unit sums, five times that
+        own = 5 * 2 ** -9 * 3 ** -0.5 if M > 12 else 1e-5
+        tol = 2 ** -8 * want.abs() + own * (1.2 * g.abs() + u.abs()) + 1e-5
+        assert ((rows.act(gu, False).double() - want).abs() <= tol).all()
 
     @pytest.mark.parametrize("M", [1, 8, 9, 16])
     @pytest.mark.parametrize("N,K", [(5120, 128), (5184, 128), (8192, 1536), (8256, 1536),

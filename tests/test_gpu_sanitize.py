@@ -5,9 +5,10 @@ checked directly: inputs and outputs are carved out of over-allocated
 buffers with canary halos on both sides, and the halos are verified bitwise
 after each op. Run under ``AMD_SERIALIZE_KERNEL=3`` (tests/sanitize_gpu.sh)
 so any kernel fault aborts at the offending launch instead of surfacing
-later. Not covered: OOB READS (those surface as faults under serialized
-launches or as numerics failures in test_gpu_kernels), and tensors that an
-op allocates itself (the slab products, their readers' bf16 rows, scratch).
+later. Outputs of over 1 MiB that an op allocates itself are led to the start of
+a block filled with canaries (``led``). Not covered: OOB READS (those surface as
+faults under serialized launches or as numerics failures in test_gpu_kernels),
+what lies below such an output, smaller ones (the slabs' readers' bf16 rows) and scratch.
 """
 
 from __future__ import annotations
@@ -61,6 +62,22 @@ class Guarded:
             hi = raw[(PAD + n) * esz:]
             assert bool((lo == CANARY).all()), f"buffer {i}: LOW canary clobbered"
             assert bool((hi == CANARY).all()), f"buffer {i}: HIGH canary clobbered"
+
+
+def led(op):
+    """op's output, which it allocates itself, from the start of a block of canaries; nothing
+    behind it may change."""
+    size = 256 << 20
+    with torch.cuda.use_mem_pool(torch.cuda.MemPool()):
+        block = torch.full((size,), CANARY, dtype=torch.uint8, device=DEV)
+        at = block.data_ptr()
+        del block
+        out = op()
+        used = -(-out.nbytes // 512) * 512   # the allocator's rounding
+        rest = torch.empty(size - used, dtype=torch.uint8, device=DEV)
+    assert out.nbytes > 1 << 20 and out.data_ptr() == at and rest.data_ptr() == at + used
+    assert bool((rest == CANARY).all()), "written behind the output"
+    return out
 
 
 @pytest.fixture()
@@ -166,6 +183,71 @@ def test_slab_products_guarded(g, M, D, H, KVH, fp8):
     if M <= 64:
         for gelu in (False, True):
             assert ops.slab_act_linear(x, g.tensor(128, K), gelu).isfinite().all()
+
+
+@pytest.mark.parametrize("M", [33, 65, 128, 129, 192, 193, 256])
+@pytest.mark.parametrize("N,K", [(16384, 640), (4160, 8192), (5120, 8192)])
+def test_ring_products_guarded(g, M, N, K):
+    x, w = g.tensor(M, K), g.tensor(N, K)
+    assert led(lambda: ops.ring_linear(x, w)).isfinite().all()
+
+
+@pytest.mark.parametrize("M", [33, 96, 129, 161, 193, 256])
+@pytest.mark.parametrize("N", [33152, 65792, 65600])
+def test_ring_pairs_guarded(g, M, N):
+    """64, 128 and 256 weight rows a workgroup."""
+    x, w = g.tensor(M, 256), g.tensor(N, 256)
+    for gelu in (False, True):
+        assert led(lambda: ops.ring_act_linear(x, w, gelu)).isfinite().all()
+
+
+@pytest.mark.parametrize("M", [17, 48, 128, 144, 160, 192, 224, 256])
+@pytest.mark.parametrize("N", [16384, 16448, 32832, 33088, 33280])
+def test_head_guarded(g, M, N):
+    """Workgroups of which the last has fewer weight rows, and token tiles of every width."""
+    x, w = g.tensor(M, 256), g.tensor(N, 256)
+    for cap in (0.0, 30.0):
+        out = led(lambda: ops.head_logits(x, w, cap))
+        assert out.dtype == torch.float32 and out.isfinite().all()
+
+
+@pytest.mark.parametrize("M", [257, 300, 700, 1153])
+@pytest.mark.parametrize("N,K", [(4096, 64), (5376, 576)])
+def test_tiles_guarded(g, M, N, K):
+    x, w = g.tensor(M, K), g.tensor(N, K)
+    for gelu in (False, True):
+        assert led(lambda: ops.tile_act_linear(x, w, gelu)).isfinite().all()
+
+
+@pytest.mark.parametrize("M", [1, 5, 9, 16])
+@pytest.mark.parametrize("H,K", [(128, 384), (2048, 128), (4352, 256)])
+@pytest.mark.parametrize("D,fp8", [(64, False), (128, True)])
+def test_few_rows_chain_guarded(g, M, H, K, D, fp8):
+    """What the steps of a layer of few rows hand each other, and the cache rows."""
+    from llmq_amd.ops import torch_ref
+
+    parts = -(-H // 8 // 4) * 4              # sums of a row: workgroups of 8 rows and more
+    residual, rows = g.tensor(M, H), g.tensor(M, H, fill="zeros")
+    kc, vc = (g.tensor(2, 1, 16, D, dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16)
+              for _ in range(2))
+    cs = g.from_values(torch_ref.build_rope_cache(64, D, 10000.0, DEV), torch.float32)
+    pos, slots = (g.from_values(torch.arange(M), torch.int64) for _ in range(2))
+    for norm in (g.tensor(H), None):
+        # sums to their last element: as many as this step leaves
+        first = g.tensor(4 * M, dtype=torch.float32)
+        assert ops._EXT.few_prep(residual, g.tensor(H), 1.0, rows, first) == 1
+        sq, n = first, 1
+        for _ in range(2):
+            assert ops._EXT.few_qkv(rows, sq, n, 1e-5, g.tensor(3 * D, H), g.tensor(3 * D), kc, vc,
+                                    pos, cs, slots).isfinite().all()
+            for N in (96, 16512):
+                assert ops._EXT.few_act(rows, sq, n, 1e-5, g.tensor(N, H), False).isfinite().all()
+            sq = g.tensor(M * parts, dtype=torch.float32)
+            n = ops._EXT.few_add(g.tensor(M, K), g.tensor(H, K), residual, norm, 1.0, rows, sq)
+            if norm is None:
+                break
+            assert 0 < n <= H // 8
+    assert residual.isfinite().all()
 
 
 def test_elementwise_and_cache_guarded(g):
