@@ -998,13 +998,14 @@ void finish_product(at::Tensor out, const at::Tensor& y, long epi) {
 // many workgroups, a last round that is no small one, and rows whose starts spread over the
 // memory channels: multiples of 1 KiB do so badly without the start of its own that a
 // workgroup of 64 rows takes, of 4 KiB worse, of 16 KiB in any form. From nine tokens on,
-// which the pairs read again for every 16 rows, it wins more. Measured (us, ring / pairs): 1 token, 2048 x
-// 2048 8.2 / 3.8, 2048 x 8192 25.3 / 8.0, 8192 x 3072 13.8 / 10.2, 9728 x 896 6.0 / 6.3, 12288 x
-// 4096 19.7 / 20.5, 16384 x 2048 13.7 / 14.4, 16384 x 8192 62 / 48, 16448 x 3072 26.9 / 21.4,
-// 17920 x 1536 14.2 / 12.9, 18432 x 2304 17.9 / 18.2, 24576 x 896 10.1 / 11.2, 28672 x 2048 26.6 / 23.3,
-// 28672 x 3584 36.0 / 37.3, 37888 x 3584 53 / 46; 9 tokens, 4096 x 896 5.2 / 3.7, 6144 x 896 5.4 /
-// 5.7, 8192 x 3072 14.9 / 12.2, 9728 x 3072 14.4 / 15.7, 16448 x 3072 26.9 / 24.5, 24640 x 2048
-// 21.8 / 24.9, 17920 x 1536 14.5 / 16.1, 28672 x 3584 35.7 / 42.4, 57344 x 8192 187 / 150.
+// which the pairs read again for every 16 rows, it wins more. Measured (us, ring / pairs): 1
+// token, 2048 x 2048 8.2 / 3.8, 2048 x 8192 25.3 / 8.0, 8192 x 3072 13.8 / 10.2, 9728 x 896
+// 6.0 / 6.3, 12288 x 4096 19.7 / 20.5, 16384 x 2048 13.7 / 14.4, 16384 x 8192 62 / 48, 16448 x
+// 3072 26.9 / 21.4, 17920 x 1536 14.2 / 12.9, 18432 x 2304 17.9 / 18.2, 24576 x 896 10.1 /
+// 11.2, 28672 x 2048 26.6 / 23.3, 28672 x 3584 36.0 / 37.3, 37888 x 3584 53 / 46; 9 tokens,
+// 4096 x 896 5.2 / 3.7, 6144 x 896 5.4 / 5.7, 8192 x 3072 14.9 / 12.2, 9728 x 3072 14.4 /
+// 15.7, 16448 x 3072 26.9 / 24.5, 24640 x 2048 21.8 / 24.9, 17920 x 1536 14.5 / 16.1, 28672 x
+// 3584 35.7 / 42.4, 57344 x 8192 187 / 150.
 bool pairs_in_ring(long M, long N, long K, long cus) {
   const bool many = M > 8;
   if (N % 64 != 0 || N <= (many && K < 1536 ? 20 : 32) * cus || K >= 8192) return false;

@@ -76,15 +76,19 @@ DEVINL int pd_total(const int* __restrict__ lens, int B, int window, int lane, i
 // (latency); two from there on, so that short pairs are not cut needlessly. Head size 64's
 // tiles are half as many keys and bytes: two where pairs of one or two tiles would be cut for
 // nothing and where one would make over 64 pieces of a pair; four beyond 2048 tiles, unless
-// pairs are short and two make one round. Measured (us, with the merge, least share of 1 / 2): 1 x 20 keys, 8 kv
-// heads 6.5 / 7.6, 8 x 60 8.3 / 7.4, 32 ragged up to 50 8.3 / 7.7, 1 x 200 8.6 / 9.4, 1 x 4000, 2 kv heads
-// 12.0 / 10.1; of 2 / 4: 200 ragged up to 100 14.7 / 16.3, 512 x 60 (three, by count) 29.4 / 24.7.
+// pairs are short and two make one round. Measured (us, with the merge, least share of 1 / 2):
+// 1 x 20 keys, 8 kv heads 6.5 / 7.6, 8 x 60 8.3 / 7.4, 32 ragged up to 50 8.3 / 7.7, 1 x 200
+// 8.6 / 9.4, 1 x 4000, 2 kv heads 12.0 / 10.1; of 2 / 4: 200 ragged up to 100 14.7 / 16.3,
+// 512 x 60 (three, by count) 29.4 / 24.7.
 template <int D>
 DEVINL int pd_share(int total, int waves, int pairs) {
   int least = total > 1024 ? 2 : 1;
   if constexpr (D == 64) {
-    if (total > 2048) least = total > 3 * pairs || total > 2 * waves ? 4 : 2;
-    else least = total > 512 || (total > pairs && total <= 2 * pairs) || total > 64 * pairs ? 2 : 1;
+    // without branches: 1 x 200 keys 8.1 us with them, 7.9 so
+    const bool two = total > 512 || (unsigned)(total - pairs - 1) < (unsigned)pairs ||
+                     total > 64 * pairs;
+    const bool four = total > 2048 && (total > 3 * pairs || total > 2 * waves);
+    least = 1 + two + 2 * four;
   }
   return max((total + waves - 1) / waves, least);
 }
