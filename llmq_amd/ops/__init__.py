@@ -313,13 +313,16 @@ def few_rows_ok(x: torch.Tensor, weights) -> bool:
 
 def few_rows_limit(layer_weights: int) -> int:
     """Rows up to which few_rows_linear serves a layer of that many weights. Its
-    workgroups own 4 to 16 weight rows and each reads all tokens again, at 16 rows as
-    many bytes as weights: the larger the matrices, the sooner that is more than the
-    launches that it saves. Beyond, the slab kernels (64 weight rows a workgroup).
-    Measured, us for six layers, few-row / slab loop: 61 M weights a layer, 8 rows 416 /
-    414, 14 rows 478 / 432; 101 M, 6 rows 581 / 580, 8 rows 625 / 588; 218 M, 4 rows
-    860 / 878, 8 rows 937 / 908; 487 M, 1 row 1648 / 1396, 4 rows 1845 / 1479; 877 M,
-    1 row 2302 / 2448, 2 rows 2368 / 2460, 16 rows 3220 / 2490 (the library's 2592)."""
+    workgroups own 8 or 16 weight rows and each reads all tokens again: the more rows, the
+    sooner that is more than the launches that it saves. Beyond, the slab loop, whose
+    workgroups own 64 weight rows and more. Measured, us a layer, few-row / slab loop: 47 M
+    weights a layer, 12 rows 48.9 / 49.2, 16 rows 51.6 / 49.0; 61 M, 8 rows 41.5 / 49.4, 16 rows
+    49.9 / 49.9; 101 M, 7 rows 56.9 / 64.0, 15 rows 65.3 / 65.6; 198 M (norms behind the products,
+    too) 4 rows 92.4 / 94.4, 10 rows 97.3 / 97.2; 218 M, 3 rows 92.9 / 100.1, 14 rows 103.1 / 102.8;
+    487 M, 2 rows 185 / 187, 3 rows 187 / 179; 566 M (such norms), 2 rows 212 / 238, 8 rows 232 /
+    243, 9 rows 276 / 245; 877 M, 2 rows 302 / 355, 13 rows 353 / 356. So the line lies where
+    the few-row loop is the faster one, but for 13 rows and more of layers under 60 M
+    weights; in most layers it would still be past the line, up to 8 to 15 rows."""
     return max(2, 800_000_000 // max(layer_weights, 1))
 
 
@@ -334,7 +337,8 @@ def few_rows_linear(
     residual: Optional[torch.Tensor] = None,  # [M, N]: added to in place and returned
 ) -> torch.Tensor:
     """out = rmsnorm(x) @ w.T (+ bias), activated or added to the residual, in
-    one launch that streams the weights once (w = [gate | up] rows with act)."""
+    one launch that streams the weights once (w = [gate | up] rows with act) and, with
+    norm, one ahead of it."""
     if _use_hip(x):
         cols = w.shape[0] // 2 if act else w.shape[0]
         out = residual if residual is not None else torch.empty(
@@ -355,7 +359,7 @@ def few_rows_qkv(
     k_cache: torch.Tensor, v_cache: torch.Tensor, positions: torch.Tensor,
     cos_sin: torch.Tensor, slot_mapping: torch.Tensor,
 ) -> torch.Tensor:
-    """few_rows_linear for q/k/v weights, then rope_and_cache, in one launch:
+    """few_rows_linear for q/k/v weights, then rope_and_cache, in the same launch:
     returns the rows [M, q+2kv] with q and k rotated."""
     if (_use_hip(x) and k_cache.shape[3] % 16 == 0
             and k_cache.dtype in (torch.bfloat16, torch.float8_e4m3fn)):

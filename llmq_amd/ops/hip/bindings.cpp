@@ -303,9 +303,10 @@ void launch_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor& kc,
     };
     using BF = __hip_bfloat16;
     using F8 = __hip_fp8_e4m3;
-    // 32 keys a tile at head size 64 (us, with the merge, 64 / 32: 1 x 200 keys, 8 kv heads 9.3
-    // / 8.1; 1 x 3000 11.2 / 10.4; 8 ragged up to 1000 10.2 / 10.4; 64 x 1040 35.2 / 34.1; 6
-    // ragged up to 15000 34.8 / 33.6). At 128 64 keys and one workgroup a CU gain on 3 ragged up
+    // 32 keys a tile at head size 64 (us, with the merge, 64 / 32: 1 x 200 keys, 8 kv heads 9.1
+    // / 7.9; 1 x 3000 11.2 / 10.4; 8 ragged up to 1000 10.2 / 10.4; 64 x 300 16.7 / 15.9; 6
+    // ragged up to 15000 34.8 / 33.6; 64 x 1040 35.7 / 36.8 call after call, but 1.3 less a
+    // layer between the products of a step: llama-3.2-1b 1440 / 1420). At 128 64 keys and one workgroup a CU gain on 3 ragged up
     // to 16000 (34.4 / 32.2) what they lose on 60 up to 800 (31.9 / 32.5).
     if (D == 64) go.template operator()<64, BF, 2, 3>();
     else if (D == 128 && !fp8) go.template operator()<128, BF, 2, 2>();

@@ -195,7 +195,9 @@ DEVINL Vec4<__hip_bfloat16> slab_store(__hip_bfloat16* p, sl_f32x4 y) {
 // Measured (us, with weights read behind the sums, three barriers a sum and rounds of eight
 // slabs -> now; a sequence of such launches): 96 rows of 3584, 9 slabs, two norms 6.8 -> 5.7;
 // 48 rows 6.4 -> 5.5; 189 rows of 3072, 10 slabs 7.5 -> 6.9; 64 rows of 2048, 8 slabs 3.8,
-// as before (with 512 channels a wave instead of 256 4.5).
+// as before (with 512 channels a wave instead of 256 4.5). Slabs that the same L2 still holds
+// from the launch before hide that: 64 rows of 3072, 8 slabs 4.4 -> 4.8; behind the products that
+// write them whole layers take 0 to 2 % less.
 constexpr int kSlabNT = 1024;
 
 // x plus the x of the lane that DPP control `CTRL` names, in the rows of 16 that ROWS has.
