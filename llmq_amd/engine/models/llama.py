@@ -276,6 +276,7 @@ class CausalLM:
         large layers): streaming products whose partial sums the norms and the rotation
         add up."""
         s = self.spec
+        own_gates = ops.ring_act_ok(h, self.layers[0].gate_up)  # all layers' have one shape
         for i, lw in enumerate(self.layers):
             w_next = self.layers[i + 1].input_norm if i + 1 < len(self.layers) else self.final_norm
             qkv = ops.slab_rope_cache(
@@ -285,7 +286,7 @@ class CausalLM:
             attn = self._attention(i, qkv, positions, kv_cache, meta, cached=True)
             h = ops.slab_add_norm(ops.ring_linear(attn, lw.o), residual, lw.post_attn_norm,
                                   lw.pre_mlp_norm, s.rms_eps, self.norm_offset)
-            if ops.ring_act_ok(h, lw.gate_up):
+            if own_gates:
                 act = ops.ring_act_linear(h, lw.gate_up, s.gelu)
             else:
                 gate_up = _proj(h, lw.gate_up)
