@@ -38,18 +38,20 @@
 // Sequential over tokens: where a portion starts cannot change a sum's order.
 constexpr int kDeltaTB = 16;
 
+// x plus the x of the lane that CTRL names: every source lane lies in the row, so the add takes
+// it as its own operand (common.h's dpp_add keeps a zero for lanes without one)
 template <int CTRL>
-DEVINL float dpp_add(float x) {
+DEVINL float delta_dpp_add(float x) {
   return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
 }
 
 // sum over the 16 lanes of a DPP row, in every lane: quad permutes (xor 1,
 // xor 2), then mirrors of half rows and rows, whose sources hold equal sums
 DEVINL float row16_sum(float x) {
-  x = dpp_add<0xB1>(x);
-  x = dpp_add<0x4E>(x);
-  x = dpp_add<0x141>(x);
-  return dpp_add<0x140>(x);
+  x = delta_dpp_add<0xB1>(x);
+  x = delta_dpp_add<0x4E>(x);
+  x = delta_dpp_add<0x141>(x);
+  return delta_dpp_add<0x140>(x);
 }
 
 template <bool FAST>
