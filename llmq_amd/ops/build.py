@@ -77,9 +77,9 @@ def build(verbose: bool = False, force: bool = False, group: str = "main") -> Pa
 
     BUILD_DIR.mkdir(exist_ok=True)
 
-    def _load() -> None:
+    def _load(name: str) -> None:
         load(
-            name=ext_name,
+            name=name,
             sources=[str(SRC)],
             extra_cflags=["-O3", "-std=c++20"],
             extra_cuda_cflags=HIPCC_FLAGS,
@@ -89,13 +89,17 @@ def build(verbose: bool = False, force: bool = False, group: str = "main") -> Pa
         )
 
     try:
-        _load()
-    except Exception:
+        _load(ext_name)
+    except OSError:
         # A stale incremental object (e.g. after a template-signature change)
-        # can link a .so with dangling device stubs — rebuild clean once.
+        # can link a .so with dangling device stubs, which does not load —
+        # rebuild clean once, under another name: torch takes a name it has
+        # built in this process as done. A compile error (RuntimeError) is the
+        # caller's: a second try only hides it.
         shutil.rmtree(BUILD_DIR, ignore_errors=True)
         BUILD_DIR.mkdir(exist_ok=True)
-        _load()
+        ext_name += "_clean"
+        _load(ext_name)
     built = BUILD_DIR / f"{ext_name}.so"
     if not built.is_file():
         candidates = list(BUILD_DIR.glob("*.so"))
