@@ -396,17 +396,21 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
   __shared__ pd_f32x2 ml[4][16];
   __shared__ PdPair pending[2];                // cut at the ends of the range
   __shared__ unsigned arrived[2];
-  // what the waves left in LDS, channels 2 e and on of the segment's heads: sum and weight
-  auto meet = [&](int e, float& top, float& sum) {
+  // What `parts` waves or groups left in LDS, channels 2 e and on of a pair's heads: sum and
+  // weight. No other part is read: it may be another pair's, and a weight of zero does not cancel
+  // an infinity there.
+  auto meet = [&](int e, int parts, float& top, float& sum) {
     const int g = e / (D / 2);
     top = -INFINITY;
     sum = 0.f;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) top = fmaxf(top, ml[v][g][0]);
+    for (int v = 0; v < 4; ++v)
+      if (v < parts) top = fmaxf(top, ml[v][g][0]);
     const float tb = top > -INFINITY ? top : 0.f;
     pd_f32x2 x = {0.f, 0.f};
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
+      if (v >= parts) break;
       const float f = __builtin_amdgcn_exp2f(ml[v][g][0] - tb);      // -inf -> 0
       sum += ml[v][g][1] * f;
       x += *reinterpret_cast<const pd_f32x2*>(mo + v * G * D + e * 2) * f;
@@ -580,7 +584,7 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
     const long slot = ((long)wg * 2 + (pieces || s_t == t_begin ? 0 : 1)) * G;
     for (int e = threadIdx.x; e < G * (D / 2); e += 256) {
       float top, sum;
-      const pd_f32x2 x = meet(e, top, sum);
+      const pd_f32x2 x = meet(e, 4, top, sum);
       if (whole) {
         finish(orow, e, x, sum);
         continue;
@@ -676,12 +680,10 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
       if (e % (D / 4) == 0) ml[group][g] = pd_f32x2{top, sum};
     }
     if (groups > 1) {
-      if ((int)tid < G)
-        for (int v = groups; v < 4; ++v) ml[v][tid][0] = -INFINITY;
       pd_barrier();
       for (int e = threadIdx.x; e < G * (D / 2); e += 256) {
         float top, sum;
-        const pd_f32x2 x = meet(e, top, sum);
+        const pd_f32x2 x = meet(e, groups, top, sum);
         finish(orow, e, x, sum);
       }
     }

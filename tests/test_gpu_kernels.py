@@ -293,6 +293,48 @@ class TestDecodePieces:
         assert_close_to_f32_ref(runs[0], ref, 2e-4, 2 ** -8)
 
 
+def _ragged_cache(lens, KVH, D, BS, fp8=False):
+    """Cache and block tables of sequences of these lengths, their blocks in no order."""
+    need = [-(-n // BS) for n in lens]
+    blocks = (torch.randperm(sum(need)) + 1).split(need)     # block 0 reserved
+    bt = torch.zeros(len(lens), max(need), dtype=torch.int32)
+    for row, mine in zip(bt, blocks):
+        row[:len(mine)] = mine
+    kc, vc = (torch.randn(sum(need) + 1, KVH, BS, D, device=DEV, dtype=torch.bfloat16)
+              for _ in range(2))
+    if fp8:
+        kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+    return kc, vc, bt.to(DEV)
+
+
+# Equal ranges of about as many tiles as two short sequences have: ranges that hold the end of
+# a pair, whole ones and the start of another, and pairs that many ranges share.
+RAGGED = [(i * 37) % 150 for i in range(300)]
+RAGGED[3], RAGGED[4], RAGGED[150], RAGGED[299] = 3000, 1500, 2100, 2999
+
+
+class TestDecodeIsolation:
+    """What one sequence's cache holds does not reach another's output: workgroups that have
+    pieces of several pairs leave both in one LDS area, and merge with fewer parts of it (G D / 4
+    over 64) than they met with."""
+
+    @pytest.mark.parametrize("D,G,KVH,fp8", [(64, 8, 3, False), (64, 5, 3, False), (64, 4, 3, False),
+                                             (128, 3, 2, False), (128, 3, 8, True),
+                                             (256, 2, 4, False), (256, 2, 2, True)])
+    def test_infinite_values(self, D, G, KVH, fp8):
+        kc, vc, bt = _ragged_cache(RAGGED, KVH, D, 16, fp8)
+        ctx = torch.tensor(RAGGED, dtype=torch.int32, device=DEV)
+        q = torch.randn(len(RAGGED), G * KVH, D, device=DEV, dtype=torch.bfloat16)
+        clean = ops.paged_decode_attention(q, kc, vc, bt, ctx, D ** -0.5)
+        for b in range(1, len(RAGGED), 3):                   # fp8 (e4m3fn) has no infinity
+            mine = bt[b, :-(-RAGGED[b] // 16)].long()
+            vc[mine] = torch.tensor(float("nan" if fp8 else "inf"), device=DEV).to(vc.dtype)
+        out = ops.paged_decode_attention(q, kc, vc, bt, ctx, D ** -0.5)
+        others = [b for b, n in enumerate(RAGGED) if b % 3 != 1 and n > 0]
+        assert torch.equal(out[others], clean[others])
+        assert not out[4].isfinite().any()
+
+
 class TestDecodeWeightBits:
     def test_head_size_64_keeps_fp32_weights(self):
         """Outputs that are not the bf16 nearest to the 64-bit result: 4e-4 of them with
