@@ -238,16 +238,18 @@ int compute_units(const at::Tensor& x) {
   return cus;
 }
 
-// The matrix-core kernel of paged_decode.hip. Workgroups: as many as are resident at
-// the variant's register use, so that every range is in work at once, and one for every pair.
-// arrivals: zeros
-// [B, KVH], used up; without it they are made here, a launch of 2 us.
-template <int D, typename TC, int NK, int OCC>
+// The matrix-core kernel of paged_decode.hip. Workgroups: as many as are resident, so that
+// every range is in work at once, and one for every pair. arrivals: zeros [B, KVH], used up;
+// without it they are made here, a launch of 2 us.
+template <int D, typename TC>
 void launch_paged_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor& kc,
                          const at::Tensor& vc, const at::Tensor& bt,
                          const at::Tensor& cl, double scale, double softcap,
                          long window, const c10::optional<at::Tensor>& arrivals) {
+  constexpr PdVariant kVariant = pd_variant(D, sizeof(TC) == 1);
+  constexpr int NK = kVariant.groups, OCC = kVariant.resident;
   using Shape = PdShape<D, TC, NK>;
+  static_assert(OCC * (4 * Shape::wave_lds(16) + 1024) <= 160 * 1024, "resident at every G");
   constexpr double kLog2e = 1.4426950408889634;
   const int B = q.size(0), KVH = kc.size(1), G = q.size(1) / KVH;
   const int bs_shift = kc.size(2) == 32 ? 5 : 4;
@@ -265,7 +267,7 @@ void launch_paged_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor&
   const at::Tensor arr = given ? *arrivals : at::zeros({B, KVH}, q.options().dtype(at::kInt));
   auto go = [&]<bool CAP>() {
     hipLaunchKernelGGL((paged_decode_kernel<D, TC, NK, OCC, CAP>), dim3(wgs), dim3(256),
-                       Shape::kLds + sizeof(float) * 4 * G * D, stream(),
+                       4 * Shape::wave_lds(G), stream(),
                        reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), out.stride(0),
                        reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()), q.stride(0),
                        reinterpret_cast<const TC*>(kc.data_ptr()),
@@ -303,24 +305,16 @@ void launch_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor& kc,
     const at::Tensor qa = rows_on_16(q);
     const at::Tensor bta = bt.stride(1) == 1 ? bt : bt.contiguous();
     at::Tensor oa = rows_start_on(out, 8) ? out : out.clone(at::MemoryFormat::Contiguous);
-    auto go = [&]<int HD, typename TC, int NK, int OCC>() {
-      launch_paged_decode<HD, TC, NK, OCC>(oa, qa, kc, vc, bta, cl, scale, softcap, window,
-                                           arrivals);
+    auto go = [&]<int HD, typename TC>() {
+      launch_paged_decode<HD, TC>(oa, qa, kc, vc, bta, cl, scale, softcap, window, arrivals);
     };
     using BF = __hip_bfloat16;
     using F8 = __hip_fp8_e4m3;
-    // 32 keys a tile at head size 64 (us, with the merge, 64 / 32: 1 x 200 keys, 8 kv heads 9.1
-    // / 7.9; 1 x 3000 11.2 / 10.4; 8 ragged up to 1000 10.2 / 10.4; 64 x 300 16.7 / 15.9; 6
-    // ragged up to 15000 34.8 / 33.6; 64 x 1040 35.7 / 36.8 call after call, but 1.3 less a
-    // layer between the products of a step: llama-3.2-1b 1440 / 1420). At 128 64 keys and one
-    // workgroup a CU gain on 3 ragged up to 16000 (34.4 / 32.2) what they lose on 60 up to 800
-    // (31.9 / 32.5). At 256 (one workgroup a CU / two): 64 ragged up to 300 30 / 22, 96 x 1064
-    // 140 / 142.
-    if (D == 64) go.template operator()<64, BF, 2, 3>();
-    else if (D == 128 && !fp8) go.template operator()<128, BF, 2, 2>();
-    else if (D == 256 && !fp8) go.template operator()<256, BF, 1, 2>();
-    else if (D == 128) go.template operator()<128, F8, 2, 3>();
-    else go.template operator()<256, F8, 1, 2>();
+    if (D == 64) go.template operator()<64, BF>();
+    else if (D == 128 && !fp8) go.template operator()<128, BF>();
+    else if (D == 256 && !fp8) go.template operator()<256, BF>();
+    else if (D == 128) go.template operator()<128, F8>();
+    else go.template operator()<256, F8>();
     if (!oa.is_same(out)) out.copy_(oa);
     return;
   } else {

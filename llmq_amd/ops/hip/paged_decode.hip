@@ -246,10 +246,20 @@ template <int D, typename TC, int NK>
 struct PdShape {
   static constexpr int kTileShift = NK == 2 ? 5 : 4;
   static constexpr int kKeys = 16 * NK;
-  static constexpr size_t kLds = 4 * sizeof(short) * (size_t)kKeys * D;
+  // LDS of a wave: its V tile, and after its last tile its sums of G heads in the same place
+  __host__ __device__ static constexpr int wave_lds(int G) {
+    return D * (kKeys * (int)sizeof(short) > G * (int)sizeof(float) ? kKeys * (int)sizeof(short)
+                                                                    : G * (int)sizeof(float));
+  }
   // the least piece of a pair: 64 KiB of keys and values
   static constexpr int kLeastPiece = 64 * 1024 / (2 * kKeys * D * (int)sizeof(TC));
 };
+
+// 16-key groups of a tile and workgroups a CU, by registers; their LDS fits at every G.
+struct PdVariant { int groups, resident; };
+constexpr PdVariant pd_variant(int D, bool fp8) {
+  return D == 64 ? PdVariant{2, 3} : D == 128 ? PdVariant{2, fp8 ? 3 : 2} : PdVariant{1, 2};
+}
 
 template <int D, typename TC, int NK, int OCC, bool CAP>
 __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
@@ -273,7 +283,8 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
-  short* const Vt = reinterpret_cast<short*>(pd_smem) + w * (KT * D);
+  const int wave_lds = PdShape<D, TC, NK>::wave_lds(NK == 2 ? 16 : G);   // 16: no more than a tile
+  short* const Vt = reinterpret_cast<short*>(pd_smem + w * wave_lds);
 
   const int wgs = gridDim.x, wg = blockIdx.x;
   const PdLens first = pd_lens(lens, B, lane, 0);
@@ -392,7 +403,7 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
                        : pd_s16x8{0, 0, 0, 0, 0, 0, 0, 0};
     }
   };
-  float* const mo = reinterpret_cast<float*>(pd_smem + PdShape<D, TC, NK>::kLds);
+  auto mo = [&](int part) { return reinterpret_cast<float*>(pd_smem + part * wave_lds); };
   __shared__ pd_f32x2 ml[4][16];
   __shared__ PdPair pending[2];                // cut at the ends of the range
   __shared__ unsigned arrived[2];
@@ -413,7 +424,7 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
       if (v >= parts) break;
       const float f = __builtin_amdgcn_exp2f(ml[v][g][0] - tb);      // -inf -> 0
       sum += ml[v][g][1] * f;
-      x += *reinterpret_cast<const pd_f32x2*>(mo + v * G * D + e * 2) * f;
+      x += *reinterpret_cast<const pd_f32x2*>(mo(v) + e * 2) * f;
     }
     return x;
   };
@@ -556,7 +567,7 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
     }
     l = across_32(across_16(l, lanes_add), lanes_add);
     if (col < G) {
-      float* to = mo + (w * G + col) * D + grp * 4;
+      float* to = mo(w) + col * D + grp * 4;   // the wave has read its last V tile
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<pd_f32x4*>(to + dt * 16) = o[dt];
       if (grp == 0) ml[w][col] = pd_f32x2{m, l};
@@ -675,8 +686,7 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
         finish(orow, e * 2 + 1, y, sum);
         continue;
       }
-      *reinterpret_cast<pd_f32x4*>(mo + group * G * D + e * 4) =
-          pd_f32x4{x[0], x[1], y[0], y[1]};
+      *reinterpret_cast<pd_f32x4*>(mo(group) + e * 4) = pd_f32x4{x[0], x[1], y[0], y[1]};
       if (e % (D / 4) == 0) ml[group][g] = pd_f32x2{top, sum};
     }
     if (groups > 1) {
