@@ -84,9 +84,37 @@ DEVINL int pd_max(int x) {                       // of values >= 0
 }
 DEVINL int pd_sum(int x) { return __builtin_amdgcn_readlane(pd_scan(x), WAVE - 1); }
 
-// Pieces of a pair of nt tiles, of up to c each; up to twice the least piece stays whole.
-DEVINL int pd_pieces(int nt, int c, int least) {
-  return nt <= 2 * least ? min(nt, 1) : (nt + c - 1) / c;
+// Here and on the host, where the deal is tested. Quotients below 2^20 are exact: the reciprocal's
+// error moves them by less than the half that keeps them off whole numbers.
+__host__ __device__ __forceinline__ float pd_rcp(float x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_rcpf(x);
+#else
+  return 1.f / x;
+#endif
+}
+__host__ __device__ __forceinline__ float pd_sqrt(float x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_sqrtf(x);
+#else
+  return sqrtf(x);
+#endif
+}
+__host__ __device__ __forceinline__ int pd_quotient(int x, float inv) {
+  return (int)(((float)x + 0.5f) * inv);
+}
+
+// Pieces of a pair of nt tiles, of up to c each; up to twice the least piece stays whole. One
+// workgroup reads the partial sums of all, each as many bytes as `thick` tiles, so that a piece has
+// at least sqrt(nt `thick`) tiles, with a factor for the merge's longer way, in whole rounds of four
+// waves. us, without that floor / with it: 1 x 16000 keys, 1 kv head of 256, 8 heads 62.6 / 30.8; 3 x
+// 16000, 2 of 128, 6 heads each 29.5 / 21.0; 1 x 16000, 8 of 64, 4 heads each 17.2 / 15.3. Factors of 1
+// to 3 are within 1 % over 86 batches; at 2 one of 4000 keys, 2 of 128, fp8 loses 13 %.
+__host__ __device__ __forceinline__ int pd_pieces(int nt, int c, int least, float thick) {
+  if (nt <= 2 * least) return nt > 0;
+  const int floor = ((int)pd_sqrt(1.5f * nt * thick) + 3) & ~3;    // four waves share them
+  const int size = c > floor ? c : floor;
+  return pd_quotient(nt + size - 1, pd_rcp((float)size));
 }
 
 // How the tiles of all pairs (in order, kv heads innermost) are dealt to `wgs` workgroups, of
@@ -120,7 +148,8 @@ DEVINL PdLens pd_lens(const int* __restrict__ lens, int B, int lane, int c) {
 
 template <int TS>
 DEVINL PdDeal pd_deal(const int* __restrict__ lens, int B, int KVH, int window, int lane,
-                      const PdLens& first, int wgs, int resident, int least, bool lone) {
+                      const PdLens& first, int wgs, int resident, int least, float thick,
+                      bool lone) {
   int tiles = 0, n0 = 0, most = 0;
   for (int c = 0; c < B; c += 4 * WAVE) {
     const PdLens l = c == 0 ? first : pd_lens(lens, B, lane, c);
@@ -129,7 +158,7 @@ DEVINL PdDeal pd_deal(const int* __restrict__ lens, int B, int KVH, int window, 
       if (c + i * WAVE >= B) break;
       const int n = pd_tiles<TS>(l.of[i], window);
       tiles += n;
-      n0 += pd_pieces(n, least, least);
+      n0 += pd_pieces(n, least, least, thick);
       most = max(most, n);
     }
   }
@@ -152,7 +181,8 @@ DEVINL PdDeal pd_deal(const int* __restrict__ lens, int B, int KVH, int window, 
 // those of one kv head before it.
 template <int TS>
 DEVINL void pd_locate(const int* __restrict__ lens, int B, int KVH, int window, int lane, int t,
-                      const PdLens& first, int piece, int least, int& b, int& len, int& before) {
+                      const PdLens& first, int piece, int least, float thick, int& b, int& len,
+                      int& before) {
   int base = 0;
   for (int c = 0; c < B; c += 4 * WAVE) {
     const PdLens l = c == 0 ? first : pd_lens(lens, B, lane, c);
@@ -160,7 +190,7 @@ DEVINL void pd_locate(const int* __restrict__ lens, int B, int KVH, int window, 
     for (int i = 0; i < 4; ++i) {
       if (c + i * WAVE >= B) break;
       int n = pd_tiles<TS>(l.of[i], window);
-      if (piece > 0) n = pd_pieces(n, piece, least);
+      if (piece > 0) n = pd_pieces(n, piece, least, thick);
       const int x = pd_scan(n);
       const unsigned long long hit = __ballot((base + x) * KVH > t);
       if (hit) {
@@ -242,6 +272,82 @@ DEVINL pd_f32x2 pd_published(const float* from) {
       reinterpret_cast<const unsigned long long*>(from), __ATOMIC_RELAXED,
       __HIP_MEMORY_SCOPE_AGENT));
 }
+
+// Two or four channels (V) of a head, their sum not yet divided by its weight.
+template <typename V>
+struct PdSum {
+  float top, weight;
+  V x;
+};
+template <typename V>
+DEVINL void pd_finish(__hip_bfloat16* to, const PdSum<V>& s) {
+  typedef __bf16 Row __attribute__((ext_vector_type(sizeof(V) / 4)));
+  const V y = s.x * (s.weight > 0.f ? 1.0f / s.weight : 0.f);
+  *reinterpret_cast<Row*>(to) = __builtin_convertvector(y, Row);
+}
+
+// The sums of a pair's pieces, of E quads of channels that are 256 quads apart and of which `live`
+// are there: pieces `group`, `group` + `groups`, .. At 32-bit offsets of rows of heads from the
+// first piece's workgroup: 64-bit places and divisions took 0.5 us (7 ragged up to 1900 keys, 2 kv
+// heads of 128, 6 heads each: 11.6 -> 11.1).
+template <int D, int E>
+DEVINL void pd_sum_pieces(PdSum<pd_f32x4> (&s)[E], const float* part_o, const float* part_ml,
+                          const PdPair& pair, int G, unsigned quad, int live, int group,
+                          int groups) {
+  const int first = __builtin_amdgcn_readfirstlane(pair.w_first);
+  const int last = __builtin_amdgcn_readfirstlane(pair.w_last) - first;
+  const unsigned head = pair.head * G, step = 2 * G;
+  const float* const from_o = part_o + (long)first * 2 * G * D;
+  const float* const from_ml = part_ml + (long)first * 2 * G * 2;
+#pragma unroll
+  for (int k = 0; k < E; ++k) s[k] = PdSum<pd_f32x4>{-INFINITY, 0.f, {0.f, 0.f, 0.f, 0.f}};
+  // N pieces from r0 on, asked for together
+  auto take = [&]<int N>(int r0) {
+    pd_f32x2 ml[E][N], x[E][N], y[E][N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int r = min(r0 + i * groups, last);  // past the end: weight zero below
+      unsigned at = r * step;
+      if (i == 0) at += r == 0 ? head : 0;
+#pragma unroll
+      for (int k = 0; k < E; ++k) {
+        const unsigned e = k < live ? quad + k * 256 : quad;
+        ml[k][i] = pd_published(from_ml + (at + e / (D / 4)) * 2);
+        const float* const o = from_o + (at * D + e * 4);
+        x[k][i] = pd_published(o);
+        y[k][i] = pd_published(o + 2);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+      float top = s[k].top;
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        if (r0 + i * groups > last) ml[k][i][0] = -INFINITY;
+        top = fmaxf(top, ml[k][i][0]);
+      }
+      const float tb = top > -INFINITY ? top : 0.f;
+      const float f0 = __builtin_amdgcn_exp2f(s[k].top - tb);
+      s[k].weight *= f0;
+      s[k].x *= f0;
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const float f = __builtin_amdgcn_exp2f(ml[k][i][0] - tb);
+        if (ml[k][i][0] > -INFINITY) {
+          s[k].weight += ml[k][i][1] * f;
+          s[k].x += __builtin_shufflevector(x[k][i], y[k][i], 0, 1, 2, 3) * f;
+        }
+      }
+      s[k].top = top;
+    }
+  };
+  constexpr int kMost = E == 4 ? 4 : 8;
+  for (int r0 = group; r0 <= last; r0 += kMost * groups) {
+    if (r0 + 2 * groups > last) take.template operator()<2>(r0);
+    else take.template operator()<kMost>(r0);
+  }
+}
+
 template <int D, typename TC, int NK>
 struct PdShape {
   static constexpr int kTileShift = NK == 2 ? 5 : 4;
@@ -295,7 +401,8 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
   // Few sequences whose least pieces all find a workgroup, without pd_deal's other sums and a
   // second scan: 150 of the 450 instructions ahead of the first load, 4 clocks each.
   int n_l = B <= WAVE ? pd_tiles<TS>(first.of[0], window) : 0;
-  n_l = pd_pieces(n_l, kLeast, kLeast);
+  const float thick = G * (2.f / (KT * (int)sizeof(TC)));
+  n_l = pd_pieces(n_l, kLeast, kLeast, thick);
   const int upto = pd_scan(n_l);               // pieces of a head of this lane's sequence and before
   const int n0 = __builtin_amdgcn_readlane(upto, WAVE - 1) * KVH;
   if (B <= WAVE && n0 <= wgs) {
@@ -305,27 +412,28 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
     nt = pd_tiles<TS>(len, window);
     const int of = __builtin_amdgcn_readlane(n_l, b);
     const int r = wg - (__builtin_amdgcn_readlane(upto, b) - of) * KVH;
-    const float inv = __builtin_amdgcn_rcpf((float)of);        // quotients below 2^20: exact
-    kh = __builtin_amdgcn_readfirstlane((int)(((float)r + 0.5f) * inv));
+    const float inv = pd_rcp((float)of);
+    kh = __builtin_amdgcn_readfirstlane(pd_quotient(r, inv));
     i0 = r - kh * of;
     w_first = wg - i0;
     w_last = w_first + of - 1;
-    const int size = __builtin_amdgcn_readfirstlane((int)(((float)(nt + of - 1) + 0.5f) * inv));
+    const int size = __builtin_amdgcn_readfirstlane(pd_quotient(nt + of - 1, inv));
     t = i0 *= size;
     t_end = min(nt, i0 + size);
   } else {
     const PdDeal deal = pd_deal<TS>(lens, B, KVH, window, lane, first, wgs, resident, kLeast,
-                                    D == 256 && !F8);
+                                    thick, D == 256 && !F8);
     share = deal.share;
     pieces = deal.piece > 0;
     t = wg * share;
     t_end = min(deal.total, t + share);
     if (t >= t_end) return;
     int before;
-    pd_locate<TS>(lens, B, KVH, window, lane, t, first, deal.piece, kLeast, b, len, before);
+    pd_locate<TS>(lens, B, KVH, window, lane, t, first, deal.piece, kLeast, thick, b, len,
+                  before);
     if (b >= B) return;
     nt = pd_tiles<TS>(len, window);
-    const int of = pieces ? pd_pieces(nt, deal.piece, kLeast) : nt;
+    const int of = pieces ? pd_pieces(nt, deal.piece, kLeast, thick) : nt;
     const int r = t - before * KVH;
     kh = r / of;
     i0 = r % of;
@@ -407,31 +515,27 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
   __shared__ pd_f32x2 ml[4][16];
   __shared__ PdPair pending[2];                // cut at the ends of the range
   __shared__ unsigned arrived[2];
-  // What `parts` waves or groups left in LDS, channels 2 e and on of a pair's heads: sum and
-  // weight. No other part is read: it may be another pair's, and a weight of zero does not cancel
-  // an infinity there.
-  auto meet = [&](int e, int parts, float& top, float& sum) {
-    const int g = e / (D / 2);
-    top = -INFINITY;
-    sum = 0.f;
+  // The W channels of a thread, number e of a pair's: two at head size 64, where four leave half the
+  // threads idle (1 x 1500 keys, 8 kv heads: 8.4 us, 8.0 so).
+  constexpr int W = D == 64 ? 2 : 4;
+  typedef float Channels __attribute__((ext_vector_type(W)));
+  // What `parts` waves or groups left of them in LDS. No other part is read: it may be another
+  // pair's, and a weight of zero does not cancel an infinity there.
+  auto meet = [&](int e, int parts) {
+    const int g = e / (D / W);
+    PdSum<Channels> s{-INFINITY, 0.f, Channels(0.f)};
 #pragma unroll
     for (int v = 0; v < 4; ++v)
-      if (v < parts) top = fmaxf(top, ml[v][g][0]);
-    const float tb = top > -INFINITY ? top : 0.f;
-    pd_f32x2 x = {0.f, 0.f};
+      if (v < parts) s.top = fmaxf(s.top, ml[v][g][0]);
+    const float tb = s.top > -INFINITY ? s.top : 0.f;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       if (v >= parts) break;
       const float f = __builtin_amdgcn_exp2f(ml[v][g][0] - tb);      // -inf -> 0
-      sum += ml[v][g][1] * f;
-      x += *reinterpret_cast<const pd_f32x2*>(mo(v) + e * 2) * f;
+      s.weight += ml[v][g][1] * f;
+      s.x += *reinterpret_cast<const Channels*>(mo(v) + e * W) * f;
     }
-    return x;
-  };
-  auto finish = [&](__hip_bfloat16* orow, int e, pd_f32x2 x, float sum) {
-    const float inv = sum > 0.f ? 1.0f / sum : 0.f;
-    *reinterpret_cast<pd_bf16x2*>(orow + e * 2) =
-        __builtin_convertvector((pd_f32x2{x[0] * inv, x[1] * inv}), pd_bf16x2);
+    return s;
   };
   int waiting = 0;
   open();
@@ -593,15 +697,17 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
     __hip_bfloat16* const orow = out + (long)s_b * out_stride + (long)s_kh * G * D;
     // a range holds at most two pieces: one from its start, one to its end
     const long slot = ((long)wg * 2 + (pieces || s_t == t_begin ? 0 : 1)) * G;
-    for (int e = threadIdx.x; e < G * (D / 2); e += 256) {
-      float top, sum;
-      const pd_f32x2 x = meet(e, 4, top, sum);
+    for (int e = threadIdx.x; e < G * (D / W); e += 256) {
+      const PdSum<Channels> s = meet(e, 4);
       if (whole) {
-        finish(orow, e, x, sum);
+        pd_finish(orow + e * W, s);
         continue;
       }
-      pd_publish(part_o + slot * D + e * 2, x);
-      if (e % (D / 2) == 0) pd_publish(part_ml + (slot + e / (D / 2)) * 2, pd_f32x2{top, sum});
+#pragma unroll
+      for (int c = 0; c < W; c += 2)
+        pd_publish(part_o + slot * D + e * W + c, pd_f32x2{s.x[c], s.x[c + 1]});
+      if (e % (D / W) == 0)
+        pd_publish(part_ml + (slot + e / (D / W)) * 2, pd_f32x2{s.top, s.weight});
     }
     if (!whole) {
       if (threadIdx.x == 0) {
@@ -628,74 +734,37 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
     const PdPair pair = pending[p];
     if ((int)arrived[p] != pair.w_last - pair.w_first) continue;
     __hip_bfloat16* const orow = out + (long)pair.b * out_stride + (long)pair.kh * G * D;
-    // 32-bit offsets from the pair's first piece, no division: those took 0.5 us (7 ragged up to
-    // 1900 keys, 2 kv heads of 128, 6 heads each: 11.6 -> 11.1).
-    const unsigned items = G * (D / 4), tid = threadIdx.x;
-    const int groups = 1 + (2 * items <= 256) + (3 * items <= 256) + (4 * items <= 256);
-    const int group = groups == 1 ? 0 : (tid >= items) + (tid >= 2 * items) + (tid >= 3 * items);
-    const int first = __builtin_amdgcn_readfirstlane(pair.w_first);
-    const int last = __builtin_amdgcn_readfirstlane(pair.w_last) - first;
-    const unsigned head = pair.head * G, step = 2 * G;
-    const float* const from_o = part_o + (long)first * 2 * G * D;
-    const float* const from_ml = part_ml + (long)first * 2 * G * 2;
-    for (unsigned e = group < groups ? tid - group * items : items; e < items; e += 256) {
-      const unsigned g = e / (D / 4);
-      float top = -INFINITY, sum = 0.f;
-      pd_f32x2 x = {0.f, 0.f}, y = {0.f, 0.f};
-      // N of the pieces that are this thread's, from r0 on: asked for together
-      auto take = [&]<int N>(int r0) {
-        pd_f32x2 pml[N], px[N], py[N];
+    const int tid = threadIdx.x, quads = G * (D / 4);
+    const int groups = 1 + (2 * quads <= 256) + (3 * quads <= 256) + (4 * quads <= 256);
+    const int group =
+        groups == 1 ? 0 : (tid >= quads) + (tid >= 2 * quads) + (tid >= 3 * quads);
+    const int e0 = tid - group * quads;
+    const int live = group < groups ? (quads - e0 + 255) / 256 : 0;      // none below zero
+    auto merge = [&]<int E>() {
+      PdSum<pd_f32x4> s[E];
+      pd_sum_pieces<D, E>(s, part_o, part_ml, pair, G, e0, live, group, groups);
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-          const int r = min(r0 + i * groups, last);          // past the end: weight zero below
-          unsigned at = r * step;
-          if (i == 0) at += r == 0 ? head : 0;
-          pml[i] = pd_published(from_ml + (at + g) * 2);
-          const float* const po = from_o + (at * D + e * 4);
-          px[i] = pd_published(po);
-          py[i] = pd_published(po + 2);
+      for (int k = 0; k < E; ++k) {
+        const int e = e0 + k * 256;
+        if (k >= live) break;
+        if (groups == 1) {
+          pd_finish(orow + e * 4, s[k]);
+        } else {
+          *reinterpret_cast<pd_f32x4*>(mo(group) + e * 4) = s[k].x;
+          if (e % (D / 4) == 0) ml[group][e / (D / 4)] = pd_f32x2{s[k].top, s[k].weight};
         }
-        float up = top;
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          if (r0 + i * groups > last) pml[i][0] = -INFINITY;
-          up = fmaxf(up, pml[i][0]);
-        }
-        const float tb = up > -INFINITY ? up : 0.f;
-        const float f0 = __builtin_amdgcn_exp2f(top - tb);
-        sum *= f0;
-        x *= f0;
-        y *= f0;
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          const float f = __builtin_amdgcn_exp2f(pml[i][0] - tb);
-          if (pml[i][0] > -INFINITY) {
-            sum += pml[i][1] * f;
-            x += px[i] * f;
-            y += py[i] * f;
-          }
-        }
-        top = up;
-      };
-      for (int r0 = group; r0 <= last; r0 += 8 * groups) {
-        if (r0 + 2 * groups > last) take.template operator()<2>(r0);
-        else take.template operator()<8>(r0);
       }
-      if (groups == 1) {
-        finish(orow, e * 2, x, sum);
-        finish(orow, e * 2 + 1, y, sum);
-        continue;
-      }
-      *reinterpret_cast<pd_f32x4*>(mo(group) + e * 4) = pd_f32x4{x[0], x[1], y[0], y[1]};
-      if (e % (D / 4) == 0) ml[group][g] = pd_f32x2{top, sum};
+    };
+    // up to D / 64 quads a thread, asked for together (1 x 200 keys, 2 kv heads of 256, 16 heads
+    // each: one after the other 15.8 us, so 12.4)
+    if (live > 0) {
+      if (D == 64 || quads <= 256) merge.template operator()<1>();
+      else if (D == 128 || quads <= 512) merge.template operator()<D == 64 ? 1 : 2>();
+      else merge.template operator()<D == 256 ? 4 : 1>();
     }
     if (groups > 1) {
       pd_barrier();
-      for (int e = threadIdx.x; e < G * (D / 2); e += 256) {
-        float top, sum;
-        const pd_f32x2 x = meet(e, groups, top, sum);
-        finish(orow, e, x, sum);
-      }
+      for (int e = tid; e < G * (D / W); e += 256) pd_finish(orow + e * W, meet(e, groups));
     }
     if (p + 1 < waiting) pd_barrier();
   }

@@ -1,5 +1,5 @@
-"""Decode attention's host side, compiled from the kernel's own source and run here without a
-GPU: what its workgroups take of a CU."""
+"""Decode attention's rules, compiled from the kernel's own source and run here without a GPU: what
+its workgroups take of a CU and how they cut a sequence."""
 
 from __future__ import annotations
 
@@ -14,6 +14,21 @@ HIPCC = shutil.which("hipcc") or shutil.which("/opt/rocm/bin/hipcc")
 SOURCE = r"""
 #include "paged_decode.hip"
 #include <cstdio>
+#include <cstring>
+
+// Pieces of the size that the kernel makes of their count: none empty, none over its size.
+void pieces(int least, int c, float thick) {
+  int most = 0;
+  for (int nt = 1; nt <= 70000; nt += nt < 3000 ? 1 : 97) {
+    const int of = pd_pieces(nt, c, least, thick);
+    const int size = pd_quotient(nt + of - 1, pd_rcp((float)of));
+    if (of < 1 || size != (nt + of - 1) / of || (long)(of - 1) * size >= nt ||
+        of > (nt + c - 1) / c || (nt <= 2 * least && of != 1) || pd_pieces(0, c, least, thick))
+      printf("%d %d %d %d\n", nt, c, of, size);
+    most = of > most ? of : most;
+  }
+  printf("%d\n", most);
+}
 
 template <int D, typename TC>
 void variant() {
@@ -23,7 +38,11 @@ void variant() {
     printf("%d %d %d %d %d\n", D, fp8, G, v.resident, 4 * PdShape<D, TC, v.groups>::wave_lds(G));
 }
 
-int main() {
+int main(int argc, char** argv) {
+  if (argc > 1 && !strcmp(argv[1], "pieces")) {
+    pieces(atoi(argv[2]), atoi(argv[3]), atof(argv[4]));
+    return 0;
+  }
   variant<64, __hip_bfloat16>();
   variant<128, __hip_bfloat16>();
   variant<256, __hip_bfloat16>();
@@ -58,3 +77,13 @@ def test_workgroups_of_a_cu_fit_its_lds(program):
     for D, fp8, G, resident, lds in program():
         of_one = -(-(lds + fixed) // granule) * granule
         assert resident * of_one <= cu, (D, fp8, G)
+
+
+@pytest.mark.parametrize("least", [4, 8])
+@pytest.mark.parametrize("longer", [0, 1, 3, 60, 1001])
+@pytest.mark.parametrize("thick", [1 / 32, 0.125, 0.375, 1.0, 2.0])
+def test_no_piece_is_empty(program, least, longer, thick):
+    out = program("pieces", least, least + longer, thick)
+    assert len(out) == 1, out[:5]                            # the largest count, no exceptions
+    # the floor: sqrt(1.5 thick nt) tiles, no more than rounded up by four
+    assert out[0][0] <= 70000 / max(least + longer, (1.5 * thick * 70000) ** 0.5 - 1) + 1

@@ -267,7 +267,9 @@ class TestDecodePieces:
 
     @pytest.mark.parametrize("D,G,KVH,fp8", [(64, 4, 8, False), (128, 6, 2, False),
                                              (128, 3, 8, True), (256, 2, 8, False),
-                                             (256, 16, 1, True)])
+                                             (256, 16, 1, True), (256, 12, 2, False),
+                                             (256, 7, 1, False), (128, 16, 2, False),
+                                             (128, 9, 1, True)])
     @pytest.mark.parametrize("lens", [
         [128], [129], [256, 257], [512, 513, 0], [9000], [3000, 17, 1], [520] * 30,
         [(i * 53) % 400 for i in range(90)], [(i * 29) % 70 for i in range(300)],
