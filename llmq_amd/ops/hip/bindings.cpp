@@ -238,9 +238,8 @@ int compute_units(const at::Tensor& x) {
   return cus;
 }
 
-// The matrix-core kernel of paged_decode.hip. Workgroups: as many as are resident, so that
-// every range is in work at once, and one for every pair. arrivals: zeros [B, KVH], used up;
-// without it they are made here, a launch of 2 us.
+// The matrix-core kernel of paged_decode.hip. arrivals: zeros [B, KVH], used up; without it they
+// are made here, a launch of 2 us.
 template <int D, typename TC>
 void launch_paged_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor& kc,
                          const at::Tensor& vc, const at::Tensor& bt,
@@ -254,9 +253,8 @@ void launch_paged_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor&
   const int B = q.size(0), KVH = kc.size(1), G = q.size(1) / KVH;
   const int bs_shift = kc.size(2) == 32 ? 5 : 4;
   const long tiles = (bt.size(1) << bs_shift) / Shape::kKeys + 1;   // of a pair, at most
-  const long most = (long)B * KVH * ((tiles + Shape::kLeastPiece - 1) / Shape::kLeastPiece);
   const long resident = (long)compute_units(q) * OCC;
-  const int wgs = (int)std::min(std::max(resident, (long)B * KVH), most);
+  const int wgs = (int)pd_workgroups((long)B * KVH, tiles, Shape::kLeastPiece, resident);
   auto opts = q.options().dtype(at::kFloat);
   at::Tensor part_o = at::empty({2L * wgs, G, D}, opts);
   at::Tensor part_ml = at::empty({2L * wgs, G, 2}, opts);

@@ -57,7 +57,7 @@ typedef __attribute__((address_space(3))) pd_bf16x4 pd_lds_bf16x4;
 
 // Tiles of 2^TS keys that a sequence's visible keys touch.
 template <int TS>
-DEVINL int pd_tiles(int len, int window) {
+__host__ __device__ __forceinline__ int pd_tiles(int len, int window) {
   if (len <= 0) return 0;
   const int lo = window > 0 && len > window ? len - window : 0;
   return ((len - 1) >> TS) - (lo >> TS) + 1;
@@ -133,6 +133,27 @@ __host__ __device__ __forceinline__ int pd_pieces(int nt, int c, int least, floa
 //     with a bf16 cache one workgroup a CU where that is 2 MiB each (96 x 1064: 143.7 / 142.3).
 struct PdDeal { int piece, share, total; };
 
+// tiles: of all pairs; most: of one; their least pieces are too many.
+__host__ __device__ __forceinline__ PdDeal pd_choose(int tiles, int most, int pairs, int wgs,
+                                                     int resident, int least, bool lone) {
+  const int share = (tiles + resident - 1) / resident;
+  const bool brief = tiles <= 3 * least * pairs;
+  if (pairs <= (brief ? wgs : resident) && most <= (brief ? 3 : 2) * share) return {most, 1, pairs};
+  const int room = resident - pairs;
+  if (room > 0) {
+    const int c = (tiles + room - 1) / room;   // sum of ceil(n / c) <= tiles / c + pairs
+    if (c * 2 <= share * 3) return {c, 1, wgs};
+  }
+  return {0, lone && share >= 64 ? 2 * share : share, tiles};
+}
+
+// Workgroups of a launch: as many as are resident, so that every range is in work at once, and
+// one for every pair. tiles: of a pair, at most.
+inline long pd_workgroups(long pairs, long tiles, int least, long resident) {
+  const long most = pairs * ((tiles + least - 1) / least), all = resident > pairs ? resident : pairs;
+  return all < most ? all : most;
+}
+
 // The lengths of sequences c + lane, c + 64 + lane, ..: four loads in flight.
 struct PdLens { int of[4]; };
 DEVINL PdLens pd_lens(const int* __restrict__ lens, int B, int lane, int c) {
@@ -165,16 +186,7 @@ DEVINL PdDeal pd_deal(const int* __restrict__ lens, int B, int KVH, int window, 
   tiles = pd_sum(tiles) * KVH;
   n0 = pd_sum(n0) * KVH;
   if (n0 <= wgs) return {least, 1, n0};
-  most = pd_max(most);
-  const int pairs = B * KVH, share = (tiles + resident - 1) / resident;
-  const bool brief = tiles <= 3 * least * pairs;
-  if (pairs <= (brief ? wgs : resident) && most <= (brief ? 3 : 2) * share) return {most, 1, pairs};
-  const int room = resident - pairs;
-  if (room > 0) {
-    const int c = (tiles + room - 1) / room;   // sum of ceil(n / c) <= tiles / c + pairs
-    if (c * 2 <= share * 3) return {c, 1, wgs};
-  }
-  return {0, lone && share >= 64 ? 2 * share : share, tiles};
+  return pd_choose(tiles, pd_max(most), B * KVH, wgs, resident, least, lone);
 }
 
 // The first sequence whose pieces or tiles reach past `t` (all pairs counted), its length and

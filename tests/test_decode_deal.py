@@ -8,11 +8,13 @@ import subprocess
 
 import pytest
 
+from decode_batches import BATCHES, VARIANTS
 from llmq_amd.ops.build import HERE, HIPCC_FLAGS
 
 HIPCC = shutil.which("hipcc") or shutil.which("/opt/rocm/bin/hipcc")
 SOURCE = r"""
 #include "paged_decode.hip"
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 
@@ -30,6 +32,32 @@ void pieces(int least, int c, float thick) {
   printf("%d\n", most);
 }
 
+// The deal of a batch on 256 CUs, after its least pieces' count and a piece's tiles; then the tiles
+// of a kv head of every sequence.
+template <int D, typename TC>
+void deal(int G, int KVH, int width, int window, char** from, char** to) {
+  constexpr PdVariant v = pd_variant(D, sizeof(TC) == 1);
+  using Shape = PdShape<D, TC, v.groups>;
+  constexpr int kLeast = Shape::kLeastPiece;
+  const float thick = G * (2.f / (Shape::kKeys * (int)sizeof(TC)));
+  const int pairs = (int)(to - from) * KVH, resident = 256 * v.resident;
+  const int wgs = (int)pd_workgroups(pairs, width / Shape::kKeys + 1, kLeast, resident);
+  int total = 0, n0 = 0, most = 0;
+  for (char** at = from; at < to; ++at) {
+    const int n = pd_tiles<Shape::kTileShift>(atoi(*at), window);
+    total += n * KVH;
+    n0 += pd_pieces(n, kLeast, kLeast, thick) * KVH;
+    most = std::max(most, n);
+  }
+  PdDeal d{kLeast, 1, n0};
+  if (n0 > wgs)
+    d = pd_choose(total, most, pairs, wgs, std::min(resident, wgs), kLeast,
+                  D == 256 && sizeof(TC) == 2);
+  printf("%d %d %d %d %d\n", n0 <= wgs, d.piece, most, d.share, d.total);
+  for (char** at = from; at < to; ++at)
+    printf("%d ", pd_tiles<Shape::kTileShift>(atoi(*at), window));
+}
+
 template <int D, typename TC>
 void variant() {
   constexpr bool fp8 = sizeof(TC) == 1;
@@ -41,6 +69,20 @@ void variant() {
 int main(int argc, char** argv) {
   if (argc > 1 && !strcmp(argv[1], "pieces")) {
     pieces(atoi(argv[2]), atoi(argv[3]), atof(argv[4]));
+    return 0;
+  }
+  if (argc > 1) {
+    const int D = atoi(argv[2]), fp8 = atoi(argv[3]);
+    auto go = [&]<int HD, typename TC>() {
+      if (D == HD && fp8 == (sizeof(TC) == 1))
+        deal<HD, TC>(atoi(argv[4]), atoi(argv[5]), atoi(argv[6]), atoi(argv[7]), argv + 8,
+                     argv + argc);
+    };
+    go.template operator()<64, __hip_bfloat16>();
+    go.template operator()<128, __hip_bfloat16>();
+    go.template operator()<256, __hip_bfloat16>();
+    go.template operator()<128, __hip_fp8_e4m3>();
+    go.template operator()<256, __hip_fp8_e4m3>();
     return 0;
   }
   variant<64, __hip_bfloat16>();
@@ -87,3 +129,36 @@ def test_no_piece_is_empty(program, least, longer, thick):
     assert len(out) == 1, out[:5]                            # the largest count, no exceptions
     # the floor: sqrt(1.5 thick nt) tiles, no more than rounded up by four
     assert out[0][0] <= 70000 / max(least + longer, (1.5 * thick * 70000) ** 0.5 - 1) + 1
+
+
+@pytest.mark.parametrize("batch", range(len(BATCHES)))
+@pytest.mark.parametrize("variant", range(len(VARIANTS)))
+def test_batches_take_their_ways(program, batch, variant):
+    """The GPU tests' batches are dealt as they are meant to be. Equal ranges hold the end of a
+    pair, whole ones and the start of another, and step over empty sequences."""
+    D, G, fp8 = VARIANTS[variant]
+    ways, lens, KVH, BS, window, _ = BATCHES[batch]
+    (least, piece, most, share, total), tiles = program(
+        "deal", D, int(fp8), G, KVH, -(-max(lens) // BS) * BS, window, *lens)
+    way = "L" if least else "R" if piece == 0 else "W" if piece == most else "P"
+    assert way == ways[variant]
+    if way == "P":
+        assert piece < most
+    if way != "R":
+        return
+    assert total == sum(tiles) * KVH
+    ends, segments = [0], []
+    for b, n in enumerate(tiles):
+        for _ in range(KVH if n else 0):
+            ends.append(ends[-1] + n)
+            segments.append(b)
+    kinds = set()
+    for lo in range(0, total, share):
+        hi = min(total, lo + share)
+        mine = [i for i, b in enumerate(segments) if ends[i] < hi and ends[i + 1] > lo]
+        cut = ends[mine[0]] < lo, ends[mine[-1] + 1] > hi
+        kinds.add((cut, len(mine) > 2))
+        seen = [segments[i] for i in mine]
+        if any(d > c + 1 for c, d in zip(seen, seen[1:])):
+            kinds.add("empty")
+    assert ((True, True), True) in kinds and "empty" in kinds

@@ -7,6 +7,8 @@ from __future__ import annotations
 import pytest
 import torch
 
+from decode_batches import BATCHES, VARIANTS
+
 pytestmark = pytest.mark.gpu
 
 if torch.cuda.is_available():
@@ -209,9 +211,8 @@ class TestDecodeAttention:
 
 
 class TestDecodeRanges:
-    """The matrix-core decode kernel deals the batch's key tiles to waves in
-    equal ranges: ranges that open, close and cross (sequence, kv head) pairs,
-    empty rows, batches over one wave's scan, block tables of any width."""
+    """The matrix-core decode kernel on batches whose least pieces all find a workgroup: short
+    and long pairs, empty rows, more sequences than one scan takes, block tables of any width."""
 
     @pytest.mark.parametrize("D,G,KVH,fp8", [
         (64, 4, 3, False), (64, 8, 1, False), (128, 1, 2, False), (128, 16, 1, False),
@@ -247,8 +248,7 @@ class TestDecodeRanges:
     ])
     @pytest.mark.parametrize("window", [0, 50])
     def test_shares_at_head_size_64(self, KVH, lens, window):
-        """Every least share of head size 64: long pairs, pairs of one and two tiles, few and
-        many."""
+        """Head size 64: long pairs, pairs of one and two tiles, few and many."""
         B, G, D = len(lens), 2, 64
         kc, vc, bt = _build_cache(B, KVH, D, 16, max(lens), torch.bfloat16)
         ctx = torch.tensor(lens, dtype=torch.int32, device=DEV)
@@ -262,8 +262,8 @@ class TestDecodeRanges:
 
 
 class TestDecodePieces:
-    """Pairs in pieces that workgroups merge where they meet: pieces of the least size, larger
-    ones, equal ranges; pairs at twice the least piece; batches over 256 lengths."""
+    """Pairs in pieces that workgroups merge where they meet: few and many, of the least size and
+    larger; pairs at twice the least piece; batches over 256 lengths."""
 
     @pytest.mark.parametrize("D,G,KVH,fp8", [(64, 4, 8, False), (128, 6, 2, False),
                                              (128, 3, 8, True), (256, 2, 8, False),
@@ -313,6 +313,27 @@ def _ragged_cache(lens, KVH, D, BS, fp8=False):
 # a pair, whole ones and the start of another, and pairs that many ranges share.
 RAGGED = [(i * 37) % 150 for i in range(300)]
 RAGGED[3], RAGGED[4], RAGGED[150], RAGGED[299] = 3000, 1500, 2100, 2999
+
+
+class TestDecodeDeals:
+    """Every way to cut a batch (test_decode_deal.py has which one each takes)."""
+
+    @pytest.mark.parametrize("batch", range(len(BATCHES)))
+    @pytest.mark.parametrize("D,G,fp8", VARIANTS)
+    def test_vs_ref(self, D, G, fp8, batch):
+        _, lens, KVH, BS, window, softcap = BATCHES[batch]
+        kc, vc, bt = _ragged_cache(lens, KVH, D, BS, fp8)
+        ctx = torch.tensor(lens, dtype=torch.int32, device=DEV)
+        q = torch.randn(len(lens), G * KVH, D, device=DEV, dtype=torch.bfloat16)
+        args = (q, kc, vc, bt, ctx, D ** -0.5, softcap, window)
+        live = ctx > 0
+        out = ops.paged_decode_attention(*args)[live]
+        live = live.cpu()
+        ref = torch_ref.paged_decode_attention(
+            q.float().cpu()[live], kc.float().cpu(), vc.float().cpu(), bt.cpu()[live],
+            ctx.cpu()[live], D ** -0.5, softcap, window)
+        # the output's bf16 rounding and fp32 sums of up to 3000 unit values, as above
+        assert_close_to_f32_ref(out.cpu(), ref, 2e-4, 2 ** -8)
 
 
 class TestDecodeIsolation:
