@@ -363,7 +363,7 @@ class CausalLM:
             x = x * math.sqrt(s.hidden_size)
             x = x.to(self.dtype)
         l0 = self.layers[0]
-        if x.is_cuda and not meta.is_prefill:             # one fill for all layers
+        if x.is_cuda and x.dtype == torch.bfloat16 and not meta.is_prefill:  # one fill for all layers
             dec = meta.decode if meta.is_mixed else meta
             dec.arrivals = torch.zeros(len(self.layers), dec.context_lens.shape[0], self.kv_heads,
                                        dtype=torch.int32, device=x.device)

@@ -195,8 +195,8 @@ def paged_decode_attention(
     window: int = 0,
     arrivals: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
-    """arrivals: int32 zeros [B, KVH] that the GPU kernel uses up; made here where a caller
-    has none (one fill can serve all layers of a step)."""
+    """arrivals: int32 zeros [B, KVH] that the GPU kernel for bf16 queries counts in and leaves
+    as zeros; made here where a caller has none (one fill can serve all layers of a step)."""
     if _use_hip(q):
         out = torch.empty_like(q)
         _EXT.paged_decode_attention(

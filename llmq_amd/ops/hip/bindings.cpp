@@ -238,8 +238,8 @@ int compute_units(const at::Tensor& x) {
   return cus;
 }
 
-// The matrix-core kernel of paged_decode.hip. arrivals: zeros [B, KVH], used up; without it they
-// are made here, a launch of 2 us.
+// The matrix-core kernel of paged_decode.hip. arrivals: zeros [B, KVH], zeros again after the
+// launch; without it they are made here, a launch of 2 us.
 template <int D, typename TC>
 void launch_paged_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor& kc,
                          const at::Tensor& vc, const at::Tensor& bt,
@@ -260,8 +260,8 @@ void launch_paged_decode(at::Tensor& out, const at::Tensor& q, const at::Tensor&
   at::Tensor part_ml = at::empty({2L * wgs, G, 2}, opts);
   const bool given = arrivals.has_value() && arrivals->defined();
   TORCH_CHECK(!given || (arrivals->scalar_type() == at::kInt && arrivals->is_contiguous() &&
-                         arrivals->numel() == (long)B * KVH && arrivals->is_cuda()),
-              "arrivals must be int32 zeros [B, kv heads]");
+                         arrivals->numel() == (long)B * KVH && arrivals->device() == q.device()),
+              "arrivals must be int32 zeros [B, kv heads] on q's device");
   const at::Tensor arr = given ? *arrivals : at::zeros({B, KVH}, q.options().dtype(at::kInt));
   auto go = [&]<bool CAP>() {
     hipLaunchKernelGGL((paged_decode_kernel<D, TC, NK, OCC, CAP>), dim3(wgs), dim3(256),

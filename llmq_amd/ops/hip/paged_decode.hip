@@ -745,6 +745,9 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
   for (int p = 0; p < waiting; ++p) {
     const PdPair pair = pending[p];
     if ((int)arrived[p] != pair.w_last - pair.w_first) continue;
+    if (threadIdx.x == 0)                      // zero again for the next launch
+      __hip_atomic_store(arrivals + pair.b * KVH + pair.kh, 0u, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
     __hip_bfloat16* const orow = out + (long)pair.b * out_stride + (long)pair.kh * G * D;
     const int tid = threadIdx.x, quads = G * (D / 4);
     const int groups = 1 + (2 * quads <= 256) + (3 * quads <= 256) + (4 * quads <= 256);

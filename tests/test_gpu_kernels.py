@@ -327,7 +327,11 @@ class TestDecodeDeals:
         q = torch.randn(len(lens), G * KVH, D, device=DEV, dtype=torch.bfloat16)
         args = (q, kc, vc, bt, ctx, D ** -0.5, softcap, window)
         live = ctx > 0
+        arrivals = torch.zeros(len(lens), KVH, dtype=torch.int32, device=DEV)
         out = ops.paged_decode_attention(*args)[live]
+        for _ in range(2):                     # the counters are left as they were found
+            assert torch.equal(ops.paged_decode_attention(*args, arrivals)[live], out)
+            assert not arrivals.any()
         live = live.cpu()
         ref = torch_ref.paged_decode_attention(
             q.float().cpu()[live], kc.float().cpu(), vc.float().cpu(), bt.cpu()[live],
