@@ -110,10 +110,13 @@ __host__ __device__ __forceinline__ int pd_quotient(int x, float inv) {
 // waves. us, without that floor / with it: 1 x 16000 keys, 1 kv head of 256, 8 heads 62.6 / 30.8; 3 x
 // 16000, 2 of 128, 6 heads each 29.5 / 21.0; 1 x 16000, 8 of 64, 4 heads each 17.2 / 15.3. Factors of 1
 // to 3 are within 1 % over 86 batches; at 2 one of 4000 keys, 2 of 128, fp8 loses 13 %.
+__host__ __device__ __forceinline__ int pd_piece(int nt, int c, float thick) {
+  const int floor = ((int)pd_sqrt(1.5f * nt * thick) + 3) & ~3;    // four waves share them
+  return c > floor ? c : floor;
+}
 __host__ __device__ __forceinline__ int pd_pieces(int nt, int c, int least, float thick) {
   if (nt <= 2 * least) return nt > 0;
-  const int floor = ((int)pd_sqrt(1.5f * nt * thick) + 3) & ~3;    // four waves share them
-  const int size = c > floor ? c : floor;
+  const int size = pd_piece(nt, c, thick);
   return pd_quotient(nt + size - 1, pd_rcp((float)size));
 }
 
@@ -172,21 +175,32 @@ DEVINL PdDeal pd_deal(const int* __restrict__ lens, int B, int KVH, int window, 
                       const PdLens& first, int wgs, int resident, int least, float thick,
                       bool lone) {
   int tiles = 0, n0 = 0, most = 0;
-  for (int c = 0; c < B; c += 4 * WAVE) {
-    const PdLens l = c == 0 ? first : pd_lens(lens, B, lane, c);
+  auto each = [&](auto f) {
+    for (int c = 0; c < B; c += 4 * WAVE) {
+      const PdLens l = c == 0 ? first : pd_lens(lens, B, lane, c);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (c + i * WAVE >= B) break;
-      const int n = pd_tiles<TS>(l.of[i], window);
-      tiles += n;
-      n0 += pd_pieces(n, least, least, thick);
-      most = max(most, n);
+      for (int i = 0; i < 4; ++i) {
+        if (c + i * WAVE >= B) break;
+        f(pd_tiles<TS>(l.of[i], window));
+      }
     }
+  };
+  each([&](int n) {
+    tiles += n;
+    n0 += n <= 2 * least ? min(n, 1) : (n + least - 1) / least;
+    most = max(most, n);
+  });
+  most = pd_max(most);
+  // Only where the longest pair's floor is over the least piece is it the count: else none of its
+  // branches (189 ragged up to 300 keys, 8 kv heads of 128: 36.0 us with them, 35.2 so).
+  if (pd_piece(most, least, thick) > least) {
+    n0 = 0;
+    each([&](int n) { n0 += pd_pieces(n, least, least, thick); });
   }
   tiles = pd_sum(tiles) * KVH;
   n0 = pd_sum(n0) * KVH;
   if (n0 <= wgs) return {least, 1, n0};
-  return pd_choose(tiles, pd_max(most), B * KVH, wgs, resident, least, lone);
+  return pd_choose(tiles, most, B * KVH, wgs, resident, least, lone);
 }
 
 // The first sequence whose pieces or tiles reach past `t` (all pairs counted), its length and
@@ -411,13 +425,16 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
   int w_first = 0, w_last = 0;                 // the workgroups of a pair in pieces
   bool pieces = true;
   // Few sequences whose least pieces all find a workgroup, without pd_deal's other sums and a
-  // second scan: 150 of the 450 instructions ahead of the first load, 4 clocks each.
-  int n_l = B <= WAVE ? pd_tiles<TS>(first.of[0], window) : 0;
+  // second scan: 150 of the 450 instructions ahead of the first load, 4 clocks each. Of many nothing
+  // is counted here (200 ragged up to 100 keys, 8 kv heads of 64: 12.3 us with it, 11.8 so).
   const float thick = G * (2.f / (KT * (int)sizeof(TC)));
-  n_l = pd_pieces(n_l, kLeast, kLeast, thick);
-  const int upto = pd_scan(n_l);               // pieces of a head of this lane's sequence and before
-  const int n0 = __builtin_amdgcn_readlane(upto, WAVE - 1) * KVH;
-  if (B <= WAVE && n0 <= wgs) {
+  int n_l = 0, upto = 0, n0 = wgs + 1;
+  if (B <= WAVE) {
+    n_l = pd_pieces(pd_tiles<TS>(first.of[0], window), kLeast, kLeast, thick);
+    upto = pd_scan(n_l);                       // pieces of a head of this lane's sequence and before
+    n0 = __builtin_amdgcn_readlane(upto, WAVE - 1) * KVH;
+  }
+  if (n0 <= wgs) {
     if (wg >= n0) return;
     b = __ffsll((long long)__ballot(upto * KVH > wg)) - 1;
     len = __builtin_amdgcn_readlane(first.of[0], b);
@@ -531,21 +548,29 @@ __global__ __launch_bounds__(256, OCC) void paged_decode_kernel(
   // threads idle (1 x 1500 keys, 8 kv heads: 8.4 us, 8.0 so).
   constexpr int W = D == 64 ? 2 : 4;
   typedef float Channels __attribute__((ext_vector_type(W)));
-  // What `parts` waves or groups left of them in LDS. No other part is read: it may be another
-  // pair's, and a weight of zero does not cancel an infinity there.
+  // What `parts` waves or groups left of them in LDS, read together. The other parts may be another
+  // pair's: a weight of zero does not cancel an infinity there, so they are put to zero.
   auto meet = [&](int e, int parts) {
     const int g = e / (D / W);
     PdSum<Channels> s{-INFINITY, 0.f, Channels(0.f)};
+    pd_f32x2 of[4];
+    Channels x[4];
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
-      if (v < parts) s.top = fmaxf(s.top, ml[v][g][0]);
+    for (int v = 0; v < 4; ++v) {
+      of[v] = ml[v][g];
+      x[v] = *reinterpret_cast<const Channels*>(mo(v) + e * W);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      if (v >= parts) of[v] = pd_f32x2{-INFINITY, 0.f}, x[v] = Channels(0.f);
+      s.top = fmaxf(s.top, of[v][0]);
+    }
     const float tb = s.top > -INFINITY ? s.top : 0.f;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      if (v >= parts) break;
-      const float f = __builtin_amdgcn_exp2f(ml[v][g][0] - tb);      // -inf -> 0
-      s.weight += ml[v][g][1] * f;
-      s.x += *reinterpret_cast<const Channels*>(mo(v) + e * W) * f;
+      const float f = __builtin_amdgcn_exp2f(of[v][0] - tb);         // -inf -> 0
+      s.weight += of[v][1] * f;
+      s.x += x[v] * f;
     }
     return s;
   };
