@@ -282,7 +282,7 @@ class CausalLM:
         for i, lw in enumerate(self.layers):
             w_next = self.layers[i + 1].input_norm if i + 1 < len(self.layers) else self.final_norm
             qkv = ops.slab_rope_cache(
-                ops.ring_linear(h, lw.qkv, ops.ROPE_READERS), lw.qkv_bias, kv_cache.k[i],
+                ops.ring_linear(h, lw.qkv, True), lw.qkv_bias, kv_cache.k[i],
                 kv_cache.v[i], positions, self.rope_cache, meta.slot_mapping,
             )
             attn = self._attention(i, qkv, positions, kv_cache, meta, cached=True)

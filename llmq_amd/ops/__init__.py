@@ -430,14 +430,11 @@ def slab_ok(x: torch.Tensor, weights, hidden: int) -> bool:
     )
 
 
-ROPE_READERS = 4  # workgroups of slab_rope_cache that read a row of the slabs
-
-
-def ring_linear(x: torch.Tensor, w: torch.Tensor, readers: int = 1) -> torch.Tensor:
+def ring_linear(x: torch.Tensor, w: torch.Tensor, for_rope: bool = False) -> torch.Tensor:
     """x @ w.T as fp32 slabs [parts, M, N] whose sum is the product, up to RING_ROWS rows.
-    readers: workgroups that will read a row of them; more parts suit more readers."""
+    for_rope: slab_rope_cache reads them, several workgroups a row; more parts suit those."""
     assert _use_hip(x)
-    return _EXT.ring_linear(x, w, readers)
+    return _EXT.ring_linear(x, w, for_rope)
 
 
 def ring_act_ok(x: torch.Tensor, w: torch.Tensor) -> bool:

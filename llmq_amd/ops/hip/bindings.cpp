@@ -721,9 +721,11 @@ void launch_slab_gemm(float* slab, __hip_bfloat16* out, long out_stride, const a
   }
 }
 
-// x W^T as fp32 slabs [parts, M, N]; their sum is the product. readers: workgroups that will
-// read a row of them.
-at::Tensor ring_linear(const at::Tensor& x, const at::Tensor& w, long readers) {
+constexpr int kRopeReaders = 4;              // workgroups of slab_rope_cache that read a row
+
+// x W^T as fp32 slabs [parts, M, N]; their sum is the product. for_rope: slab_rope_cache will
+// read them, else slab_add_norm, a workgroup a row.
+at::Tensor ring_linear(const at::Tensor& x, const at::Tensor& w, bool for_rope) {
   CHECK_GPU(x);
   TORCH_CHECK(slab_rows_ok(x, w, kRingRows),
               "ring_linear: 1 to 256 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
@@ -736,7 +738,7 @@ at::Tensor ring_linear(const at::Tensor& x, const at::Tensor& w, long readers) {
     launch_slab_gemm<kSlabSums>(slab.data_ptr<float>(), nullptr, 0, x, w);
     return slab;
   }
-  const RingPlan plan = ring_plan(M, N, K, compute_units(x), std::max(readers, 1L));
+  const RingPlan plan = ring_plan(M, N, K, compute_units(x), for_rope ? kRopeReaders : 1);
   at::Tensor slabs = at::empty({plan.parts, M, N}, opts);
   float* p = slabs.data_ptr<float>();
   auto go = [&]<int TT, bool ROT>() {
@@ -949,7 +951,7 @@ at::Tensor slab_linear(const at::Tensor& x, const at::Tensor& w) {
   CHECK_GPU(x);
   TORCH_CHECK(slab_rows_ok(x, w, kSlabRows),
               "slab_linear: 1 to 128 bf16 rows on 16 bytes, K a multiple of 128, N of 64");
-  return ring_linear(x, w, 1);
+  return ring_linear(x, w, false);
 }
 
 at::Tensor slab_act_linear(const at::Tensor& x, const at::Tensor& w, bool gelu) {
@@ -1298,8 +1300,6 @@ at::Tensor slab_add_norm(const at::Tensor& slabs, at::Tensor residual,
   return h;
 }
 
-constexpr int kRopeReaders = 4;              // workgroups a row
-
 // bf16 rows [M, (heads + 2 kv heads) D] of the summed slabs + bias, q and k rotated;
 // k and v also into the paged cache.
 at::Tensor slab_rope_cache(const at::Tensor& slabs, c10::optional<at::Tensor> bias,
@@ -1372,7 +1372,7 @@ at::Tensor prompt_layers(at::Tensor h, at::Tensor residual, at::TensorList weigh
     const c10::optional<at::Tensor> bias =
         biases.empty() ? none : c10::make_optional(biases[i]);
     const at::Tensor qkv =
-        slab ? slab_rope_cache(ring_linear(h, w[0], kRopeReaders), bias, k_caches[i],
+        slab ? slab_rope_cache(ring_linear(h, w[0], true), bias, k_caches[i],
                                v_caches[i], positions, cos_sin, slots)
              : at::linear(h, w[0], bias);
     const long kv_heads = k_caches[i].size(1);
@@ -1394,7 +1394,7 @@ at::Tensor prompt_layers(at::Tensor h, at::Tensor residual, at::TensorList weigh
     auto project_add_norm = [&](const at::Tensor& a, const at::Tensor& wt,
                                 const at::Tensor* post, const at::Tensor& norm) {
       if (slab)
-        return slab_add_norm(ring_linear(a, wt, 1), residual,
+        return slab_add_norm(ring_linear(a, wt, false), residual,
                              post ? c10::make_optional(*post) : none, norm, eps, offset);
       at::Tensor y = at::linear(a, wt);
       if (post) norm_add_norm(y, residual, *post, norm, eps, offset);
@@ -1531,7 +1531,7 @@ TORCH_LIBRARY(llmq_amd, m) {
   m.def("few_qkv(Tensor g, Tensor sq, int n, float eps, Tensor w, Tensor? bias, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor positions, Tensor cos_sin, Tensor slots) -> Tensor");
   m.def("few_act(Tensor g, Tensor sq, int n, float eps, Tensor w, bool gelu) -> Tensor");
   m.def("slab_linear(Tensor x, Tensor w) -> Tensor");
-  m.def("ring_linear(Tensor x, Tensor w, int readers=1) -> Tensor");
+  m.def("ring_linear(Tensor x, Tensor w, bool for_rope=False) -> Tensor");
   m.def("ring_head(Tensor x, Tensor w, float cap) -> Tensor");
   m.def("ring_act_ok(Tensor x, Tensor w) -> bool");
   m.def("ring_act_linear(Tensor x, Tensor w, bool gelu) -> Tensor");
