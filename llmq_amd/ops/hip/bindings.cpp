@@ -771,8 +771,8 @@ void launch_ring_act(__hip_bfloat16* out, long out_stride, const at::Tensor& x,
   const long rows = ring_act_rows(w.size(0), compute_units(x));
   const int steps = (int)(w.size(1) / kRingBK);
   // over 192 tokens two groups of 128, and as many workgroups (us, one group / two: 16384 x
-  // 2048, 200 rows 26.9 / 23.7, 256 rows 27.1 / 24.8; 16384 x 3072, the same 38.9 / 36.5, 39.4 /
-  // 35.6; two of 96: 192 rows 23.5 / 23.2, 36.3 / 35.8, 161 rows 23.1 / 23.6)
+  // 2048, 200 rows 26.5 / 23.6, 256 rows 27.1 / 24.5; 16384 x 3072, the same 39.0 / 34.2, 40.7 /
+  // 35.2; two of 96: 192 rows 23.5 / 23.2, 36.3 / 35.8, 161 rows 23.1 / 23.6)
   if (rows == 64 && x.size(0) > 192 && w.size(0) % 128 == 0)
     return launch_ring<8, 4, 2, 4, 1, 4, EPI, false, 2>(nullptr, out, out_stride, x, w, 1, steps);
   ring_tiles(x.size(0), [&]<int TT>() {

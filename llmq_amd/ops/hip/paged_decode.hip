@@ -6,12 +6,12 @@
 // Bound by the cache's bytes: at 16 query columns the products take a few percent
 // of the matrix cores, so everything here serves to keep loads in flight on all
 // CUs until the last byte has come. Measured (us; before = a wave a range, waves' pieces
-// merged by a second launch): 1 x 200 keys, 8 kv heads of 64: 7.3 -> 4.8; 16 ragged up to 300,
-// the same: 10.3 -> 7.1; 64 x 1040, the same: 33.6 -> 26.6 (136 MB); 7 ragged up to 1900, 2 of
-// 128: 11.7 -> 10.8; 189 ragged up to 1100, 8 of 128: 99 -> 87.4 (473 MB, 5.4 TB/s); 3 ragged
-// up to 16000, the same: 44.5 -> 38.5; 96 x 1064, 8 of 256, capped: 159 -> 142.3 (837 MB, 5.9
-// TB/s); 64 ragged up to 300, the same: 26 -> 22.1; 48 ragged up to 2000, 8 of 256, fp8: 51.2
-// -> 46.9; 1 x 1000, 8 of 64: 7.9 -> 7.3. Below about 100 MB the launch, the walk from
+// merged by a second launch): 1 x 200 keys, 8 kv heads of 64: 7.6 -> 4.6; 16 ragged up to 300,
+// the same: 10.7 -> 7.0; 1 x 1000: 8.7 -> 8.1; 64 x 1040: 33.4 -> 26.2 (136 MB); 7 ragged up to
+// 1900, 2 of 128, 6 heads each: 12.0 -> 10.6; 189 ragged up to 1100, 8 of 128: 97 -> 87 (5.4 TB/s);
+// 3 ragged up to 16000, the same: 33.8 -> 28.9; 96 x 1064, 8 of 256, capped: 156 -> 142 (837 MB,
+// 5.9 TB/s); 64 ragged up to 300, the same: 26.3 -> 24.9; 48 ragged up to 2000, fp8: 52.1 -> 48.5;
+// 64 x 1040, 2 of 256, 16 heads each: 41.5 -> 39.2. Below about 100 MB the launch, the walk from
 // lengths to block table to keys and every instruction around it (4 clocks each) count most.
 //
 //   - The work is cut in tiles of 16 NK keys of one (sequence, kv head) pair, in order, and
@@ -127,9 +127,10 @@ __host__ __device__ __forceinline__ int pd_pieces(int nt, int c, int least, floa
 //     12000 keys, 8 kv heads of 64 26.4 us, of 64 15.2) where all find a workgroup;
 //   - whole pairs unless the longest is over twice the mean share; short ones (three least pieces
 //     in the mean) up to three times, and also more of them than run at a time. us, whole / equal
-//     ranges: 64 x 1040, 8 of 64 26.6 / 33; 200 ragged up to 100, the same 12.1 / 16.3; 200 up to
-//     400, 8 of 256 (3.5 least pieces) 77.3 / 80.1, 150 up to 500 (4.4) 73.2 / 70.9; 48 up to
-//     2000, 8 of 256, fp8 (2.45 times) 57.8 / 46.9;
+//     ranges: 64 x 1040, 8 of 64 26.6 / 33; 120 ragged up to 700, the same 25.1 / 29.0; 200 up to
+//     700, 8 of 128, fp8 40.0 / 45.3; 100 up to 300, 8 of 256 35.7 / 38.9; 120 up to 400, the same,
+//     fp8 33.3 / 37.9; 200 up to 400, 8 of 256 (3.5 least pieces) 77.3 / 80.1, 150 up to 500 (4.4)
+//     73.2 / 70.9; 48 up to 2000, 8 of 256, fp8 (2.45 times) 57.8 / 46.9;
 //   - pieces that surely find a workgroup, where they are at most 1.5 mean shares (24 ragged up
 //     to 1500, 8 of 256, 1.6: 43.3, equal ranges 38.8);
 //   - equal ranges, whose ends cut pairs and whose segments follow each other; at head size 256
@@ -387,7 +388,13 @@ struct PdShape {
   static constexpr int kLeastPiece = 64 * 1024 / (2 * kKeys * D * (int)sizeof(TC));
 };
 
-// 16-key groups of a tile and workgroups a CU, by registers; their LDS fits at every G.
+// 16-key groups of a tile and workgroups a CU, by registers; their LDS fits at every G. us, so / else:
+// head size 64, four groups and two workgroups: 16 ragged up to 300 keys 6.9 / 7.8, 64 x 1040 26.3 /
+// 28.6, 200 ragged up to 100 12.6 / 17.4, 6 ragged up to 15000 31.1 / 30.5; 128, four and one: 189
+// ragged up to 1100 86.3 / 104, 60 up to 800 29.4 / 35.0, 3 up to 16000 28.5 / 28.2, two and one: 86.3
+// / 91.8, 29.4 / 32.6, 28.5 / 27.8; 256, one and one: 64 up to 300 24.6 / 29.1, 40 up to 500 26.2 /
+// 28.8; fp8 of 128, two and two: 189 up to 1100 53.8 / 54.0, 3 up to 16000 22.4 / 20.5, four and two: 53.8
+// / 59.1, 22.4 / 20.7; of 256, one and one: 48 up to 2000 48.8 / 66.3, 100 up to 500 35.4 / 37.3.
 struct PdVariant { int groups, resident; };
 constexpr PdVariant pd_variant(int D, bool fp8) {
   return D == 64 ? PdVariant{2, 3} : D == 128 ? PdVariant{2, fp8 ? 3 : 2} : PdVariant{1, 2};
