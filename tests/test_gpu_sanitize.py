@@ -16,6 +16,8 @@ from __future__ import annotations
 import pytest
 import torch
 
+from decode_batches import BATCHES, VARIANTS
+
 pytestmark = pytest.mark.gpu
 
 if torch.cuda.is_available():
@@ -104,6 +106,24 @@ def test_decode_attention_guarded(g, D, G, KVH, BS, fp8, softcap, window):
         ops._EXT.paged_decode_attention(out[:n], q[:n], kc, vc, bt[:n], ctx[:n], D ** -0.5,
                                         softcap, window)
         assert out[:n].isfinite().all()
+
+
+@pytest.mark.parametrize("batch", range(len(BATCHES)))
+@pytest.mark.parametrize("D,G,fp8", VARIANTS)
+def test_decode_deals_guarded(g, D, G, fp8, batch):
+    """Every way to cut a batch (test_decode_deal.py has which one each takes)."""
+    _, lens, KVH, BS, window, softcap = BATCHES[batch]
+    need = [-(-n // BS) for n in lens]
+    kc, vc = (g.tensor(sum(need) + 1, KVH, BS, D,
+                       dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16) for _ in range(2))
+    table = torch.zeros(len(lens), max(need))
+    for row, mine in zip(table, torch.arange(1, sum(need) + 1).split(need)):
+        row[:len(mine)] = mine
+    q, out = (g.tensor(len(lens), G * KVH, D) for _ in range(2))
+    bt, ctx = g.from_values(table, torch.int32), g.from_values(torch.tensor(lens), torch.int32)
+    arrivals = g.tensor(len(lens), KVH, dtype=torch.int32, fill="zeros")
+    ops._EXT.paged_decode_attention(out, q, kc, vc, bt, ctx, D ** -0.5, softcap, window, arrivals)
+    assert out[ctx > 0].isfinite().all() and not arrivals.any()
 
 
 @pytest.mark.parametrize("D,H,KVH", [(64, 4, 2), (64, 3, 1), (128, 6, 2), (256, 16, 8),
